@@ -33,32 +33,58 @@ constexpr int kWaves = 4;          // waves per workgroup, side by side in x
 constexpr int kLdsBudget = 64 * 1024;
 
 // ------------------------------------------------------------------------- template staging
-template <int TYPE, int KIND>
-__global__ __launch_bounds__(256) void template_prep(const char *tpl, int tw, int th, int tstep,
-                                                      int nch, int ch, int pitch, void *out,
-                                                      double *sums)
+// The staged template and its sums, by one workgroup (the sums have one fixed order and no
+// second launch).  Bound by memory latency: up to kPrepWide threads, K elements per thread in
+// flight (one for templates of that many elements or fewer, which start sooner), (row, column)
+// stepped along with the element index instead of divided out.  64x64: 9.0 -> 5.0 us, 256x256:
+// 122 -> 35 us against 256 threads with one element in flight.
+constexpr int kPrepWide = 1024;
+
+template <int TYPE, int KIND, int K>
+__global__ __launch_bounds__(kPrepWide) void template_prep(const char *tpl, int tw, int th,
+                                                           int tstep, int nch, int ch, int pitch,
+                                                           void *out, double *sums)
 {
-   __shared__ double red[2][4];
+   __shared__ double red[2][kPrepWide / 64];
    double s2 = 0, s1 = 0;
-   const int n = pitch * th;
-   for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      const int v = i / pitch, u = i - v * pitch;
-      double val = 0;
-      if (u < tw) val = (double)ld<TYPE>(tpl + (size_t)v * tstep, u * nch + ch);
-      if (KIND == 0) static_cast<float *>(out)[i] = (float)val;
-      else if (KIND == 1) static_cast<double *>(out)[i] = val;
-      else static_cast<int32_t *>(out)[i] = (int32_t)val;
-      s2 += val * val;
-      s1 += val;
+   const int n = pitch * th, B = blockDim.x;
+   const int dv = B / pitch, du = B - dv * pitch;
+   int v = threadIdx.x / pitch, u = threadIdx.x - v * pitch;
+   for (int i0 = threadIdx.x; i0 < n; i0 += K * B) {
+      double val[K];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+         val[k] = i0 + k * B < n && u < tw ? (double)ld<TYPE>(tpl + (size_t)v * tstep, u * nch + ch)
+                                           : 0.0;
+         u += du;
+         v += dv;
+         if (u >= pitch) {
+            u -= pitch;
+            ++v;
+         }
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+         const int i = i0 + k * B;
+         if (i < n) {
+            if (KIND == 0) static_cast<float *>(out)[i] = (float)val[k];
+            else if (KIND == 1) static_cast<double *>(out)[i] = val[k];
+            else static_cast<int32_t *>(out)[i] = (int32_t)val[k];
+         }
+         const double q = val[k] * val[k];
+         s2 += q;
+         s1 += val[k];
+      }
    }
    s2 = wave_sum(s2);
    s1 = wave_sum(s1);
-   const int wave = threadIdx.x >> 6;
+   const int wave = threadIdx.x >> 6, waves = B >> 6;
    if ((threadIdx.x & 63) == 0) { red[0][wave] = s2; red[1][wave] = s1; }
    __syncthreads();
-   if (threadIdx.x == 0) {
-      sums[0] = red[0][0] + red[0][1] + red[0][2] + red[0][3];
-      sums[1] = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+   if (threadIdx.x < 2) {
+      double t = red[threadIdx.x][0];
+      for (int w = 1; w < waves; ++w) t += red[threadIdx.x][w];
+      sums[threadIdx.x] = t;
    }
 }
 
@@ -755,17 +781,23 @@ void launch_template_prep(hipStream_t s, const View &t, int channel, int pitch, 
                           void *out, double *sums)
 {
    KernelTimer kt(s, "template_prep");
+   const long long n = (long long)pitch * t.height;
+   const int threads = n >= kPrepWide ? kPrepWide : n <= 64 ? 64 : (int)((n + 63) / 64 * 64);
    OCIP_TYPE_SWITCH(t.type, TT, {
       const char *p = static_cast<const char *>(t.ptr);
-      if (kind == 0)
-         template_prep<TT, 0><<<1, 256, 0, s>>>(p, t.width, t.height, t.step, t.channels,
-                                                channel, pitch, out, sums);
-      else if (kind == 1)
-         template_prep<TT, 1><<<1, 256, 0, s>>>(p, t.width, t.height, t.step, t.channels,
-                                                channel, pitch, out, sums);
-      else
-         template_prep<TT, 2><<<1, 256, 0, s>>>(p, t.width, t.height, t.step, t.channels,
-                                                channel, pitch, out, sums);
+      auto go = [&](auto kernel) {
+         kernel<<<1, threads, 0, s>>>(p, t.width, t.height, t.step, t.channels, channel, pitch, out,
+                                      sums);
+      };
+      if (n <= kPrepWide) {
+         if (kind == 0) go(template_prep<TT, 0, 1>);
+         else if (kind == 1) go(template_prep<TT, 1, 1>);
+         else go(template_prep<TT, 2, 1>);
+      } else {
+         if (kind == 0) go(template_prep<TT, 0, 8>);
+         else if (kind == 1) go(template_prep<TT, 1, 8>);
+         else go(template_prep<TT, 2, 8>);
+      }
    });
    launch_check("template_prep");
 }
