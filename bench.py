@@ -36,7 +36,7 @@ sys.path.insert(0, ROOT)
 
 PEAK_TFLOPS = {"bf16": 2500.0, "f16": 2500.0, "bf16x3": 2500.0, "f32": 157.3}
 PREC_CODE = {"f32": 0, "bf16": 1, "f16": 2, "bf16x3": 3}
-DOMINANT = {"f32": "prox_tile_f32", "bf16": "crosscorr_mfma", "f16": "crosscorr_mfma",
+DOMINANT = {"f32": "crosscorr_mfma_split", "bf16": "crosscorr_mfma", "f16": "crosscorr_mfma",
             "bf16x3": "crosscorr_mfma"}
 
 

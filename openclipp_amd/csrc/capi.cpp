@@ -131,12 +131,12 @@ void throw_if(cl_int code, const char *what)
 // ---- proximity driver ---------------------------------------------------------------------
 
 // FP64 exclusive sum-of-squares integral of channel c of S into c.integ.
-const double *sqr_integral_for(Context &c, const Image &S, int channel)
+const double *sqr_integral_for(Context &c, const Image &S, int channel, unsigned *peak = nullptr)
 {
    View v = view(S);
    c.integ.ensure(excl_bytes(v.width, v.height));
    c.integ_aux.ensure(integral_aux_bytes(v.width, v.height));
-   launch_integral(c.stream, v, channel, true, c.integ.ptr, 0, -1, c.integ_aux.ptr);
+   launch_integral(c.stream, v, channel, true, c.integ.ptr, 0, -1, c.integ_aux.ptr, peak);
    return c.integ.as<double>();
 }
 
@@ -172,6 +172,22 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
       c.stats.ensure(int_mfma_work_bytes(tw, th));
       launch_int_mfma(c.stream, op, view(S), view(T), c.tmpl.sums.as<double>(),
                       static_cast<float *>(D.dev), D.desc.Step, c.stats.ptr);
+      D.in_device = true;
+      return;
+   }
+   // CrossCorr_Norm of F32 images: split-FP16 MFMA where the path applies
+   if (precision == ocipPrecisionF32 && split_ncc_ok(op, view(S), view(T))) {
+      const size_t head = 256;   // the peaks, ahead of the path's work buffer
+      c.stats.ensure(head + split_ncc_work_bytes(view(S), view(T)));
+      unsigned *peaks = c.stats.as<unsigned>();
+      launch_template_prep(c.stream, view(T), 0, tpitch, 0, c.tmpl.data.ptr,
+                           c.tmpl.sums.as<double>(), peaks + 1);
+      const double *integ = sqr_integral_for(c, S, 0, peaks);
+      const SplitFlags f = launch_split_ncc(c.stream, view(S), view(T), c.tmpl.sums.as<double>(),
+                                            integ, peaks, static_cast<float *>(D.dev), D.desc.Step,
+                                            c.stats.as<char>() + head);
+      launch_proximity_flagged(c.stream, view(S), view(T), D.dev, D.desc.Step, c.tmpl.data.ptr,
+                               tpitch, c.tmpl.sums.as<double>(), integ, f);
       D.in_device = true;
       return;
    }

@@ -125,6 +125,18 @@ __device__ __forceinline__ float inv_sqrt(double p)
    return (float)(1.0 / sqrt(p));
 }
 
+// 1 / sqrt(p) to FP64 accuracy short of the last bits (relative error below 2^-43): one Newton step
+// on the FP32 reciprocal square root, a fifth of the FP64 square root and division's
+// instructions; outside float range the FP64 functions.  p = 0 gives +inf, p < 0 NaN.
+__device__ __forceinline__ double rsqrt64(double p)
+{
+   if (p >= 1e-30 && p <= 1e30) {
+      const double y = (double)__builtin_amdgcn_rsqf((float)p);
+      return y * __builtin_fma(-0.5 * p * y, y, 1.5);
+   }
+   return 1.0 / sqrt(p);
+}
+
 // Window sum of the Norm denominators: the template window of output (x, y) with origin at
 // (-tw/2, -th/2) (cl-files/ImageProximityFFT.cl:55-84 gives the same window).
 __device__ __forceinline__ double window_sqsum(const double *__restrict__ I, int W, int H,

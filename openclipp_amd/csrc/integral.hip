@@ -32,7 +32,9 @@ struct IntegralAux {
    //   colsum  [RB][W]     column sums per tile row, then exclusive-scanned over tile rows
    //   rowsum  [H][CB]     row sums per tile column, then exclusive-scanned over tile columns
    //   tiletot [RB][CB]    tile totals, then 2-D exclusive-scanned (corner carries)
+   //   tilepeak [RB][CB]   (unsigned) high word of the tile's largest f
    double *colsum, *rowsum, *tiletot;
+   unsigned *tilepeak;
    int CB, RB;
 };
 
@@ -47,6 +49,7 @@ IntegralAux aux_layout(void *base, int W, int H)
    a.colsum = p;
    a.rowsum = a.colsum + (size_t)a.RB * W;
    a.tiletot = a.rowsum + (size_t)H * a.CB;
+   a.tilepeak = reinterpret_cast<unsigned *>(a.tiletot + (size_t)a.RB * a.CB);
    return a;
 }
 
@@ -79,8 +82,9 @@ __device__ __forceinline__ void load_row(const char *src, int step, int y, int y
    }
 }
 
-// 1. per-tile aggregates: column sums, row sums, tile total
-template <int TYPE, bool SQR, bool VEC>
+// 1. per-tile aggregates: column sums, row sums, tile total (and the tile's peak where the
+// caller wants the image's: f >= 0 then)
+template <int TYPE, bool SQR, bool VEC, bool PEAK>
 __global__ __launch_bounds__(kThreads) void integral_aggregate(const char *src, int W, int H,
                                                                 int step, int nch, int ch,
                                                                 IntegralAux aux)
@@ -93,6 +97,7 @@ __global__ __launch_bounds__(kThreads) void integral_aggregate(const char *src, 
    const int x0 = cb * kCW + threadIdx.x * kVec;
    const int y0 = rb * kRH, y1 = min(y0 + kRH, H);
    double col[kVec] = {0, 0, 0, 0};
+   unsigned peak = 0;
    for (int y = y0; y < y1; y += kRowUnroll) {
       double v[kRowUnroll][kVec];
 #pragma unroll
@@ -108,6 +113,12 @@ __global__ __launch_bounds__(kThreads) void integral_aggregate(const char *src, 
          }
          part[y - y0 + r][threadIdx.x] = rs;   // rows past y1 hold 0 and are not summed
       }
+      if (PEAK) {
+#pragma unroll
+         for (int r = 0; r < kRowUnroll; ++r)
+#pragma unroll
+            for (int j = 0; j < kVec; ++j) peak = max(peak, (unsigned)__double2hiint(v[r][j]) & 0x7fffffffu);
+      }
    }
 #pragma unroll
    for (int j = 0; j < kVec; ++j)
@@ -121,6 +132,11 @@ __global__ __launch_bounds__(kThreads) void integral_aggregate(const char *src, 
    }
    const double tot = wave_sum(rs);
    if (threadIdx.x == 0) aux.tiletot[(size_t)rb * aux.CB + cb] = tot;
+   if (PEAK) {
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) peak = max(peak, (unsigned)__shfl_xor((int)peak, d, 64));
+      if (threadIdx.x == 0) aux.tilepeak[(size_t)rb * aux.CB + cb] = peak;
+   }
 }
 
 // exclusive scan in place of n values at p[0], p[stride], ...
@@ -143,9 +159,23 @@ __device__ __forceinline__ void exclusive_scan_strided(double *p, int n, size_t 
 
 // 2. carries.  blockIdx.y = 0: column sums over tile rows, one thread per column;
 //              blockIdx.y = 1: row sums over tile columns, one thread per row;
-//              blockIdx.y = 2: 2-D exclusive scan of the tile totals (block 0 only).
-__global__ __launch_bounds__(256) void integral_carries(int W, int H, IntegralAux aux)
+//              blockIdx.y = 2: 2-D exclusive scan of the tile totals (block 0);
+//              blockIdx.y = 3: the largest tile peak into *peak (block 0, where wanted).
+__global__ __launch_bounds__(256) void integral_carries(int W, int H, IntegralAux aux,
+                                                        unsigned *peak)
 {
+   if (blockIdx.y == 3) {
+      if (blockIdx.x) return;
+      __shared__ unsigned red[4];
+      unsigned m = 0;
+      for (int k = threadIdx.x; k < aux.RB * aux.CB; k += 256) m = max(m, aux.tilepeak[k]);
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, d, 64));
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+      __syncthreads();
+      if (threadIdx.x == 0) *peak = max(max(red[0], red[1]), max(red[2], red[3]));
+      return;
+   }
    const int i = blockIdx.x * 256 + threadIdx.x;
    if (blockIdx.y == 0) {
       if (i < W) exclusive_scan_strided(aux.colsum + i, aux.RB, (size_t)W);
@@ -269,24 +299,30 @@ __global__ __launch_bounds__(kThreads) void integral_final(const char *src, int 
 size_t integral_aux_bytes(int W, int H)
 {
    size_t CB = cdiv(W, kCW), RB = cdiv(H, kRH);
-   return (RB * W + (size_t)H * CB + RB * CB) * sizeof(double);
+   return (RB * W + (size_t)H * CB + RB * CB) * sizeof(double) + RB * CB * sizeof(unsigned);
 }
 
 template <int TT, bool VEC>
 static void launch_integral_t(hipStream_t s, const char *src, const View &v, int channel,
-                              bool sqr, void *out, int ostep, int mode, bool ovec, IntegralAux aux)
+                              bool sqr, void *out, int ostep, int mode, bool ovec, IntegralAux aux,
+                              unsigned *peak)
 {
    const int W = v.width, H = v.height;
    dim3 grid(aux.CB, aux.RB);
    KernelTimer kt(s, "integral");
-   if (sqr)
-      integral_aggregate<TT, true, VEC><<<grid, kThreads, 0, s>>>(src, W, H, v.step, v.channels,
-                                                                 channel, aux);
-   else
-      integral_aggregate<TT, false, VEC><<<grid, kThreads, 0, s>>>(src, W, H, v.step, v.channels,
-                                                                  channel, aux);
+   auto aggregate = [&](auto kernel) {
+      kernel<<<grid, kThreads, 0, s>>>(src, W, H, v.step, v.channels, channel, aux);
+   };
+   if (peak) {
+      if constexpr (TT == SImage::F32) aggregate(integral_aggregate<TT, true, VEC, true>);
+      else fail(CL_INVALID_VALUE, "the peak of F32 images only");
+   } else if (sqr) {
+      aggregate(integral_aggregate<TT, true, VEC, false>);
+   } else {
+      aggregate(integral_aggregate<TT, false, VEC, false>);
+   }
    launch_check("integral_aggregate");
-   integral_carries<<<dim3(cdiv(W > H ? W : H, 256), 3), 256, 0, s>>>(W, H, aux);
+   integral_carries<<<dim3(cdiv(W > H ? W : H, 256), peak ? 4 : 3), 256, 0, s>>>(W, H, aux, peak);
    launch_check("integral_carries");
    char *o = static_cast<char *>(out);
 #define OCIP_FINAL(SQ, M, OV) \
@@ -302,7 +338,7 @@ static void launch_integral_t(hipStream_t s, const char *src, const View &v, int
 }
 
 void launch_integral(hipStream_t s, const View &v, int channel, bool sqr, void *out, int ostep,
-                     int out_type, void *auxp)
+                     int out_type, void *auxp, unsigned *peak)
 {
    IntegralAux aux = aux_layout(auxp, v.width, v.height);
    const char *src = static_cast<const char *>(v.ptr);
@@ -315,8 +351,8 @@ void launch_integral(hipStream_t s, const View &v, int channel, bool sqr, void *
    const bool ovec = mode != 2 && (ostep % (4 * osz)) == 0 &&
                      (reinterpret_cast<uintptr_t>(out) % (4 * osz)) == 0;
    OCIP_TYPE_SWITCH(v.type, TT, {
-      if (vec) launch_integral_t<TT, true>(s, src, v, channel, sqr, out, ostep, mode, ovec, aux);
-      else launch_integral_t<TT, false>(s, src, v, channel, sqr, out, ostep, mode, ovec, aux);
+      if (vec) launch_integral_t<TT, true>(s, src, v, channel, sqr, out, ostep, mode, ovec, aux, peak);
+      else launch_integral_t<TT, false>(s, src, v, channel, sqr, out, ostep, mode, ovec, aux, peak);
    });
 }
 

@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256) void ncc_scale_direct(const double *__restrict
 
 int kc_for(int tw) { return tw <= 97 ? std::max(2, (tw + 31 + 15) / 16) : 6; }
 int nub_for(int tw) { return tw <= 97 ? 1 : (tw + mfma::kBlockW - 1) / mfma::kBlockW; }
-int planes_for(int precision) { return precision == mfma::kBF16x3 ? 2 : 1; }
+int planes_for(int precision) { return mfma::planes_of(precision); }
 
 struct Geometry {
    int ldsp, vb;
@@ -906,6 +906,73 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
                                      run, {16, 14, 4, 2});
    KernelTimer kt(s, "crosscorr_mfma");
    run(variant);
+}
+
+// ======================================================================= split FP16
+constexpr int kSplitNT = 4;
+
+// Where the path is taken: prox_tile_f32 costs about 4 us + Mpx (12 us + 0.044 us taps) where it
+// forms the window sums in its tiles, and this path 58 us (seven launches, the integral's
+// three among them) + Mpx (7 us + 0.0055 us taps), equal at Mpx (taps + 142) = 1420: it is taken from
+// 1600 on (1900^2/16x16 88 against 82 us, 1000x3000/24x24 110 against 96, 1400^2/24x24 77
+// against 87).  Where prox_tile_f32 needs the integral too, it pays its launches as well:
+// taken from 200 taps or 2 Mpx on (160x120/31x31 90 against 67 us, 2048x512/16x16 68 against 64,
+// 2048x1024/5x5 79 against 73; 2048x512/5x5 55 against 63).
+// OCIP_SPLIT_NCC=0 turns the path off (prox_tile_f32 then computes the maps), 1 has it take
+// every call that it can.
+bool split_ncc_ok(int op, const View &S, const View &T)
+{
+   const char *e = getenv("OCIP_SPLIT_NCC");
+   if ((e && e[0] == '0') || op != kCCNorm) return false;
+   if (S.type != SImage::F32 || T.type != SImage::F32 || S.channels != 1) return false;
+   const int tw = T.width, th = T.height;
+   // one template column block; the staged tile's planes in LDS
+   if (tw <= 0 || th <= 0 || tw > 97 || th > 256) return false;
+   if (pair_geometry(kc2_for(tw), kSplitNT, th, mfma::kLdsMax, 2).vb < 1) return false;
+   if (e && e[0] == '1') return true;
+   const long long px = (long long)S.width * S.height, taps = (long long)tw * th;
+   return prox_norm_from_tile(op, S, T) ? px * (taps + 142) >= 1600000000LL
+                                        : taps >= 200 || px >= 1 << 21;
+}
+
+size_t split_ncc_work_bytes(const View &S, const View &T)
+{
+   const size_t tiles = (size_t)((S.width + 63) / 64) * ((S.height + mfma::kPairRows - 1) / mfma::kPairRows);
+   return pair_frag_bytes(mfma::kF16x3, T.width, T.height) + (1 + tiles) * sizeof(unsigned);
+}
+
+SplitFlags launch_split_ncc(hipStream_t s, const View &S, const View &T, const double *tsums,
+                            const double *integ, const unsigned *peaks, float *dst, int dstep,
+                            void *work)
+{
+   const int tw = T.width, th = T.height, KC2 = kc2_for(tw), NT = kSplitNT;
+   u16x8 *g0 = static_cast<u16x8 *>(work);
+   u16x8 *g1 = g0 + pair_frag_count(tw, th) * 64;
+   unsigned *any = reinterpret_cast<unsigned *>(static_cast<char *>(work) +
+                                                pair_frag_bytes(mfma::kF16x3, tw, th));
+   {
+      KernelTimer kt(s, "template_prep");
+      mfma::launch_split_prep(s, BatchDesc{static_cast<const char *>(T.ptr), tw, th, T.step, KC2,
+                                           1, g0, g1, nullptr}, peaks, any);
+   }
+   const Geometry g = pair_geometry(KC2, NT, th, mfma::kLdsMax, 2);
+   SingleLaunch L;
+   L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw, th, 1,
+                        g0, g1, tsums, integ, dst, dstep, g.vb,
+                        ((tw / 2) % 4 == 0 && rows_aligned(S)) ? 1 : 0};
+   L.a.peaks = peaks;
+   L.a.any = any;
+   L.a.flags = any + 1;
+   L.KC = KC2;
+   L.NT = NT;
+   L.mode = mfma::kModeNCC;
+   L.ldsp = g.ldsp;
+   L.lds = g.lds;
+   L.grid = dim3((S.width + 16 * NT - 1) / (16 * NT),
+                 (S.height + mfma::kPairRows - 1) / mfma::kPairRows);
+   KernelTimer kt(s, "crosscorr_mfma_split");
+   mfma::launch_split_pair(s, L);
+   return SplitFlags{any, any + 1, (int)L.grid.x, 16 * NT, mfma::kPairRows};
 }
 
 // ======================================================================= exact integer sums

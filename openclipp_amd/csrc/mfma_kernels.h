@@ -41,7 +41,14 @@ constexpr int kBlockW = 64;             // template column block for wide templa
 // dynamic LDS budget: the 160 KiB of a CU less room for the kernels' static LDS
 constexpr int kLdsMax = 160 * 1024 - 256;
 
-enum { kBF16 = 1, kF16 = 2, kBF16x3 = 3 };
+// kF16x3 (ocipCrossCorr_Norm of F32 images): split FP16, s = s_hi + s_lo of s scaled by a power of
+// two so that the image's largest magnitude lies in (2^14, 2^15], the template likewise.  hi
+// takes 11 significant bits and lo the next 11 to 13 (down to 2^-24, FP16 subnormals, which the
+// matrix cores keep), so a value within 2^15 of the largest is held to 2^-24 of itself, the rounding
+// unit of FP32, and every value to 2^-40 of the largest; the three products hi hi, hi lo, lo hi
+// leave out lo lo, at most 2^-24 of the product.
+enum { kBF16 = 1, kF16 = 2, kBF16x3 = 3, kF16x3 = 4 };
+__host__ __device__ constexpr int planes_of(int P) { return P == kBF16x3 || P == kF16x3 ? 2 : 1; }
 // kModeCC: the CrossCorr map (the single-template call; CrossCorr_Norm scales it in place
 // afterwards); kModeNCC / kModeSSDN: the batch kernel's epilogues from the FP64 integral;
 // kModeInt: the row-pair kernel on 8-bit integer images, exact integer sums (any of the
@@ -63,6 +70,11 @@ struct TileArgs {
    // kModeInt (exact sums of 8-bit integer images): element type of source and template
    // (kSrcU8 / kSrcS8), the op (ProxOp) and the steps between the int32 flushes
    int src8 = 0, op = 0, flush = 0;
+   // kF16x3: the peaks of source and template (split_range), the source's scale, the word that any
+   // flagged tile sets, and the tile's flag (non-zero: prox_tile_f32_flagged computes it again)
+   const unsigned *peaks = nullptr;
+   unsigned *any = nullptr, *flags = nullptr;
+   float scale = 1.f;
 };
 
 // Several sources of one size and template with crosscorr_mfma in one launch: the source, its
@@ -123,13 +135,45 @@ __device__ __forceinline__ unsigned short to_f16(float f)
    return __builtin_bit_cast(unsigned short, (_Float16)f);
 }
 
-// 16-bit encodings of a float for plane 0 (and plane 1 for split BF16)
+// What the split-FP16 sums of an image and a template need of their magnitudes.  peaks[0], [1]:
+// the high words of the largest s^2 and t^2 in FP64 (infinities and NaN compare above
+// everything finite).  n: taps.
+//   ok        the split holds: finite values, and every product and sum well inside FP32's range
+//             (smax tmax >= 2^-60 and n smax tmax <= 2^120), so that it loses nothing that the FP32
+//             sums of prox_tile_f32 keep
+//   ks, kt    the scales 2^ks, 2^kt
+//   unscale   2^-(ks + kt)
+//   least_ss  the least window sum of s^2 for which s's error, at most 2^-40 smax, stays within
+//             2^-24 of the window's root mean square
+struct SplitRange {
+   bool ok;
+   int ks, kt;
+   double unscale, least_ss;
+};
+__device__ __forceinline__ SplitRange split_range(const unsigned *peaks, int n)
+{
+   const unsigned hs = peaks[0], ht = peaks[1];
+   const double s2 = __hiloint2double((int)hs, 0), t2 = __hiloint2double((int)ht, 0);
+   SplitRange r;
+   // smax^2 < 2^(e + 1) with e the exponent of s2: smax < 2^ceil((e + 1) / 2)
+   r.ks = 15 - (((int)(hs >> 20) - 1023 + 2) >> 1);
+   r.kt = 15 - (((int)(ht >> 20) - 1023 + 2) >> 1);
+   const double p = s2 * t2, nn = (double)n * (double)n;
+   r.ok = hs < 0x7ff00000u && ht < 0x7ff00000u && p >= 0x1p-120 && p * nn <= 0x1p240 &&
+          abs(r.ks) <= 126 && abs(r.kt) <= 126;
+   r.unscale = __hiloint2double((1023 - (r.ks + r.kt)) << 20, 0);
+   r.least_ss = (double)n * s2 * 0x1p-32;
+   return r;
+}
+__device__ __forceinline__ float pow2f(int k) { return __uint_as_float((unsigned)(127 + k) << 23); }
+
+// 16-bit encodings of a float for plane 0 (and plane 1 for the split precisions)
 template <int P> __device__ __forceinline__ void encode(float f, unsigned short &p0,
                                                         unsigned short &p1)
 {
-   if (P == kF16) {
+   if (P == kF16 || P == kF16x3) {
       p0 = to_f16(f);
-      p1 = 0;
+      p1 = P == kF16x3 ? to_f16(f - (float)__builtin_bit_cast(_Float16, p0)) : (unsigned short)0;
    } else {
       p0 = to_bf16(f);
       p1 = P == kBF16x3 ? to_bf16(f - from_bf16(p0)) : (unsigned short)0;
@@ -209,7 +253,7 @@ __global__ __launch_bounds__(256) void single_prep(BatchDesc d)
 template <int P>
 __device__ __forceinline__ f32x16 mma(u16x8 a, u16x8 b, f32x16 c)
 {
-   if (P == kF16)
+   if (P == kF16 || P == kF16x3)
       return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                     __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
@@ -295,7 +339,7 @@ template <int P, int LCOLS, bool SRC8 = false>
 __device__ __forceinline__ void stage_rows(const TileArgs &a, unsigned short *lds, int ldsp,
                                            size_t plane, int row0, int col0, int nrows)
 {
-   constexpr int NPL = P == kBF16x3 ? 2 : 1;
+   constexpr int NPL = planes_of(P);
    constexpr int groups = LCOLS / 8;
    const int W = a.W, H = a.H;
    const int total = nrows * groups;
@@ -381,7 +425,7 @@ __device__ __forceinline__ void stage_rows(const TileArgs &a, unsigned short *ld
 #pragma unroll
          for (int i = 0; i < 8; ++i) {
             unsigned short e0, e1;
-            encode<P>(f[k][i], e0, e1);
+            encode<P>(P == kF16x3 ? f[k][i] * a.scale : f[k][i], e0, e1);
             h0[i] = e0;
             h1[i] = e1;
          }
@@ -397,7 +441,7 @@ template <int P, int KC, int NT, int MODE>
 __device__ __forceinline__ void mfma_tile(const TileArgs &a, int bx, int by, unsigned short *lds,
                                           int ldsp)
 {
-   constexpr int NPL = P == kBF16x3 ? 2 : 1;
+   constexpr int NPL = planes_of(P);
    constexpr int lcols = lcols_for(KC, NT);
    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
    const int x0 = bx * 32 * NT, y0 = by * kTileRows;
@@ -566,7 +610,7 @@ __host__ __device__ constexpr int pair_frag_steps(int th, int nub)
 template <int P>
 __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep, int tw, int th,
                                                     int KC, int nub, int f, int lane, u16x8 *frag,
-                                                    u16x8 *frag1, int src8)
+                                                    u16x8 *frag1, int src8, float scale = 1.f)
 {
    const int S = pair_frag_steps(th, nub);
    const int kc = f % KC, s = (f / KC) % S, ub = f / (KC * S);
@@ -581,12 +625,12 @@ __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep,
       const int u = 16 * kc + kb + i - dx;
       const float t = (v < th && u >= 0 && u < wb) ? tmpl_elem(trow, u0 + u, src8) : 0.f;
       unsigned short h0, h1;
-      encode<P>(t, h0, h1);
+      encode<P>(P == kF16x3 ? t * scale : t, h0, h1);
       h[i] = h0;
       l[i] = h1;
    }
    frag[(size_t)f * 64 + lane] = h;
-   if (P == kBF16x3) frag1[(size_t)f * 64 + lane] = l;   // split BF16: the lo plane
+   if (planes_of(P) == 2) frag1[(size_t)f * 64 + lane] = l;   // the lo plane
 }
 
 // Fragments of the row-pair kernel, one per wavefront, the FP64 sum of squares (same order
@@ -642,7 +686,7 @@ __device__ __forceinline__ void pair_mfma(f32x16 (&acc)[NT], const unsigned shor
    u16x8 a0[NA];
 #pragma unroll
    for (int c = 0; c < NA; ++c) a0[c] = *reinterpret_cast<const u16x8 *>(ab + 16 * c);
-   if constexpr (P != kBF16x3) {
+   if constexpr (planes_of(P) == 1) {
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
@@ -687,7 +731,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    constexpr bool INT = MODE == kModeInt;
    // operand planes: two for split BF16 (hi and lo), the lo plane of the staged rows at
    // `plane` 16-bit elements past the hi plane (the rows a band of a.vb steps stages)
-   constexpr int NPL = P == kBF16x3 ? 2 : 1;
+   constexpr int NPL = planes_of(P);
    const size_t plane = NPL == 2 ? (size_t)(kTileRows - 2 + 2 * a.vb) * ldsp : 0;
    constexpr int lcols = pair_lcols(KC, NT);
    constexpr int C = 16 * NT;
@@ -900,6 +944,11 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    if constexpr (NORM) {
       const double tt = tmpl_sqsum(a);
       const bool v4 = a.dstep % 16 == 0 && reinterpret_cast<uintptr_t>(a.dst) % 16 == 0;
+      // kF16x3: the sums' scale undone, the division in FP64 (as prox_tile_f32 has it), and
+      // outputs whose window is too dark for the split (split_range)
+      SplitRange sr;
+      if constexpr (P == kF16x3) sr = split_range(a.peaks, a.tw * a.th);
+      int dark = 0;
       auto finish = [&](int i0, const Corners &q) {
 #pragma unroll
          for (int u = 0; u < kEpiGroups; ++u) {
@@ -913,8 +962,13 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                const double ss = (q[u][3][e] - q[u][2][e]) - (q[u][1][e] - q[u][0][e]);
-               const double num = MODE == kModeNCC ? (double)cc[e] : ss - 2.0 * (double)cc[e] + tt;
-               v[e] = (float)num * inv_sqrt(ss * tt);
+               if constexpr (P == kF16x3) {
+                  v[e] = (float)((double)cc[e] * sr.unscale * rsqrt64(ss * tt));
+                  dark |= cc[e] != 0.f && ss < sr.least_ss && x + e < a.W;
+               } else {
+                  const double num = MODE == kModeNCC ? (double)cc[e] : ss - 2.0 * (double)cc[e] + tt;
+                  v[e] = (float)num * inv_sqrt(ss * tt);
+               }
             }
             gmem_f32 *o = out_row(a, y) + x;
             if (v4 && x + 4 <= a.W) {
@@ -935,6 +989,13 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
          if (i0 + kEpiGroups < kNormIters) {
             if (i0 + 2 * kEpiGroups < kNormIters) load_corners(i0 + 2 * kEpiGroups, qa);
             finish(i0 + kEpiGroups, qb);
+         }
+      }
+      if constexpr (P == kF16x3) {
+         dark = __syncthreads_or(dark);
+         if (threadIdx.x == 0) {
+            *a.flags = (unsigned)dark;
+            if (dark) *a.any = 1u;
          }
       }
       return;
@@ -969,7 +1030,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
 // workgroup per CU at these template widths, and whose three fragment sets would spill at 2).
 __host__ __device__ constexpr int pair_waves(int P, int KC, int NT, int MODE)
 {
-   return NT <= 4 && MODE == kModeCC && P != kBF16x3 ? 3 : P == kBF16x3 && NT == 6 && KC >= 7 ? 1 : 2;
+   return NT <= 4 && MODE == kModeCC && planes_of(P) == 1 ? 3 : P == kBF16x3 && NT == 6 && KC >= 7 ? 1 : 2;
 }
 
 // One 127 x 16 NT tile per workgroup, XCD-aware order (the single-template call): tiles_x *
@@ -987,6 +1048,15 @@ void crosscorr_mfma_pair(TileArgs a, int ldsp, int tiles_x, int tiles, ZImages z
       a.src = z.src[zi];
       a.dst = z.dst[zi];
       a.sstep = z.sstep[zi];
+   }
+   if constexpr (P == kF16x3) {
+      const SplitRange sr = split_range(a.peaks, a.tw * a.th);
+      a.flags += t;
+      if (!sr.ok) {
+         if (threadIdx.x == 0) *a.flags = *a.any = 1u;
+         return;
+      }
+      a.scale = pow2f(sr.ks);
    }
    pair_tile<P, KC, NT, MODE>(a, t % tiles_x, t / tiles_x, reinterpret_cast<unsigned short *>(lds_v),
                               ldsp);
@@ -1373,6 +1443,9 @@ template <int P> void launch_single_prep(hipStream_t s, const BatchDesc &d);
 template <int P> void launch_pair(hipStream_t s, const SingleLaunch &L);
 template <int P> void launch_pair_prep(hipStream_t s, const BatchDesc &d);
 template <int P> void launch_strip(hipStream_t s, const SingleLaunch &L, int tiles_y, int q_rows);
+// CrossCorr_Norm on split FP16 (mfma_f16x3.hip): the fragments, and the row-pair kernel
+void launch_split_prep(hipStream_t s, const BatchDesc &d, const unsigned *peaks, unsigned *any);
+void launch_split_pair(hipStream_t s, const SingleLaunch &L);
 template <int P> void launch_batch_prep(hipStream_t s, const BatchDesc *descs, int n);
 // the batch on the row-pair tile (BF16, FP16): its kernel and its fragments
 template <int P> void launch_pair_batch(hipStream_t s, const BatchLaunch &L);

@@ -166,14 +166,16 @@ inline size_t excl_bytes(int W, int H) { return excl_pitch(W) * ((size_t)H + 1) 
 //   out_type F32/F64 with inclusive same-size layout (public API), or
 //   out_type = -1: the internal exclusive layout above (out_step ignored).
 size_t integral_aux_bytes(int width, int height);
+// peak (sqr of F32 images, may be null): receives the high word of the largest f.
 void launch_integral(hipStream_t s, const View &src, int channel, bool sqr, void *out,
-                     int out_step, int out_type, void *aux);
+                     int out_step, int out_type, void *aux, unsigned *peak = nullptr);
 
 // Template staging: converts the template to the kernels' compute type with a row pitch of
 // `pitch` elements (zero padding), and writes FP64 sum(t^2), sum(t) to sums[0..1].
-// kind 0: float, 1: double, 2: int32.
+// kind 0: float, 1: double, 2: int32.  peak (may be null): receives the high word of the largest
+// t^2 in FP64.
 void launch_template_prep(hipStream_t s, const View &tpl, int channel, int pitch, int kind,
-                          void *out, double *sums);
+                          void *out, double *sums, unsigned *peak = nullptr);
 
 // Plain (VALU) proximity for any type/channel count.  `integ` is the exclusive FP64
 // sum-of-squares integral of the source for the Norm ops (null for the others).
@@ -183,6 +185,25 @@ void launch_proximity(hipStream_t s, int op, const View &src, const View &tpl, v
 // The plain Norm ops on F32 sources whose template fits one LDS band form the window sums
 // of s^2 inside the tile kernel (launch_proximity with no integral)
 bool prox_norm_from_tile(int op, const View &src, const View &tpl);
+
+// CrossCorr_Norm of F32 1-channel images on split-FP16 MFMA (as accurate as the FP32 sums of
+// launch_proximity, mfma_kernels.h): split_ncc_ok tells whether the path takes the call.  peaks
+// (launch_integral's of the source, launch_template_prep's of the template, in this order)
+// and integ come first; the tiles that the split cannot hold are then computed by
+// launch_proximity_flagged, from the flags (one per tile_w x tile_h outputs, tiles_x a row)
+// that launch_split_ncc left in `work`.
+struct SplitFlags {
+   const unsigned *any, *flags;   // any: 0 where no tile is flagged
+   int tiles_x, tile_w, tile_h;
+};
+bool split_ncc_ok(int op, const View &src, const View &T);
+size_t split_ncc_work_bytes(const View &src, const View &T);
+SplitFlags launch_split_ncc(hipStream_t s, const View &src, const View &T, const double *tsums,
+                            const double *integ, const unsigned *peaks, float *dst, int dst_step,
+                            void *work);
+void launch_proximity_flagged(hipStream_t s, const View &src, const View &T, void *dst,
+                              int dst_step, const void *tstage, int tpitch, const double *tsums,
+                              const double *integ, const SplitFlags &f);
 
 // MFMA cross-correlation (F32 1-channel source and template), precision 1..3.
 // The template's fragments and sum of squares (tsums[0]) are built from T in the call.

@@ -43,10 +43,13 @@ constexpr int kPrepWide = 1024;
 template <int TYPE, int KIND, int K>
 __global__ __launch_bounds__(kPrepWide) void template_prep(const char *tpl, int tw, int th,
                                                            int tstep, int nch, int ch, int pitch,
-                                                           void *out, double *sums)
+                                                           void *out, double *sums,
+                                                           unsigned *peak)
 {
    __shared__ double red[2][kPrepWide / 64];
+   __shared__ unsigned redp[kPrepWide / 64];
    double s2 = 0, s1 = 0;
+   unsigned top = 0;
    const int n = pitch * th, B = blockDim.x;
    const int dv = B / pitch, du = B - dv * pitch;
    int v = threadIdx.x / pitch, u = threadIdx.x - v * pitch;
@@ -74,17 +77,26 @@ __global__ __launch_bounds__(kPrepWide) void template_prep(const char *tpl, int 
          const double q = val[k] * val[k];
          s2 += q;
          s1 += val[k];
+         top = max(top, (unsigned)__double2hiint(q) & 0x7fffffffu);
       }
    }
    s2 = wave_sum(s2);
    s1 = wave_sum(s1);
    const int wave = threadIdx.x >> 6, waves = B >> 6;
-   if ((threadIdx.x & 63) == 0) { red[0][wave] = s2; red[1][wave] = s1; }
+   if (peak) {
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) top = max(top, (unsigned)__shfl_xor((int)top, d, 64));
+   }
+   if ((threadIdx.x & 63) == 0) { red[0][wave] = s2; red[1][wave] = s1; redp[wave] = top; }
    __syncthreads();
    if (threadIdx.x < 2) {
       double t = red[threadIdx.x][0];
       for (int w = 1; w < waves; ++w) t += red[threadIdx.x][w];
       sums[threadIdx.x] = t;
+   }
+   if (threadIdx.x == 2 && peak) {
+      for (int w = 0; w < waves; ++w) top = max(top, redp[w]);
+      *peak = top;
    }
 }
 
@@ -267,23 +279,16 @@ __device__ __forceinline__ void tile_sqsums(float *lds, int ldsw, int tw, int th
    for (int r = 0; r < R; ++r) ss[r] = sb[(size_t)lane * C4 + colbase + r];
 }
 
+// One output tile (x0, y0).  Starts with a barrier, so consecutive calls may reuse the LDS.
 template <int OP, int TYPE, int R>
-__global__ __launch_bounds__(256) void prox_tile_f32(const char *src, int W, int H, int sstep,
-                                                      int nch, int ch,
-                                                      const float *__restrict__ tp, int tpitch,
-                                                      int tw, int th,
-                                                      const double *__restrict__ tsums,
-                                                      const double *__restrict__ integ,
-                                                      char *dst, int dstep, int vb, int ldsw,
-                                                      int cx, int cy)
+__device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int H, int sstep,
+                                         int nch, int ch, const float *__restrict__ tp, int tpitch,
+                                         int tw, int th, const double *__restrict__ tsums,
+                                         const double *__restrict__ integ, char *dst, int dstep,
+                                         int vb, int ldsw, int cx, int cy, int x0, int y0)
 {
-   extern __shared__ float lds[];
    constexpr int U = 8;
    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-   // one-dimensional grid in XCD-aware tile order
-   const int tiles_x = (W + kWaves * R - 1) / (kWaves * R);
-   const int tile = xcd_tile(blockIdx.x, gridDim.x);
-   const int x0 = (tile % tiles_x) * (kWaves * R), y0 = (tile / tiles_x) * kTileRows;
    const int ncols = kWaves * R + tw - 1;
    const int nfull = tw / U, rem = tw - nfull * U;
    const int colbase = wave * R;
@@ -349,6 +354,55 @@ __global__ __launch_bounds__(256) void prox_tile_f32(const char *src, int W, int
    for (int r = 0; r < R; ++r) {
       const int ox = x0 + colbase + r;
       if (ox < W) drow[ox * nch + ch] = acc[r];
+   }
+}
+
+template <int OP, int TYPE, int R>
+__global__ __launch_bounds__(256) void prox_tile_f32(const char *src, int W, int H, int sstep,
+                                                      int nch, int ch,
+                                                      const float *__restrict__ tp, int tpitch,
+                                                      int tw, int th,
+                                                      const double *__restrict__ tsums,
+                                                      const double *__restrict__ integ,
+                                                      char *dst, int dstep, int vb, int ldsw,
+                                                      int cx, int cy)
+{
+   extern __shared__ float lds[];
+   // one-dimensional grid in XCD-aware tile order
+   const int tiles_x = (W + kWaves * R - 1) / (kWaves * R);
+   const int tile = xcd_tile(blockIdx.x, gridDim.x);
+   tile_f32<OP, TYPE, R>(lds, src, W, H, sstep, nch, ch, tp, tpitch, tw, th, tsums, integ, dst,
+                         dstep, vb, ldsw, cx, cy, (tile % tiles_x) * (kWaves * R),
+                         (tile / tiles_x) * kTileRows);
+}
+
+// CrossCorr_Norm of the tiles that the split-FP16 kernel flagged (SplitFlags): a workgroup walks
+// every gridDim.x-th tile and computes those that a flagged tile of that kernel overlaps.  With
+// no tile flagged it ends at once (4 us at 4096^2).
+template <int R>
+__global__ __launch_bounds__(256) void prox_tile_f32_flagged(const char *src, int W, int H,
+                                                              int sstep,
+                                                              const float *__restrict__ tp,
+                                                              int tpitch, int tw, int th,
+                                                              const double *__restrict__ tsums,
+                                                              const double *__restrict__ integ,
+                                                              char *dst, int dstep, int vb,
+                                                              int ldsw, SplitFlags f)
+{
+   extern __shared__ float lds[];
+   if (*f.any == 0u) return;
+   const int tiles_x = (W + kWaves * R - 1) / (kWaves * R);
+   const int tiles = tiles_x * ((H + kTileRows - 1) / kTileRows);
+   for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+      const int x0 = (t % tiles_x) * (kWaves * R), y0 = (t / tiles_x) * kTileRows;
+      const int bx1 = min(x0 + kWaves * R, W) - 1, by1 = min(y0 + kTileRows, H) - 1;
+      bool any = false;
+      for (int by = y0 / f.tile_h; by <= by1 / f.tile_h; ++by)
+         for (int bx = x0 / f.tile_w; bx <= bx1 / f.tile_w; ++bx)
+            any |= f.flags[by * f.tiles_x + bx] != 0u;
+      if (any)
+         tile_f32<kCCNorm, SImage::F32, R>(lds, src, W, H, sstep, 1, 0, tp, tpitch, tw, th, tsums,
+                                           integ, dst, dstep, vb, ldsw, tw / 2, th / 2, x0, y0);
    }
 }
 
@@ -778,7 +832,7 @@ int lds_pitch(int ncols)
 }  // namespace
 
 void launch_template_prep(hipStream_t s, const View &t, int channel, int pitch, int kind,
-                          void *out, double *sums)
+                          void *out, double *sums, unsigned *peak)
 {
    KernelTimer kt(s, "template_prep");
    const long long n = (long long)pitch * t.height;
@@ -787,7 +841,7 @@ void launch_template_prep(hipStream_t s, const View &t, int channel, int pitch, 
       const char *p = static_cast<const char *>(t.ptr);
       auto go = [&](auto kernel) {
          kernel<<<1, threads, 0, s>>>(p, t.width, t.height, t.step, t.channels, channel, pitch, out,
-                                      sums);
+                                      sums, peak);
       };
       if (n <= kPrepWide) {
          if (kind == 0) go(template_prep<TT, 0, 1>);
@@ -815,6 +869,22 @@ bool prox_norm_from_tile(int op, const View &S, const View &T)
    if (rows_fit < T.height) return false;   // one band
    return tile_sqsum_offset(kTileRows + T.height - 1, ldsw) + tile_sqsum_lds(R, T.height) <=
           (size_t)kLdsBudget;
+}
+
+void launch_proximity_flagged(hipStream_t s, const View &S, const View &T, void *dst, int dstep,
+                              const void *tstage, int tpitch, const double *tsums,
+                              const double *integ, const SplitFlags &f)
+{
+   constexpr int R = 16;
+   const int W = S.width, H = S.height, tw = T.width, th = T.height;
+   const int ldsw = lds_pitch(kWaves * R + tw - 1);
+   const int vb = min(th, kLdsBudget / (ldsw * 4) - (kTileRows - 1));   // >= 1: split_ncc_ok
+   const int tiles = ((W + kWaves * R - 1) / (kWaves * R)) * ((H + kTileRows - 1) / kTileRows);
+   KernelTimer kt(s, "prox_flagged");
+   prox_tile_f32_flagged<R><<<min(tiles, 512), 256, (size_t)(kTileRows + vb - 1) * ldsw * 4, s>>>(
+       static_cast<const char *>(S.ptr), W, H, S.step, static_cast<const float *>(tstage), tpitch,
+       tw, th, tsums, integ, static_cast<char *>(dst), dstep, vb, ldsw, f);
+   launch_check("prox_flagged");
 }
 
 template <int OP>
