@@ -752,9 +752,8 @@ void launch_crosscorr_mfma(hipStream_t s, int precision, bool norm, const View &
          else mfma::launch_pair_prep<mfma::kBF16x3>(s, d);
       }
    }
-   // staged columns start at x0 - tw/2 + 64 ub + 8 g with x0 a multiple of 64 (crosscorr_mfma)
-   // or 16 (row-pair kernels): 16-byte aligned when tw/2 is a multiple of 4 and the rows are
-   // 16-byte aligned
+   // the strip kernel's ring columns start at x0 - tw/2 + 4 g with x0 a multiple of 64: 16-byte
+   // aligned when tw/2 is a multiple of 4 and the rows are 16-byte aligned
    const int vec = ((tw / 2) % 4 == 0 && rows_aligned(S)) ? 1 : 0;
    auto run = [&](int variant) {
       SingleLaunch L;
@@ -781,7 +780,7 @@ void launch_crosscorr_mfma(hipStream_t s, int precision, bool norm, const View &
          const int NT = variant - 10;
          const Geometry g = pair_geometry(KC2, NT, th, mfma::kLdsMax, planes_for(precision));
          L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw,
-                              th, nub, g0, g1, tsums, integ, dst, dstep, g.vb, vec};
+                              th, nub, g0, g1, tsums, integ, dst, dstep, g.vb, 0};
          L.KC = KC2;
          L.NT = NT;
          L.ldsp = g.ldsp;
@@ -796,7 +795,7 @@ void launch_crosscorr_mfma(hipStream_t s, int precision, bool norm, const View &
       const int NT = variant;
       const Geometry g = geometry(precision, KC, NT, th);
       L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw, th,
-                           nub, f0, f1, tsums, integ, dst, dstep, g.vb, vec};
+                           nub, f0, f1, tsums, integ, dst, dstep, g.vb, 0};
       L.KC = KC;
       L.NT = NT;
       L.ldsp = g.ldsp;
@@ -870,13 +869,10 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
       for (int i0 = 0; i0 < n; i0 += mfma::kZImages) {
          SingleLaunch L;
          L.z.n = std::min(mfma::kZImages, n - i0);
-         // 16-byte staging loads: tw/2 a multiple of 4 and every source's rows 16-byte aligned
-         int vec = (tw / 2) % 4 == 0;
          for (int k = 0; k < L.z.n; ++k) {
             L.z.src[k] = src[i0 + k];
             L.z.dst[k] = dst[i0 + k];
             L.z.sstep[k] = sstep[i0 + k];
-            if (reinterpret_cast<uintptr_t>(src[i0 + k]) % 16 || sstep[i0 + k] % 16) vec = 0;
          }
          L.mode = mfma::kModeCC;
          L.NT = NT;
@@ -884,13 +880,13 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
          L.lds = g.lds;
          if (pair) {
             L.a = mfma::TileArgs{src[i0], W, H, sstep[i0], tw, th, nub, g0, g1, sums, nullptr,
-                                 dst[i0], dstep, g.vb, vec};
+                                 dst[i0], dstep, g.vb, 0};
             L.KC = KC2;
             L.grid = dim3((W + 16 * NT - 1) / (16 * NT), (H + mfma::kPairRows - 1) / mfma::kPairRows);
             mfma::launch_pair<mfma::kBF16x3>(s, L);
          } else {
             L.a = mfma::TileArgs{src[i0], W, H, sstep[i0], tw, th, nub, f0, f1, sums, nullptr,
-                                 dst[i0], dstep, vb, vec};
+                                 dst[i0], dstep, vb, 0};
             L.KC = KC;
             L.grid = dim3((W + 32 * NT - 1) / (32 * NT), (H + mfma::kTileRows - 1) / mfma::kTileRows);
             mfma::launch_single<mfma::kBF16x3>(s, L);
@@ -958,8 +954,7 @@ SplitFlags launch_split_ncc(hipStream_t s, const View &S, const View &T, const d
    const Geometry g = pair_geometry(KC2, NT, th, mfma::kLdsMax, 2);
    SingleLaunch L;
    L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw, th, 1,
-                        g0, g1, tsums, integ, dst, dstep, g.vb,
-                        ((tw / 2) % 4 == 0 && rows_aligned(S)) ? 1 : 0};
+                        g0, g1, tsums, integ, dst, dstep, g.vb, 0};
    L.a.peaks = peaks;
    L.a.any = any;
    L.a.flags = any + 1;
@@ -1217,12 +1212,8 @@ void launch_int_mfma(hipStream_t s, int op, const View &S, const View &T, double
    const Geometry g = pair_geometry(KC2, 4, th);
    SingleLaunch L;
    L.mode = mfma::kModeInt;
-   // 8-byte staging loads: staged columns start at 64 bx - tw/2 + 8 g, so tw/2 a multiple of 8,
-   // and 8-byte aligned rows
-   const int vec8 = (tw / 2) % 8 == 0 && S.step % 8 == 0 &&
-                    reinterpret_cast<uintptr_t>(S.ptr) % 8 == 0;
    L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw, th, 1,
-                        g0, nullptr, tsums, nullptr, dst, dstep, g.vb, vec8};
+                        g0, nullptr, tsums, nullptr, dst, dstep, g.vb, 0};
    L.a.src8 = src8;
    L.a.op = op;
    // steps between the int32 flushes: each step adds one template row of products
@@ -1380,7 +1371,6 @@ void run_batch_mfma(hipStream_t s, BatchCache *cache, int num_cus, int precision
          L.W = S.width;
          L.H = S.height;
          L.sstep = S.step;
-         L.vec = rows_aligned(S) ? 1 : 0;
          L.integ = e->integ.as<double>();
          L.items = ditems + k.first;
          L.nitems = k.count;

@@ -32,7 +32,7 @@ template <int KC, int NT, int MODE> void batch(hipStream_t s, const BatchLaunch 
 {
    auto k = crosscorr_mfma_batch<P, KC, NT, MODE>;
    allow_lds(k);
-   k<<<L.grid, 256, L.lds, s>>>(L.src, L.W, L.H, L.sstep, L.vec, L.integ, L.items, L.nitems,
+   k<<<L.grid, 256, L.lds, s>>>(L.src, L.W, L.H, L.sstep, L.integ, L.items, L.nitems,
                                 L.tiles_x, L.tiles_y, L.counter, L.ldsp);
 }
 
@@ -75,7 +75,7 @@ template <int KC, int NT, int MODE> void pair_batch(hipStream_t s, const BatchLa
 {
    auto k = crosscorr_mfma_pair_batch<P, KC, NT, MODE>;
    allow_lds(k);
-   k<<<L.grid, 256, L.lds, s>>>(L.src, L.W, L.H, L.sstep, L.vec, L.integ, L.items, L.nitems,
+   k<<<L.grid, 256, L.lds, s>>>(L.src, L.W, L.H, L.sstep, L.integ, L.items, L.nitems,
                                 L.tiles_x, L.tiles_y, L.counter, L.ldsp);
 }
 

@@ -66,7 +66,7 @@ struct TileArgs {
    float *dst;
    int dstep;
    int vb;                       // template rows per LDS band
-   int vec;                      // 16-byte staging loads allowed
+   int vec;                      // 16-byte ring loads allowed (crosscorr_mfma_strip)
    // kModeInt (exact sums of 8-bit integer images): element type of source and template
    // (kSrcU8 / kSrcS8), the op (ProxOp) and the steps between the int32 flushes
    int src8 = 0, op = 0, flush = 0;
@@ -269,12 +269,12 @@ typedef const u16x8 __attribute__((address_space(1))) *gfrag_ptr;
 // The same for the output maps and the template sums, whose pointers the batch kernels also
 // read from a table: stores through a flat pointer count against the LDS wait counter too, so
 // an epilogue's LDS reads would wait for every earlier store of the thread.
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef __attribute__((address_space(1))) float gmem_f32;
 typedef __attribute__((address_space(1))) f32x4_t gmem_f32x4;
 typedef __attribute__((address_space(1))) char gmem_char;
 typedef __attribute__((address_space(1))) int gmem_i32;
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x4_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef __attribute__((address_space(1))) i32x4_t gmem_i32x4;
 __device__ __forceinline__ gmem_f32 *out_row(const TileArgs &a, int y)
 {
@@ -333,7 +333,11 @@ __device__ __forceinline__ void row_mfma(f32x16 (&acc)[NT], const unsigned short
 }
 
 // Stage source rows [row0, row0 + nrows) x columns [col0, col0 + LCOLS) into LDS as 16-bit
-// values (zero outside the image), 8 columns per item, four items per thread in flight.
+// values (zero outside the image), 8 columns per item, four items per thread in flight, each
+// item two 16-byte loads (one 8-byte load of 8-bit sources) whatever its alignment.  Against
+// eight loads of single elements wherever tw/2 or the row pitch left the columns unaligned:
+// CrossCorr_Norm BF16 4096^2/63x64 220 -> 187 us, 4095-wide 8-bit SqrDistance 32x32 167 -> 118 us,
+// 48 BF16 templates of 8..96 px on 2048^2 2217 -> 1966 us; aligned calls unchanged.
 // SRC8: the source holds 8-bit integers (a.src8 gives the sign), exact in BF16.
 template <int P, int LCOLS, bool SRC8 = false>
 __device__ __forceinline__ void stage_rows(const TileArgs &a, unsigned short *lds, int ldsp,
@@ -357,9 +361,8 @@ __device__ __forceinline__ void stage_rows(const TileArgs &a, unsigned short *ld
             const bool rowin = it < total && sy >= 0 && sy < H;
             const unsigned char *brow = reinterpret_cast<const unsigned char *>(a.src) +
                                         (size_t)(rowin ? sy : 0) * a.sstep;
-            if (a.vec && rowin && sx >= 0 && sx + 8 <= W) {
-               // a.vec: 8-byte aligned rows and staged columns starting on multiples of 8
-               const uint2 q = *reinterpret_cast<const uint2 *>(brow + sx);
+            if (rowin && sx >= 0 && sx + 8 <= W) {
+               const u32x2_u q = *reinterpret_cast<const u32x2_u *>(brow + sx);
                lo[k] = q.x;
                hi[k] = q.y;
             } else {
@@ -403,9 +406,9 @@ __device__ __forceinline__ void stage_rows(const TileArgs &a, unsigned short *ld
          const bool rowin = it < total && sy >= 0 && sy < H;
          const float *srow = reinterpret_cast<const float *>(
              reinterpret_cast<const char *>(a.src) + (size_t)(rowin ? sy : 0) * a.sstep);
-         if (a.vec && rowin && sx >= 0 && sx + 8 <= W) {
-            const float4 q0 = *reinterpret_cast<const float4 *>(srow + sx);
-            const float4 q1 = *reinterpret_cast<const float4 *>(srow + sx + 4);
+         if (rowin && sx >= 0 && sx + 8 <= W) {
+            const f32x4_u q0 = *reinterpret_cast<const f32x4_u *>(srow + sx);
+            const f32x4_u q1 = *reinterpret_cast<const f32x4_u *>(srow + sx + 4);
             f[k][0] = q0.x; f[k][1] = q0.y; f[k][2] = q0.z; f[k][3] = q0.w;
             f[k][4] = q1.x; f[k][5] = q1.y; f[k][6] = q1.z; f[k][7] = q1.w;
          } else {
@@ -551,7 +554,7 @@ void crosscorr_mfma(TileArgs a, int ldsp, int tiles_x, int tiles, ZImages z)
 // held to two waves per SIMD, the two workgroups per CU that the LDS allows.
 template <int P, int KC, int NT, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void crosscorr_mfma_batch(const float *src, int W, int H, int sstep, int vec,
+void crosscorr_mfma_batch(const float *src, int W, int H, int sstep,
                           const double *integ, const BatchItem *__restrict__ items, int nitems,
                           int tiles_x, int tiles_y, unsigned *counter, int ldsp)
 {
@@ -569,9 +572,8 @@ void crosscorr_mfma_batch(const float *src, int W, int H, int sstep, int vec,
       if (it >= total) break;
       const BatchItem b = items[it / tiles];
       const int tile = it - (it / tiles) * tiles;
-      // 16-byte staging loads: aligned rows (vec) and tw/2 a multiple of 4
       TileArgs a{src, W, H, sstep, b.tw, b.th, b.nub, b.frag0, b.frag1, b.tsums, integ,
-                 b.dst, b.dstep, b.vb, (vec && (b.tw / 2) % 4 == 0) ? 1 : 0};
+                 b.dst, b.dstep, b.vb, 0};
       mfma_tile<P, KC, NT, MODE>(a, tile % tiles_x, tile / tiles_x,
                                  reinterpret_cast<unsigned short *>(lds_v), ldsp);
    }
@@ -848,7 +850,6 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    constexpr int kIntIters = (kPairRows * (C / 4) + 255) / 256;
    int4 ssq[INT ? kIntIters : 1];
    if constexpr (INT) {
-      const bool v4 = a.dstep % 16 == 0 && reinterpret_cast<uintptr_t>(a.dst) % 16 == 0;
 #pragma unroll
       for (int i = 0; i < kIntIters; ++i) {
          const int k = threadIdx.x + 256 * i;
@@ -857,7 +858,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
          ssq[i] = make_int4(0, 0, 0, 0);
          if (a.op == kCC || k >= kPairRows * (C / 4) || y >= a.H || x >= a.W) continue;
          const gmem_i32 *oi = reinterpret_cast<const gmem_i32 *>(out_row(a, y) + x);
-         if (v4 && x + 4 <= a.W) {
+         if (x + 4 <= a.W) {
             const i32x4_t q = *reinterpret_cast<const gmem_i32x4 *>(oi);
             ssq[i] = make_int4(q[0], q[1], q[2], q[3]);
          } else {
@@ -904,7 +905,6 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
       // sum of squares SS, an exact int32 that ss_box8 left in the map), as prox_tile_int forms
       // it; four consecutive columns per thread, one 16-byte store where the row allows
       const double tt = a.tsums[0];
-      const bool v4 = a.dstep % 16 == 0 && reinterpret_cast<uintptr_t>(a.dst) % 16 == 0;
 #pragma unroll
       for (int i = 0; i < kIntIters; ++i) {
          const int k = threadIdx.x + 256 * i;
@@ -927,7 +927,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
                v[e] = a.op == kSSD ? (float)d : (float)(d / sqrt(ss * tt));
             }
          }
-         if (v4 && x + 4 <= a.W) {
+         if (x + 4 <= a.W) {
             *reinterpret_cast<gmem_f32x4 *>(o) = f32x4_t{v[0], v[1], v[2], v[3]};
          } else {
 #pragma unroll
@@ -937,13 +937,11 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
       }
       return;
    }
-   // rows 1..127 are whole.  16-byte aligned output rows: four consecutive columns per
-   // thread (the tile pitch keeps them 16-byte aligned in LDS too), one at a time at the
-   // right edge; otherwise consecutive threads take consecutive columns
+   // rows 1..127 are whole: four consecutive columns per thread (the tile pitch keeps them
+   // 16-byte aligned in LDS), one at a time at the right edge
    static_assert(TP % 4 == 0 && C % 4 == 0, "16-byte groups of the LDS tile");
    if constexpr (NORM) {
       const double tt = tmpl_sqsum(a);
-      const bool v4 = a.dstep % 16 == 0 && reinterpret_cast<uintptr_t>(a.dst) % 16 == 0;
       // kF16x3: the sums' scale undone, the division in FP64 (as prox_tile_f32 has it), and
       // outputs whose window is too dark for the split (split_range)
       SplitRange sr;
@@ -971,7 +969,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
                }
             }
             gmem_f32 *o = out_row(a, y) + x;
-            if (v4 && x + 4 <= a.W) {
+            if (x + 4 <= a.W) {
                *reinterpret_cast<gmem_f32x4 *>(o) = f32x4_t{v[0], v[1], v[2], v[3]};
             } else {
 #pragma unroll
@@ -1000,27 +998,18 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
       }
       return;
    }
-   if (a.dstep % 16 == 0 && reinterpret_cast<uintptr_t>(a.dst) % 16 == 0) {
-      for (int k = threadIdx.x; k < kPairRows * (C / 4); k += 256) {
-         const int r = k / (C / 4), c = 4 * (k - r * (C / 4));
-         const int y = Y0 + r, x = x0 + c;
-         if (y >= a.H || x >= a.W) continue;
-         gmem_f32 *o = out_row(a, y) + x;
-         const float4 q = *reinterpret_cast<const float4 *>(&tile[(r + 1) * TP + c]);
-         if (x + 4 <= a.W) {
-            *reinterpret_cast<gmem_f32x4 *>(o) = f32x4_t{q.x, q.y, q.z, q.w};
-         } else {
-            o[0] = q.x;
-            if (x + 1 < a.W) o[1] = q.y;
-            if (x + 2 < a.W) o[2] = q.z;
-         }
-      }
-   } else {
-      for (int k = threadIdx.x; k < kPairRows * C; k += 256) {
-         const int r = k / C, c = k - r * C;
-         const int y = Y0 + r, x = x0 + c;
-         if (y >= a.H || x >= a.W) continue;
-         out_row(a, y)[x] = tile[(r + 1) * TP + c];
+   for (int k = threadIdx.x; k < kPairRows * (C / 4); k += 256) {
+      const int r = k / (C / 4), c = 4 * (k - r * (C / 4));
+      const int y = Y0 + r, x = x0 + c;
+      if (y >= a.H || x >= a.W) continue;
+      gmem_f32 *o = out_row(a, y) + x;
+      const float4 q = *reinterpret_cast<const float4 *>(&tile[(r + 1) * TP + c]);
+      if (x + 4 <= a.W) {
+         *reinterpret_cast<gmem_f32x4 *>(o) = f32x4_t{q.x, q.y, q.z, q.w};
+      } else {
+         o[0] = q.x;
+         if (x + 1 < a.W) o[1] = q.y;
+         if (x + 2 < a.W) o[2] = q.z;
       }
    }
 }
@@ -1075,7 +1064,7 @@ constexpr int kPairBatchBands = kXcds * kSubBands;
 
 template <int P, int KC, int NT, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void crosscorr_mfma_pair_batch(const float *src, int W, int H, int sstep, int vec,
+void crosscorr_mfma_pair_batch(const float *src, int W, int H, int sstep,
                                const double *integ, const BatchItem *__restrict__ items,
                                int nitems, int tiles_x, int tiles_y, unsigned *counter, int ldsp)
 {
@@ -1098,9 +1087,8 @@ void crosscorr_mfma_pair_batch(const float *src, int W, int H, int sstep, int ve
          if (it >= total) break;
          const BatchItem b = items[it / bt];
          const int tile = t0 + (it - (it / bt) * bt);
-         // 16-byte staging loads: aligned rows (vec) and tw/2 a multiple of 4
          TileArgs a{src, W, H, sstep, b.tw, b.th, b.nub, b.frag0, nullptr, b.tsums, integ,
-                    b.dst, b.dstep, b.vb, (vec && (b.tw / 2) % 4 == 0) ? 1 : 0};
+                    b.dst, b.dstep, b.vb, 0};
          pair_tile<P, KC, NT, MODE>(a, tile % tiles_x, tile / tiles_x,
                                     reinterpret_cast<unsigned short *>(lds_v), ldsp);
       }
@@ -1427,7 +1415,7 @@ struct SingleLaunch {
 
 struct BatchLaunch {
    const float *src;
-   int W, H, sstep, vec;
+   int W, H, sstep;
    const double *integ;
    const BatchItem *items;
    int nitems, tiles_x, tiles_y;
