@@ -162,14 +162,14 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
    const int esz = kind == 1 ? 8 : 4;
    const int tpitch = tpitch_for(tw);
    c.tmpl.data.ensure((size_t)tpitch * (th > 0 ? th : 1) * esz);
-   c.tmpl.sums.ensure(2 * sizeof(double));
+   c.tmpl.sums.ensure(4 * sizeof(double));
 
    // SqrDistance on 8-bit sources is formed from the cross term and the window sums of
    // squares, which come from the integral as for the Norm ops
    const bool ssd8 = op == kSSD && (type == SImage::U8 || type == SImage::S8);
    // 8-bit integer images: exact sums on BF16 MFMA where the path applies
    if (precision == ocipPrecisionF32 && int_mfma_ok(op, view(S), view(T))) {
-      c.stats.ensure(int_mfma_work_bytes(tw, th));
+      c.stats.ensure(int_mfma_work_bytes(view(S), view(T)));
       launch_int_mfma(c.stream, op, view(S), view(T), c.tmpl.sums.as<double>(),
                       static_cast<float *>(D.dev), D.desc.Step, c.stats.ptr);
       D.in_device = true;
@@ -271,7 +271,7 @@ void run_backward_batch(uint n, const ocipImage *hs, ocipImage ht, const ocipIma
    const int W = S[0]->desc.Width, H = S[0]->desc.Height;
    const int tpitch = tpitch_for(tw);
    c.tmpl.data.ensure((size_t)tpitch * th * sizeof(float));
-   c.tmpl.sums.ensure(2 * sizeof(double));
+   c.tmpl.sums.ensure(4 * sizeof(double));
    c.integ_aux.ensure(integral_aux_bytes(W, H));
    launch_template_prep(c.stream, view(T), 0, tpitch, 0, c.tmpl.data.ptr, c.tmpl.sums.as<double>());
    c.work.ensure(backward_work_bytes((int)n, W, H, tw, th, tpitch));
@@ -817,7 +817,7 @@ static ocipError run_proximity_fft(int op, ocipProgram Program, ocipImage Source
       const double *integ = op == kCC ? nullptr : sqr_integral_for(c, S, 0);
       const int tpitch = tpitch_for(T.desc.Width);
       c.tmpl.data.ensure((size_t)tpitch * T.desc.Height * sizeof(float));
-      c.tmpl.sums.ensure(2 * sizeof(double));
+      c.tmpl.sums.ensure(4 * sizeof(double));
       launch_template_prep(c.stream, view(T), 0, tpitch, 0, c.tmpl.data.ptr, c.tmpl.sums.as<double>());
       launch_proximity_fft(c.stream, p.fft, op, view(S), view(T), integ, c.tmpl.sums.as<double>(),
                            D.dev, (int)D.desc.Step);

@@ -1021,13 +1021,17 @@ __device__ __forceinline__ void wave_incl_scan(int (&x)[N])
 template <int NCH, bool SIGNED, bool BST>
 __global__ __launch_bounds__(64) void ss_box8(const unsigned char *__restrict__ src, int W,
                                               int H, int sstep, int tw, int th,
-                                              char *__restrict__ dst, int dstep, int bands)
+                                              char *__restrict__ dst, int dstep, int bands,
+                                              size_t plane8, size_t planef)
 {
    extern __shared__ int ring[];   // th x 64: lane's R of the last th rows
    constexpr int U = 8;            // rows per batch of loads (two batches in flight)
    const int lane = threadIdx.x;
    // consecutive blocks (one XCD's run) side by side along a band share halo columns in L2
    const int b = xcd_tile(blockIdx.x, gridDim.x);
+   // blockIdx.y = channel
+   src += blockIdx.y * plane8;
+   dst += blockIdx.y * planef;
    const int cblks = gridDim.x / bands;
    const int band = b / cblks, cblk = b % cblks;
    const int x0 = cblk * 64, y0 = band * kBoxBand;
@@ -1156,28 +1160,129 @@ __global__ __launch_bounds__(64) void ss_box8(const unsigned char *__restrict__ 
 // chunks of 128 columns: P up to index 63 + tw (the 63 + tw staged columns and one past)
 static int ss_box8_chunks(int tw) { return 63 + tw < 128 ? 1 : 2; }
 
+// Interleaved 8-bit channels into planes of their own (row pitch plane8_step, plane pitch H rows),
+// zeros between the width and the pitch, and the planes of the map back into interleaved
+// channels: the kernels between them take every channel of an image in one launch, as
+// 1-channel images with wide loads and stores (with the channels' maps interleaved by those
+// kernels themselves, 4 bytes of every 16 a store, the row-pair kernel ran 60 instead of 40 us
+// at 1280x960/24x24).  Four pixels per thread.  Bound by HBM: 2 W H NCH and 8 W H NCH bytes.
+static int plane8_step(int W) { return (W + 15) / 16 * 16; }
+
+template <int NCH>
+__global__ __launch_bounds__(256) void split_planes8(const unsigned char *__restrict__ src, int W,
+                                                     int H, int sstep,
+                                                     unsigned char *__restrict__ dst, int dstep)
+{
+   const int k = blockIdx.x * 256 + threadIdx.x, groups = dstep / 4;
+   const int y = k / groups, x = 4 * (k - y * groups);
+   if (y >= H) return;
+   const unsigned char *row = src + (size_t)y * sstep;
+   uint32_t q[NCH];   // the 4 NCH bytes of the thread's pixels
+   if (x + 4 <= W) {
+      typedef uint32_t u32_u __attribute__((aligned(1)));
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) q[i] = reinterpret_cast<const u32_u *>(row + x * NCH)[i];
+   } else {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) q[i] = 0;
+#pragma unroll
+      for (int i = 0; i < 4 * NCH; ++i)
+         if (x + i / NCH < W) q[i / 4] |= (uint32_t)row[x * NCH + i] << (8 * (i % 4));
+   }
+#pragma unroll
+   for (int c = 0; c < NCH; ++c) {
+      uint32_t v = 0;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+         const int i = p * NCH + c;
+         v |= (q[i / 4] >> (8 * (i % 4)) & 0xffu) << (8 * p);
+      }
+      *reinterpret_cast<uint32_t *>(dst + ((size_t)c * H + y) * dstep + x) = v;
+   }
+}
+
+template <int NCH>
+__global__ __launch_bounds__(256) void join_planes(const float *__restrict__ src, int W, int H,
+                                                   int sstep, float *__restrict__ dst, int dstep)
+{
+   const int k = blockIdx.x * 256 + threadIdx.x, groups = sstep / 16;
+   const int y = k / groups, x = 4 * (k - y * groups);
+   if (y >= H) return;
+   float v[4 * NCH];
+#pragma unroll
+   for (int c = 0; c < NCH; ++c) {
+      const float4 q = *reinterpret_cast<const float4 *>(
+          reinterpret_cast<const char *>(src) + ((size_t)c * H + y) * sstep + 4 * x);
+      v[c] = q.x; v[NCH + c] = q.y; v[2 * NCH + c] = q.z; v[3 * NCH + c] = q.w;
+   }
+   float *d = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + (size_t)y * dstep) + x * NCH;
+   if (x + 4 <= W) {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+         reinterpret_cast<f32x4_u *>(d)[i] = f32x4_u{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+   } else {
+#pragma unroll
+      for (int i = 0; i < 4 * NCH; ++i)
+         if (x + i / NCH < W) d[i] = v[i];
+   }
+}
+
+// one thread per 4 columns of a plane
+static unsigned plane_blocks(int H, int step) { return (unsigned)(((long long)H * (step / 4) + 255) / 256); }
+
 bool int_mfma_ok(int op, const View &S, const View &T)
 {
    const char *e = getenv("OCIP_INT_MFMA");
    if ((e && e[0] == '0') || op == kSAD) return false;
-   if ((S.type != SImage::U8 && S.type != SImage::S8) || S.channels != 1 || T.type != S.type)
-      return false;
+   if ((S.type != SImage::U8 && S.type != SImage::S8) || T.type != S.type) return false;
+   if (S.channels != 1 && S.channels != 2 && S.channels != 4) return false;
    const int tw = T.width, th = T.height;
    // (templates of one column block; ss_box8: byte offsets of the image below kBoxOob)
    if (tw <= 0 || th <= 0 || tw > 97 || th > 97) return false;
-   if ((long long)S.height * S.step >= kBoxOob) return false;
+   if ((long long)S.height * std::max((long long)S.step, (long long)plane8_step(S.width)) >= kBoxOob)
+      return false;
    const long long mp = int_max_product(S.type);
    if ((long long)tw * mp >= (1LL << 24) || (long long)tw * th * mp >= (1LL << 31)) return false;
    return pair_geometry(kc2_for(tw), 4, th).vb >= 1;
 }
 
-size_t int_mfma_work_bytes(int tw, int th) { return pair_frag_bytes(mfma::kBF16, tw, th); }
+size_t int_mfma_work_bytes(const View &S, const View &T)
+{
+   // several channels: a plane of bytes and a plane of the map each
+   const size_t planes = S.channels > 1 ? 5 * (size_t)S.channels * S.height * plane8_step(S.width) : 0;
+   return S.channels * pair_frag_bytes(mfma::kBF16, T.width, T.height) + planes;
+}
 
-void launch_int_mfma(hipStream_t s, int op, const View &S, const View &T, double *tsums,
+void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, double *tsums,
                      float *dst, int dstep, void *work)
 {
-   const int tw = T.width, th = T.height, KC2 = kc2_for(tw);
-   const int src8 = S.type == SImage::U8 ? mfma::kSrcU8 : mfma::kSrcS8;
+   const int tw = T.width, th = T.height, KC2 = kc2_for(tw), nch = image.channels;
+   const int src8 = image.type == SImage::U8 ? mfma::kSrcU8 : mfma::kSrcS8;
+   const size_t frag_bytes = pair_frag_bytes(mfma::kBF16, tw, th);
+   // S, map: the image and its map, or (several channels) their first planes, the others plane8
+   // and planef bytes apart
+   View S = image;
+   float *map = dst;
+   int mstep = dstep;
+   size_t plane8 = 0, planef = 0;
+   if (nch > 1) {
+      KernelTimer kt(s, "split_planes8");
+      unsigned char *planes = static_cast<unsigned char *>(work) + nch * frag_bytes;
+      S.ptr = planes;
+      S.step = plane8_step(S.width);
+      S.channels = 1;
+      plane8 = (size_t)S.height * S.step;
+      map = reinterpret_cast<float *>(planes + nch * plane8);
+      mstep = 4 * S.step;
+      planef = (size_t)S.height * mstep;
+      auto go = [&](auto kernel) {
+         kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(
+             static_cast<const unsigned char *>(image.ptr), S.width, S.height, image.step, planes,
+             S.step);
+      };
+      if (nch == 2) go(split_planes8<2>); else go(split_planes8<4>);
+      launch_check("split_planes8");
+   }
    if (op != kCC) {
       // the window sums of s^2 go to the map first; the MFMA kernel's epilogue reads them
       KernelTimer kt(s, "ss_box8");
@@ -1185,12 +1290,13 @@ void launch_int_mfma(hipStream_t s, int op, const View &S, const View &T, double
       const int cblks = (S.width + 63) / 64;
       const size_t lds = (size_t)th * 64 * sizeof(int);   // th <= 97: below 64 KiB
       auto go = [&](auto kernel) {
-         kernel<<<bands * cblks, 64, lds, s>>>(static_cast<const unsigned char *>(S.ptr), S.width,
-                                               S.height, S.step, tw, th,
-                                               reinterpret_cast<char *>(dst), dstep, bands);
+         kernel<<<dim3(bands * cblks, nch), 64, lds, s>>>(static_cast<const unsigned char *>(S.ptr),
+                                                         S.width, S.height, S.step, tw, th,
+                                                         reinterpret_cast<char *>(map), mstep,
+                                                         bands, plane8, planef);
       };
       const bool sgn = src8 == mfma::kSrcS8;
-      const bool bst = (long long)S.height * dstep < kBoxOob;
+      const bool bst = (long long)S.height * mstep < kBoxOob;
 #define OCIP_BOX_CASE(NCH)                                                                      \
    if (sgn) { if (bst) go(ss_box8<NCH, true, true>); else go(ss_box8<NCH, true, false>); }      \
    else { if (bst) go(ss_box8<NCH, false, true>); else go(ss_box8<NCH, false, false>); }
@@ -1207,14 +1313,20 @@ void launch_int_mfma(hipStream_t s, int op, const View &S, const View &T, double
       KernelTimer kt(s, "template_prep");
       BatchDesc d{static_cast<const char *>(T.ptr), tw, th, T.step, KC2, 1, g0, nullptr, tsums};
       d.src8 = src8;
+      d.nch = nch;
+      d.fragch = frag_bytes / sizeof(u16x8);
       mfma::launch_pair_prep<mfma::kBF16>(s, d);
    }
    const Geometry g = pair_geometry(KC2, 4, th);
    SingleLaunch L;
    L.mode = mfma::kModeInt;
    L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw, th, 1,
-                        g0, nullptr, tsums, nullptr, dst, dstep, g.vb, 0};
+                        g0, nullptr, tsums, nullptr, map, mstep, g.vb, 0};
    L.a.src8 = src8;
+   L.a.nch = nch;
+   L.a.plane8 = plane8;
+   L.a.planef = planef;
+   L.a.fragch = frag_bytes / sizeof(u16x8);
    L.a.op = op;
    // steps between the int32 flushes: each step adds one template row of products
    L.a.flush = (int)(((1LL << 24) - 1) / ((long long)tw * int_max_product(S.type)));
@@ -1223,8 +1335,19 @@ void launch_int_mfma(hipStream_t s, int op, const View &S, const View &T, double
    L.ldsp = g.ldsp;
    L.lds = g.lds;
    L.grid = dim3((S.width + 63) / 64, (S.height + mfma::kPairRows - 1) / mfma::kPairRows);
-   KernelTimer kt(s, "crosscorr_mfma_int");
-   mfma::launch_pair<mfma::kBF16>(s, L);
+   {
+      KernelTimer kt(s, "crosscorr_mfma_int");
+      mfma::launch_pair<mfma::kBF16>(s, L);
+   }
+   if (nch > 1) {
+      KernelTimer kt(s, "join_planes");
+      auto go = [&](auto kernel) {
+         kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(map, S.width, S.height, mstep, dst,
+                                                               dstep);
+      };
+      if (nch == 2) go(join_planes<2>); else go(join_planes<4>);
+      launch_check("join_planes");
+   }
 }
 
 // ======================================================================= batch

@@ -70,6 +70,10 @@ struct TileArgs {
    // kModeInt (exact sums of 8-bit integer images): element type of source and template
    // (kSrcU8 / kSrcS8), the op (ProxOp) and the steps between the int32 flushes
    int src8 = 0, op = 0, flush = 0;
+   // kModeInt: channels, the bytes from one channel's plane of the source and of the map to the
+   // next, and the 16-byte vectors from one channel's fragments to the next
+   int nch = 1;
+   size_t plane8 = 0, planef = 0, fragch = 0;
    // kF16x3: the peaks of source and template (split_range), the source's scale, the word that any
    // flagged tile sets, and the tile's flag (non-zero: prox_tile_f32_flagged computes it again)
    const unsigned *peaks = nullptr;
@@ -104,6 +108,10 @@ struct BatchDesc {
    u16x8 *frag0, *frag1;
    double *sums;
    int src8 = 0;                 // template elements: F32 (0), U8 (kSrcU8), S8 (kSrcS8)
+   // interleaved channels (8-bit templates), the one described, and the vectors from one channel's
+   // fragments to the next
+   int nch = 1, ch = 0;
+   size_t fragch = 0;
 };
 
 // 8-bit integer element types of kModeInt (their values and products are exact in BF16 and
@@ -222,7 +230,8 @@ __device__ __forceinline__ void template_sqsum(const BatchDesc &d, double *red)
       for (int i = 0; i < 16; ++i) {
          const int k = k0 + 256 * i;
          const int v = k / pitch, u = k - v * pitch;
-         t[i] = (k < total && u < d.tw) ? tmpl_elem(d.tptr + (size_t)v * d.tstep, u, d.src8) : 0.f;
+         t[i] = (k < total && u < d.tw)
+                    ? tmpl_elem(d.tptr + (size_t)v * d.tstep, u * d.nch + d.ch, d.src8) : 0.f;
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) s2 += (double)t[i] * (double)t[i];
@@ -612,7 +621,8 @@ __host__ __device__ constexpr int pair_frag_steps(int th, int nub)
 template <int P>
 __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep, int tw, int th,
                                                     int KC, int nub, int f, int lane, u16x8 *frag,
-                                                    u16x8 *frag1, int src8, float scale = 1.f)
+                                                    u16x8 *frag1, int src8, float scale = 1.f,
+                                                    int nch = 1, int ch = 0)
 {
    const int S = pair_frag_steps(th, nub);
    const int kc = f % KC, s = (f / KC) % S, ub = f / (KC * S);
@@ -625,7 +635,7 @@ __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep,
 #pragma unroll
    for (int i = 0; i < 8; ++i) {
       const int u = 16 * kc + kb + i - dx;
-      const float t = (v < th && u >= 0 && u < wb) ? tmpl_elem(trow, u0 + u, src8) : 0.f;
+      const float t = (v < th && u >= 0 && u < wb) ? tmpl_elem(trow, (u0 + u) * nch + ch, src8) : 0.f;
       unsigned short h0, h1;
       encode<P>(P == kF16x3 ? t * scale : t, h0, h1);
       h[i] = h0;
@@ -636,11 +646,14 @@ __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep,
 }
 
 // Fragments of the row-pair kernel, one per wavefront, the FP64 sum of squares (same order
-// as single_prep) in the last block, alongside.
+// as single_prep) in the last block, alongside; blockIdx.y = channel (sums[0] per channel).
 template <int P>
 __global__ __launch_bounds__(256) void pair_prep(BatchDesc d)
 {
    __shared__ double red[4];
+   d.ch = blockIdx.y;
+   d.sums += d.ch;
+   d.frag0 += d.ch * d.fragch;
    if (blockIdx.x == gridDim.x - 1) {
       template_sqsum(d, red);
       return;
@@ -649,7 +662,7 @@ __global__ __launch_bounds__(256) void pair_prep(BatchDesc d)
    const int f = blockIdx.x * 4 + (threadIdx.x >> 6);
    if (f < nfrag)
       build_pair_fragment<P>(d.tptr, d.tstep, d.tw, d.th, d.KC, d.nub, f, threadIdx.x & 63,
-                             d.frag0, d.frag1, d.src8);
+                             d.frag0, d.frag1, d.src8, 1.f, d.nch, d.ch);
 }
 
 // Batch: for template blockIdx.y, workgroups 0 .. gridDim.x - 2 build its fragments (in the
@@ -1032,11 +1045,20 @@ void crosscorr_mfma_pair(TileArgs a, int ldsp, int tiles_x, int tiles, ZImages z
 {
    extern __shared__ u16x8 lds_v[];
    const int zi = blockIdx.x / tiles;
-   const int t = xcd_tile(blockIdx.x - zi * tiles, tiles);
+   int t = xcd_tile(blockIdx.x - zi * tiles, tiles);
    if (z.n) {
       a.src = z.src[zi];
       a.dst = z.dst[zi];
       a.sstep = z.sstep[zi];
+   }
+   if constexpr (MODE == kModeInt) {
+      // channel by channel
+      const int ch = blockIdx.x / tiles;
+      t = xcd_tile(blockIdx.x - ch * tiles, tiles);
+      a.src = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.src) + ch * a.plane8);
+      a.dst = reinterpret_cast<float *>(reinterpret_cast<char *>(a.dst) + ch * a.planef);
+      a.frag0 += ch * a.fragch;
+      a.tsums += ch;
    }
    if constexpr (P == kF16x3) {
       const SplitRange sr = split_range(a.peaks, a.tw * a.th);

@@ -235,10 +235,10 @@ void noalloc_scratch_init(int device);
 void *noalloc_scratch(int device);
 
 // Exact integer sums of 8-bit images on BF16 MFMA (CrossCorr, CrossCorr_Norm, SqrDistance,
-// SqrDistance_Norm of U8/S8 1-channel images): int_mfma_ok tells whether the path takes the
-// call; tsums[0] receives sum t^2.  The maps equal prox_tile_int's bit for bit.
+// SqrDistance_Norm of U8/S8 images, every channel in one launch): int_mfma_ok tells whether the
+// path takes the call; tsums[ch] receives sum t^2.  The maps equal prox_tile_int's bit for bit.
 bool int_mfma_ok(int op, const View &src, const View &T);
-size_t int_mfma_work_bytes(int tw, int th);
+size_t int_mfma_work_bytes(const View &src, const View &T);
 void launch_int_mfma(hipStream_t s, int op, const View &src, const View &T, double *tsums,
                      float *dst, int dst_step, void *work);
 
