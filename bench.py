@@ -125,7 +125,7 @@ def fft_bench(ocip, src, steps):
         ocip.check(ocip.lib.ocipPrepareImageProximityFFT(ctypes.byref(prog), S.handle, T.handle))
         tpix = W * H * tw * th
         fn = lambda: ocip.lib.ocipCrossCorrFFT_Norm(prog, S.handle, T.handle, D.handle)
-        ms, _ = time_steps(ocip, fn, steps, 1, "fft_cols_pair")
+        ms, _ = time_steps(ocip, fn, steps, 1, "fft_cols")
         row = {"fft_value": round(tpix / (ms * 1e-3) / 1e9, 3), "fft_ms_per_step": round(ms, 3)}
         if name == "t256":
             fn2 = lambda: ocip.lib.ocipCrossCorr_NormEx(S.handle, T.handle, D.handle, 1)

@@ -815,12 +815,7 @@ static ocipError run_proximity_fft(int op, ocipProgram Program, ocipImage Source
       send_if_needed(c, S);
       send_if_needed(c, T);
       const double *integ = op == kCC ? nullptr : sqr_integral_for(c, S, 0);
-      const int tpitch = tpitch_for(T.desc.Width);
-      c.tmpl.data.ensure((size_t)tpitch * T.desc.Height * sizeof(float));
-      c.tmpl.sums.ensure(4 * sizeof(double));
-      launch_template_prep(c.stream, view(T), 0, tpitch, 0, c.tmpl.data.ptr, c.tmpl.sums.as<double>());
-      launch_proximity_fft(c.stream, p.fft, op, view(S), view(T), integ, c.tmpl.sums.as<double>(),
-                           D.dev, (int)D.desc.Step);
+      launch_proximity_fft(c.stream, p.fft, op, view(S), view(T), integ, D.dev, (int)D.desc.Step);
       D.in_device = true;
    });
 }

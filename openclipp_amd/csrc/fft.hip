@@ -12,16 +12,22 @@
 // zero border.
 //
 // This build computes in FP64 complex arithmetic (the reference uses clFFT in single
-// precision and an F32 integral) with its own mixed-radix (2, 3, 4, 5, 8, 9) Stockham FFT in LDS:
-//   pass 1 (fft_rows_pack): one workgroup per row y of the packed image z = s + i t (source
-//          and template share one complex transform), FFT along x, written transposed;
-//   pass 2 (fft_cols_pair): one workgroup per pair of spectrum columns (kx, -kx): FFT along y
-//          of both, the spectra of s and t separated by Hermitian symmetry
-//          (S = (Z(k) + conj Z(-k)) / 2, T = (Z(k) - conj Z(-k)) / 2i), the product
-//          conj(S conj T) / (Wb Hb), FFT along y again (an inverse transform of conjugated
-//          data), written transposed;
-//   pass 3 (fft_rows_epi): one workgroup per output row: FFT along x, real part (the
-//          conjugations cancel in it), the epilogue of the op, stored as float.
+// precision and an F32 integral) with its own mixed-radix (2, 3, 4, 5, 8, 9) Stockham FFT in LDS.
+// Every image is real, so only the spectrum columns kx <= Wb / 2 are formed and rows travel in
+// pairs, two real rows a, b as one complex row a + i b:
+//   pass 1 (fft_rows_pair): one workgroup per pair of rows of the source or the template, FFT
+//          along x, the two half spectra separated by Hermitian symmetry
+//          (A = (Z(k) + conj Z(-k)) / 2, B = (Z(k) - conj Z(-k)) / 2i), written transposed;
+//          rows outside the images are never formed;
+//   pass 2 (fft_cols): one workgroup per spectrum column kx: FFT along y of the template's column
+//          T, then of the source's S, the product conj(S conj T) / (Wb Hb), FFT along y again (an
+//          inverse transform of conjugated data), rows y < H written transposed;
+//   pass 3 (fft_rows_epi): one workgroup per pair of output rows: their half spectra completed
+//          (Q(-k) = conj Q(k)) and packed as Q_a + i Q_b, FFT along x, real and imaginary part the
+//          two correlation rows, the epilogue of the op, stored as float.
+// Against one complex transform of source + i template over the whole padded image: half the rows
+// in passes 1 and 3, three column transforms instead of four, half the intermediate bytes.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -31,10 +37,18 @@ namespace ocip {
 
 namespace {
 
-constexpr int kFftThreads = 1024;
 constexpr int kFftMaxStages = 24;
 // one row of complex doubles in the 160 KiB of LDS (less room for static LDS)
 constexpr int kFftMaxLen = (160 * 1024 - 256) / 16;
+constexpr int kFftThreads = 1024;
+// Workgroups of the proximity passes for transforms of up to kFftSmallLen points: 8 wavefronts, two
+// on each SIMD, with 128 registers and half a CU's LDS (lengths up to about 4600 with their
+// twiddles), so that two workgroups share a CU and one computes while the other waits at a
+// barrier or for memory.  4320 points: 278 + 110 + 118 us for the three passes at 4096^2/256x256
+// against 350 + 131 + 162 us with 10 wavefronts (640 threads, one round for a radix-8 stage), whose
+// 3 + 3 + 2 + 2 on the SIMDs leaves no room for a second workgroup.  Longer transforms take
+// kFftThreads, one workgroup per CU.
+constexpr int kFftSmallThreads = 512, kFftSmallLen = kFftMaxLen / 2;
 
 struct FftPlan {
    int n, nstages, twsize;
@@ -180,17 +194,17 @@ __device__ __forceinline__ void lds_barrier()
 // butterfly b (k = b mod span) takes x[b + j n/R], multiplies input j by w^(j k),
 // w = exp(-2 pi i / (span R)), and writes DFT output j to x[(b - k) R + k + j span].  All
 // inputs are read into registers before any output is written (one buffer).
-template <int R>
+template <int R, int THREADS, int MAXN>
 __device__ __forceinline__ void fft_stage(double2 *x, int n, int nseq, int span,
                                           const double2 *__restrict__ tw)
 {
-   constexpr int MAXB = (kFftMaxLen / R + kFftThreads - 1) / kFftThreads;
+   constexpr int MAXB = (MAXN / R + THREADS - 1) / THREADS;
    const int m = n / R, total = m * nseq;
    const float rm = 1.0f / (float)m, rs = 1.0f / (float)span;
    double2 u[MAXB][R];
 #pragma unroll
    for (int q = 0; q < MAXB; ++q) {
-      const int g = threadIdx.x + q * kFftThreads;
+      const int g = threadIdx.x + q * THREADS;
       if (g < total) {
          int b, k;
          const int seq = nseq == 1 ? (b = g, 0) : div_small(g, m, rm, b);
@@ -213,7 +227,7 @@ __device__ __forceinline__ void fft_stage(double2 *x, int n, int nseq, int span,
    lds_barrier();
 #pragma unroll
    for (int q = 0; q < MAXB; ++q) {
-      const int g = threadIdx.x + q * kFftThreads;
+      const int g = threadIdx.x + q * THREADS;
       if (g < total) {
          int b, k;
          const int seq = nseq == 1 ? (b = g, 0) : div_small(g, m, rm, b);
@@ -228,9 +242,8 @@ __device__ __forceinline__ void fft_stage(double2 *x, int n, int nseq, int span,
 
 // Forward FFT (unnormalised) of nseq sequences of length P.n in LDS, natural order in and out;
 // tw: the plan's twiddles, in LDS.
-// LARGE: the plan may hold radix-8 and radix-9 stages (row plans only: the column kernels,
-// which hold two columns, have no registers to spare for them)
-template <bool LARGE = false>
+// LARGE: the plan may hold radix-8 and radix-9 stages.  THREADS threads, at most MAXN points in all.
+template <bool LARGE = false, int THREADS = kFftThreads, int MAXN = kFftMaxLen>
 __device__ __forceinline__ void lds_fft(double2 *x, int nseq, const FftPlan *__restrict__ P, const double2 *tw)
 {
    const int n = P->n, ns = P->nstages;
@@ -238,137 +251,232 @@ __device__ __forceinline__ void lds_fft(double2 *x, int nseq, const FftPlan *__r
       const double2 *t = tw + P->twoff[s];
       const int span = P->span[s];
       switch (P->radix[s]) {
-      case 2: fft_stage<2>(x, n, nseq, span, t); break;
-      case 3: fft_stage<3>(x, n, nseq, span, t); break;
-      case 4: fft_stage<4>(x, n, nseq, span, t); break;
+      case 2: fft_stage<2, THREADS, MAXN>(x, n, nseq, span, t); break;
+      case 3: fft_stage<3, THREADS, MAXN>(x, n, nseq, span, t); break;
+      case 4: fft_stage<4, THREADS, MAXN>(x, n, nseq, span, t); break;
       case 8:
-         if constexpr (LARGE) fft_stage<8>(x, n, nseq, span, t);
+         if constexpr (LARGE) fft_stage<8, THREADS, MAXN>(x, n, nseq, span, t);
          break;
       case 9:
-         if constexpr (LARGE) fft_stage<9>(x, n, nseq, span, t);
+         if constexpr (LARGE) fft_stage<9, THREADS, MAXN>(x, n, nseq, span, t);
          break;
-      default: fft_stage<5>(x, n, nseq, span, t); break;
+      default: fft_stage<5, THREADS, MAXN>(x, n, nseq, span, t); break;
       }
    }
 }
 
 
-// One workgroup per row (passes 1 and 3) or column pair (pass 2).  Passes 1 and 2 take their
-// rows in XCD-aware order (xcd_tile): the workgroups of one XCD take consecutive rows, so the
-// transposed 16-byte stores of neighbouring rows fill the same lines of that XCD's L2.
+// Pitch of the transposed half spectra of h rows: whole 128-byte lines, and one more so that the
+// columns of a power-of-two height do not meet in the same cache sets and channels (pass 1 at 4096^2: 161 -> 156 us).
+__host__ __device__ constexpr int spectrum_pitch(int h) { return (h + 7) / 8 * 8 + 8; }
 
-// Pass 1: row y of z = s + i t (s at (tw/2, th/2), t at (0, 0), zero elsewhere), FFT along
-// x, stored transposed: out[kx * Hb + y].
-__global__ __launch_bounds__(kFftThreads) void fft_rows_pack(const char *__restrict__ S, int W,
-                                                             int H, int sstep,
-                                                             const char *__restrict__ T, int tw,
-                                                             int th, int tstep, int Hb,
-                                                             const FftPlan *__restrict__ pw,
-                                                             const double2 *__restrict__ tww,
-                                                             double2 *__restrict__ out)
-{
-   extern __shared__ double2 fbuf[];
-   const int Wb = pw->n, cx = tw / 2;
-   const int y = xcd_tile(blockIdx.x, gridDim.x);
-   double2 *ltw = fbuf + Wb;
-   for (int i = threadIdx.x; i < pw->twsize; i += kFftThreads) ltw[i] = tww[i];
-   const int sy = y - th / 2;
-   const bool srow = sy >= 0 && sy < H, trow = y < th;
-   const float *sr = reinterpret_cast<const float *>(S + (size_t)(srow ? sy : 0) * sstep);
-   const float *tr = reinterpret_cast<const float *>(T + (size_t)(trow ? y : 0) * tstep);
-   for (int x = threadIdx.x; x < Wb; x += kFftThreads) {
-      const int sx = x - cx;
-      const double sv = (srow && sx >= 0 && sx < W) ? (double)sr[sx] : 0.0;
-      const double tv = (trow && x < tw) ? (double)tr[x] : 0.0;
-      fbuf[x] = make_double2(sv, tv);
-   }
-   lds_barrier();
-   lds_fft<true>(fbuf, 1, pw, ltw);
-   for (int x = threadIdx.x; x < Wb; x += kFftThreads) out[(size_t)x * Hb + y] = fbuf[x];
-}
+// Passes 1 and 2 take their work in XCD-aware order (xcd_tile): the workgroups of one XCD take
+// consecutive row pairs or columns, so the transposed stores of neighbours fill the same lines
+// of that XCD's L2.
+template <bool SMALL> struct FftShape {
+   static constexpr int threads = SMALL ? kFftSmallThreads : kFftThreads;
+   static constexpr int maxn = SMALL ? kFftSmallLen : kFftMaxLen;
+};
+// (both shapes come to four wavefronts per SIMD)
+#define OCIP_FFT_BOUNDS(SMALL) \
+   __launch_bounds__(FftShape<SMALL>::threads) \
+       __attribute__((amdgpu_waves_per_eu(4, 4)))
 
-// Spectrum product at k from Z(k) = z1 and Z(-k) = z2, conjugated for the inverse transform.
-__device__ __forceinline__ double2 spectrum_product(double2 z1, double2 z2, double scale)
+// Pass 1: rows 2 j, 2 j + 1 of the source (j < (H + 1) / 2, at x = tw/2 of the padded row) or,
+// after those, of the template (at x = 0), zero elsewhere, FFT along x, both half spectra stored
+// transposed: outs[kx * spectrum_pitch(H) + y], outt likewise (32 bytes a column).  The
+// template's pairs also leave their FP64 sum of t^2 in tpart.
+template <bool SMALL>
+__global__ OCIP_FFT_BOUNDS(SMALL) void fft_rows_pair(const char *__restrict__ S, int W, int H,
+                                                     int sstep, const char *__restrict__ T, int tw,
+                                                     int th, int tstep,
+                                                     const FftPlan *__restrict__ pw,
+                                                     const double2 *__restrict__ tww,
+                                                     double2 *__restrict__ outs,
+                                                     double2 *__restrict__ outt,
+                                                     double *__restrict__ tpart)
 {
-   const double2 s = cscale(cadd(z1, cconj(z2)), 0.5);           // FFT of the source
-   const double2 t = cscale(mul_mi(csub(z1, cconj(z2))), 0.5);   // FFT of the template
-   return cconj(cscale(cmul(s, cconj(t)), scale));
-}
-
-// Pass 2: spectrum columns kx and Wb - kx (rows of the transposed array), kx = 0..Wb/2: FFT
-// along y, product, FFT along y again; stored transposed (rows y < H only): out[y * Wb + kx].
-__global__ __launch_bounds__(kFftThreads) void fft_cols_pair(const double2 *__restrict__ in, int Wb,
-                                                             int H, const FftPlan *__restrict__ ph,
-                                                             const double2 *__restrict__ twh,
-                                                             double scale,
-                                                             double2 *__restrict__ out)
-{
-   extern __shared__ double2 fbuf[];
-   const int Hb = ph->n;
-   double2 *ltw = fbuf + 2 * Hb;
-   for (int i = threadIdx.x; i < ph->twsize; i += kFftThreads) ltw[i] = twh[i];
-   {
-      const int kx = xcd_tile(blockIdx.x, gridDim.x);
-      const int kx2 = (Wb - kx) % Wb;
-      const int nseq = kx2 == kx ? 1 : 2;
-      double2 *A = fbuf, *B = nseq == 2 ? fbuf + Hb : fbuf;
-      for (int y = threadIdx.x; y < Hb; y += kFftThreads) {
-         A[y] = in[(size_t)kx * Hb + y];
-         if (nseq == 2) B[y] = in[(size_t)kx2 * Hb + y];
-      }
-      lds_barrier();
-      lds_fft(fbuf, nseq, ph, ltw);
-      // the four entries of a pair (ky, -ky) of both columns are read and written by one thread
-      for (int ky = threadIdx.x; ky <= Hb / 2; ky += kFftThreads) {
-         const int ky2 = ky == 0 ? 0 : Hb - ky;
-         const double2 a1 = A[ky], a2 = A[ky2], b1 = B[ky], b2 = B[ky2];
-         A[ky] = spectrum_product(a1, b2, scale);
-         A[ky2] = spectrum_product(a2, b1, scale);
-         if (nseq == 2) {
-            B[ky] = spectrum_product(b1, a2, scale);
-            B[ky2] = spectrum_product(b2, a1, scale);
-         }
-      }
-      lds_barrier();
-      lds_fft(fbuf, nseq, ph, ltw);
-      for (int y = threadIdx.x; y < H; y += kFftThreads) {
-         out[(size_t)y * Wb + kx] = A[y];
-         if (nseq == 2) out[(size_t)y * Wb + kx2] = B[y];
-      }
-   }
-}
-
-// Pass 3: output row y < H: FFT along x, real part = the correlation, the op's epilogue
-// (ImageProximityFFT.cl:86-147, in FP64 with SS from the FP64 integral).
-__global__ __launch_bounds__(kFftThreads) void fft_rows_epi(const double2 *__restrict__ in, int W,
-                                                            int H, const FftPlan *__restrict__ pw,
-                                                            const double2 *__restrict__ tww,
-                                                            int op, int tw, int th,
-                                                            const double *__restrict__ integ,
-                                                            const double *__restrict__ tsums,
-                                                            char *__restrict__ dst, int dstep)
-{
+   constexpr int THREADS = FftShape<SMALL>::threads;
    extern __shared__ double2 fbuf[];
    const int Wb = pw->n;
    double2 *ltw = fbuf + Wb;
-   for (int i = threadIdx.x; i < pw->twsize; i += kFftThreads) ltw[i] = tww[i];
-   const double tt = op == kCC ? 0.0 : tsums[0];
-   {
-      const int y = blockIdx.x;
-      for (int x = threadIdx.x; x < Wb; x += kFftThreads) fbuf[x] = in[(size_t)y * Wb + x];
+   for (int i = threadIdx.x; i < pw->twsize; i += THREADS) ltw[i] = tww[i];
+   const int pairs = (H + 1) / 2, g = xcd_tile(blockIdx.x, gridDim.x);
+   const bool tpl = g >= pairs;
+   const int y = 2 * (tpl ? g - pairs : g);
+   const int w = tpl ? tw : W, h = tpl ? th : H, x0 = tpl ? 0 : tw / 2;
+   const char *base = (tpl ? T : S) + (size_t)y * (tpl ? tstep : sstep);
+   const float *ra = reinterpret_cast<const float *>(base);
+   const bool two = y + 1 < h;   // (a row alone is read twice and counted once)
+   const float *rb = two ? reinterpret_cast<const float *>(base + (tpl ? tstep : sstep)) : ra;
+   // E elements a thread in flight (unconditional loads, from column 0 outside the row)
+   constexpr int E = 4;
+   double t2 = 0.0;
+#pragma unroll 1
+   for (int xb = threadIdx.x; xb < Wb; xb += E * THREADS) {
+      float va[E], vb[E];
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+         const int sx = xb + i * THREADS - x0;
+         const int c = sx >= 0 && sx < w ? sx : 0;
+         va[i] = ra[c];
+         vb[i] = rb[c];
+      }
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+         const int x = xb + i * THREADS, sx = x - x0;
+         const bool in = sx >= 0 && sx < w;
+         const double a = in ? (double)va[i] : 0.0, b = in && two ? (double)vb[i] : 0.0;
+         if (x < Wb) fbuf[x] = make_double2(a, b);
+         t2 += a * a + b * b;
+      }
+   }
+   lds_barrier();
+   lds_fft<true, THREADS, FftShape<SMALL>::maxn>(fbuf, 1, pw, ltw);
+   const int hp = spectrum_pitch(h);
+   double2 *out = (tpl ? outt : outs) + y;
+   for (int k = threadIdx.x; k <= Wb / 2; k += THREADS) {
+      const double2 z = fbuf[k], zc = cconj(fbuf[k == 0 ? 0 : Wb - k]);
+      double2 *o = out + (size_t)k * hp;
+      o[0] = cscale(cadd(z, zc), 0.5);
+      o[1] = cscale(mul_mi(csub(z, zc)), 0.5);
+   }
+   if (tpl) {
+      // the twiddles are not read any more: their LDS takes the waves' sums
+      double *red = reinterpret_cast<double *>(fbuf + Wb);
+      t2 = wave_sum(t2);
       lds_barrier();
-      lds_fft<true>(fbuf, 1, pw, ltw);
-      float *drow = reinterpret_cast<float *>(dst + (size_t)y * dstep);
-      for (int x = threadIdx.x; x < W; x += kFftThreads) {
-         const double cc = fbuf[x].x;
-         double v = cc;
-         if (op != kCC) {
-            const double ss = window_sqsum(integ, W, H, x, y, tw, th);
-            if (op == kCCNorm) v = cc / sqrt(ss * tt);
-            else if (op == kSSD) v = ss - 2.0 * cc + tt;
-            else v = (ss - 2.0 * cc + tt) / sqrt(ss * tt);
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t2;
+      lds_barrier();
+      if (threadIdx.x == 0) {
+         t2 = 0.0;
+         for (int i = 0; i < THREADS / 64; ++i) t2 += red[i];
+         tpart[g - pairs] = t2;
+      }
+   }
+}
+
+// Pass 2: spectrum column kx <= Wb / 2: FFT along y of the template's column (at y = 0) and of the
+// source's (at y = th/2), the conjugated product, FFT along y again; rows y < H stored
+// transposed: out[y * half + kx].  One column in LDS at a time, the template's spectrum in
+// registers meanwhile.
+template <bool SMALL>
+__global__ OCIP_FFT_BOUNDS(SMALL) void fft_cols(const double2 *__restrict__ ins,
+                                                const double2 *__restrict__ inT, int half, int H,
+                                                int th, const FftPlan *__restrict__ ph,
+                                                const double2 *__restrict__ twh, double scale,
+                                                double2 *__restrict__ out)
+{
+   constexpr int THREADS = FftShape<SMALL>::threads, MAXN = FftShape<SMALL>::maxn;
+   constexpr int PER = (kFftSmallLen + THREADS - 1) / THREADS;   // Hb <= kFftSmallLen (fft_sizes)
+   extern __shared__ double2 fbuf[];
+   const int Hb = ph->n, kx = xcd_tile(blockIdx.x, gridDim.x), cy = th / 2;
+   double2 *ltw = fbuf + Hb;
+   for (int i = threadIdx.x; i < ph->twsize; i += THREADS) ltw[i] = twh[i];
+   const double2 *tc = inT + (size_t)kx * spectrum_pitch(th);
+   const double2 *sc = ins + (size_t)kx * spectrum_pitch(H);
+   const double2 zero = make_double2(0.0, 0.0);
+   for (int y = threadIdx.x; y < Hb; y += THREADS) fbuf[y] = y < th ? tc[y] : zero;
+   lds_barrier();
+   lds_fft<true, THREADS, MAXN>(fbuf, 1, ph, ltw);
+   double2 t[PER];
+#pragma unroll
+   for (int i = 0; i < PER; ++i) {
+      const int y = threadIdx.x + i * THREADS;
+      if (y < Hb) {
+         t[i] = fbuf[y];
+         fbuf[y] = y >= cy && y < H + cy ? sc[y - cy] : zero;   // (its own entry)
+      }
+   }
+   lds_barrier();
+   lds_fft<true, THREADS, MAXN>(fbuf, 1, ph, ltw);
+#pragma unroll
+   for (int i = 0; i < PER; ++i) {
+      const int y = threadIdx.x + i * THREADS;
+      if (y < Hb) fbuf[y] = cconj(cscale(cmul(fbuf[y], cconj(t[i])), scale));
+   }
+   lds_barrier();
+   lds_fft<true, THREADS, MAXN>(fbuf, 1, ph, ltw);
+   for (int y = threadIdx.x; y < H; y += THREADS) out[(size_t)y * half + kx] = fbuf[y];
+}
+
+// Pass 3: output rows 2 j and 2 j + 1: FFT along x of Q_a + i Q_b = the two correlation rows, the
+// op's epilogue (ImageProximityFFT.cl:86-147, in FP64 with SS from the FP64 integral and
+// TT = the sum of the ntpart sums of tpart).
+template <bool SMALL>
+__global__ OCIP_FFT_BOUNDS(SMALL) void fft_rows_epi(const double2 *__restrict__ in, int half, int W,
+                                                    int H, const FftPlan *__restrict__ pw,
+                                                    const double2 *__restrict__ tww, int op, int tw,
+                                                    int th, const double *__restrict__ integ,
+                                                    const double *__restrict__ tpart, int ntpart,
+                                                    char *__restrict__ dst, int dstep)
+{
+   constexpr int THREADS = FftShape<SMALL>::threads;
+   extern __shared__ double2 fbuf[];
+   const int Wb = pw->n, y = 2 * blockIdx.x;
+   const bool two = y + 1 < H;
+   double2 *ltw = fbuf + Wb;
+   for (int i = threadIdx.x; i < pw->twsize; i += THREADS) ltw[i] = tww[i];
+   const double2 *qa = in + (size_t)y * half, *qb = two ? qa + half : qa;
+   {
+      constexpr int PER = (FftShape<SMALL>::maxn / 2 + THREADS) / THREADS;
+      double2 a[PER], b[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+         const int k = min((int)threadIdx.x + i * THREADS, half - 1);
+         a[i] = qa[k];
+         b[i] = qb[k];
+      }
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+         const int k = threadIdx.x + i * THREADS;
+         if (k >= half) break;
+         fbuf[k] = cadd(a[i], mul_pi(b[i]));
+         if (k > 0 && k < Wb - k) fbuf[Wb - k] = cadd(cconj(a[i]), mul_pi(cconj(b[i])));
+      }
+   }
+   lds_barrier();
+   lds_fft<true, THREADS, FftShape<SMALL>::maxn>(fbuf, 1, pw, ltw);
+   double tt = 0.0;
+   if (op != kCC) {
+      // every wavefront sums the parts alike
+      for (int i = threadIdx.x & 63; i < ntpart; i += 64) tt += tpart[i];
+      tt = wave_sum(tt);
+   }
+   float *da = reinterpret_cast<float *>(dst + (size_t)y * dstep);
+   float *db = reinterpret_cast<float *>(dst + (size_t)(two ? y + 1 : y) * dstep);
+   if (op == kCC) {
+      for (int x = threadIdx.x; x < W; x += THREADS) {
+         const double2 c = fbuf[x];
+         da[x] = (float)c.x;
+         if (two) db[x] = (float)c.y;
+      }
+      return;
+   }
+   // E columns' window sums at a time: all their integral corners in flight
+   constexpr int E = 2;
+   for (int x0 = threadIdx.x; x0 < W; x0 += E * THREADS) {
+      double ss[E][2];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+         const int x = min(x0 + e * THREADS, W - 1);
+         ss[e][0] = window_sqsum(integ, W, H, x, y, tw, th);
+         ss[e][1] = window_sqsum(integ, W, H, x, y + 1, tw, th);
+      }
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+         const int x = x0 + e * THREADS;
+         if (x >= W) break;
+         const double2 c = fbuf[x];
+         const double cc[2] = {c.x, c.y};
+         float v[2];
+#pragma unroll
+         for (int r = 0; r < 2; ++r) {
+            const double d = op == kCCNorm ? cc[r] : ss[e][r] - 2.0 * cc[r] + tt;
+            v[r] = (float)(op == kSSD ? d : d * rsqrt64(ss[e][r] * tt));
          }
-         drow[x] = (float)v;
+         da[x] = v[0];
+         if (two) db[x] = v[1];
       }
    }
 }
@@ -519,8 +627,9 @@ void make_plan(int n, FftPlan &p, std::vector<double2> &table, bool large)
    p.twsize = (int)table.size() - base;
 }
 
-// LDS of the three passes: data plus the plan's twiddles, in complex doubles
-size_t row_lds(const FftPlan &p) { return (size_t)(p.n + p.twsize) * sizeof(double2); }
+// LDS of a pass: data plus the plan's twiddles, in complex doubles (at least the waves' sums of
+// fft_rows_pair); pair_lds: two columns (the path's limit on the padded height)
+size_t row_lds(const FftPlan &p) { return (size_t)(p.n + std::max(p.twsize, 8)) * sizeof(double2); }
 size_t pair_lds(const FftPlan &p) { return (size_t)(2 * p.n + p.twsize) * sizeof(double2); }
 
 }  // namespace
@@ -544,13 +653,15 @@ int fft_padded_length(int n)
 struct FftState {
    int Wb = 0, Hb = 0, hbase = 0;   // hbase: first twiddle of the height plan
    FftPlan pw{}, ph{};
-   DevBuf twid, plans, a, b;   // plans: pw and ph, read by the kernels
+   DevBuf twid, plans, a, b, t, tpart;   // plans: pw and ph, read by the kernels
    ~FftState()
    {
       twid.release();
       plans.release();
       a.release();
       b.release();
+      t.release();
+      tpart.release();
    }
 };
 
@@ -584,7 +695,7 @@ void fft_prepare(hipStream_t s, FftState *st, int W, int H, int tw, int th)
    std::vector<double2> table;  // the width plan's twiddles, then the height plan's
    make_plan(Wb, st->pw, table, true);
    st->hbase = (int)table.size();
-   make_plan(Hb, st->ph, table, false);
+   make_plan(Hb, st->ph, table, true);
    st->twid.ensure(table.size() * sizeof(double2));
    hip_check(hipMemcpyAsync(st->twid.ptr, table.data(), table.size() * sizeof(double2),
                             hipMemcpyHostToDevice, s), "twiddles");
@@ -592,15 +703,22 @@ void fft_prepare(hipStream_t s, FftState *st, int W, int H, int tw, int th)
    st->plans.ensure(sizeof(both));
    hip_check(hipMemcpyAsync(st->plans.ptr, both, sizeof(both), hipMemcpyHostToDevice, s), "plans");
    hip_check(hipStreamSynchronize(s), "twiddles");
-   st->a.ensure((size_t)Wb * Hb * sizeof(double2));
-   st->b.ensure((size_t)Wb * Hb * sizeof(double2));
+   // half spectra of the source's and the template's rows (transposed) and of the map's rows, for
+   // any image and template of this padded size
+   const size_t half = Wb / 2 + 1;
+   st->a.ensure(half * spectrum_pitch(Hb) * sizeof(double2));
+   st->b.ensure(half * Hb * sizeof(double2));
+   st->t.ensure(half * spectrum_pitch(Hb) * sizeof(double2));
+   st->tpart.ensure((size_t)((Hb + 1) / 2) * sizeof(double));
    st->Wb = Wb;
    st->Hb = Hb;
    static bool lds_set = false;
    if (!lds_set) {
-      for (const void *k : {reinterpret_cast<const void *>(fft_rows_pack),
-                            reinterpret_cast<const void *>(fft_cols_pair),
-                            reinterpret_cast<const void *>(fft_rows_epi)})
+      for (const void *k : {reinterpret_cast<const void *>(fft_rows_pair<true>),
+                            reinterpret_cast<const void *>(fft_rows_pair<false>),
+                            reinterpret_cast<const void *>(fft_cols<true>),
+                            reinterpret_cast<const void *>(fft_rows_epi<true>),
+                            reinterpret_cast<const void *>(fft_rows_epi<false>)})
          hip_check(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        kFftMaxLen * (int)sizeof(double2)),
                    "lds attribute");
@@ -609,31 +727,42 @@ void fft_prepare(hipStream_t s, FftState *st, int W, int H, int tw, int th)
 }
 
 void launch_proximity_fft(hipStream_t s, FftState *st, int op, const View &S, const View &T,
-                          const double *integ, const double *tsums, void *dst, int dstep)
+                          const double *integ, void *dst, int dstep)
 {
    fft_prepare(s, st, S.width, S.height, T.width, T.height);
-   const int Wb = st->Wb, Hb = st->Hb;
+   const int Wb = st->Wb, Hb = st->Hb, half = Wb / 2 + 1;
    const double2 *tww = static_cast<const double2 *>(st->twid.ptr), *twh = tww + st->hbase;
    double2 *a = static_cast<double2 *>(st->a.ptr), *b = static_cast<double2 *>(st->b.ptr);
+   double2 *t = static_cast<double2 *>(st->t.ptr);
+   double *tpart = static_cast<double *>(st->tpart.ptr);
    const FftPlan *plans = static_cast<const FftPlan *>(st->plans.ptr);
+   const int spairs = (S.height + 1) / 2, tpairs = (T.height + 1) / 2;
+   const bool small = Wb <= kFftSmallLen;
+   const int threads = small ? kFftSmallThreads : kFftThreads;
    {
-      KernelTimer kt(s, "fft_rows_pack");
-      fft_rows_pack<<<Hb, kFftThreads, row_lds(st->pw), s>>>(
-          static_cast<const char *>(S.ptr), S.width, S.height, S.step,
-          static_cast<const char *>(T.ptr), T.width, T.height, T.step, Hb, plans, tww, a);
-      launch_check("fft_rows_pack");
+      KernelTimer kt(s, "fft_rows_pair");
+      auto go = [&](auto kernel) {
+         kernel<<<spairs + tpairs, threads, row_lds(st->pw), s>>>(
+             static_cast<const char *>(S.ptr), S.width, S.height, S.step,
+             static_cast<const char *>(T.ptr), T.width, T.height, T.step, plans, tww, a, t, tpart);
+      };
+      if (small) go(fft_rows_pair<true>); else go(fft_rows_pair<false>);
+      launch_check("fft_rows_pair");
    }
    {
-      KernelTimer kt(s, "fft_cols_pair");
-      fft_cols_pair<<<Wb / 2 + 1, kFftThreads, pair_lds(st->ph), s>>>(
-          a, Wb, S.height, plans + 1, twh, 1.0 / ((double)Wb * Hb), b);
-      launch_check("fft_cols_pair");
+      KernelTimer kt(s, "fft_cols");
+      fft_cols<true><<<half, kFftSmallThreads, row_lds(st->ph), s>>>(
+          a, t, half, S.height, T.height, plans + 1, twh, 1.0 / ((double)Wb * Hb), b);
+      launch_check("fft_cols");
    }
    {
       KernelTimer kt(s, "fft_rows_epi");
-      fft_rows_epi<<<S.height, kFftThreads, row_lds(st->pw), s>>>(
-          b, S.width, S.height, plans, tww, op, T.width, T.height, integ, tsums,
-          static_cast<char *>(dst), dstep);
+      auto go = [&](auto kernel) {
+         kernel<<<spairs, threads, row_lds(st->pw), s>>>(
+             b, half, S.width, S.height, plans, tww, op, T.width, T.height, integ, tpart, tpairs,
+             static_cast<char *>(dst), dstep);
+      };
+      if (small) go(fft_rows_epi<true>); else go(fft_rows_epi<false>);
       launch_check("fft_rows_epi");
    }
 }

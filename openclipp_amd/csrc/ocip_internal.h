@@ -262,12 +262,12 @@ void launch_backward_batch(hipStream_t s, int n, const View *S, const View *G1, 
 
 // Proximity through 2-D FFTs (FP64): op kSSD, kSSDNorm, kCC or kCCNorm on an F32 1-channel
 // source and template into an F32 dest.  integ: the exclusive FP64 sum-of-squares integral
-// (all ops but kCC); tsums[0] = sum t^2.  fft_sizes gives the padded transform size or
+// (all ops but kCC).  fft_sizes gives the padded transform size or
 // CL_INVALID_IMAGE_SIZE when the image is too big for the path.
 cl_int fft_sizes(int W, int H, int tw, int th, int *Wb, int *Hb);
 void fft_prepare(hipStream_t s, FftState *st, int W, int H, int tw, int th);
 void launch_proximity_fft(hipStream_t s, FftState *st, int op, const View &S, const View &T,
-                          const double *integ, const double *tsums, void *dst, int dstep);
+                          const double *integ, void *dst, int dstep);
 
 // Generic 2-D FFT (F32 or F64): forward real W x H -> half spectrum (W/2 + 1) x H of
 // interleaved complex values, inverse back, unnormalised.  fft_plain_sizes: CL_SUCCESS or
