@@ -361,6 +361,12 @@ __global__ __launch_bounds__(kThreads) void weight_corr(const char *M, int mstep
 constexpr int kTgRows = 32, kTgCols = 128;
 constexpr int kTgPRows = kTgRows + 31;       // staged source rows
 constexpr int kTgMCols = kTgCols + 32;       // staged map columns (31 to the left, 1 spare)
+// LDS pitch of the source rows: an odd multiple of 16 bytes, so that the 16-byte A reads of 8
+// consecutive rows fall on distinct banks (at a pitch of 256 bytes all of them met in one
+// group: 300 -> 145 us for 16 x 1024^2 with 31x31); map copies half the banks apart, so that the even lanes' B reads from
+// one copy and the odd lanes' from the other do not meet
+constexpr int kTgPPitch = kTgCols + 8;
+constexpr int kTgMCopy = kTgRows * kTgMCols + 64;
 
 typedef __bf16 tg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float tg_f32x16 __attribute__((ext_vector_type(16)));
@@ -393,8 +399,8 @@ __global__ __launch_bounds__(256) void tgrad_mfma(const char *Ms, int mstep, siz
    float *partial = partials + blockIdx.y * pzstride;
    // planes: source hi, source lo (kTgPRows x kTgCols); map hi, lo, each in two copies
    // (kTgRows x kTgMCols)
-   __shared__ unsigned short ps[2][kTgPRows * kTgCols];
-   __shared__ unsigned short ms[2][2][kTgRows * kTgMCols];
+   __shared__ __attribute__((aligned(16))) unsigned short ps[2][kTgPRows * kTgPPitch];
+   __shared__ __attribute__((aligned(16))) unsigned short ms[2][2][kTgMCopy];
    const int cx = tw / 2, cy = th / 2;
    const int tx = blockIdx.x % tasks_x, ty = blockIdx.x / tasks_x;
    const int xb = tx * kTgCols, y0 = ty * kTgRows;
@@ -429,9 +435,10 @@ __global__ __launch_bounds__(256) void tgrad_mfma(const char *Ms, int mstep, siz
    for (int it = 0; it < kPIt; ++it) {
       const int k = threadIdx.x + 256 * it;
       if (k >= kTgPRows * kTgCols) break;
+      const int at = k + 8 * (k / kTgCols);   // row k / kTgCols at the pitch
       const unsigned short h = tg_hi(pf[it]);
-      ps[0][k] = h;
-      ps[1][k] = tg_lo(pf[it], h);
+      ps[0][at] = h;
+      ps[1][at] = tg_lo(pf[it], h);
    }
 #pragma unroll
    for (int it = 0; it < kMIt; ++it) {
@@ -452,8 +459,8 @@ __global__ __launch_bounds__(256) void tgrad_mfma(const char *Ms, int mstep, siz
    for (int r = wave; r < kTgRows; r += 4) {
       if (y0 + r >= H) break;
       // A: source row (task row r + m), columns 16 kb + 8 g .. + 7
-      const unsigned short *ah = &ps[0][(r + mn) * kTgCols + 8 * g];
-      const unsigned short *al = &ps[1][(r + mn) * kTgCols + 8 * g];
+      const unsigned short *ah = &ps[0][(r + mn) * kTgPPitch + 8 * g];
+      const unsigned short *al = &ps[1][(r + mn) * kTgPPitch + 8 * g];
 #pragma unroll 2
       for (int kb = 0; kb < kTgCols / 16; ++kb) {
          if (xb + 16 * kb >= W) break;
