@@ -15,6 +15,8 @@
 //   3. final     : per tile, the in-tile 2-D scan (a running column sum per lane and one
 //                  wavefront scan per row) plus the three carries.
 // HBM traffic: 2 x source + 1 x output (+ small aggregates).
+#include <type_traits>
+
 #include "device_common.h"
 
 namespace ocip {
@@ -53,84 +55,110 @@ IntegralAux aux_layout(void *base, int W, int H)
    return a;
 }
 
-template <class T> struct alignas(4 * sizeof(T)) Vec4 {
+// Four elements read or written at once, at the element's own alignment (see f32x4_u)
+template <class T> struct __attribute__((packed, aligned(alignof(T)))) Vec4 {
    T v[4];
 };
 
-// f(s) for the lane's 4 columns of row y (0 outside [0, y1) x [0, W)).  VEC: 1-channel rows
-// whose 4-element groups are aligned, read with one vector load.
-template <int TYPE, bool SQR, bool VEC>
-__device__ __forceinline__ void load_row(const char *src, int step, int y, int y1, int x0, int W,
-                                         int nch, int ch, double (&v)[kVec])
+// The lane's 4 elements of a row as loaded, unconditionally, so that many rows can be in flight in
+// ragged tiles too: rows from y1 on read the row before, columns from W on the last ones inside
+// (VEC: 1-channel rows of at least 4 elements, one vector load at column min(x0, W - 4)).
+template <int TYPE, bool VEC>
+__device__ __forceinline__ Vec4<typename ElemT<TYPE>::type>
+load_raw(const char *src, int step, int y, int y1, int x0, int W, int nch, int ch)
 {
    typedef typename ElemT<TYPE>::type T;
-   const char *row = src + (size_t)(y < y1 ? y : 0) * step;
-   if (VEC && y < y1 && x0 + kVec <= W) {
-      const Vec4<T> q = *reinterpret_cast<const Vec4<T> *>(row + (size_t)x0 * sizeof(T));
+   const char *row = src + (size_t)min(y, y1 - 1) * step;
+   if (VEC) return *reinterpret_cast<const Vec4<T> *>(row + (size_t)min(x0, W - 4) * sizeof(T));
+   Vec4<T> q;
 #pragma unroll
-      for (int j = 0; j < kVec; ++j) {
-         const double f = (double)q.v[j];
-         v[j] = SQR ? f * f : f;
-      }
-      return;
-   }
+   for (int j = 0; j < kVec; ++j) q.v[j] = ld<TYPE>(row, min(x0 + j, W - 1) * nch + ch);
+   return q;
+}
+
+// f(s) for the lane's 4 columns of row y from load_raw's elements, 0 outside [0, y1) x [0, W).
+// WHOLE: the tile lies inside the image.
+template <bool WHOLE, bool SQR, bool VEC, class A, class T>
+__device__ __forceinline__ void values(const Vec4<T> &q, int y, int y1, int x0, int W, A (&v)[kVec])
+{
+   const int d = VEC && !WHOLE ? x0 - min(x0, W - 4) : 0;   // the vector starts d columns early
 #pragma unroll
    for (int j = 0; j < kVec; ++j) {
-      const int x = x0 + j;
-      const double f = (y < y1 && x < W) ? (double)ld<TYPE>(row, x * nch + ch) : 0.0;
+      T e = q.v[j];
+      if (!WHOLE) {
+#pragma unroll
+         for (int k = j + 1; k < kVec; ++k)
+            if (d == k - j) e = q.v[k];
+         if (y >= y1 || x0 + j >= W) e = (T)0;
+      }
+      const A f = (A)e;
       v[j] = SQR ? f * f : f;
    }
 }
 
+// body(whole) with whole = std::true_type for tiles wholly inside the image, false_type for others
+template <class F> __device__ __forceinline__ void by_tile(int cb, int rb, int W, int H, F &&body)
+{
+   if ((cb + 1) * kCW <= W && (rb + 1) * kRH <= H) body(std::true_type());
+   else body(std::false_type());
+}
+
 // 1. per-tile aggregates: column sums, row sums, tile total (and the tile's peak where the
-// caller wants the image's: f >= 0 then)
+// caller wants the image's: f >= 0 then).  Bound by memory latency: kAggRows rows of raw elements
+// are in flight per lane and converted afterwards, 8-bit images are summed in int32 (a tile's
+// column holds at most 32 x 255^2), and two lanes share each row's sum (U8 4096^2: 16 -> 7 us,
+// F32: 17 -> 15 us; rows of odd pitch took one load per element before: 3001x2003 F32 66 -> 29 us for
+// all three launches).
+constexpr int kAggRows = 16;
+
 template <int TYPE, bool SQR, bool VEC, bool PEAK>
 __global__ __launch_bounds__(kThreads) void integral_aggregate(const char *src, int W, int H,
                                                                 int step, int nch, int ch,
                                                                 IntegralAux aux)
 {
-   // each lane's partial row sums, rows x lanes (odd pitch: lane r's walk along row r
-   // spreads over the banks); lane r then sums row r in lane order
-   __shared__ double part[kRH][kThreads + 1];
-   static_assert(kRH % kRowUnroll == 0 && kRH <= kThreads, "rows of the tile");
+   constexpr bool kInt = TYPE == SImage::U8 || TYPE == SImage::S8;
+   typedef typename std::conditional<kInt, int, double>::type A;
+   // each lane's partial row sums, rows x lanes (odd pitch: the walks along the rows spread
+   // over the banks); lanes r and r + 32 then sum the halves of row r in lane order
+   __shared__ A part[kRH][kThreads + 1];
+   static_assert(kRH % kAggRows == 0 && 2 * kRH == kThreads, "rows of the tile");
    const int cb = blockIdx.x, rb = blockIdx.y;
    const int x0 = cb * kCW + threadIdx.x * kVec;
    const int y0 = rb * kRH, y1 = min(y0 + kRH, H);
-   double col[kVec] = {0, 0, 0, 0};
+   A col[kVec] = {0, 0, 0, 0};
    unsigned peak = 0;
-   for (int y = y0; y < y1; y += kRowUnroll) {
-      double v[kRowUnroll][kVec];
+   by_tile(cb, rb, W, H, [&](auto whole) {
+      for (int y = y0; y < y1; y += kAggRows) {
+         Vec4<typename ElemT<TYPE>::type> q[kAggRows];
 #pragma unroll
-      for (int r = 0; r < kRowUnroll; ++r)
-         load_row<TYPE, SQR, VEC>(src, step, y + r, y1, x0, W, nch, ch, v[r]);
+         for (int r = 0; r < kAggRows; ++r)
+            q[r] = load_raw<TYPE, VEC>(src, step, y + r, y1, x0, W, nch, ch);
 #pragma unroll
-      for (int r = 0; r < kRowUnroll; ++r) {
-         double rs = 0;
+         for (int r = 0; r < kAggRows; ++r) {
+            A v[kVec], rs = 0;
+            values<decltype(whole)::value, SQR, VEC>(q[r], y + r, y1, x0, W, v);
 #pragma unroll
-         for (int j = 0; j < kVec; ++j) {
-            col[j] += v[r][j];
-            rs += v[r][j];
+            for (int j = 0; j < kVec; ++j) {
+               col[j] += v[j];
+               rs += v[j];
+               if (PEAK) peak = max(peak, (unsigned)__double2hiint((double)v[j]) & 0x7fffffffu);
+            }
+            part[y - y0 + r][threadIdx.x] = rs;   // rows past y1 hold 0 and are not summed
          }
-         part[y - y0 + r][threadIdx.x] = rs;   // rows past y1 hold 0 and are not summed
       }
-      if (PEAK) {
-#pragma unroll
-         for (int r = 0; r < kRowUnroll; ++r)
-#pragma unroll
-            for (int j = 0; j < kVec; ++j) peak = max(peak, (unsigned)__double2hiint(v[r][j]) & 0x7fffffffu);
-      }
-   }
+   });
 #pragma unroll
    for (int j = 0; j < kVec; ++j)
-      if (x0 + j < W) aux.colsum[(size_t)rb * W + x0 + j] = col[j];
+      if (x0 + j < W) aux.colsum[(size_t)rb * W + x0 + j] = (double)col[j];
    __syncthreads();
-   const int r = threadIdx.x;
-   double rs = 0;
-   if (r < y1 - y0) {
-      for (int l = 0; l < kThreads; ++l) rs += part[r][l];
-      aux.rowsum[(size_t)(y0 + r) * aux.CB + cb] = rs;
-   }
-   const double tot = wave_sum(rs);
+   const int r = threadIdx.x & 31, l0 = threadIdx.x & 32;
+   A rs = 0;
+   if (r < y1 - y0)
+#pragma unroll 8
+      for (int l = 0; l < 32; ++l) rs += part[r][l0 + l];
+   rs += __shfl_xor(rs, 32, 64);
+   if (r < y1 - y0 && l0 == 0) aux.rowsum[(size_t)(y0 + r) * aux.CB + cb] = (double)rs;
+   const double tot = wave_sum(l0 == 0 ? (double)rs : 0.0);
    if (threadIdx.x == 0) aux.tiletot[(size_t)rb * aux.CB + cb] = tot;
    if (PEAK) {
 #pragma unroll
@@ -157,7 +185,45 @@ __device__ __forceinline__ void exclusive_scan_strided(double *p, int n, size_t 
    }
 }
 
-// 2. carries.  blockIdx.y = 0: column sums over tile rows, one thread per column;
+// Exclusive scans down n rows (W elements apart) of COLS adjacent columns, in place, by one
+// workgroup of 256 threads: 256 / COLS groups of rows, one per thread of a column, whose sums
+// go through LDS; up to K rows of a group stay in registers between the two passes, more are read
+// again.  One round trip to memory where a thread per column took n / 32: the carries of 4096^2
+// (128 tile rows) 10.0 -> 6.0 us.
+template <int COLS, int K>
+__device__ __forceinline__ void scan_columns(double *base, int n, size_t W, int x, int xend)
+{
+   constexpr int GROUPS = 256 / COLS;
+   __shared__ double total[GROUPS][COLS];
+   const int c = threadIdx.x % COLS, g = threadIdx.x / COLS;
+   const int per = cdiv(n, GROUPS), k0 = min(g * per, n), k1 = min(k0 + per, n);
+   double *p = base + min(x + c, xend - 1);
+   double v[K], sum = 0.0;
+   for (int k = k0; k < k1; k += K) {
+#pragma unroll
+      for (int i = 0; i < K; ++i) v[i] = k + i < k1 ? p[(size_t)(k + i) * W] : 0.0;
+#pragma unroll
+      for (int i = 0; i < K; ++i) sum += v[i];
+   }
+   __syncthreads();   // (an earlier call's totals are read)
+   total[g][c] = sum;
+   __syncthreads();
+   double acc = 0.0;
+   for (int w = 0; w < g; ++w) acc += total[w][c];
+   for (int k = k0; k < k1; k += K) {
+      if (per > K) {
+#pragma unroll
+         for (int i = 0; i < K; ++i) v[i] = k + i < k1 ? p[(size_t)(k + i) * W] : 0.0;
+      }
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+         if (k + i < k1 && x + c < xend) p[(size_t)(k + i) * W] = acc;
+         acc += v[i];
+      }
+   }
+}
+
+// 2. carries.  blockIdx.y = 0: column sums over tile rows, 64 columns a block;
 //              blockIdx.y = 1: row sums over tile columns, one thread per row;
 //              blockIdx.y = 2: 2-D exclusive scan of the tile totals (block 0);
 //              blockIdx.y = 3: the largest tile peak into *peak (block 0, where wanted).
@@ -178,7 +244,7 @@ __global__ __launch_bounds__(256) void integral_carries(int W, int H, IntegralAu
    }
    const int i = blockIdx.x * 256 + threadIdx.x;
    if (blockIdx.y == 0) {
-      if (i < W) exclusive_scan_strided(aux.colsum + i, aux.RB, (size_t)W);
+      if (blockIdx.x * 64 < W) scan_columns<64, 32>(aux.colsum, aux.RB, W, blockIdx.x * 64, W);
    } else if (blockIdx.y == 1) {
       if (i < H) exclusive_scan_strided(aux.rowsum + (size_t)i * aux.CB, aux.CB, 1);
    } else if (blockIdx.x == 0) {
@@ -187,16 +253,16 @@ __global__ __launch_bounds__(256) void integral_carries(int W, int H, IntegralAu
       for (int rb = threadIdx.x; rb < aux.RB; rb += 256)
          exclusive_scan_strided(aux.tiletot + (size_t)rb * aux.CB, aux.CB, 1);
       __syncthreads();
-      for (int cb = threadIdx.x; cb < aux.CB; cb += 256)
-         exclusive_scan_strided(aux.tiletot + cb, aux.RB, (size_t)aux.CB);
+      for (int cb = 0; cb < aux.CB; cb += 16)
+         scan_columns<16, 8>(aux.tiletot, aux.RB, aux.CB, cb, aux.CB);
    }
 }
 
-// 4 output values of a row at column x0 (j = 0..3), vector store when OVEC and in range
-template <class T, bool OVEC>
+// 4 output values of a row at column x0 (j = 0..3)
+template <class T>
 __device__ __forceinline__ void store4(T *o, int x0, int W, const double (&val)[kVec])
 {
-   if (OVEC && x0 + kVec <= W) {
+   if (x0 + kVec <= W) {
       Vec4<T> q;
 #pragma unroll
       for (int j = 0; j < kVec; ++j) q.v[j] = (T)val[j];
@@ -209,8 +275,8 @@ __device__ __forceinline__ void store4(T *o, int x0, int W, const double (&val)[
 }
 
 // 3. final pass.  OUT: 0 = F32 inclusive, 1 = F64 inclusive (both with the caller's pitch),
-// 2 = the internal exclusive layout.  OVEC: output rows allow aligned 4-element stores.
-template <int TYPE, bool SQR, bool VEC, int OUT, bool OVEC>
+// 2 = the internal exclusive layout.
+template <int TYPE, bool SQR, bool VEC, int OUT>
 __global__ __launch_bounds__(kThreads) void integral_final(const char *src, int W, int H,
                                                             int step, int nch, int ch,
                                                             IntegralAux aux, char *out,
@@ -252,46 +318,52 @@ __global__ __launch_bounds__(kThreads) void integral_final(const char *src, int 
 
    double colrun[kVec] = {0, 0, 0, 0};
    double py = 0;
-   for (int y = y0; y < y1; y += kRowUnroll) {
-      double v[kRowUnroll][kVec];
-      double rc[kRowUnroll];
+   by_tile(cb, rb, W, H, [&](auto whole) {
+      for (int y = y0; y < y1; y += kRowUnroll) {
+         Vec4<typename ElemT<TYPE>::type> q[kRowUnroll];
+         double v[kRowUnroll][kVec];
+         double rc[kRowUnroll];
 #pragma unroll
-      for (int r = 0; r < kRowUnroll; ++r) {
-         load_row<TYPE, SQR, VEC>(src, step, y + r, y1, x0, W, nch, ch, v[r]);
-         rc[r] = y + r < y1 ? aux.rowsum[(size_t)(y + r) * aux.CB + cb] : 0.0;
-      }
-      // the lane's prefixes of the batch's rows, then their wavefront scans together
-      double p[kRowUnroll][kVec], inc[kRowUnroll];
-#pragma unroll
-      for (int r = 0; r < kRowUnroll; ++r) {
-         double loc = 0;
-#pragma unroll
-         for (int j = 0; j < kVec; ++j) {
-            colrun[j] += v[r][j];
-            loc += colrun[j];
-            p[r][j] = loc;
+         for (int r = 0; r < kRowUnroll; ++r) {
+            q[r] = load_raw<TYPE, VEC>(src, step, y + r, y1, x0, W, nch, ch);
+            rc[r] = aux.rowsum[(size_t)min(y + r, y1 - 1) * aux.CB + cb];   // (unused from y1 on)
          }
-         inc[r] = loc;
-      }
-      wave_incl_scan_f64<kRowUnroll>(inc);
 #pragma unroll
-      for (int r = 0; r < kRowUnroll; ++r) {
-         py += rc[r];
-         const double base = corner + py + (inc[r] - p[r][kVec - 1]);
-         const int yy = y + r;
-         if (yy >= y1) continue;
-         double val[kVec];
+         for (int r = 0; r < kRowUnroll; ++r)
+            values<decltype(whole)::value, SQR, VEC>(q[r], y + r, y1, x0, W, v[r]);
+         // the lane's prefixes of the batch's rows, then their wavefront scans together
+         double p[kRowUnroll][kVec], inc[kRowUnroll];
 #pragma unroll
-         for (int j = 0; j < kVec; ++j) val[j] = base + p[r][j] + px[j];
-         if (OUT == 0)
-            store4<float, OVEC>(reinterpret_cast<float *>(out + (size_t)yy * ostep), x0, W, val);
-         else if (OUT == 1)
-            store4<double, OVEC>(reinterpret_cast<double *>(out + (size_t)yy * ostep), x0, W, val);
-         else
-            store4<double, true>(reinterpret_cast<double *>(out) + (size_t)(yy + 1) * P +
-                                     kExclOffset + 1, x0, W, val);
+         for (int r = 0; r < kRowUnroll; ++r) {
+            double loc = 0;
+#pragma unroll
+            for (int j = 0; j < kVec; ++j) {
+               colrun[j] += v[r][j];
+               loc += colrun[j];
+               p[r][j] = loc;
+            }
+            inc[r] = loc;
+         }
+         wave_incl_scan_f64<kRowUnroll>(inc);
+#pragma unroll
+         for (int r = 0; r < kRowUnroll; ++r) {
+            py += rc[r];
+            const double base = corner + py + (inc[r] - p[r][kVec - 1]);
+            const int yy = y + r;
+            if (yy >= y1) continue;
+            double val[kVec];
+#pragma unroll
+            for (int j = 0; j < kVec; ++j) val[j] = base + p[r][j] + px[j];
+            if (OUT == 0)
+               store4<float>(reinterpret_cast<float *>(out + (size_t)yy * ostep), x0, W, val);
+            else if (OUT == 1)
+               store4<double>(reinterpret_cast<double *>(out + (size_t)yy * ostep), x0, W, val);
+            else
+               store4<double>(reinterpret_cast<double *>(out) + (size_t)(yy + 1) * P +
+                                        kExclOffset + 1, x0, W, val);
+         }
       }
-   }
+   });
 }
 
 }  // namespace
@@ -304,7 +376,7 @@ size_t integral_aux_bytes(int W, int H)
 
 template <int TT, bool VEC>
 static void launch_integral_t(hipStream_t s, const char *src, const View &v, int channel,
-                              bool sqr, void *out, int ostep, int mode, bool ovec, IntegralAux aux,
+                              bool sqr, void *out, int ostep, int mode, IntegralAux aux,
                               unsigned *peak)
 {
    const int W = v.width, H = v.height;
@@ -322,15 +394,14 @@ static void launch_integral_t(hipStream_t s, const char *src, const View &v, int
       aggregate(integral_aggregate<TT, false, VEC, false>);
    }
    launch_check("integral_aggregate");
-   integral_carries<<<dim3(cdiv(W > H ? W : H, 256), peak ? 4 : 3), 256, 0, s>>>(W, H, aux, peak);
+   integral_carries<<<dim3(max(cdiv(W, 64), cdiv(H, 256)), peak ? 4 : 3), 256, 0, s>>>(W, H, aux, peak);
    launch_check("integral_carries");
    char *o = static_cast<char *>(out);
-#define OCIP_FINAL(SQ, M, OV) \
-   integral_final<TT, SQ, VEC, M, OV><<<grid, kThreads, 0, s>>>(src, W, H, v.step, v.channels, channel, aux, o, ostep)
+#define OCIP_FINAL(SQ, M) \
+   integral_final<TT, SQ, VEC, M><<<grid, kThreads, 0, s>>>(src, W, H, v.step, v.channels, channel, aux, o, ostep)
 #define OCIP_FINAL_M(SQ)                                                    \
-   if (mode == 2) OCIP_FINAL(SQ, 2, true);                                  \
-   else if (mode == 1) { if (ovec) OCIP_FINAL(SQ, 1, true); else OCIP_FINAL(SQ, 1, false); } \
-   else { if (ovec) OCIP_FINAL(SQ, 0, true); else OCIP_FINAL(SQ, 0, false); }
+   if (mode == 2) OCIP_FINAL(SQ, 2);                                        \
+   else if (mode == 1) OCIP_FINAL(SQ, 1); else OCIP_FINAL(SQ, 0);
    if (sqr) { OCIP_FINAL_M(true) } else { OCIP_FINAL_M(false) }
 #undef OCIP_FINAL_M
 #undef OCIP_FINAL
@@ -343,16 +414,10 @@ void launch_integral(hipStream_t s, const View &v, int channel, bool sqr, void *
    IntegralAux aux = aux_layout(auxp, v.width, v.height);
    const char *src = static_cast<const char *>(v.ptr);
    const int mode = out_type == SImage::F32 ? 0 : (out_type == SImage::F64 ? 1 : 2);
-   const int esz = elem_size(v.type);
-   // 4-element vector loads: one channel, rows and base aligned to 4 elements
-   const bool vec = v.channels == 1 && (v.step % (4 * esz)) == 0 &&
-                    (reinterpret_cast<uintptr_t>(v.ptr) % (4 * esz)) == 0;
-   const int osz = mode == 0 ? 4 : 8;
-   const bool ovec = mode != 2 && (ostep % (4 * osz)) == 0 &&
-                     (reinterpret_cast<uintptr_t>(out) % (4 * osz)) == 0;
+   const bool vec = v.channels == 1 && v.width >= 4;
    OCIP_TYPE_SWITCH(v.type, TT, {
-      if (vec) launch_integral_t<TT, true>(s, src, v, channel, sqr, out, ostep, mode, ovec, aux, peak);
-      else launch_integral_t<TT, false>(s, src, v, channel, sqr, out, ostep, mode, ovec, aux, peak);
+      if (vec) launch_integral_t<TT, true>(s, src, v, channel, sqr, out, ostep, mode, aux, peak);
+      else launch_integral_t<TT, false>(s, src, v, channel, sqr, out, ostep, mode, aux, peak);
    });
 }
 
