@@ -29,6 +29,7 @@ __device__ __forceinline__ typename ElemT<TYPE>::type ld(const char *row, int i)
 // only 4-byte aligned addresses and a 4- or 8-byte one none, at one more cache line for the
 // wavefront, so image rows need no particular pitch, width or template offset for them.
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double f64x2_u __attribute__((ext_vector_type(2), aligned(8)));
 typedef uint32_t u32x2_u __attribute__((ext_vector_type(2), aligned(1)));
 
 // Dispatch a runtime SImage type to a template parameter.

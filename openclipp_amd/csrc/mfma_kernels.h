@@ -835,8 +835,36 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    constexpr int kEpiGroups = 2;
    constexpr bool NORM = MODE == kModeNCC || MODE == kModeSSDN;
    typedef double Corners[kEpiGroups][4][4];   // [group][corner][e]
+   // INNER: every window of the tile lies inside the image: no clamps, each corner's four values
+   // as two 16-byte loads (48 BF16 templates of 8..96 px on 2048^2: 1900 -> 1823 us)
+   const bool inner = x0 >= cx && x0 + C - cx + a.tw <= a.W && Y0 >= cy &&
+                      Y0 + kPairRows - cy + a.th <= a.H;
    auto load_corners = [&](int i0, Corners &q) {
       const size_t ip = excl_pitch(a.W);
+      if (inner) {
+#pragma unroll
+         for (int u = 0; u < kEpiGroups; ++u) {
+            const int k = threadIdx.x + 256 * (i0 + u);
+            const int r = min(k / (C / 4), kPairRows - 1), c = 4 * (k - (k / (C / 4)) * (C / 4));
+            const double *p = a.integ + (size_t)(Y0 + r - cy) * ip + (kExclOffset + x0 + c - cx);
+            const double *p1 = p + (size_t)a.th * ip;
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+               const f64x2_u v0 = *reinterpret_cast<const f64x2_u *>(p + e);
+               const f64x2_u v1 = *reinterpret_cast<const f64x2_u *>(p1 + e);
+               const f64x2_u v2 = *reinterpret_cast<const f64x2_u *>(p + a.tw + e);
+               const f64x2_u v3 = *reinterpret_cast<const f64x2_u *>(p1 + a.tw + e);
+#pragma unroll
+               for (int h = 0; h < 2; ++h) {
+                  q[u][0][e + h] = v0[h];
+                  q[u][1][e + h] = v1[h];
+                  q[u][2][e + h] = v2[h];
+                  q[u][3][e + h] = v3[h];
+               }
+            }
+         }
+         return;
+      }
 #pragma unroll
       for (int u = 0; u < kEpiGroups; ++u) {
          const int k = threadIdx.x + 256 * (i0 + u);
