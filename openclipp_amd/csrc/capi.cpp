@@ -204,6 +204,12 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
                                c.tmpl.sums.as<double>(), integ, (float *)D.dev, D.desc.Step,
                                c.stats.ptr);
       } else {
+         // (a map written over its own template needs the template staged first)
+         if (T.dev != D.dev && prox_template_in_place(op, view(S), view(T), integ != nullptr)) {
+            launch_proximity(c.stream, op, view(S), view(T), D.dev, D.desc.Step, T.dev,
+                             (int)(T.desc.Step / sizeof(float)), nullptr, integ, ch);
+            continue;
+         }
          launch_template_prep(c.stream, view(T), ch, tpitch, kind, c.tmpl.data.ptr,
                               c.tmpl.sums.as<double>());
          launch_proximity(c.stream, op, view(S), view(T), D.dev, D.desc.Step, c.tmpl.data.ptr,

@@ -907,13 +907,13 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
 // ======================================================================= split FP16
 constexpr int kSplitNT = 4;
 
-// Where the path is taken: prox_tile_f32 costs about 4 us + Mpx (12 us + 0.044 us taps) where it
-// forms the window sums in its tiles, and this path 58 us (seven launches, the integral's
-// three among them) + Mpx (7 us + 0.0055 us taps), equal at Mpx (taps + 142) = 1420: it is taken from
-// 1600 on (1900^2/16x16 88 against 82 us, 1000x3000/24x24 110 against 96, 1400^2/24x24 77
-// against 87).  Where prox_tile_f32 needs the integral too, it pays its launches as well:
-// taken from 200 taps or 2 Mpx on (160x120/31x31 90 against 67 us, 2048x512/16x16 68 against 64,
-// 2048x1024/5x5 79 against 73; 2048x512/5x5 55 against 63).
+// Where the path is taken: prox_tile_f32 costs about 2 us + Mpx (11 us + 0.04 us taps) where it
+// forms the window sums in its tiles, and this path 46 us (seven launches, the integral's
+// three among them) + Mpx (5 us + 0.006 us taps), equal near Mpx (taps + 142) = 1420, where it is
+// taken from (1900^2/16x16 78 against 66 us, 1000x3000/24x24 96 against 79; 1400^2/24x24 66
+// against 73, 1000x3000/16x16 61 against 67).  Where prox_tile_f32 needs the integral too, it pays
+// its launches as well: taken from 200 taps or 2 Mpx on (160x120/31x31 78 against 57 us,
+// 2048x512/16x16 54 against 50, 2048x1024/5x5 56 against 55; 2048x512/5x5 40 against 47).
 // OCIP_SPLIT_NCC=0 turns the path off (prox_tile_f32 then computes the maps), 1 has it take
 // every call that it can.
 bool split_ncc_ok(int op, const View &S, const View &T)
@@ -927,7 +927,7 @@ bool split_ncc_ok(int op, const View &S, const View &T)
    if (pair_geometry(kc2_for(tw), kSplitNT, th, mfma::kLdsMax, 2).vb < 1) return false;
    if (e && e[0] == '1') return true;
    const long long px = (long long)S.width * S.height, taps = (long long)tw * th;
-   return prox_norm_from_tile(op, S, T) ? px * (taps + 142) >= 1600000000LL
+   return prox_norm_from_tile(op, S, T) ? px * (taps + 142) >= 1420000000LL
                                         : taps >= 200 || px >= 1 << 21;
 }
 

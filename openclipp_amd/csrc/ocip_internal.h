@@ -182,6 +182,9 @@ void launch_template_prep(hipStream_t s, const View &tpl, int channel, int pitch
 void launch_proximity(hipStream_t s, int op, const View &src, const View &tpl, void *dst,
                       int dst_step, const void *tstage, int tpitch, const double *tsums,
                       const double *integ, int channel);
+// 1-channel F32 templates that launch_proximity reads in place (tstage = the image, tpitch its
+// pitch in floats, tsums null): no staging launch.
+bool prox_template_in_place(int op, const View &src, const View &tpl, bool have_integral);
 // The plain Norm ops on F32 sources whose template fits one LDS band form the window sums
 // of s^2 inside the tile kernel (launch_proximity with no integral)
 bool prox_norm_from_tile(int op, const View &src, const View &tpl);

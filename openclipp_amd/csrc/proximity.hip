@@ -168,15 +168,14 @@ __device__ __forceinline__ void stage_tile_f32(float *lds, int ldsw, int nrows, 
    }
 }
 
-// stage_tile_f32 for 1-channel F32 rows whose staged columns start 16-byte aligned (sx0 a
-// multiple of 4, 16-byte aligned rows): groups of four columns, one 16-byte load each where
-// the group lies wholly inside the image, eight groups per thread in flight; the same values
-// in LDS.
+// stage_tile_f32 for 1-channel F32 images: groups of four columns, one 16-byte load each (at any
+// alignment) where the group lies wholly inside the image, eight groups per thread in flight;
+// the same values in the columns that the taps read (up to ncols + 2).
 __device__ __forceinline__ void stage_tile_f32_v4(float *lds, int ldsw, int nrows, int ncols,
                                                   const char *src, int W, int H, int sstep,
                                                   int sx0, int sy0)
 {
-   const int gpr = ldsw / 4, n4 = nrows * gpr;
+   const int gpr = (ncols + 6) / 4, n4 = nrows * gpr;   // columns 0 .. ncols + 2, within the pitch
    // group i = r gpr + g, (r, g) stepped along with i (256 groups a step) instead of divided out
    const int dq = 256 / gpr, dr = 256 - dq * gpr;
    int r = threadIdx.x / gpr, g = threadIdx.x - r * gpr;
@@ -192,7 +191,8 @@ __device__ __forceinline__ void stage_tile_f32_v4(float *lds, int ldsw, int nrow
          const bool rowin = i < n4 && sy >= 0 && sy < H;
          const float *srow = reinterpret_cast<const float *>(src + (size_t)(rowin ? sy : 0) * sstep);
          if (rowin && c + 4 <= ncols && sx >= 0 && sx + 4 <= W) {
-            v[k] = *reinterpret_cast<const float4 *>(srow + sx);
+            const f32x4_u q = *reinterpret_cast<const f32x4_u *>(srow + sx);
+            v[k] = make_float4(q[0], q[1], q[2], q[3]);
          } else {
             float e[4];
 #pragma unroll
@@ -296,11 +296,21 @@ __device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int
    float acc[R];
 #pragma unroll
    for (int r = 0; r < R; ++r) acc[r] = 0.f;
-   // 16-byte staging loads: 1-channel F32 rows, staged columns from x0 - cx with x0 a
-   // multiple of 4 R and cx a multiple of 4, 16-byte aligned rows; for the 16-output tiles of
-   // large images (2.24 -> 2.09-2.12 ms at 4096^2 / 64x64)
-   const bool v4 = R == 16 && TYPE == SImage::F32 && nch == 1 && (cx & 3) == 0 &&
-                   (sstep & 15) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+   const bool v4 = TYPE == SImage::F32 && nch == 1;
+   // sum t^2 where the host passes none: each workgroup its own from the template (in place), the
+   // loads under the staging's
+   __shared__ double red[4];
+   if ((OP == kSSDNorm || OP == kCCNorm) && !tsums) {
+      double t2 = 0.0;
+      const int n = tw * th;
+      for (int i = threadIdx.x; i < n; i += 256) {
+         const int v = i / tw;
+         const double t = (double)tp[(size_t)v * tpitch + (i - v * tw)];
+         t2 = fma(t, t, t2);
+      }
+      t2 = wave_sum(t2);
+      if (lane == 0) red[wave] = t2;
+   }
 
    for (int v0 = 0; v0 < th; v0 += vb) {
       const int nv = min(vb, th - v0);
@@ -333,7 +343,7 @@ __device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int
 
    const int oy = y0 + lane;
    if (OP == kSSDNorm || OP == kCCNorm) {
-      const double tt = tsums[0];
+      const double tt = tsums ? tsums[0] : red[0] + red[1] + red[2] + red[3];
       double ss[R];
       if (integ) {
          // all integral corners of the R outputs first, then the divisions
@@ -346,10 +356,17 @@ __device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int
       }
       if (oy >= H) return;
 #pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] = (float)((double)acc[r] / sqrt(ss[r] * tt));
+      for (int r = 0; r < R; ++r) acc[r] = (float)((double)acc[r] * rsqrt64(ss[r] * tt));
    }
    if (oy >= H) return;
    float *drow = reinterpret_cast<float *>(dst + (size_t)oy * dstep);
+   if (nch == 1 && x0 + colbase + R <= W) {
+#pragma unroll
+      for (int r = 0; r < R; r += 4)
+         *reinterpret_cast<f32x4_u *>(drow + x0 + colbase + r) =
+             f32x4_u{acc[r], acc[r + 1], acc[r + 2], acc[r + 3]};
+      return;
+   }
 #pragma unroll
    for (int r = 0; r < R; ++r) {
       const int ox = x0 + colbase + r;
@@ -885,6 +902,20 @@ void launch_proximity_flagged(hipStream_t s, const View &S, const View &T, void 
        static_cast<const char *>(S.ptr), W, H, S.step, static_cast<const float *>(tstage), tpitch,
        tw, th, tsums, integ, static_cast<char *>(dst), dstep, vb, ldsw, f);
    launch_check("prox_flagged");
+}
+
+// The tile kernel reads an F32 template's rows as scalar loads wherever they lie, and for the Norm
+// ops each workgroup sums t^2 by itself, up to kTileTaps taps (four a thread); past that, or with
+// the denominators from the integral, template_prep's launch costs less than the sums.
+// (SqrDistance_Norm 1024^2/16x16 30.6 -> 22.2 us with the vector staging and stores.)
+bool prox_template_in_place(int op, const View &S, const View &T, bool have_integral)
+{
+   constexpr int kTileTaps = 1024;
+   if (S.type != SImage::F32 || S.channels != 1 || T.width <= 0 || T.height <= 0) return false;
+   const int ncols = kWaves * tile_r(S.width, T.width, T.height) + T.width - 1;
+   if (kLdsBudget / (lds_pitch(ncols) * 4) - (kTileRows - 1) < 1) return false;   // prox_direct
+   const bool norm = op == kSSDNorm || op == kCCNorm;
+   return !norm || (!have_integral && T.width * T.height <= kTileTaps);
 }
 
 template <int OP>
