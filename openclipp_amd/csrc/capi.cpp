@@ -392,9 +392,12 @@ ocipError ocip_API ocipInitialize(ocipContext *ContextPtr, const char *Preferred
          c->name = p.name;
          if (p.gcnArchName[0]) c->name += std::string(" (") + p.gcnArchName + ")";
          c->num_cus = p.multiProcessorCount;
+         hip_check(hipHostMalloc(&c->host_out, kHostOutBytes, hipHostMallocDefault), "pinned memory");
          hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "stream");
          noalloc_scratch_init(c->device);
       } catch (...) {
+         if (c->stream) (void)hipStreamDestroy(c->stream);
+         if (c->host_out) (void)hipHostFree(c->host_out);
          delete c;
          throw;
       }
@@ -423,6 +426,7 @@ ocipError ocip_API ocipUninitialize(ocipContext Context)
       batch_cache_destroy(c->batch);
       c->batch = nullptr;
       (void)hipStreamDestroy(c->stream);
+      (void)hipHostFree(c->host_out);
       c->magic = 0;
       delete c;
    });
@@ -745,7 +749,7 @@ static ocipError run_minmax(ocipProgram Program, ocipImage Source, double *Resul
       send_if_needed(c, S);
       DevBuf &buf = Program ? reinterpret_cast<ocip::Program *>(Program)->scratch : c.stats;
       buf.ensure(minmax_partials_bytes(S.desc.Width, S.desc.Height));
-      launch_minmax(c.stream, want_max, view(S), buf.ptr, Result, IndexX, IndexY);
+      launch_minmax(c.stream, want_max, view(S), buf.ptr, c.host_out, Result, IndexX, IndexY);
    });
 }
 
@@ -774,7 +778,7 @@ static ocipError run_sum(ocipProgram Program, ocipImage Source, double *Result, 
       send_if_needed(c, S);
       DevBuf &buf = Program ? reinterpret_cast<ocip::Program *>(Program)->scratch : c.stats;
       buf.ensure(sum_partials_bytes(S.desc.Width, S.desc.Height));
-      launch_sum(c.stream, sqr, view(S), buf.ptr, Result);
+      launch_sum(c.stream, sqr, view(S), buf.ptr, c.host_out, Result);
    });
 }
 

@@ -100,6 +100,8 @@ struct TemplateBuf {
    DevBuf sums;      // [0] = sum t^2 (double), [1] = sum t (double)
 };
 
+constexpr size_t kHostOutBytes = 16 * 1024;
+
 struct Context {
    uint32_t magic = kContextMagic;
    int device = 0;
@@ -111,6 +113,7 @@ struct Context {
    DevBuf integ_aux;      // integral scan aggregates
    DevBuf stats;          // reduction partials for MinIndx / MaxIndx, MFMA fragments
    DevBuf work;           // gradient workspace
+   void *host_out = nullptr;   // kHostOutBytes of pinned memory that reductions leave results in
    BatchCache *batch = nullptr;  // recorded batch graphs (mfma.hip)
 };
 
@@ -280,13 +283,14 @@ void fft_plain_prepare(hipStream_t s, FftState *st, int W, int H);
 void launch_fft(hipStream_t s, FftState *st, bool forward, const View &real, const View &cplx);
 
 // Per-channel sum (sqr = false) or sum of squares of an image into result[0..channels),
-// blocking.  partials: sum_partials_bytes of device scratch.
+// blocking.  partials: sum_partials_bytes of device scratch; host_out: the context's.
 size_t sum_partials_bytes(int width, int height);
-void launch_sum(hipStream_t s, bool sqr, const View &src, void *partials, double *result);
+void launch_sum(hipStream_t s, bool sqr, const View &src, void *partials, void *host_out,
+                double *result);
 // Min / max of a 1-channel image and the pixel holding it, in the reference's reduction order
 // (its tie-breaks and float partials), blocking.
 size_t minmax_partials_bytes(int width, int height);
-void launch_minmax(hipStream_t s, bool want_max, const View &src, void *partials,
+void launch_minmax(hipStream_t s, bool want_max, const View &src, void *partials, void *host_out,
                    double *host_result, int *ix, int *iy);
 
 }  // namespace ocip
