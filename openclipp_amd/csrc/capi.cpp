@@ -175,6 +175,13 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
       D.in_device = true;
       return;
    }
+   // 8-bit AbsDistance: its own tile kernel
+   if (precision == ocipPrecisionF32 && sad8_ok(op, view(S), view(T))) {
+      c.stats.ensure(sad8_work_bytes(view(S), view(T)));
+      launch_sad8(c.stream, view(S), view(T), D.dev, D.desc.Step, c.stats.ptr);
+      D.in_device = true;
+      return;
+   }
    // CrossCorr_Norm of F32 images: split-FP16 MFMA where the path applies
    if (precision == ocipPrecisionF32 && split_ncc_ok(op, view(S), view(T))) {
       const size_t head = 256;   // the peaks, ahead of the path's work buffer

@@ -1230,6 +1230,29 @@ __global__ __launch_bounds__(256) void join_planes(const float *__restrict__ src
 // one thread per 4 columns of a plane
 static unsigned plane_blocks(int H, int step) { return (unsigned)(((long long)H * (step / 4) + 255) / 256); }
 
+size_t planes8_bytes(const View &S)
+{
+   return S.channels > 1 ? (size_t)S.channels * S.height * plane8_step(S.width) : 0;
+}
+
+View launch_planes8(hipStream_t s, const View &image, void *planes, size_t *plane8)
+{
+   KernelTimer kt(s, "split_planes8");
+   View S = image;
+   S.ptr = planes;
+   S.step = plane8_step(image.width);
+   S.channels = 1;
+   *plane8 = (size_t)S.height * S.step;
+   auto go = [&](auto kernel) {
+      kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(
+          static_cast<const unsigned char *>(image.ptr), S.width, S.height, image.step,
+          static_cast<unsigned char *>(planes), S.step);
+   };
+   if (image.channels == 2) go(split_planes8<2>); else go(split_planes8<4>);
+   launch_check("split_planes8");
+   return S;
+}
+
 bool int_mfma_ok(int op, const View &S, const View &T)
 {
    const char *e = getenv("OCIP_INT_MFMA");
@@ -1249,7 +1272,7 @@ bool int_mfma_ok(int op, const View &S, const View &T)
 size_t int_mfma_work_bytes(const View &S, const View &T)
 {
    // several channels: a plane of bytes and a plane of the map each
-   const size_t planes = S.channels > 1 ? 5 * (size_t)S.channels * S.height * plane8_step(S.width) : 0;
+   const size_t planes = 5 * planes8_bytes(S);
    return S.channels * pair_frag_bytes(mfma::kBF16, T.width, T.height) + planes;
 }
 
@@ -1266,22 +1289,11 @@ void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, do
    int mstep = dstep;
    size_t plane8 = 0, planef = 0;
    if (nch > 1) {
-      KernelTimer kt(s, "split_planes8");
-      unsigned char *planes = static_cast<unsigned char *>(work) + nch * frag_bytes;
-      S.ptr = planes;
-      S.step = plane8_step(S.width);
-      S.channels = 1;
-      plane8 = (size_t)S.height * S.step;
+      char *planes = static_cast<char *>(work) + nch * frag_bytes;
+      S = launch_planes8(s, image, planes, &plane8);
       map = reinterpret_cast<float *>(planes + nch * plane8);
       mstep = 4 * S.step;
       planef = (size_t)S.height * mstep;
-      auto go = [&](auto kernel) {
-         kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(
-             static_cast<const unsigned char *>(image.ptr), S.width, S.height, image.step, planes,
-             S.step);
-      };
-      if (nch == 2) go(split_planes8<2>); else go(split_planes8<4>);
-      launch_check("split_planes8");
    }
    if (op != kCC) {
       // the window sums of s^2 go to the map first; the MFMA kernel's epilogue reads them

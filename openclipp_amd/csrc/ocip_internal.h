@@ -240,6 +240,16 @@ constexpr size_t kNoAllocSumsBytes = 256;   // template sums ahead of the fragme
 void noalloc_scratch_init(int device);
 void *noalloc_scratch(int device);
 
+// The interleaved channels (2 or 4) of an 8-bit image as 1-channel planes in `planes`
+// (planes8_bytes): the view of the first, the others *plane8 bytes apart.
+size_t planes8_bytes(const View &image);
+View launch_planes8(hipStream_t s, const View &image, void *planes, size_t *plane8);
+
+// AbsDistance of 8-bit images (every channel in one launch), exact int32 sums.
+bool sad8_ok(int op, const View &src, const View &T);
+size_t sad8_work_bytes(const View &src, const View &T);
+void launch_sad8(hipStream_t s, const View &src, const View &T, void *dst, int dst_step, void *work);
+
 // Exact integer sums of 8-bit images on BF16 MFMA (CrossCorr, CrossCorr_Norm, SqrDistance,
 // SqrDistance_Norm of U8/S8 images, every channel in one launch): int_mfma_ok tells whether the
 // path takes the call; tsums[ch] receives sum t^2.  The maps equal prox_tile_int's bit for bit.

@@ -22,6 +22,8 @@
 //                  templates too wide for the LDS tile).
 // Norm denominators come from the FP64 sum-of-squares integral of the source (exclusive,
 // (W+1) x (H+1) layout) by four corners and the FP64 sum of squares of the template.
+#include <algorithm>
+
 #include "device_common.h"
 
 namespace ocip {
@@ -491,75 +493,11 @@ __device__ __forceinline__ uint32_t pack4(int32_t a, int32_t b, int32_t c, int32
    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
-// Four taps at once on packed bytes: v_dot4_u32_u8 / v_dot4_i32_i8 for the cross term,
-// v_sad_u8 (bytes kept in 0..255 by sad_key) for AbsDistance.
-template <int OP, int TYPE> __device__ __forceinline__ int32_t itap4(int32_t acc, uint32_t s, uint32_t t)
+// Four taps at once on packed bytes: v_dot4_u32_u8 / v_dot4_i32_i8.
+template <int TYPE> __device__ __forceinline__ int32_t itap4(int32_t acc, uint32_t s, uint32_t t)
 {
-   if (OP == kSAD) return (int32_t)__builtin_amdgcn_sad_u8(s, t, (uint32_t)acc);
    if (TYPE == SImage::S8) return __builtin_amdgcn_sdot4((int32_t)s, (int32_t)t, acc, false);
    return (int32_t)__builtin_amdgcn_udot4(s, t, (uint32_t)acc, false);
-}
-
-// AbsDistance on 8-bit sources: the staged tile's keyed values (sad_key) repacked in place as
-// P(c) = bytes (v[c], v[c + 4], v[c + 8], v[c + 12]) for the columns c < ncols (the tile was
-// staged ncols + 12 columns wide, within the pitch), so that the 16 taps u0 .. u0 + 15 of the
-// output at window column x are four v_sad_u8 of P(x + k) against the template bytes
-// (t[u0 + k], t[u0 + k + 4], t[u0 + k + 8], t[u0 + k + 12]), k < 4, with no byte
-// realignment.  Rounds of 8 elements per thread in increasing order: every read of a round
-// (elements i .. i + 12) precedes its writes (elements i) at a barrier, and later rounds read
-// only elements no earlier round wrote.
-template <int TYPE>
-__device__ __forceinline__ void pack_sad8(int32_t *lds, int ldsw, int nrows, int ncols)
-{
-   const int n = nrows * ldsw;
-   // column c = i % ldsw stepped along with i (256 elements a step)
-   const int dr = 256 % ldsw;
-   int c = threadIdx.x % ldsw;
-   for (int i0 = 0; i0 < n; i0 += 256 * 8) {
-      uint32_t p[8];
-      bool in[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-         const int i = i0 + threadIdx.x + 256 * k;
-         in[k] = i < n && c < ncols;
-         p[k] = 0;
-         if (in[k])
-            p[k] = pack4(sad_key<kSAD, TYPE, int32_t>(lds[i]), sad_key<kSAD, TYPE, int32_t>(lds[i + 4]),
-                         sad_key<kSAD, TYPE, int32_t>(lds[i + 8]),
-                         sad_key<kSAD, TYPE, int32_t>(lds[i + 12]));
-         c += dr;
-         if (c >= ldsw) c -= ldsw;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-         const int i = i0 + threadIdx.x + 256 * k;
-         if (in[k]) lds[i] = (int32_t)p[k];
-      }
-      __syncthreads();
-   }
-}
-
-// AbsDistance on 8-bit sources: the staged template (int32 per column, row pitch tpitch) gets,
-// in each block of 16 columns, the four dwords of the block's keyed bytes that the repacked
-// tile meets, in place at the block's first four columns: dword k = bytes of columns 16 b + k,
-// + 4, + 8, + 12, a zero byte for a column past the template (a last partial block).  One
-// thread per (row, block).
-__host__ __device__ constexpr int sad8_blocks(int tw) { return (tw + 15) / 16; }
-
-template <int TYPE>
-__global__ __launch_bounds__(256) void sad8_template_pack(int32_t *tp, int tpitch, int tw, int th)
-{
-   const int nb = sad8_blocks(tw);
-   const int i = blockIdx.x * 256 + threadIdx.x;
-   if (i >= nb * th) return;
-   const int v = i / nb, b = i - v * nb;
-   int32_t *blk = tp + (size_t)v * tpitch + 16 * b;
-   int32_t t[16];
-#pragma unroll
-   for (int k = 0; k < 16; ++k) t[k] = 16 * b + k < tw ? sad_key<kSAD, TYPE, int32_t>(blk[k]) : 0;
-#pragma unroll
-   for (int k = 0; k < 4; ++k) blk[k] = (int32_t)pack4(t[k], t[k + 4], t[k + 8], t[k + 12]);
 }
 
 // With int32 sums (8-bit sources) SqrDistance and SqrDistance_Norm take the cross term only,
@@ -584,11 +522,7 @@ __global__ __launch_bounds__(256) void prox_tile_int(const char *src, int W, int
    constexpr int TOP = kViaCC ? kCC : OP;   // the op of each tap
    // 8-bit sources with int32 sums: four taps per instruction on packed bytes
    constexpr bool kPacked = sizeof(ACC) == 4 && (TYPE == SImage::U8 || TYPE == SImage::S8) &&
-                            (TOP == kCC || TOP == kCCNorm || TOP == kSAD);
-   // AbsDistance on 8-bit sources: the tile repacked by pack_sad8 (the host sized the pitch
-   // for ncols + 12 staged columns), the template's full 16-column blocks by
-   // sad8_template_pack
-   constexpr bool kSad8 = kPacked && TOP == kSAD;
+                            (TOP == kCC || TOP == kCCNorm);
    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
    const int x0 = blockIdx.x * (kWaves * R), y0 = blockIdx.y * kTileRows;
    const int cx = tw / 2, cy = th / 2;
@@ -602,76 +536,12 @@ __global__ __launch_bounds__(256) void prox_tile_int(const char *src, int W, int
    for (int v0 = 0; v0 < th; v0 += vb) {
       const int nv = min(vb, th - v0);
       __syncthreads();
-      stage_tile_int<TYPE>(ldsi, ldsw, kTileRows + nv - 1, kSad8 ? ncols + 12 : ncols, src, W,
+      stage_tile_int<TYPE>(ldsi, ldsw, kTileRows + nv - 1, ncols, src, W,
                            H, sstep, nch, ch, x0 - cx, y0 - cy + v0);
       __syncthreads();
-      if constexpr (kSad8) pack_sad8<TYPE>(ldsi, ldsw, kTileRows + nv - 1, ncols);
       for (int v = 0; v < nv; ++v) {
          const int32_t *lrow = ldsi + (size_t)(lane + v) * ldsw + colbase;
          const int32_t *trow = tp + (size_t)(v0 + v) * tpitch;
-         if constexpr (kSad8) {
-            // 16 taps per step: the window's P values of columns u0 .. u0 + R + 2 (16-byte
-            // reads from a 16-byte aligned column: ldsw, colbase and u0 are multiples of 4),
-            // four v_sad_u8 per output; the last tw % 16 taps in one masked step of the same
-            // kind
-            int u0 = 0;
-            for (; u0 + 16 <= tw; u0 += 16) {
-               uint32_t pw[R + 4];
-               // (an empty asm with a memory clobber: each step reads its window afresh as 16-byte
-               // loads, rather than the compiler carrying one dword over from the step before
-               // and reading the rest as conflicting 4-byte loads)
-               asm volatile("" ::: "memory");
-               const int4 *w4 = reinterpret_cast<const int4 *>(lrow + u0);
-#pragma unroll
-               for (int m = 0; m < (R + 4) / 4; ++m) {
-                  const int4 q4 = w4[m];
-                  pw[4 * m] = (uint32_t)q4.x; pw[4 * m + 1] = (uint32_t)q4.y;
-                  pw[4 * m + 2] = (uint32_t)q4.z; pw[4 * m + 3] = (uint32_t)q4.w;
-               }
-               // the block's four packed template dwords (sad8_template_pack)
-               uint32_t tq[4];
-#pragma unroll
-               for (int k = 0; k < 4; ++k) tq[k] = (uint32_t)trow[u0 + k];
-#pragma unroll
-               for (int r = 0; r < R; ++r)
-#pragma unroll
-                  for (int k = 0; k < 4; ++k)
-                     acc[r] = (ACC)__builtin_amdgcn_sad_u8(pw[r + k], tq[k], (uint32_t)acc[r]);
-            }
-            if (u0 < tw) {
-               // a last block of 1 to 15 taps: the same step, each P masked to the bytes of
-               // taps inside the template (its packed template dword holds zeros past it), so
-               // that every other byte adds |0 - 0|, and the dwords k >= rem, which hold no
-               // tap, skipped.  The window reads stay inside the row pitch: columns up to
-               // colbase + u0 + 19 <= ncols + 3.
-               const int rem = tw - u0;
-               asm volatile("" ::: "memory");
-               uint32_t pw[R + 4];
-               const int4 *w4 = reinterpret_cast<const int4 *>(lrow + u0);
-#pragma unroll
-               for (int m = 0; m < (R + 4) / 4; ++m) {
-                  const int4 q4 = w4[m];
-                  pw[4 * m] = (uint32_t)q4.x; pw[4 * m + 1] = (uint32_t)q4.y;
-                  pw[4 * m + 2] = (uint32_t)q4.z; pw[4 * m + 3] = (uint32_t)q4.w;
-               }
-               uint32_t tq[4], mk[4];
-#pragma unroll
-               for (int k = 0; k < 4; ++k) {
-                  tq[k] = (uint32_t)trow[u0 + k];
-                  // bytes j of tap u0 + k + 4 j < tw: (rem - k + 3) / 4 of them
-                  const int nbytes = (rem - k + 3) >> 2;
-                  mk[k] = nbytes >= 4 ? 0xffffffffu : (1u << (8 * nbytes)) - 1u;
-               }
-#pragma unroll
-               for (int k = 0; k < 4; ++k) {
-                  if (k >= rem) break;
-#pragma unroll
-                  for (int r = 0; r < R; ++r)
-                     acc[r] = (ACC)__builtin_amdgcn_sad_u8(pw[r + k] & mk[k], tq[k], (uint32_t)acc[r]);
-               }
-            }
-            continue;
-         }
          // the template row in chunks of kIntU columns: kIntU template values and the
          // R + kIntU - 1 window values they meet, then R x kIntU taps (exact integer sums,
          // so the order is free); LDS columns used: colbase .. colbase + R + tw - 2 (the
@@ -693,17 +563,13 @@ __global__ __launch_bounds__(256) void prox_tile_int(const char *src, int W, int
                   const int4 v4 = w4[m];
                   sw[4 * m] = v4.x; sw[4 * m + 1] = v4.y; sw[4 * m + 2] = v4.z; sw[4 * m + 3] = v4.w;
                }
-#pragma unroll
-               for (int j = 0; j < 4 * NQ; ++j) sw[j] = sad_key<TOP, TYPE, ACC>(sw[j]);
                uint32_t q[NQ], tq[kIntU / 4];
 #pragma unroll
                for (int m = 0; m < NQ; ++m) q[m] = pack4(sw[4 * m], sw[4 * m + 1], sw[4 * m + 2], sw[4 * m + 3]);
 #pragma unroll
                for (int g = 0; g < kIntU / 4; ++g)
-                  tq[g] = pack4(sad_key<TOP, TYPE, ACC>(trow[u0 + 4 * g]),
-                                sad_key<TOP, TYPE, ACC>(trow[u0 + 4 * g + 1]),
-                                sad_key<TOP, TYPE, ACC>(trow[u0 + 4 * g + 2]),
-                                sad_key<TOP, TYPE, ACC>(trow[u0 + 4 * g + 3]));
+                  tq[g] = pack4(trow[u0 + 4 * g], trow[u0 + 4 * g + 1], trow[u0 + 4 * g + 2],
+                                trow[u0 + 4 * g + 3]);
 #pragma unroll
                for (int g = 0; g < kIntU / 4; ++g)
 #pragma unroll
@@ -711,7 +577,7 @@ __global__ __launch_bounds__(256) void prox_tile_int(const char *src, int W, int
                      const int j = r + 4 * g;
                      const uint32_t pj = (j & 3) == 0 ? q[j >> 2]
                                          : __builtin_amdgcn_alignbyte(q[(j >> 2) + 1], q[j >> 2], j & 3);
-                     acc[r] = itap4<TOP, TYPE>(acc[r], pj, tq[g]);
+                     acc[r] = itap4<TYPE>(acc[r], pj, tq[g]);
                   }
             }
          }
@@ -802,6 +668,197 @@ __global__ __launch_bounds__(256) void prox_tile_int(const char *src, int W, int
    }
 }
 
+// ------------------------------------------------------------------------- 8-bit AbsDistance
+// Exact int32 sums, four v_sad_u8 per 16 taps and output.  The staged tile holds, for each column c,
+// the dword P(c) of the keyed bytes (sad_key) of columns c, c + 4, c + 8, c + 12, so that the
+// taps u0 .. u0 + 15 of the output at window column x are |P(x + u0 + k) - Q(u0 + k)|, k < 4, bytewise,
+// with Q the template's bytes in the same order (sad8_template): no realignment by bytes.  A
+// group of four columns' P is the 4 x 4 byte transpose of 16 source bytes, so the tile is staged
+// from one 16-byte load (at any alignment) and eight byte permutes per group, straight into LDS.
+// Bound by VALU issue (sads) and the window reads.  1919x1079/31x23 46.7 -> 32.5 us, 4096^2/32x32
+// 260 -> 160 us against staging as int32, two LDS passes of repacking and a second template
+// launch.  8 outputs per thread at every size: 16 ran 4096^2/32x32 in 157 us, but 640x480/48x48 in
+// 54 instead of 38, 2500x2001/61x64 in 306 instead of 267.
+constexpr int kSad8R = 8;
+constexpr int sad8_blocks(int tw) { return (tw + 15) / 16; }
+// columns of P that a tile's outputs read, in whole groups
+constexpr int sad8_cols(int tw) { return kWaves * kSad8R + 16 * (sad8_blocks(tw) - 1) + 4; }
+
+__device__ __forceinline__ void transpose4x4(const uint32_t (&q)[4], uint32_t (&p)[4])
+{
+   const uint32_t t0 = __builtin_amdgcn_perm(q[1], q[0], 0x05010400u);   // 0 4 1 5
+   const uint32_t t1 = __builtin_amdgcn_perm(q[1], q[0], 0x07030602u);   // 2 6 3 7
+   const uint32_t t2 = __builtin_amdgcn_perm(q[3], q[2], 0x05010400u);   // 8 12 9 13
+   const uint32_t t3 = __builtin_amdgcn_perm(q[3], q[2], 0x07030602u);   // 10 14 11 15
+   p[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
+   p[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
+   p[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
+   p[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+}
+
+// Q of a template: four dwords per row and block of 16 columns, zero bytes past the row; channel
+// blockIdx.y of nch.  One thread per (row, block).
+template <int TYPE>
+__global__ __launch_bounds__(256) void sad8_template(const unsigned char *tpl, int tw, int th,
+                                                     int tstep, int nch, uint32_t *out)
+{
+   const int nb = sad8_blocks(tw);
+   const int i = blockIdx.x * 256 + threadIdx.x, ch = blockIdx.y;
+   if (i >= nb * th) return;
+   const int v = i / nb, b = i - v * nb;
+   const unsigned char *row = tpl + (size_t)v * tstep;
+   uint32_t q[4] = {0, 0, 0, 0}, p[4];
+#pragma unroll
+   for (int k = 0; k < 16; ++k) {
+      const int u = 16 * b + k;
+      const uint32_t t = u < tw ? row[u * nch + ch] ^ (TYPE == SImage::S8 ? 0x80u : 0u) : 0u;
+      q[k / 4] |= t << (8 * (k % 4));
+   }
+   transpose4x4(q, p);
+#pragma unroll
+   for (int k = 0; k < 4; ++k) out[((size_t)ch * th * nb + i) * 4 + k] = p[k];
+}
+
+// Channel blockIdx.y: its plane plane8 bytes after the one before, its Q likewise.
+template <int TYPE>
+__global__ __launch_bounds__(256) void prox_sad8(const unsigned char *src, int W, int H, int sstep,
+                                                 size_t plane8, const uint32_t *__restrict__ tq,
+                                                 int tw, int th, char *dst, int dstep, int nch,
+                                                 int vb, int ldsw)
+{
+   extern __shared__ uint32_t ldsp[];
+   constexpr int R = kSad8R;
+   constexpr uint32_t kKey = TYPE == SImage::S8 ? 0x80808080u : 0u;
+   typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
+   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ch = blockIdx.y;
+   const int tiles_x = (W + kWaves * R - 1) / (kWaves * R);
+   const int tile = xcd_tile(blockIdx.x, gridDim.x);
+   const int x0 = (tile % tiles_x) * (kWaves * R), y0 = (tile / tiles_x) * kTileRows;
+   const int nb = sad8_blocks(tw), gpr = sad8_cols(tw) / 4;
+   const int colbase = wave * R, sx0 = x0 - tw / 2;
+   src += ch * plane8;
+   tq += (size_t)ch * th * nb * 4;
+
+   uint32_t acc[R];
+#pragma unroll
+   for (int r = 0; r < R; ++r) acc[r] = 0;
+   for (int v0 = 0; v0 < th; v0 += vb) {
+      const int nv = min(vb, th - v0), sy0 = y0 - th / 2 + v0;
+      const int items = (kTileRows + nv - 1) * gpr;
+      __syncthreads();
+      {
+         // group i = r gpr + g, (r, g) stepped along with i; eight groups in flight
+         constexpr int K = 8;
+         const int dq = 256 / gpr, dr = 256 - dq * gpr;
+         int r = threadIdx.x / gpr, g = threadIdx.x - r * gpr;
+         for (int i0 = threadIdx.x; i0 < items; i0 += 256 * K) {
+            uint32_t q[K][4];
+            int at[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+               const int sx = sx0 + 4 * g, sy = sy0 + r;
+               at[k] = r * ldsw + 4 * g;
+               const bool rowin = i0 + 256 * k < items && sy >= 0 && sy < H;
+               const unsigned char *row = src + (size_t)(rowin ? sy : 0) * sstep;
+               if (rowin && sx >= 0 && sx + 16 <= W) {
+                  const u32x4_b b = *reinterpret_cast<const u32x4_b *>(row + sx);
+#pragma unroll
+                  for (int j = 0; j < 4; ++j) q[k][j] = b[j];
+               } else {
+#pragma unroll
+                  for (int j = 0; j < 4; ++j) q[k][j] = 0;
+                  if (rowin && sx + 16 > 0 && sx < W) {
+#pragma unroll
+                     for (int j = 0; j < 16; ++j) {
+                        const int x = sx + j;
+                        if (x >= 0 && x < W) q[k][j / 4] |= (uint32_t)row[x] << (8 * (j % 4));
+                     }
+                  }
+               }
+               g += dr;
+               r += dq;
+               if (g >= gpr) {
+                  g -= gpr;
+                  ++r;
+               }
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+               if (i0 + 256 * k >= items) break;
+               uint32_t p[4];
+#pragma unroll
+               for (int j = 0; j < 4; ++j) q[k][j] ^= kKey;
+               transpose4x4(q[k], p);
+               *reinterpret_cast<uint4 *>(ldsp + at[k]) = make_uint4(p[0], p[1], p[2], p[3]);
+            }
+         }
+      }
+      __syncthreads();
+      for (int v = 0; v < nv; ++v) {
+         const uint32_t *lrow = ldsp + (size_t)(lane + v) * ldsw + colbase;
+         const uint32_t *trow = tq + (size_t)(v0 + v) * nb * 4;
+         auto window = [&](int u0, uint32_t (&pw)[R + 4]) {
+            // (an empty asm with a memory clobber: each step reads its window afresh as 16-byte
+            // loads, rather than the compiler carrying one dword over from the step before
+            // and reading the rest as conflicting 4-byte loads)
+            asm volatile("" ::: "memory");
+            const uint4 *w4 = reinterpret_cast<const uint4 *>(lrow + u0);
+#pragma unroll
+            for (int m = 0; m < (R + 4) / 4; ++m) {
+               const uint4 a = w4[m];
+               pw[4 * m] = a.x; pw[4 * m + 1] = a.y; pw[4 * m + 2] = a.z; pw[4 * m + 3] = a.w;
+            }
+         };
+         int u0 = 0;
+         for (; u0 + 16 <= tw; u0 += 16) {
+            uint32_t pw[R + 4], t[4];
+            window(u0, pw);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) t[k] = trow[u0 / 4 + k];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+               for (int k = 0; k < 4; ++k) acc[r] = __builtin_amdgcn_sad_u8(pw[r + k], t[k], acc[r]);
+         }
+         if (u0 < tw) {
+            // a last block of 1 to 15 taps: dword k has the bytes j of the taps u0 + k + 4 j < tw,
+            // the others masked out of P (they are zero in Q)
+            const int rem = tw - u0;
+            uint32_t pw[R + 4];
+            window(u0, pw);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+               const int nbytes = (rem - k + 3) >> 2;
+               const uint32_t t = trow[u0 / 4 + k];
+               if (nbytes >= 4) {
+#pragma unroll
+                  for (int r = 0; r < R; ++r) acc[r] = __builtin_amdgcn_sad_u8(pw[r + k], t, acc[r]);
+               } else if (nbytes > 0) {
+                  const uint32_t mk = (1u << (8 * nbytes)) - 1u;
+#pragma unroll
+                  for (int r = 0; r < R; ++r)
+                     acc[r] = __builtin_amdgcn_sad_u8(pw[r + k] & mk, t, acc[r]);
+               }
+            }
+         }
+      }
+   }
+   const int oy = y0 + lane;
+   if (oy >= H) return;
+   float *drow = reinterpret_cast<float *>(dst + (size_t)oy * dstep);
+   const int ox = x0 + colbase;
+   if (nch == 1 && ox + R <= W) {
+#pragma unroll
+      for (int r = 0; r < R; r += 4)
+         *reinterpret_cast<f32x4_u *>(drow + ox + r) =
+             f32x4_u{(float)acc[r], (float)acc[r + 1], (float)acc[r + 2], (float)acc[r + 3]};
+      return;
+   }
+#pragma unroll
+   for (int r = 0; r < R; ++r)
+      if (ox + r < W) drow[(ox + r) * nch + ch] = (float)acc[r];
+}
+
 // ------------------------------------------------------------------------- direct
 template <int OP, int TYPE, class REALT, class STAGED>
 __global__ __launch_bounds__(256) void prox_direct(const char *src, int W, int H, int sstep,
@@ -888,6 +945,64 @@ bool prox_norm_from_tile(int op, const View &S, const View &T)
           (size_t)kLdsBudget;
 }
 
+// The tile of prox_sad8 in LDS: pitch and template rows per band (0: it does not fit)
+static void sad8_tile(int tw, int th, int &ldsw, int &vb)
+{
+   ldsw = sad8_cols(tw);
+   while (ldsw % 32 != 4) ldsw += 4;   // 16-byte reads of consecutive rows on different banks
+   vb = std::max(0, std::min(th, kLdsBudget / (ldsw * 4) - (kTileRows - 1)));
+}
+
+bool sad8_ok(int op, const View &S, const View &T)
+{
+   if (op != kSAD || (S.type != SImage::U8 && S.type != SImage::S8)) return false;
+   if (S.channels != 1 && S.channels != 2 && S.channels != 4) return false;
+   if (T.width <= 0 || T.height <= 0 || (long long)T.width * T.height * 65025LL >= (1LL << 31))
+      return false;   // int32 sums
+   int ldsw, vb;
+   sad8_tile(T.width, T.height, ldsw, vb);
+   return vb >= 1;
+}
+
+static size_t sad8_template_bytes(const View &T)
+{
+   return ((size_t)T.channels * T.height * sad8_blocks(T.width) * 16 + 255) / 256 * 256;
+}
+
+size_t sad8_work_bytes(const View &S, const View &T)
+{
+   return sad8_template_bytes(T) + planes8_bytes(S);
+}
+
+void launch_sad8(hipStream_t s, const View &image, const View &T, void *dst, int dstep, void *work)
+{
+   const int tw = T.width, th = T.height, nch = image.channels, R = kSad8R;
+   uint32_t *tq = static_cast<uint32_t *>(work);
+   View S = image;
+   size_t plane8 = 0;
+   if (nch > 1) S = launch_planes8(s, image, static_cast<char *>(work) + sad8_template_bytes(T), &plane8);
+   int ldsw, vb;
+   sad8_tile(tw, th, ldsw, vb);
+   const unsigned tiles = ((S.width + kWaves * R - 1) / (kWaves * R)) * ((S.height + kTileRows - 1) / kTileRows);
+   const size_t lds = (size_t)(kTileRows + vb - 1) * ldsw * 4;
+   const int items = sad8_blocks(tw) * th;
+   auto go = [&](auto prep, auto kernel) {
+      {
+         KernelTimer kt(s, "template_prep");
+         prep<<<dim3((items + 255) / 256, nch), 256, 0, s>>>(
+             static_cast<const unsigned char *>(T.ptr), tw, th, T.step, nch, tq);
+         launch_check("sad8_template");
+      }
+      KernelTimer kt(s, "prox_tile_int");
+      kernel<<<dim3(tiles, nch), 256, lds, s>>>(static_cast<const unsigned char *>(S.ptr), S.width,
+                                                S.height, S.step, plane8, tq, tw, th,
+                                                static_cast<char *>(dst), dstep, nch, vb, ldsw);
+      launch_check("prox_sad8");
+   };
+   if (S.type == SImage::U8) go(sad8_template<SImage::U8>, prox_sad8<SImage::U8>);
+   else go(sad8_template<SImage::S8>, prox_sad8<SImage::S8>);
+}
+
 void launch_proximity_flagged(hipStream_t s, const View &S, const View &T, void *dst, int dstep,
                               const void *tstage, int tpitch, const double *tsums,
                               const double *integ, const SplitFlags &f)
@@ -936,8 +1051,7 @@ static void launch_op(hipStream_t s, const View &S, const View &T, void *dst, in
    const long long taps = (long long)tw * th;
    const bool fits32 = bits8 ? taps * 65025LL < (1LL << 31)
                              : OP == kSAD && taps * 65535LL < (1LL << 31);
-   // AbsDistance on 8-bit sources with int32 sums stages 12 more columns (pack_sad8)
-   const int ldsw = lds_pitch(ncols + (OP == kSAD && bits8 && fits32 ? 12 : 0));
+   const int ldsw = lds_pitch(ncols);
    const int rows_fit = kLdsBudget / (ldsw * 4) - (kTileRows - 1);
    const bool tiled = S.type != SImage::F64 && rows_fit >= 1 && th > 0 && tw > 0;
 
@@ -984,18 +1098,6 @@ static void launch_op(hipStream_t s, const View &S, const View &T, void *dst, in
        tsums, integ, static_cast<char *>(dst), dstep, vb, ldsw)
 
    if (small_int) {
-      if (OP == kSAD && bits8 && fits32 && sad8_blocks(tw) > 0) {
-         // the packed template blocks of the tile's AbsDistance loop (in the staged template,
-         // which the next call stages again)
-         KernelTimer kt(s, "template_prep");
-         const int items = sad8_blocks(tw) * th;
-         int32_t *tp = static_cast<int32_t *>(const_cast<void *>(tstage));
-         OCIP_TYPE_SWITCH(S.type, TT, {
-            if constexpr (TT == SImage::U8 || TT == SImage::S8)
-               sad8_template_pack<TT><<<(items + 255) / 256, 256, 0, s>>>(tp, tpitch, tw, th);
-         });
-         launch_check("sad8_template_pack");
-      }
       KernelTimer kt(s, "prox_tile_int");
       OCIP_TYPE_SWITCH(S.type, TT, {
          if (fits32) {
