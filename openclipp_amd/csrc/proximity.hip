@@ -930,14 +930,25 @@ void launch_template_prep(hipStream_t s, const View &t, int channel, int pitch, 
    launch_check("template_prep");
 }
 
-// Output columns per lane of the tiled kernels
-static int tile_r(int W, int tw, int th) { return (W >= 2048 || tw * th >= 1024) ? 16 : 8; }
+// Output columns per lane of the tiled kernels: 8, twice the workgroups and less staged at once, or
+// 16, fewer LDS reads per tap, for images that fill the GPU with such tiles and templates of
+// up to 1024 taps (F32 CrossCorr 4096^2: 8x8 57 us with 16, 64 with 8; 64x64 1994, 1951; 640x480/48x48
+// SqrDistance 172, 104; 2500x2001/61x64 AbsDistance 856, 695).  The F32 Norm ops, whose window sums
+// come from tiles of 8 but from an integral with 16, take 16 only where the integral is the
+// smaller part (SqrDistance_Norm 4096^2: 8x8 282, 189; 16x16 297, 323; 2048^2/16x16 103, 81).
+static int tile_r(int op, const View &S, const View &T)
+{
+   const long long px = (long long)S.width * S.height, taps = (long long)T.width * T.height;
+   const bool norm = S.type == SImage::F32 && (op == kSSDNorm || op == kCCNorm);
+   if (taps >= 1024 || px < (norm ? 8 : 4) * (1 << 20) || (norm && taps < 200)) return 8;
+   return 16;
+}
 
 bool prox_norm_from_tile(int op, const View &S, const View &T)
 {
    if ((op != kSSDNorm && op != kCCNorm) || S.type != SImage::F32 || T.width <= 0 || T.height <= 0)
       return false;
-   const int R = tile_r(S.width, T.width, T.height);
+   const int R = tile_r(op, S, T);
    const int ldsw = lds_pitch(kWaves * R + T.width - 1);
    const int rows_fit = kLdsBudget / (ldsw * 4) - (kTileRows - 1);
    if (rows_fit < T.height) return false;   // one band
@@ -1027,7 +1038,7 @@ bool prox_template_in_place(int op, const View &S, const View &T, bool have_inte
 {
    constexpr int kTileTaps = 1024;
    if (S.type != SImage::F32 || S.channels != 1 || T.width <= 0 || T.height <= 0) return false;
-   const int ncols = kWaves * tile_r(S.width, T.width, T.height) + T.width - 1;
+   const int ncols = kWaves * tile_r(op, S, T) + T.width - 1;
    if (kLdsBudget / (lds_pitch(ncols) * 4) - (kTileRows - 1) < 1) return false;   // prox_direct
    const bool norm = op == kSSDNorm || op == kCCNorm;
    return !norm || (!have_integral && T.width * T.height <= kTileTaps);
@@ -1042,7 +1053,7 @@ static void launch_op(hipStream_t s, const View &S, const View &T, void *dst, in
    const char *src = static_cast<const char *>(S.ptr);
    const bool small_int = S.type == SImage::U8 || S.type == SImage::S8 ||
                           S.type == SImage::U16 || S.type == SImage::S16;
-   const int R = tile_r(W, tw, th);
+   const int R = tile_r(OP, S, T);
    const int ncols = kWaves * R + tw - 1;
    // int32 accumulation is exact when taps * max|term| < 2^31: 8-bit sources up to 33025
    // taps, and AbsDistance on 16-bit sources up to 32768 taps; the other 16-bit cases
