@@ -981,21 +981,23 @@ static int int_max_product(int type) { return type == SImage::U8 ? 255 * 255 : 1
 
 // Window sums of s^2 of an 8-bit image, exact in int32, into the map `dst` (as int32 bits):
 // SS(x, y) = sum over the template window of (x, y) (origin (-tw/2, -th/2), zero outside the
-// image).  One wavefront per 64 output columns and a band of kBoxBand output rows, streaming
-// down the band's th - 1 + kBoxBand source rows.  For each row:
-//  * the squares q of its 63 + tw columns from x0 - tw/2, two adjacent columns per lane (NCH
-//    chunks of 128 columns; zero outside the image through the range of a buffer resource);
-//  * their exclusive prefix along the row, P[i] = sum of q over columns < i: a wavefront
-//    inclusive scan of the lanes' pair sums (DPP row shifts and row broadcasts), the chunk
-//    carry through readlane; integers, exact;
-//  * for output column x0 + x (lane x from here on), R(x) = P[x + tw] - P[x], both prefixes
-//    fetched from the lanes that hold them with ds_bpermute;
-//  * a per-lane ring of the last th rows' R in LDS: V += R - R(th rows up); from the th-th
-//    row on, V is the sum of the output row th - 1 rows up, stored as one 256-byte row segment.
-// Integer arithmetic throughout (every value below 2^31, checked by the host), so the sums are
-// exact in any order.
-constexpr int kBoxBand = 64;
-constexpr int kBoxOob = 0x40000000;   // a byte offset past any image this kernel takes
+// image).  One wavefront per band of box_band(th) output rows and 256 source columns, four adjacent
+// ones per lane, i.e. box_cols(tw) output columns:
+//  * each lane's four column sums of squares over the window's rows, running down the band: the
+//    squares of the rows entering the window (a dword each) less those of the rows leaving it;
+//  * per output row the inclusive prefix I of the column sums along the row: the lane's own four,
+//    a wavefront scan of the lanes' totals (DPP row shifts and broadcasts; U rows at once), then
+//    SS(i) = I[i + tw - 1] - I[i - 1]: the subtrahends are the lane's own, the minuends come through
+//    LDS; one 16-byte store per lane and row.
+// Integer arithmetic modulo 2^32 throughout and every result below 2^31 (checked by the host), so
+// the sums are exact in any order.  Bound by issue and the map's store: about 44 instructions per
+// row and 225 outputs (tw = 32) where a lane per output column with a ring of row sums in LDS
+// took 35 per 64 (4096^2/32x32: 38 -> 22 us).
+// Output rows per wavefront: 16, or 32 where the th - 1 rows before the first would outweigh them
+// (more wavefronts hide the chains' latency: colour 1280x960/24x24 15 us with 16, 18 with 32, 25 with 64)
+constexpr int box_band(int th) { return th <= 48 ? 16 : 32; }
+constexpr int kBoxOob = 0x40000000;   // a byte count past any image this kernel takes
+constexpr int box_cols(int tw) { return (256 - (tw - 1)) / 4 * 4; }
 
 // Inclusive scans across the 64 lanes of N values at once (the N scans interleaved, so that
 // each DPP step's wait on the previous one is filled by the others): within rows of 16 lanes
@@ -1018,147 +1020,108 @@ __device__ __forceinline__ void wave_incl_scan(int (&x)[N])
    for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x143, 0xc, 0xf, false);
 }
 
-template <int NCH, bool SIGNED, bool BST>
+template <bool SIGNED>
 __global__ __launch_bounds__(64) void ss_box8(const unsigned char *__restrict__ src, int W,
                                               int H, int sstep, int tw, int th,
                                               char *__restrict__ dst, int dstep, int bands,
                                               size_t plane8, size_t planef)
 {
-   extern __shared__ int ring[];   // th x 64: lane's R of the last th rows
-   constexpr int U = 8;            // rows per batch of loads (two batches in flight)
+   constexpr int U = 4;                          // rows at once (their loads one batch ahead)
+   __shared__ int pre[U][256 + 100];             // (lanes past the outputs read up to tw + 2 past 256)
+   typedef uint32_t u32_u __attribute__((aligned(1)));
+   typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
    const int lane = threadIdx.x;
    // consecutive blocks (one XCD's run) side by side along a band share halo columns in L2
    const int b = xcd_tile(blockIdx.x, gridDim.x);
    // blockIdx.y = channel
    src += blockIdx.y * plane8;
    dst += blockIdx.y * planef;
-   const int cblks = gridDim.x / bands;
+   const int cblks = gridDim.x / bands, cols = box_cols(tw);
    const int band = b / cblks, cblk = b % cblks;
-   const int x0 = cblk * 64, y0 = band * kBoxBand;
+   const int x0 = cblk * cols, y0 = band * box_band(th);
    const int cx = tw / 2, cy = th / 2;
-   const int n = min(kBoxBand, H - y0);
-   const int steps = n + th - 1;
-   // lane holds columns x0 - cx + 128 k + 2 lane + e (e = 0, 1) of chunk k
-   int coff[NCH][2];
+   const int n = min(box_band(th), H - y0);
+   // the lane's columns c .. c + 3 from the dword at column min(max(c, 0), W - 4), shifted into
+   // place, zero outside the image (mask 0: wholly outside)
+   const int c = x0 - cx + 4 * lane, cl = min(max(c, 0), W - 4);
+   const int lsh = min(max(-c, 0), 3) * 8, rsh = min(max(c - cl, 0), 3) * 8;
+   const uint32_t mask = c <= -4 || c >= W ? 0u : 0xffffffffu;
+   auto load = [&](int y) -> uint32_t {
+      return *reinterpret_cast<const u32_u *>(src + (size_t)min(max(y, 0), H - 1) * sstep + cl);
+   };
+   auto place = [&](uint32_t v, int y) -> uint32_t {
+      return (unsigned)y < (unsigned)H ? (v << lsh) >> rsh & mask : 0u;
+   };
+   auto elem = [&](uint32_t v, int e) -> int {
+      return SIGNED ? (int)(v << (24 - 8 * e)) >> 24 : (int)(v >> (8 * e) & 0xffu);
+   };
+   // column sums lead - lag: squares are only ever added (sums that took squares off were compiled
+   // into byte dot products that added them)
+   int lead[4] = {0, 0, 0, 0}, lag[4] = {0, 0, 0, 0};
+   // the th - 1 rows before the first output row's last
+   for (int j0 = 0; j0 < th - 1; j0 += 8) {
+      uint32_t v[8];
 #pragma unroll
-   for (int k = 0; k < NCH; ++k)
+      for (int j = 0; j < 8; ++j) v[j] = load(y0 - cy + j0 + j);
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-         const int c = x0 - cx + 128 * k + 2 * lane + e;
-         coff[k][e] = c >= 0 && c < W ? c : kBoxOob;
+      for (int j = 0; j < 8; ++j) {
+         const uint32_t q = j0 + j < th - 1 ? place(v[j], y0 - cy + j0 + j) : 0u;
+#pragma unroll
+         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(q, e), elem(q, e));
       }
-   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-       const_cast<unsigned char *>(src), (short)0, H * sstep, 0x00020000);
-   // (bytes kept as loaded until used, so that the loop carries no conversion that would wait
-   // for the loads in flight).  A row outside the image takes the row offset 2 kBoxOob, a
-   // column outside it the column offset kBoxOob: every sum with either is past the range (and
-   // below 2^32); rows past the band's last step load real rows whose sums are never used.
-   auto load = [&](int j0, unsigned char (&v)[U][NCH][2]) {
+   }
+   uint32_t in[U], out[U];
+   auto fetch = [&](int r) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-         const int sy = y0 - cy + j0 + u;
-         const unsigned roff = (unsigned)sy < (unsigned)H ? (unsigned)(sy * sstep) : 2u * kBoxOob;
-#pragma unroll
-         for (int k = 0; k < NCH; ++k)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-               const unsigned o = roff + (unsigned)coff[k][e];
-               v[u][k][e] = __builtin_amdgcn_raw_buffer_load_b8(rsrc, (int)o, 0, 0);
-            }
+         in[u] = load(y0 - cy + th - 1 + r + u);
+         out[u] = load(y0 - cy + r + u);
       }
    };
-   // P[x] at lane x / 2 of chunk 0 (element x % 2); P[x + tw] at lane ((x + tw) % 128) / 2
-   // of chunk (x + tw) / 128 (element (x + tw) % 2)
-   const int ia = lane, ib = lane + tw;
-   const int la = (ia >> 1) * 4, lb = ((ib & 127) >> 1) * 4;
-   const bool oa = ia & 1, ob = ib & 1, cb = ib >= 128;
-   int *const myring = ring + lane;
-   int V = 0, slot = 0;
-   // BST (maps of fewer than kBoxOob bytes): buffer stores, the column offset kBoxOob past
-   // the image's width dropping a lane's store; otherwise stores through a pointer
-   int *orow = reinterpret_cast<int *>(dst + (size_t)y0 * dstep) + x0 + lane;
-   const bool xin = x0 + lane < W;
-   const __amdgpu_buffer_rsrc_t drsrc =
-       __builtin_amdgcn_make_buffer_rsrc(dst, (short)0, BST ? H * dstep : 0, 0x00020000);
-   const int xoff = xin ? (x0 + lane) * 4 : kBoxOob;
-   int yoff = y0 * dstep;
-   unsigned char va[U][NCH][2], vb[U][NCH][2];
-   auto process = [&](int j0, const unsigned char (&v)[U][NCH][2]) {
-      // the batch's row sums first (independent rows: their scans and lane exchanges
-      // interleave, two rows at a time; rows past the band read real rows or zeros, and their
-      // sums are never used), then the ring and the running sums in order
-      int R[U];
-#pragma unroll
-      for (int u = 0; u < U; u += 2) {
-         int q0[2 * NCH], t[2 * NCH], inc[2 * NCH];
-#pragma unroll
-         for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int k = 0; k < NCH; ++k) {
-               int e0 = v[u + h][k][0], e1 = v[u + h][k][1];
-               if (SIGNED) {
-                  e0 = (int)(signed char)e0;
-                  e1 = (int)(signed char)e1;
-               }
-               q0[h * NCH + k] = e0 * e0;
-               t[h * NCH + k] = inc[h * NCH + k] = e0 * e0 + e1 * e1;
-            }
-         wave_incl_scan<2 * NCH>(inc);
-#pragma unroll
-         for (int h = 0; h < 2; ++h) {
-            int E0[NCH], E1[NCH];
-            int carry = 0;
-#pragma unroll
-            for (int k = 0; k < NCH; ++k) {
-               const int i = inc[h * NCH + k] + carry;
-               E0[k] = i - t[h * NCH + k];
-               E1[k] = E0[k] + q0[h * NCH + k];
-               carry = __builtin_amdgcn_readlane(i, 63);
-            }
-            const int a0 = __builtin_amdgcn_ds_bpermute(la, E0[0]);
-            const int a1 = __builtin_amdgcn_ds_bpermute(la, E1[0]);
-            int b0 = __builtin_amdgcn_ds_bpermute(lb, E0[0]);
-            int b1 = __builtin_amdgcn_ds_bpermute(lb, E1[0]);
-            if constexpr (NCH == 2) {
-               // P[x + tw] in chunk 1 for the lanes with x + tw >= 128
-               const int c0 = __builtin_amdgcn_ds_bpermute(lb, E0[1]);
-               const int c1 = __builtin_amdgcn_ds_bpermute(lb, E1[1]);
-               b0 = cb ? c0 : b0;
-               b1 = cb ? c1 : b1;
-            }
-            R[u + h] = (ob ? b1 : b0) - (oa ? a1 : a0);
-         }
-      }
+   fetch(0);
+   const int x = x0 + 4 * lane;
+   const bool mine = 4 * lane < cols && x < W;
+   for (int r0 = 0; r0 < n; r0 += U) {
+      int q[U][4], inc[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-         const int j = j0 + u;
-         if (j >= steps) break;
-         const int old = myring[slot * 64];
-         myring[slot * 64] = R[u];
-         V += R[u] - (j >= th ? old : 0);
-         if (++slot == th) slot = 0;
-         if (j >= th - 1) {
-            if (BST) {
-               __builtin_amdgcn_raw_buffer_store_b32(V, drsrc, (int)((unsigned)yoff + (unsigned)xoff), 0, 0);
-               yoff += dstep;
-            } else {
-               if (xin) *orow = V;
-               orow = reinterpret_cast<int *>(reinterpret_cast<char *>(orow) + dstep);
-            }
+         const uint32_t a = place(in[u], y0 - cy + th - 1 + r0 + u), o = place(out[u], y0 - cy + r0 + u);
+#pragma unroll
+         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(a, e), elem(a, e));
+         q[u][0] = lead[0] - lag[0];
+#pragma unroll
+         for (int e = 1; e < 4; ++e) q[u][e] = q[u][e - 1] + (lead[e] - lag[e]);
+         inc[u] = q[u][3];
+#pragma unroll
+         for (int e = 0; e < 4; ++e) lag[e] += __mul24(elem(o, e), elem(o, e));
+      }
+      if (r0 + U < n) fetch(r0 + U);
+      wave_incl_scan<U>(inc);
+      __syncthreads();   // the reads of the batch before are done
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         inc[u] -= q[u][3];   // the sums of the lanes before
+         *reinterpret_cast<int4 *>(&pre[u][4 * lane]) =
+             make_int4(inc[u] + q[u][0], inc[u] + q[u][1], inc[u] + q[u][2], inc[u] + q[u][3]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         const int *p = &pre[u][4 * lane + tw - 1];
+         const int s0 = p[0] - inc[u], s1 = p[1] - inc[u] - q[u][0], s2 = p[2] - inc[u] - q[u][1],
+                   s3 = p[3] - inc[u] - q[u][2];
+         if (!mine || r0 + u >= n) continue;
+         int *o = reinterpret_cast<int *>(dst + (size_t)(y0 + r0 + u) * dstep) + x;
+         if (x + 4 <= W) {
+            *reinterpret_cast<i32x4_u *>(o) = i32x4_u{s0, s1, s2, s3};
+         } else {
+            o[0] = s0;
+            if (x + 1 < W) o[1] = s1;
+            if (x + 2 < W) o[2] = s2;
          }
       }
-   };
-   load(0, va);
-   for (int j0 = 0; j0 < steps; j0 += 2 * U) {
-      load(j0 + U, vb);
-      process(j0, va);
-      load(j0 + 2 * U, va);
-      process(j0 + U, vb);
    }
 }
-
-// chunks of 128 columns: P up to index 63 + tw (the 63 + tw staged columns and one past)
-static int ss_box8_chunks(int tw) { return 63 + tw < 128 ? 1 : 2; }
 
 // Interleaved 8-bit channels into planes of their own (row pitch plane8_step, plane pitch H rows),
 // zeros between the width and the pitch, and the planes of the map back into interleaved
@@ -1260,8 +1223,8 @@ bool int_mfma_ok(int op, const View &S, const View &T)
    if ((S.type != SImage::U8 && S.type != SImage::S8) || T.type != S.type) return false;
    if (S.channels != 1 && S.channels != 2 && S.channels != 4) return false;
    const int tw = T.width, th = T.height;
-   // (templates of one column block; ss_box8: byte offsets of the image below kBoxOob)
-   if (tw <= 0 || th <= 0 || tw > 97 || th > 97) return false;
+   // (templates of one column block; ss_box8: dwords of four columns)
+   if (tw <= 0 || th <= 0 || tw > 97 || th > 97 || (S.width < 4 && op != kCC)) return false;
    if ((long long)S.height * std::max((long long)S.step, (long long)plane8_step(S.width)) >= kBoxOob)
       return false;
    const long long mp = int_max_product(S.type);
@@ -1298,26 +1261,15 @@ void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, do
    if (op != kCC) {
       // the window sums of s^2 go to the map first; the MFMA kernel's epilogue reads them
       KernelTimer kt(s, "ss_box8");
-      const int bands = (S.height + kBoxBand - 1) / kBoxBand;
-      const int cblks = (S.width + 63) / 64;
-      const size_t lds = (size_t)th * 64 * sizeof(int);   // th <= 97: below 64 KiB
+      const int bands = (S.height + box_band(th) - 1) / box_band(th);
+      const int cblks = (S.width + box_cols(tw) - 1) / box_cols(tw);
       auto go = [&](auto kernel) {
-         kernel<<<dim3(bands * cblks, nch), 64, lds, s>>>(static_cast<const unsigned char *>(S.ptr),
-                                                         S.width, S.height, S.step, tw, th,
-                                                         reinterpret_cast<char *>(map), mstep,
-                                                         bands, plane8, planef);
+         kernel<<<dim3(bands * cblks, nch), 64, 0, s>>>(static_cast<const unsigned char *>(S.ptr),
+                                                       S.width, S.height, S.step, tw, th,
+                                                       reinterpret_cast<char *>(map), mstep, bands,
+                                                       plane8, planef);
       };
-      const bool sgn = src8 == mfma::kSrcS8;
-      const bool bst = (long long)S.height * mstep < kBoxOob;
-#define OCIP_BOX_CASE(NCH)                                                                      \
-   if (sgn) { if (bst) go(ss_box8<NCH, true, true>); else go(ss_box8<NCH, true, false>); }      \
-   else { if (bst) go(ss_box8<NCH, false, true>); else go(ss_box8<NCH, false, false>); }
-      if (ss_box8_chunks(tw) == 1) {
-         OCIP_BOX_CASE(1)
-      } else {
-         OCIP_BOX_CASE(2)
-      }
-#undef OCIP_BOX_CASE
+      if (src8 == mfma::kSrcS8) go(ss_box8<true>); else go(ss_box8<false>);
       launch_check("ss_box8");
    }
    u16x8 *g0 = static_cast<u16x8 *>(work);
