@@ -946,6 +946,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
       // sum of squares SS, an exact int32 that ss_box8 left in the map), as prox_tile_int forms
       // it; four consecutive columns per thread, one 16-byte store where the row allows
       const double tt = a.tsums[0];
+      const int itt = (int)tt;
 #pragma unroll
       for (int i = 0; i < kIntIters; ++i) {
          const int k = threadIdx.x + 256 * i;
@@ -959,14 +960,12 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
          float v[4];
 #pragma unroll
          for (int e = 0; e < 4; ++e) {
-            if (a.op == kCC) {
-               v[e] = (float)ci[e];
-            } else {
-               const double ss = (double)si[e];
-               const double cd = (double)ci[e];
-               const double d = (a.op == kSSD || a.op == kSSDNorm) ? ss - 2.0 * cd + tt : cd;
-               v[e] = a.op == kSSD ? (float)d : (float)(d / sqrt(ss * tt));
-            }
+            // (every sum is an exact integer below 2^31, so int32 arithmetic rounds to float as
+            // the FP64 expression does)
+            const int d = a.op == kSSD || a.op == kSSDNorm ? si[e] - 2 * ci[e] + itt : ci[e];
+            v[e] = a.op == kCC || a.op == kSSD
+                       ? (float)d
+                       : (float)((double)d * rsqrt64((double)si[e] * tt));
          }
          if (x + 4 <= a.W) {
             *reinterpret_cast<gmem_f32x4 *>(o) = f32x4_t{v[0], v[1], v[2], v[3]};

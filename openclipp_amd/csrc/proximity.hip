@@ -650,7 +650,7 @@ __global__ __launch_bounds__(256) void prox_tile_int(const char *src, int W, int
          for (int r = 0; r < 4; ++r) {
             const double c = (double)acc[g + r];
             const double d = kViaCC ? ss[r] - 2.0 * c + tt : c;
-            const float v = OP == kSSD ? (float)d : (float)(d / sqrt(ss[r] * tt));
+            const float v = OP == kSSD ? (float)d : (float)(d * rsqrt64(ss[r] * tt));
             const int ox = x0 + colbase + g + r;
             if (ox < W) drow[ox * nch + ch] = v;
          }
