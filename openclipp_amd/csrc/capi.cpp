@@ -167,11 +167,19 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
    // SqrDistance on 8-bit sources is formed from the cross term and the window sums of
    // squares, which come from the integral as for the Norm ops
    const bool ssd8 = op == kSSD && (type == SImage::U8 || type == SImage::S8);
-   // 8-bit integer images: exact sums on BF16 MFMA where the path applies
+   // integer images: exact sums on int8 MFMA where the paths apply
    if (precision == ocipPrecisionF32 && int_mfma_ok(op, view(S), view(T))) {
       c.stats.ensure(int_mfma_work_bytes(view(S), view(T)));
-      launch_int_mfma(c.stream, op, view(S), view(T), c.tmpl.sums.as<double>(),
-                      static_cast<float *>(D.dev), D.desc.Step, c.stats.ptr);
+      launch_int_mfma(c.stream, op, view(S), view(T), static_cast<float *>(D.dev), D.desc.Step,
+                      c.stats.ptr);
+      D.in_device = true;
+      return;
+   }
+   if (precision == ocipPrecisionF32 && int16_mfma_ok(op, view(S), view(T))) {
+      c.stats.ensure(i8_work_bytes(view(T)));
+      const double *integ = norm ? sqr_integral_for(c, S, 0) : nullptr;
+      launch_int16_mfma(c.stream, op, view(S), view(T), integ, static_cast<float *>(D.dev),
+                        D.desc.Step, c.stats.ptr);
       D.in_device = true;
       return;
    }

@@ -970,350 +970,6 @@ SplitFlags launch_split_ncc(hipStream_t s, const View &S, const View &T, const d
    return SplitFlags{any, any + 1, (int)L.grid.x, 16 * NT, mfma::kPairRows};
 }
 
-// ======================================================================= exact integer sums
-// 8-bit integer images through the row-pair kernel (kModeInt): the exact cross term of
-// CrossCorr, CrossCorr_Norm, SqrDistance and SqrDistance_Norm on BF16 MFMA, and the window
-// sums of s^2 from ss_box8.  Limits: templates up to 97 x 97 (one template column block, and
-// the rows ss_box8 stages), one row's products below 2^24 (the flush period is at least one
-// step) and the whole sum below 2^31 (int32), the LDS tiles.  OCIP_INT_MFMA=0 turns the
-// path off (the VALU kernel prox_tile_int then computes the same maps).
-static int int_max_product(int type) { return type == SImage::U8 ? 255 * 255 : 128 * 128; }
-
-// Window sums of s^2 of an 8-bit image, exact in int32, into the map `dst` (as int32 bits):
-// SS(x, y) = sum over the template window of (x, y) (origin (-tw/2, -th/2), zero outside the
-// image).  One wavefront per band of box_band(th) output rows and 256 source columns, four adjacent
-// ones per lane, i.e. box_cols(tw) output columns:
-//  * each lane's four column sums of squares over the window's rows, running down the band: the
-//    squares of the rows entering the window (a dword each) less those of the rows leaving it;
-//  * per output row the inclusive prefix I of the column sums along the row: the lane's own four,
-//    a wavefront scan of the lanes' totals (DPP row shifts and broadcasts; U rows at once), then
-//    SS(i) = I[i + tw - 1] - I[i - 1]: the subtrahends are the lane's own, the minuends come through
-//    LDS; one 16-byte store per lane and row.
-// Integer arithmetic modulo 2^32 throughout and every result below 2^31 (checked by the host), so
-// the sums are exact in any order.  Bound by issue and the map's store: about 44 instructions per
-// row and 225 outputs (tw = 32) where a lane per output column with a ring of row sums in LDS
-// took 35 per 64 (4096^2/32x32: 38 -> 22 us).
-// Output rows per wavefront: 16, or 32 where the th - 1 rows before the first would outweigh them
-// (more wavefronts hide the chains' latency: colour 1280x960/24x24 15 us with 16, 18 with 32, 25 with 64)
-constexpr int box_band(int th) { return th <= 48 ? 16 : 32; }
-constexpr int kBoxOob = 0x40000000;   // a byte count past any image this kernel takes
-constexpr int box_cols(int tw) { return (256 - (tw - 1)) / 4 * 4; }
-
-// Inclusive scans across the 64 lanes of N values at once (the N scans interleaved, so that
-// each DPP step's wait on the previous one is filled by the others): within rows of 16 lanes
-// (lanes without a source add 0), then rows 1 and 3 take the last lane of rows 0 and 2, rows
-// 2 and 3 the last lane of row 1.
-template <int N>
-__device__ __forceinline__ void wave_incl_scan(int (&x)[N])
-{
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x111, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x112, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x114, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x118, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x142, 0xa, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x143, 0xc, 0xf, false);
-}
-
-template <bool SIGNED>
-__global__ __launch_bounds__(64) void ss_box8(const unsigned char *__restrict__ src, int W,
-                                              int H, int sstep, int tw, int th,
-                                              char *__restrict__ dst, int dstep, int bands,
-                                              size_t plane8, size_t planef)
-{
-   constexpr int U = 4;                          // rows at once (their loads one batch ahead)
-   __shared__ int pre[U][256 + 100];             // (lanes past the outputs read up to tw + 2 past 256)
-   typedef uint32_t u32_u __attribute__((aligned(1)));
-   typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
-   const int lane = threadIdx.x;
-   // consecutive blocks (one XCD's run) side by side along a band share halo columns in L2
-   const int b = xcd_tile(blockIdx.x, gridDim.x);
-   // blockIdx.y = channel
-   src += blockIdx.y * plane8;
-   dst += blockIdx.y * planef;
-   const int cblks = gridDim.x / bands, cols = box_cols(tw);
-   const int band = b / cblks, cblk = b % cblks;
-   const int x0 = cblk * cols, y0 = band * box_band(th);
-   const int cx = tw / 2, cy = th / 2;
-   const int n = min(box_band(th), H - y0);
-   // the lane's columns c .. c + 3 from the dword at column min(max(c, 0), W - 4), shifted into
-   // place, zero outside the image (mask 0: wholly outside)
-   const int c = x0 - cx + 4 * lane, cl = min(max(c, 0), W - 4);
-   const int lsh = min(max(-c, 0), 3) * 8, rsh = min(max(c - cl, 0), 3) * 8;
-   const uint32_t mask = c <= -4 || c >= W ? 0u : 0xffffffffu;
-   auto load = [&](int y) -> uint32_t {
-      return *reinterpret_cast<const u32_u *>(src + (size_t)min(max(y, 0), H - 1) * sstep + cl);
-   };
-   auto place = [&](uint32_t v, int y) -> uint32_t {
-      return (unsigned)y < (unsigned)H ? (v << lsh) >> rsh & mask : 0u;
-   };
-   auto elem = [&](uint32_t v, int e) -> int {
-      return SIGNED ? (int)(v << (24 - 8 * e)) >> 24 : (int)(v >> (8 * e) & 0xffu);
-   };
-   // column sums lead - lag: squares are only ever added (sums that took squares off were compiled
-   // into byte dot products that added them)
-   int lead[4] = {0, 0, 0, 0}, lag[4] = {0, 0, 0, 0};
-   // the th - 1 rows before the first output row's last
-   for (int j0 = 0; j0 < th - 1; j0 += 8) {
-      uint32_t v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = load(y0 - cy + j0 + j);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-         const uint32_t q = j0 + j < th - 1 ? place(v[j], y0 - cy + j0 + j) : 0u;
-#pragma unroll
-         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(q, e), elem(q, e));
-      }
-   }
-   uint32_t in[U], out[U];
-   auto fetch = [&](int r) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         in[u] = load(y0 - cy + th - 1 + r + u);
-         out[u] = load(y0 - cy + r + u);
-      }
-   };
-   fetch(0);
-   const int x = x0 + 4 * lane;
-   const bool mine = 4 * lane < cols && x < W;
-   for (int r0 = 0; r0 < n; r0 += U) {
-      int q[U][4], inc[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         const uint32_t a = place(in[u], y0 - cy + th - 1 + r0 + u), o = place(out[u], y0 - cy + r0 + u);
-#pragma unroll
-         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(a, e), elem(a, e));
-         q[u][0] = lead[0] - lag[0];
-#pragma unroll
-         for (int e = 1; e < 4; ++e) q[u][e] = q[u][e - 1] + (lead[e] - lag[e]);
-         inc[u] = q[u][3];
-#pragma unroll
-         for (int e = 0; e < 4; ++e) lag[e] += __mul24(elem(o, e), elem(o, e));
-      }
-      if (r0 + U < n) fetch(r0 + U);
-      wave_incl_scan<U>(inc);
-      __syncthreads();   // the reads of the batch before are done
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         inc[u] -= q[u][3];   // the sums of the lanes before
-         *reinterpret_cast<int4 *>(&pre[u][4 * lane]) =
-             make_int4(inc[u] + q[u][0], inc[u] + q[u][1], inc[u] + q[u][2], inc[u] + q[u][3]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         const int *p = &pre[u][4 * lane + tw - 1];
-         const int s0 = p[0] - inc[u], s1 = p[1] - inc[u] - q[u][0], s2 = p[2] - inc[u] - q[u][1],
-                   s3 = p[3] - inc[u] - q[u][2];
-         if (!mine || r0 + u >= n) continue;
-         int *o = reinterpret_cast<int *>(dst + (size_t)(y0 + r0 + u) * dstep) + x;
-         if (x + 4 <= W) {
-            *reinterpret_cast<i32x4_u *>(o) = i32x4_u{s0, s1, s2, s3};
-         } else {
-            o[0] = s0;
-            if (x + 1 < W) o[1] = s1;
-            if (x + 2 < W) o[2] = s2;
-         }
-      }
-   }
-}
-
-// Interleaved 8-bit channels into planes of their own (row pitch plane8_step, plane pitch H rows),
-// zeros between the width and the pitch, and the planes of the map back into interleaved
-// channels: the kernels between them take every channel of an image in one launch, as
-// 1-channel images with wide loads and stores (with the channels' maps interleaved by those
-// kernels themselves, 4 bytes of every 16 a store, the row-pair kernel ran 60 instead of 40 us
-// at 1280x960/24x24).  Four pixels per thread.  Bound by HBM: 2 W H NCH and 8 W H NCH bytes.
-static int plane8_step(int W) { return (W + 15) / 16 * 16; }
-
-template <int NCH>
-__global__ __launch_bounds__(256) void split_planes8(const unsigned char *__restrict__ src, int W,
-                                                     int H, int sstep,
-                                                     unsigned char *__restrict__ dst, int dstep)
-{
-   const int k = blockIdx.x * 256 + threadIdx.x, groups = dstep / 4;
-   const int y = k / groups, x = 4 * (k - y * groups);
-   if (y >= H) return;
-   const unsigned char *row = src + (size_t)y * sstep;
-   uint32_t q[NCH];   // the 4 NCH bytes of the thread's pixels
-   if (x + 4 <= W) {
-      typedef uint32_t u32_u __attribute__((aligned(1)));
-#pragma unroll
-      for (int i = 0; i < NCH; ++i) q[i] = reinterpret_cast<const u32_u *>(row + x * NCH)[i];
-   } else {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i) q[i] = 0;
-#pragma unroll
-      for (int i = 0; i < 4 * NCH; ++i)
-         if (x + i / NCH < W) q[i / 4] |= (uint32_t)row[x * NCH + i] << (8 * (i % 4));
-   }
-#pragma unroll
-   for (int c = 0; c < NCH; ++c) {
-      uint32_t v = 0;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-         const int i = p * NCH + c;
-         v |= (q[i / 4] >> (8 * (i % 4)) & 0xffu) << (8 * p);
-      }
-      *reinterpret_cast<uint32_t *>(dst + ((size_t)c * H + y) * dstep + x) = v;
-   }
-}
-
-template <int NCH>
-__global__ __launch_bounds__(256) void join_planes(const float *__restrict__ src, int W, int H,
-                                                   int sstep, float *__restrict__ dst, int dstep)
-{
-   const int k = blockIdx.x * 256 + threadIdx.x, groups = sstep / 16;
-   const int y = k / groups, x = 4 * (k - y * groups);
-   if (y >= H) return;
-   float v[4 * NCH];
-#pragma unroll
-   for (int c = 0; c < NCH; ++c) {
-      const float4 q = *reinterpret_cast<const float4 *>(
-          reinterpret_cast<const char *>(src) + ((size_t)c * H + y) * sstep + 4 * x);
-      v[c] = q.x; v[NCH + c] = q.y; v[2 * NCH + c] = q.z; v[3 * NCH + c] = q.w;
-   }
-   float *d = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + (size_t)y * dstep) + x * NCH;
-   if (x + 4 <= W) {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i)
-         reinterpret_cast<f32x4_u *>(d)[i] = f32x4_u{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-   } else {
-#pragma unroll
-      for (int i = 0; i < 4 * NCH; ++i)
-         if (x + i / NCH < W) d[i] = v[i];
-   }
-}
-
-// one thread per 4 columns of a plane
-static unsigned plane_blocks(int H, int step) { return (unsigned)(((long long)H * (step / 4) + 255) / 256); }
-
-size_t planes8_bytes(const View &S)
-{
-   return S.channels > 1 ? (size_t)S.channels * S.height * plane8_step(S.width) : 0;
-}
-
-View launch_planes8(hipStream_t s, const View &image, void *planes, size_t *plane8)
-{
-   KernelTimer kt(s, "split_planes8");
-   View S = image;
-   S.ptr = planes;
-   S.step = plane8_step(image.width);
-   S.channels = 1;
-   *plane8 = (size_t)S.height * S.step;
-   auto go = [&](auto kernel) {
-      kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(
-          static_cast<const unsigned char *>(image.ptr), S.width, S.height, image.step,
-          static_cast<unsigned char *>(planes), S.step);
-   };
-   if (image.channels == 2) go(split_planes8<2>); else go(split_planes8<4>);
-   launch_check("split_planes8");
-   return S;
-}
-
-bool int_mfma_ok(int op, const View &S, const View &T)
-{
-   const char *e = getenv("OCIP_INT_MFMA");
-   if ((e && e[0] == '0') || op == kSAD) return false;
-   if ((S.type != SImage::U8 && S.type != SImage::S8) || T.type != S.type) return false;
-   if (S.channels != 1 && S.channels != 2 && S.channels != 4) return false;
-   const int tw = T.width, th = T.height;
-   // (templates of one column block; ss_box8: dwords of four columns)
-   if (tw <= 0 || th <= 0 || tw > 97 || th > 97 || (S.width < 4 && op != kCC)) return false;
-   if ((long long)S.height * std::max((long long)S.step, (long long)plane8_step(S.width)) >= kBoxOob)
-      return false;
-   const long long mp = int_max_product(S.type);
-   if ((long long)tw * mp >= (1LL << 24) || (long long)tw * th * mp >= (1LL << 31)) return false;
-   return pair_geometry(kc2_for(tw), 4, th).vb >= 1;
-}
-
-size_t int_mfma_work_bytes(const View &S, const View &T)
-{
-   // several channels: a plane of bytes and a plane of the map each
-   const size_t planes = 5 * planes8_bytes(S);
-   return S.channels * pair_frag_bytes(mfma::kBF16, T.width, T.height) + planes;
-}
-
-void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, double *tsums,
-                     float *dst, int dstep, void *work)
-{
-   const int tw = T.width, th = T.height, KC2 = kc2_for(tw), nch = image.channels;
-   const int src8 = image.type == SImage::U8 ? mfma::kSrcU8 : mfma::kSrcS8;
-   const size_t frag_bytes = pair_frag_bytes(mfma::kBF16, tw, th);
-   // S, map: the image and its map, or (several channels) their first planes, the others plane8
-   // and planef bytes apart
-   View S = image;
-   float *map = dst;
-   int mstep = dstep;
-   size_t plane8 = 0, planef = 0;
-   if (nch > 1) {
-      char *planes = static_cast<char *>(work) + nch * frag_bytes;
-      S = launch_planes8(s, image, planes, &plane8);
-      map = reinterpret_cast<float *>(planes + nch * plane8);
-      mstep = 4 * S.step;
-      planef = (size_t)S.height * mstep;
-   }
-   if (op != kCC) {
-      // the window sums of s^2 go to the map first; the MFMA kernel's epilogue reads them
-      KernelTimer kt(s, "ss_box8");
-      const int bands = (S.height + box_band(th) - 1) / box_band(th);
-      const int cblks = (S.width + box_cols(tw) - 1) / box_cols(tw);
-      auto go = [&](auto kernel) {
-         kernel<<<dim3(bands * cblks, nch), 64, 0, s>>>(static_cast<const unsigned char *>(S.ptr),
-                                                       S.width, S.height, S.step, tw, th,
-                                                       reinterpret_cast<char *>(map), mstep, bands,
-                                                       plane8, planef);
-      };
-      if (src8 == mfma::kSrcS8) go(ss_box8<true>); else go(ss_box8<false>);
-      launch_check("ss_box8");
-   }
-   u16x8 *g0 = static_cast<u16x8 *>(work);
-   {
-      KernelTimer kt(s, "template_prep");
-      BatchDesc d{static_cast<const char *>(T.ptr), tw, th, T.step, KC2, 1, g0, nullptr, tsums};
-      d.src8 = src8;
-      d.nch = nch;
-      d.fragch = frag_bytes / sizeof(u16x8);
-      mfma::launch_pair_prep<mfma::kBF16>(s, d);
-   }
-   const Geometry g = pair_geometry(KC2, 4, th);
-   SingleLaunch L;
-   L.mode = mfma::kModeInt;
-   L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw, th, 1,
-                        g0, nullptr, tsums, nullptr, map, mstep, g.vb, 0};
-   L.a.src8 = src8;
-   L.a.nch = nch;
-   L.a.plane8 = plane8;
-   L.a.planef = planef;
-   L.a.fragch = frag_bytes / sizeof(u16x8);
-   L.a.op = op;
-   // steps between the int32 flushes: each step adds one template row of products
-   L.a.flush = (int)(((1LL << 24) - 1) / ((long long)tw * int_max_product(S.type)));
-   L.KC = KC2;
-   L.NT = 4;
-   L.ldsp = g.ldsp;
-   L.lds = g.lds;
-   L.grid = dim3((S.width + 63) / 64, (S.height + mfma::kPairRows - 1) / mfma::kPairRows);
-   {
-      KernelTimer kt(s, "crosscorr_mfma_int");
-      mfma::launch_pair<mfma::kBF16>(s, L);
-   }
-   if (nch > 1) {
-      KernelTimer kt(s, "join_planes");
-      auto go = [&](auto kernel) {
-         kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(map, S.width, S.height, mstep, dst,
-                                                               dstep);
-      };
-      if (nch == 2) go(join_planes<2>); else go(join_planes<4>);
-      launch_check("join_planes");
-   }
-}
-
 // ======================================================================= batch
 struct BatchEntry {
    hipGraphExec_t exec = nullptr;

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void split_prep(BatchDesc d, const unsigned *_
    const int f = blockIdx.x * 4 + (threadIdx.x >> 6);
    if (f < nfrag && sr.ok)
       build_pair_fragment<kF16x3>(d.tptr, d.tstep, d.tw, d.th, d.KC, 1, f, threadIdx.x & 63,
-                                  d.frag0, d.frag1, 0, pow2f(sr.kt));
+                                  d.frag0, d.frag1, pow2f(sr.kt));
 }
 
 template <int KC> void pair(hipStream_t s, const SingleLaunch &L)

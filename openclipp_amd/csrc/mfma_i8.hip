@@ -1,0 +1,772 @@
+// mfma_i8.hip -- exact cross terms of 8- and 16-bit integer images on int8 matrix cores.
+//
+// v_mfma_i32_32x32x32_i8 takes 32 source columns per instruction (a BF16 product takes 16) and adds
+// into int32, so sums are exact without flushes.  Source values become signed bytes,
+//   S8   s                                                                         K = 0
+//   U8   s - 128                                                                   K = 128
+//   S16  s - 128   = 256 h + l, h the high byte, l the low byte - 128              K = 128
+//   U16  s - 32896 = 256 h + l, h the high byte - 128, l the low byte - 128        K = 32896
+// (pixels outside the image: 0 - K), template values t signed digits of base 256 (one for S8, two
+// for U8, three for 16-bit types, the top one 0 or 1), and
+//   sum s t = sum over the pairs of digits of 256^(place of both) sum s_i t_j + K sum t,
+// one int32 sum per place, put together in FP64 (16-bit: exact below 2^53) or int32.  SqrDistance
+// of U8 takes t - 128 in one digit instead: a difference keeps when both lose 128.
+//
+// The contraction is the row-pair one of mfma_kernels.h (crosscorr_mfma_pair) with chunks of 32 source
+// columns: MFMA column n = 16 dy + dx, output row Y0 - 1 + 32 w + m + dy,
+//   B_kc[k][n] = t(32 kc + k - dx, 2 s + 1 - dy), KC = ceil((tw + 15) / 32),
+// 127 output rows by 16 NT columns per workgroup, the whole template's source rows staged at once.
+// Lane l of a fragment holds row or column l % 32 and k = 16 (l / 32) + i, i < 16; A and B share
+// that order, so any order of the instruction's own gives the same sums.
+#include <algorithm>
+
+#include "mfma_kernels.h"
+
+namespace ocip {
+
+namespace {
+
+using mfma::kPairRows;
+using mfma::kTileRows;
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
+typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef const i32x4 __attribute__((address_space(1))) *gfrag_i8;
+
+constexpr bool is16(int type) { return type == SImage::U16 || type == SImage::S16; }
+// digits of a source value, digits of a template value (U8: 1 = both less 128), places
+__host__ __device__ constexpr int i8_npa(int type) { return type == SImage::U16 || type == SImage::S16 ? 2 : 1; }
+
+__host__ __device__ constexpr int i8_chunks(int tw) { return (tw + 15 + 31) / 32; }
+__host__ __device__ constexpr int i8_steps(int th) { return (th + 1) / 2; }
+// n-tiles of 16 columns per wavefront.  8-bit: two, against four SqrDistance 4096^2/32x32 50 -> 47.6 us,
+// colour CrossCorr_Norm 1280x960/24x24 42 -> 33 (twice the wavefronts per SIMD), one 60 and 33.5.
+// 16-bit: one, against two CrossCorr_Norm 2048x1536/31x31 60 -> 51 us (48x48 of 4000x3000 233 -> 248).
+__host__ __device__ constexpr int i8_nt(int npa) { return npa == 1 ? 2 : 1; }
+__host__ __device__ constexpr int i8_lcols(int npa, int KC) { return 16 * (i8_nt(npa) - 1) + 32 * KC; }
+
+// B fragments (NPB digits, lowest first) of channel blockIdx.y, one (row pair, chunk) per wavefront;
+// the last block the sums of the template: sums[2 ch] = sum t^2 (of t - 128 for U8 in one digit),
+// sums[2 ch + 1] = sum t.
+template <int TYPE, int NPB>
+__global__ __launch_bounds__(256) void i8_prep(const char *tpl, int tw, int th, int tstep, int nch,
+                                               i32x4 *frag, double *sums)
+{
+   constexpr bool kKey = TYPE == SImage::U8 && NPB == 1;
+   __shared__ double red[2][4];
+   const int ch = blockIdx.y, KC = i8_chunks(tw), S = i8_steps(th);
+   if (blockIdx.x == gridDim.x - 1) {
+      double s2 = 0.0, s1 = 0.0;
+      const int n = tw * th;
+      for (int i0 = threadIdx.x; i0 < n; i0 += 256 * 8) {
+         int t[8];
+#pragma unroll
+         for (int k = 0; k < 8; ++k) {
+            const int i = min(i0 + 256 * k, n - 1), v = i / tw, u = i - v * tw;
+            t[k] = (int)ld<TYPE>(tpl + (size_t)v * tstep, u * nch + ch);
+         }
+#pragma unroll
+         for (int k = 0; k < 8; ++k) {
+            const double q = i0 + 256 * k < n ? (double)(kKey ? t[k] - 128 : t[k]) : 0.0;
+            s2 += q * q;
+            s1 += q;
+         }
+      }
+      s2 = wave_sum(s2);
+      s1 = wave_sum(s1);
+      if ((threadIdx.x & 63) == 0) {
+         red[0][threadIdx.x >> 6] = s2;
+         red[1][threadIdx.x >> 6] = s1;
+      }
+      __syncthreads();
+      if (threadIdx.x < 2)
+         sums[2 * ch + threadIdx.x] = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] +
+                                      red[threadIdx.x][3];
+      return;
+   }
+   const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+   if (f >= S * KC) return;
+   const int s = f / KC, kc = f - s * KC;
+   const int n = lane & 31, dy = n >> 4, dx = n & 15, kb = 16 * (lane >> 5);
+   const int v = 2 * s + 1 - dy;
+   const char *row = tpl + (size_t)(v < th ? v : 0) * tstep;
+   uint32_t q[NPB][4];
+#pragma unroll
+   for (int p = 0; p < NPB; ++p)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[p][i] = 0;
+#pragma unroll
+   for (int i = 0; i < 16; ++i) {
+      const int u = 32 * kc + kb + i - dx;
+      int t = (int)ld<TYPE>(row, min(max(u, 0), tw - 1) * nch + ch);   // (in range: all 16 in flight)
+      t = v < th && u >= 0 && u < tw ? (kKey ? t - 128 : t) : 0;
+#pragma unroll
+      for (int p = 0; p < NPB; ++p) {
+         const int digit = (int)(int8_t)t;
+         q[p][i / 4] |= ((uint32_t)digit & 0xffu) << (8 * (i % 4));
+         t = (t - digit) >> 8;
+      }
+   }
+   i32x4 *out = frag + ((size_t)(ch * S * KC + f) * NPB) * 64 + lane;
+#pragma unroll
+   for (int p = 0; p < NPB; ++p)
+      out[64 * p] = i32x4{(int)q[p][0], (int)q[p][1], (int)q[p][2], (int)q[p][3]};
+}
+
+struct I8Args {
+   const unsigned char *src;
+   int W, H, sstep;
+   int tw, th;
+   const i32x4 *frag;
+   const double *sums;          // i8_prep
+   // 8-bit ops but CrossCorr: the int32 window sums of s^2 (of (s - 128)^2 for U8 in one digit) lie
+   // in dst; 16-bit CrossCorr_Norm: the integral of s^2
+   const double *integ;
+   float *dst;
+   int dstep, op;
+   size_t plane8, planef;       // bytes from one channel's source and map to the next
+};
+
+// Source rows [row0, row0 + nrows) x columns [col0, col0 + 16 groups) as signed bytes, 16 columns
+// per item, at byte pitch ldsp (plane h at `plane` bytes past plane l).
+template <int TYPE, int GROUPS>
+__device__ __forceinline__ void stage_i8(const I8Args &a, const unsigned char *src, unsigned char *lds,
+                                         int ldsp, int plane, int row0, int col0, int nrows)
+{
+   constexpr bool B16 = is16(TYPE);
+   constexpr int ND = B16 ? 8 : 4;   // dwords of 16 elements
+   constexpr int K = 4;              // items in flight
+   constexpr uint32_t kFlip = 0x80808080u;
+   const int total = nrows * GROUPS;
+   for (int it0 = threadIdx.x; it0 < total; it0 += 256 * K) {
+      uint32_t q[K][ND];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+         const int it = it0 + 256 * k, r = it / GROUPS, g = it - r * GROUPS;
+         const int sy = row0 + r, sx = col0 + 16 * g;
+         const bool rowin = it < total && sy >= 0 && sy < a.H;
+         const unsigned char *row = src + (size_t)(rowin ? sy : 0) * a.sstep;
+         if (rowin && sx >= 0 && sx + 16 <= a.W) {
+#pragma unroll
+            for (int j = 0; j < ND / 4; ++j) {
+               const u32x4_b b = *reinterpret_cast<const u32x4_b *>(row + sx * (B16 ? 2 : 1) + 16 * j);
+#pragma unroll
+               for (int e = 0; e < 4; ++e) q[k][4 * j + e] = b[e];
+            }
+         } else {
+#pragma unroll
+            for (int j = 0; j < ND; ++j) q[k][j] = 0;
+            if (rowin && sx + 16 > 0 && sx < a.W) {
+#pragma unroll
+               for (int j = 0; j < 16; ++j) {
+                  const int x = sx + j;
+                  if (x < 0 || x >= a.W) continue;
+                  if (B16) q[k][j / 2] |= (uint32_t)reinterpret_cast<const uint16_t *>(row)[x] << (16 * (j % 2));
+                  else q[k][j / 4] |= (uint32_t)row[x] << (8 * (j % 4));
+               }
+            }
+         }
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+         const int it = it0 + 256 * k, r = it / GROUPS, g = it - r * GROUPS;
+         if (it >= total) break;
+         uint4 *at = reinterpret_cast<uint4 *>(lds + (size_t)r * ldsp + 16 * g);
+         if constexpr (B16) {
+            uint32_t lo[4], hi[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+               lo[j] = __builtin_amdgcn_perm(q[k][2 * j + 1], q[k][2 * j], 0x06040200u) ^ kFlip;
+               hi[j] = __builtin_amdgcn_perm(q[k][2 * j + 1], q[k][2 * j], 0x07050301u);
+               if (TYPE == SImage::U16) hi[j] ^= kFlip;
+            }
+            *at = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+            *reinterpret_cast<uint4 *>(lds + plane + (size_t)r * ldsp + 16 * g) =
+                make_uint4(hi[0], hi[1], hi[2], hi[3]);
+         } else {
+            if (TYPE == SImage::U8) {
+#pragma unroll
+               for (int j = 0; j < 4; ++j) q[k][j] ^= kFlip;
+            }
+            *at = make_uint4(q[k][0], q[k][1], q[k][2], q[k][3]);
+         }
+      }
+   }
+}
+
+__device__ __forceinline__ i32x16 mma_i8(i32x4 a, i32x4 b, i32x16 c)
+{
+   return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+}
+
+// Bound by latency (staging, then the products, then the epilogue, two to six workgroups per CU over
+// one another) above the map's bytes (8-bit SqrDistance 4096^2/32x32: 49 us, 144 MB = 28 us at the copy rate) and
+// the MFMAs (U16 2048x1536/31x31: 51 us, of it 22 in the products, 17 us of MFMA issue).  Against
+// BF16 products flushed into int32 every few rows: SqrDistance 4096^2/32x32 82 -> 49 us, colour
+// CrossCorr_Norm 1280x960/24x24 37.5 -> 33 us; 16-bit images against the tile kernel's int64 sums:
+// 120 -> 51 us.  More wavefronts per SIMD by bounds on the registers (3, 4): no faster, spills at 4.
+template <int TYPE, int NPB, int KC>
+__global__ __launch_bounds__(256, is16(TYPE) && KC > 2 ? 1 : 2)
+void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
+{
+   constexpr bool B16 = is16(TYPE);
+   constexpr int NPA = i8_npa(TYPE), NL = NPA + NPB - 1;
+   constexpr int NT = i8_nt(NPA), C = 16 * NT, NA = NT + 2 * KC - 2;
+   typedef typename std::conditional<B16, double, int>::type V;   // a half row's cross term
+   constexpr int TP = C + (B16 ? 2 : 4);                          // pitch of the paired tile
+   extern __shared__ uint4 lds_v[];
+   unsigned char *lds = reinterpret_cast<unsigned char *>(lds_v);
+   const int ch = blockIdx.x / tiles;
+   const int t = xcd_tile(blockIdx.x - ch * tiles, tiles);
+   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+   const int x0 = (t % tiles_x) * C, Y0 = (t / tiles_x) * kPairRows;
+   const int S = i8_steps(a.th), nrows = kTileRows - 2 + 2 * S, plane = nrows * ldsp;
+   const unsigned char *src = a.src + ch * a.plane8;
+   char *dst = reinterpret_cast<char *>(a.dst) + ch * a.planef;
+   const gfrag_i8 fr = (gfrag_i8)(a.frag + (size_t)ch * S * KC * NPB * 64 + lane);
+   const double tt = a.sums[2 * ch], t1 = a.sums[2 * ch + 1];
+
+   // LDS row r = source row Y0 - cy + r; wave w reads rows 32 w + m + 2 s
+   stage_i8<TYPE, i8_lcols(NPA, KC) / 16>(a, src, lds, ldsp, plane, Y0 - a.th / 2, x0 - a.tw / 2, nrows);
+   __syncthreads();
+   i32x16 acc[NL][NT];
+#pragma unroll
+   for (int l = 0; l < NL; ++l)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int i = 0; i < 16; ++i) acc[l][j][i] = 0;
+   // (a wave whose output rows all lie below the image has nothing to multiply)
+   if (Y0 - 1 + 32 * wave < a.H) {
+      i32x4 b[2][KC][NPB];
+      auto fetch = [&](int s, i32x4 (&q)[KC][NPB]) {
+#pragma unroll
+         for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int p = 0; p < NPB; ++p) q[kc][p] = fr[(size_t)((s * KC + kc) * NPB + p) * 64];
+      };
+      const unsigned char *arow = lds + (size_t)(wave * 32 + (lane & 31)) * ldsp + 16 * (lane >> 5);
+      auto step = [&](int s, const i32x4 (&q)[KC][NPB]) {
+         i32x4 x[NPA][NA];
+#pragma unroll
+         for (int c = 0; c < NA; ++c)
+#pragma unroll
+            for (int p = 0; p < NPA; ++p)
+               x[p][c] = *reinterpret_cast<const i32x4 *>(arow + p * plane + (size_t)(2 * s) * ldsp + 16 * c);
+#pragma unroll
+         for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+               // digit of s, digit of t: neighbours never add into the same place
+               constexpr int kA[6] = {0, 1, 0, 1, 1, 0}, kB[6] = {0, 1, 1, 2, 0, 2};
+               if (kA[k] >= NPA || kB[k] >= NPB) continue;
+#pragma unroll
+               for (int j = 0; j < NT; ++j)
+                  acc[kA[k] + kB[k]][j] =
+                      mma_i8(x[kA[k] < NPA ? kA[k] : 0][j + 2 * kc], q[kc][kB[k] < NPB ? kB[k] : 0],
+                             acc[kA[k] + kB[k] < NL ? kA[k] + kB[k] : 0][j]);
+            }
+      };
+      fetch(0, b[0]);
+      int s = 0;
+      for (; s + 1 < S; s += 2) {
+         // keep each prefetch ahead of the MFMAs of the step before it
+         fetch(s + 1, b[1]);
+         __builtin_amdgcn_sched_barrier(0);
+         step(s, b[0]);
+         fetch(min(s + 2, S - 1), b[0]);
+         __builtin_amdgcn_sched_barrier(0);
+         step(s + 1, b[1]);
+      }
+      if (s < S) step(s, b[0]);
+   }
+
+   // Pair the halves in LDS: tile row r = 32 w + m + dy holds output row Y0 - 1 + r; C fragment: lane
+   // holds column n = lane % 32, rows m = 8 (i / 4) + 4 (lane / 32) + i % 4.
+   V *tile = reinterpret_cast<V *>(lds);
+   const int n = lane & 31, dy = n >> 4, dx = n & 15;
+   const int rb = 32 * wave + 4 * (lane >> 5) + dy;
+   auto half = [&](int j, int i) -> V {
+      V v = (V)acc[NL - 1][j][i];
+#pragma unroll
+      for (int l = NL - 2; l >= 0; --l) v = v * (V)256 + (V)acc[l][j][i];
+      return v;
+   };
+   __syncthreads();
+   if (dy) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int i = 0; i < 16; ++i) tile[(rb + 8 * (i / 4) + (i % 4)) * TP + 16 * j + dx] = half(j, i);
+   }
+   __syncthreads();
+   if (!dy) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int i = 0; i < 16; ++i) tile[(rb + 8 * (i / 4) + (i % 4)) * TP + 16 * j + dx] += half(j, i);
+   }
+   __syncthreads();
+   // four consecutive columns per thread
+   const int itt = (int)tt;
+   constexpr int K = TYPE == SImage::U16 ? 32896 : TYPE == SImage::S16 || (TYPE == SImage::U8 && NPB == 2) ? 128 : 0;
+   const V kt = (V)K * (V)t1;
+   const int cx = a.tw / 2, cy = a.th / 2;
+   const size_t ip = excl_pitch(a.W);
+   for (int g = threadIdx.x; g < kPairRows * (C / 4); g += 256) {
+      const int r = g / (C / 4), c = 4 * (g - r * (C / 4));
+      const int y = Y0 + r, x = x0 + c;
+      if (y >= a.H || x >= a.W) continue;
+      const V *cc = &tile[(r + 1) * TP + c];
+      float *o = reinterpret_cast<float *>(dst + (size_t)y * a.dstep) + x;
+      const bool whole = x + 4 <= a.W;
+      float v[4];
+      if constexpr (B16) {
+         if (a.op == kCC) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (float)(cc[e] + kt);
+         } else {
+            double ss[4];
+            if (x >= cx && x - cx + a.tw + 3 <= a.W && y >= cy && y - cy + a.th <= a.H) {
+               const double *p = a.integ + (size_t)(y - cy) * ip + (kExclOffset + x - cx);
+               const double *p1 = p + (size_t)a.th * ip;
+#pragma unroll
+               for (int e = 0; e < 4; e += 2) {
+                  const f64x2_u v0 = *reinterpret_cast<const f64x2_u *>(p + e);
+                  const f64x2_u v1 = *reinterpret_cast<const f64x2_u *>(p1 + e);
+                  const f64x2_u v2 = *reinterpret_cast<const f64x2_u *>(p + a.tw + e);
+                  const f64x2_u v3 = *reinterpret_cast<const f64x2_u *>(p1 + a.tw + e);
+#pragma unroll
+                  for (int h = 0; h < 2; ++h) ss[e + h] = (v3[h] - v2[h]) - (v1[h] - v0[h]);
+               }
+            } else {
+#pragma unroll
+               for (int e = 0; e < 4; ++e) ss[e] = window_sqsum(a.integ, a.W, a.H, x + e, y, a.tw, a.th);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (float)((cc[e] + kt) * rsqrt64(ss[e] * tt));
+         }
+      } else {
+         int ss[4] = {0, 0, 0, 0};
+         if (a.op != kCC) {
+            if (whole) {
+               const i32x4_u q = *reinterpret_cast<const i32x4_u *>(o);
+#pragma unroll
+               for (int e = 0; e < 4; ++e) ss[e] = q[e];
+            } else {
+#pragma unroll
+               for (int e = 0; e < 4; ++e)
+                  if (x + e < a.W) ss[e] = reinterpret_cast<const int *>(o)[e];
+            }
+         }
+#pragma unroll
+         for (int e = 0; e < 4; ++e) {
+            const int cross = cc[e] + kt;
+            const int d = a.op == kSSD || a.op == kSSDNorm ? ss[e] - 2 * cross + itt : cross;
+            v[e] = a.op == kCC || a.op == kSSD ? (float)d
+                                               : (float)((double)d * rsqrt64((double)ss[e] * tt));
+         }
+      }
+      if (whole) {
+         *reinterpret_cast<f32x4_u *>(o) = f32x4_u{v[0], v[1], v[2], v[3]};
+      } else {
+#pragma unroll
+         for (int e = 0; e < 4; ++e)
+            if (x + e < a.W) o[e] = v[e];
+      }
+   }
+}
+
+template <int TYPE, int NPB>
+void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
+{
+   constexpr int NPA = i8_npa(TYPE), NT = i8_nt(NPA);
+   constexpr bool B16 = is16(TYPE);
+   a.src = static_cast<const unsigned char *>(S.ptr);
+   a.W = S.width; a.H = S.height; a.sstep = S.step;
+   a.tw = T.width; a.th = T.height;
+   const int KC = i8_chunks(a.tw), steps = i8_steps(a.th), nch = T.channels;
+   {
+      KernelTimer kt(s, "template_prep");
+      i8_prep<TYPE, NPB><<<dim3((steps * KC + 3) / 4 + 1, nch), 256, 0, s>>>(
+          static_cast<const char *>(T.ptr), a.tw, a.th, T.step, nch, const_cast<i32x4 *>(a.frag),
+          const_cast<double *>(a.sums));
+      launch_check("i8_prep");
+   }
+   // an odd multiple of 16 bytes: the A reads of 8 consecutive rows on distinct banks
+   int ldsp = i8_lcols(NPA, KC);
+   if (ldsp % 32 == 0) ldsp += 16;
+   const size_t staging = (size_t)NPA * (kTileRows - 2 + 2 * steps) * ldsp;
+   const size_t pairing = (size_t)(kTileRows + 1) * (16 * NT + (B16 ? 2 : 4)) * (B16 ? 8 : 4);
+   const size_t lds = std::max(staging, pairing);
+   const int tiles_x = (a.W + 16 * NT - 1) / (16 * NT), tiles_y = (a.H + kPairRows - 1) / kPairRows;
+   KernelTimer kt(s, "crosscorr_mfma_int");
+   auto go = [&](auto kernel) {
+      if (lds > 64 * 1024)
+         hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                   "lds attribute");
+      kernel<<<tiles_x * tiles_y * nch, 256, lds, s>>>(a, ldsp, tiles_x, tiles_x * tiles_y);
+   };
+   switch (KC) {
+   case 1: go(crosscorr_i8<TYPE, NPB, 1>); break;
+   case 2: go(crosscorr_i8<TYPE, NPB, 2>); break;
+   case 3: go(crosscorr_i8<TYPE, NPB, 3>); break;
+   case 4: go(crosscorr_i8<TYPE, NPB, 4>); break;
+   default: fail(CL_INVALID_VALUE, "template width");
+   }
+   launch_check("crosscorr_i8");
+}
+
+// ------------------------------------------------------------------------- window sums, planes
+// Window sums of s^2 of an 8-bit image, exact in int32, into the map `dst` (as int32 bits):
+// SS(x, y) = sum over the template window of (x, y) (origin (-tw/2, -th/2), zero outside the
+// image).  One wavefront per band of box_band(th) output rows and 256 source columns, four adjacent
+// ones per lane, i.e. box_cols(tw) output columns:
+//  * each lane's four column sums of squares over the window's rows, running down the band: the
+//    squares of the rows entering the window (a dword each) less those of the rows leaving it;
+//  * per output row the inclusive prefix I of the column sums along the row: the lane's own four,
+//    a wavefront scan of the lanes' totals (DPP row shifts and broadcasts; U rows at once), then
+//    SS(i) = I[i + tw - 1] - I[i - 1]: the subtrahends are the lane's own, the minuends come through
+//    LDS; one 16-byte store per lane and row.
+// Integer arithmetic modulo 2^32 throughout and every result below 2^31 (checked by the host), so
+// the sums are exact in any order.  Bound by issue and the map's store: about 44 instructions per
+// row and 225 outputs (tw = 32) where a lane per output column with a ring of row sums in LDS
+// took 35 per 64 (4096^2/32x32: 38 -> 22 us).
+// Output rows per wavefront: 16, or 32 where the th - 1 rows before the first would outweigh them
+// (more wavefronts hide the chains' latency: colour 1280x960/24x24 15 us with 16, 18 with 32, 25 with 64)
+constexpr int box_band(int th) { return th <= 48 ? 16 : 32; }
+constexpr int kBoxOob = 0x40000000;   // a byte count past any image this kernel takes
+constexpr int box_cols(int tw) { return (256 - (tw - 1)) / 4 * 4; }
+
+// Inclusive scans across the 64 lanes of N values at once (the N scans interleaved, so that
+// each DPP step's wait on the previous one is filled by the others): within rows of 16 lanes
+// (lanes without a source add 0), then rows 1 and 3 take the last lane of rows 0 and 2, rows
+// 2 and 3 the last lane of row 1.
+template <int N>
+__device__ __forceinline__ void wave_incl_scan(int (&x)[N])
+{
+#pragma unroll
+   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x111, 0xf, 0xf, false);
+#pragma unroll
+   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x112, 0xf, 0xf, false);
+#pragma unroll
+   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x114, 0xf, 0xf, false);
+#pragma unroll
+   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x118, 0xf, 0xf, false);
+#pragma unroll
+   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x142, 0xa, 0xf, false);
+#pragma unroll
+   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x143, 0xc, 0xf, false);
+}
+
+// FLIP: of s - 128 (U8).
+template <bool SIGNED, bool FLIP>
+__global__ __launch_bounds__(64) void ss_box8(const unsigned char *__restrict__ src, int W,
+                                              int H, int sstep, int tw, int th,
+                                              char *__restrict__ dst, int dstep, int bands,
+                                              size_t plane8, size_t planef)
+{
+   constexpr int U = 4;                          // rows at once (their loads one batch ahead)
+   __shared__ int pre[U][256 + 100];             // (lanes past the outputs read up to tw + 2 past 256)
+   typedef uint32_t u32_u __attribute__((aligned(1)));
+   typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+   const int lane = threadIdx.x;
+   // consecutive blocks (one XCD's run) side by side along a band share halo columns in L2
+   const int b = xcd_tile(blockIdx.x, gridDim.x);
+   // blockIdx.y = channel
+   src += blockIdx.y * plane8;
+   dst += blockIdx.y * planef;
+   const int cblks = gridDim.x / bands, cols = box_cols(tw);
+   const int band = b / cblks, cblk = b % cblks;
+   const int x0 = cblk * cols, y0 = band * box_band(th);
+   const int cx = tw / 2, cy = th / 2;
+   const int n = min(box_band(th), H - y0);
+   // the lane's columns c .. c + 3 from the dword at column min(max(c, 0), W - 4), shifted into
+   // place, zero outside the image (mask 0: wholly outside)
+   const int c = x0 - cx + 4 * lane, cl = min(max(c, 0), W - 4);
+   const int lsh = min(max(-c, 0), 3) * 8, rsh = min(max(c - cl, 0), 3) * 8;
+   const uint32_t mask = c <= -4 || c >= W ? 0u : 0xffffffffu;
+   auto load = [&](int y) -> uint32_t {
+      return *reinterpret_cast<const u32_u *>(src + (size_t)min(max(y, 0), H - 1) * sstep + cl);
+   };
+   auto place = [&](uint32_t v, int y) -> uint32_t {
+      return ((unsigned)y < (unsigned)H ? (v << lsh) >> rsh & mask : 0u) ^ (FLIP ? 0x80808080u : 0u);
+   };
+   auto elem = [&](uint32_t v, int e) -> int {
+      return SIGNED ? (int)(v << (24 - 8 * e)) >> 24 : (int)(v >> (8 * e) & 0xffu);
+   };
+   // column sums lead - lag: squares are only ever added (sums that took squares off were compiled
+   // into byte dot products that added them)
+   int lead[4] = {0, 0, 0, 0}, lag[4] = {0, 0, 0, 0};
+   // the th - 1 rows before the first output row's last
+   for (int j0 = 0; j0 < th - 1; j0 += 8) {
+      uint32_t v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = load(y0 - cy + j0 + j);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+         const uint32_t q = j0 + j < th - 1 ? place(v[j], y0 - cy + j0 + j) : 0u;
+#pragma unroll
+         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(q, e), elem(q, e));
+      }
+   }
+   uint32_t in[U], out[U];
+   auto fetch = [&](int r) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         in[u] = load(y0 - cy + th - 1 + r + u);
+         out[u] = load(y0 - cy + r + u);
+      }
+   };
+   fetch(0);
+   const int x = x0 + 4 * lane;
+   const bool mine = 4 * lane < cols && x < W;
+   for (int r0 = 0; r0 < n; r0 += U) {
+      int q[U][4], inc[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         const uint32_t a = place(in[u], y0 - cy + th - 1 + r0 + u), o = place(out[u], y0 - cy + r0 + u);
+#pragma unroll
+         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(a, e), elem(a, e));
+         q[u][0] = lead[0] - lag[0];
+#pragma unroll
+         for (int e = 1; e < 4; ++e) q[u][e] = q[u][e - 1] + (lead[e] - lag[e]);
+         inc[u] = q[u][3];
+#pragma unroll
+         for (int e = 0; e < 4; ++e) lag[e] += __mul24(elem(o, e), elem(o, e));
+      }
+      if (r0 + U < n) fetch(r0 + U);
+      wave_incl_scan<U>(inc);
+      __syncthreads();   // the reads of the batch before are done
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         inc[u] -= q[u][3];   // the sums of the lanes before
+         *reinterpret_cast<int4 *>(&pre[u][4 * lane]) =
+             make_int4(inc[u] + q[u][0], inc[u] + q[u][1], inc[u] + q[u][2], inc[u] + q[u][3]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         const int *p = &pre[u][4 * lane + tw - 1];
+         const int s0 = p[0] - inc[u], s1 = p[1] - inc[u] - q[u][0], s2 = p[2] - inc[u] - q[u][1],
+                   s3 = p[3] - inc[u] - q[u][2];
+         if (!mine || r0 + u >= n) continue;
+         int *o = reinterpret_cast<int *>(dst + (size_t)(y0 + r0 + u) * dstep) + x;
+         if (x + 4 <= W) {
+            *reinterpret_cast<i32x4_u *>(o) = i32x4_u{s0, s1, s2, s3};
+         } else {
+            o[0] = s0;
+            if (x + 1 < W) o[1] = s1;
+            if (x + 2 < W) o[2] = s2;
+         }
+      }
+   }
+}
+
+// Interleaved 8-bit channels into planes of their own (row pitch plane8_step, plane pitch H rows),
+// zeros between the width and the pitch, and the planes of the map back into interleaved
+// channels: the kernels between them take every channel of an image in one launch, as
+// 1-channel images with wide loads and stores (with the channels' maps interleaved by those
+// kernels themselves, 4 bytes of every 16 a store, the row-pair kernel ran 60 instead of 40 us
+// at 1280x960/24x24).  Four pixels per thread.  Bound by HBM: 2 W H NCH and 8 W H NCH bytes.
+int plane8_step(int W) { return (W + 15) / 16 * 16; }
+
+template <int NCH>
+__global__ __launch_bounds__(256) void split_planes8(const unsigned char *__restrict__ src, int W,
+                                                     int H, int sstep,
+                                                     unsigned char *__restrict__ dst, int dstep)
+{
+   const int k = blockIdx.x * 256 + threadIdx.x, groups = dstep / 4;
+   const int y = k / groups, x = 4 * (k - y * groups);
+   if (y >= H) return;
+   const unsigned char *row = src + (size_t)y * sstep;
+   uint32_t q[NCH];   // the 4 NCH bytes of the thread's pixels
+   if (x + 4 <= W) {
+      typedef uint32_t u32_u __attribute__((aligned(1)));
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) q[i] = reinterpret_cast<const u32_u *>(row + x * NCH)[i];
+   } else {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) q[i] = 0;
+#pragma unroll
+      for (int i = 0; i < 4 * NCH; ++i)
+         if (x + i / NCH < W) q[i / 4] |= (uint32_t)row[x * NCH + i] << (8 * (i % 4));
+   }
+#pragma unroll
+   for (int c = 0; c < NCH; ++c) {
+      uint32_t v = 0;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+         const int i = p * NCH + c;
+         v |= (q[i / 4] >> (8 * (i % 4)) & 0xffu) << (8 * p);
+      }
+      *reinterpret_cast<uint32_t *>(dst + ((size_t)c * H + y) * dstep + x) = v;
+   }
+}
+
+template <int NCH>
+__global__ __launch_bounds__(256) void join_planes(const float *__restrict__ src, int W, int H,
+                                                   int sstep, float *__restrict__ dst, int dstep)
+{
+   const int k = blockIdx.x * 256 + threadIdx.x, groups = sstep / 16;
+   const int y = k / groups, x = 4 * (k - y * groups);
+   if (y >= H) return;
+   float v[4 * NCH];
+#pragma unroll
+   for (int c = 0; c < NCH; ++c) {
+      const float4 q = *reinterpret_cast<const float4 *>(
+          reinterpret_cast<const char *>(src) + ((size_t)c * H + y) * sstep + 4 * x);
+      v[c] = q.x; v[NCH + c] = q.y; v[2 * NCH + c] = q.z; v[3 * NCH + c] = q.w;
+   }
+   float *d = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + (size_t)y * dstep) + x * NCH;
+   if (x + 4 <= W) {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+         reinterpret_cast<f32x4_u *>(d)[i] = f32x4_u{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+   } else {
+#pragma unroll
+      for (int i = 0; i < 4 * NCH; ++i)
+         if (x + i / NCH < W) d[i] = v[i];
+   }
+}
+
+// one thread per 4 columns of a plane
+static unsigned plane_blocks(int H, int step) { return (unsigned)(((long long)H * (step / 4) + 255) / 256); }
+
+}  // namespace
+
+size_t planes8_bytes(const View &S)
+{
+   return S.channels > 1 ? (size_t)S.channels * S.height * plane8_step(S.width) : 0;
+}
+
+View launch_planes8(hipStream_t s, const View &image, void *planes, size_t *plane8)
+{
+   KernelTimer kt(s, "split_planes8");
+   View S = image;
+   S.ptr = planes;
+   S.step = plane8_step(image.width);
+   S.channels = 1;
+   *plane8 = (size_t)S.height * S.step;
+   auto go = [&](auto kernel) {
+      kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(
+          static_cast<const unsigned char *>(image.ptr), S.width, S.height, image.step,
+          static_cast<unsigned char *>(planes), S.step);
+   };
+   if (image.channels == 2) go(split_planes8<2>); else go(split_planes8<4>);
+   launch_check("split_planes8");
+   return S;
+}
+
+bool int_mfma_ok(int op, const View &S, const View &T)
+{
+   const char *e = getenv("OCIP_INT_MFMA");
+   if ((e && e[0] == '0') || op == kSAD) return false;
+   if ((S.type != SImage::U8 && S.type != SImage::S8) || T.type != S.type) return false;
+   if (S.channels != 1 && S.channels != 2 && S.channels != 4) return false;
+   const int tw = T.width, th = T.height;
+   // (ss_box8: dwords of four columns)
+   if (tw <= 0 || th <= 0 || tw > 97 || th > 97 || (S.width < 4 && op != kCC)) return false;
+   if ((long long)S.height * std::max((long long)S.step, (long long)plane8_step(S.width)) >= kBoxOob)
+      return false;
+   // the whole sum in int32
+   return (long long)tw * th * (S.type == SImage::U8 ? 255 * 255 : 128 * 128) < (1LL << 31);
+}
+
+// Sums (two per channel), then the fragments of every channel (three digits at most).
+constexpr size_t kSumsBytes = 256;
+
+size_t i8_work_bytes(const View &T)
+{
+   const size_t n = 3 * (size_t)T.channels * i8_steps(T.height) * i8_chunks(T.width) * 64 * sizeof(i32x4);
+   return kSumsBytes + (n + 255) / 256 * 256;
+}
+
+size_t int_mfma_work_bytes(const View &S, const View &T)
+{
+   // several channels: a plane of bytes and a plane of the map each
+   return i8_work_bytes(T) + 5 * planes8_bytes(S);
+}
+
+static I8Args work_args(int op, void *work)
+{
+   I8Args a{};
+   a.sums = static_cast<const double *>(work);
+   a.frag = reinterpret_cast<const i32x4 *>(static_cast<const char *>(work) + kSumsBytes);
+   a.op = op;
+   return a;
+}
+
+void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, float *dst, int dstep,
+                     void *work)
+{
+   const int nch = image.channels;
+   // S, map: the image and its map, or (several channels) their first planes, the others plane8
+   // and planef bytes apart
+   View S = image;
+   I8Args a = work_args(op, work);
+   a.dst = dst;
+   a.dstep = dstep;
+   if (nch > 1) {
+      char *planes = static_cast<char *>(work) + i8_work_bytes(T);
+      S = launch_planes8(s, image, planes, &a.plane8);
+      a.dst = reinterpret_cast<float *>(planes + nch * a.plane8);
+      a.dstep = 4 * S.step;
+      a.planef = (size_t)S.height * a.dstep;
+   }
+   if (op != kCC) {
+      // the window sums of s^2 go to the map first; the MFMA kernel's epilogue reads them
+      KernelTimer kt(s, "ss_box8");
+      const int bands = (S.height + box_band(T.height) - 1) / box_band(T.height);
+      const int cblks = (S.width + box_cols(T.width) - 1) / box_cols(T.width);
+      auto go = [&](auto kernel) {
+         kernel<<<dim3(bands * cblks, nch), 64, 0, s>>>(static_cast<const unsigned char *>(S.ptr),
+                                                       S.width, S.height, S.step, T.width, T.height,
+                                                       reinterpret_cast<char *>(a.dst), a.dstep, bands,
+                                                       a.plane8, a.planef);
+      };
+      if (T.type == SImage::S8) go(ss_box8<true, false>);
+      else if (op == kSSD) go(ss_box8<true, true>);
+      else go(ss_box8<false, false>);
+      launch_check("ss_box8");
+   }
+   if (T.type == SImage::S8) launch_i8<SImage::S8, 1>(s, a, S, T);
+   else if (op == kSSD) launch_i8<SImage::U8, 1>(s, a, S, T);
+   else launch_i8<SImage::U8, 2>(s, a, S, T);
+   if (nch > 1) {
+      KernelTimer kt(s, "join_planes");
+      auto go = [&](auto kernel) {
+         kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(a.dst, S.width, S.height, a.dstep, dst,
+                                                               dstep);
+      };
+      if (nch == 2) go(join_planes<2>); else go(join_planes<4>);
+      launch_check("join_planes");
+   }
+}
+
+// Every size up to the widest template of four chunks: against the tile kernel, CrossCorr 160x120/2x2
+// 9.2 -> 8.2 us, 640x480/3x3 11.1 -> 10.0, 1920x1080/11x11 27 -> 17, /49x49 232 -> 45, /113x128
+// 1355 -> 204.  (The height keeps the staged rows within the LDS and the sums within int32.)
+bool int16_mfma_ok(int op, const View &S, const View &T)
+{
+   const char *e = getenv("OCIP_INT_MFMA");
+   if ((e && e[0] == '0') || (op != kCC && op != kCCNorm)) return false;
+   if (!is16(S.type) || T.type != S.type || S.channels != 1) return false;
+   return T.width > 0 && T.height > 0 && i8_chunks(T.width) <= 4 && T.height <= 128;
+}
+
+void launch_int16_mfma(hipStream_t s, int op, const View &S, const View &T, const double *integ,
+                       float *dst, int dstep, void *work)
+{
+   I8Args a = work_args(op, work);
+   a.integ = integ;
+   a.dst = dst;
+   a.dstep = dstep;
+   if (S.type == SImage::U16) launch_i8<SImage::U16, 3>(s, a, S, T);
+   else launch_i8<SImage::S16, 3>(s, a, S, T);
+}
+
+}  // namespace ocip

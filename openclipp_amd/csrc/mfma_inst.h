@@ -41,16 +41,11 @@ template <int KC, int NT, int MODE> void pair(hipStream_t s, const SingleLaunch 
    auto k = crosscorr_mfma_pair<P, KC, NT, MODE>;
    allow_lds(k);
    const int tiles = L.grid.x * L.grid.y;
-   k<<<tiles * std::max(1, L.z.n) * L.a.nch, 256, L.lds, s>>>(L.a, L.ldsp, (int)L.grid.x, tiles, L.z);
+   k<<<tiles * std::max(1, L.z.n), 256, L.lds, s>>>(L.a, L.ldsp, (int)L.grid.x, tiles, L.z);
 }
 
 template <int KC> void pair_mode(hipStream_t s, const SingleLaunch &L)
 {
-   if (L.mode == kModeInt) {
-      if constexpr (P == kBF16) pair<KC, 4, kModeInt>(s, L);
-      else fail(CL_INVALID_VALUE, "exact integer sums take BF16 operands");
-      return;
-   }
    if (L.NT == 4) pair<KC, 4, kModeCC>(s, L); else pair<KC, 6, kModeCC>(s, L);
 }
 
@@ -160,7 +155,7 @@ template <> void launch_pair<P>(hipStream_t s, const SingleLaunch &L)
 template <> void launch_pair_prep<P>(hipStream_t s, const BatchDesc &d)
 {
    const int nfrag = d.nub * pair_frag_steps(d.th, d.nub) * d.KC;
-   pair_prep<P><<<dim3((nfrag + 3) / 4 + 1, d.nch), 256, 0, s>>>(d);   // + 1: the sum of squares
+   pair_prep<P><<<(nfrag + 3) / 4 + 1, 256, 0, s>>>(d);   // + 1: the sum of squares
    launch_check("pair_prep");
 }
 

@@ -50,10 +50,8 @@ constexpr int kLdsMax = 160 * 1024 - 256;
 enum { kBF16 = 1, kF16 = 2, kBF16x3 = 3, kF16x3 = 4 };
 __host__ __device__ constexpr int planes_of(int P) { return P == kBF16x3 || P == kF16x3 ? 2 : 1; }
 // kModeCC: the CrossCorr map (the single-template call; CrossCorr_Norm scales it in place
-// afterwards); kModeNCC / kModeSSDN: the batch kernel's epilogues from the FP64 integral;
-// kModeInt: the row-pair kernel on 8-bit integer images, exact integer sums (any of the
-// four cross-term ops, TileArgs::op)
-enum { kModeCC = 0, kModeNCC = 1, kModeSSDN = 2, kModeInt = 3 };
+// afterwards); kModeNCC / kModeSSDN: the batch kernel's epilogues from the FP64 integral
+enum { kModeCC = 0, kModeNCC = 1, kModeSSDN = 2 };
 
 // Arguments of one output tile computation.
 struct TileArgs {
@@ -67,13 +65,6 @@ struct TileArgs {
    int dstep;
    int vb;                       // template rows per LDS band
    int vec;                      // 16-byte ring loads allowed (crosscorr_mfma_strip)
-   // kModeInt (exact sums of 8-bit integer images): element type of source and template
-   // (kSrcU8 / kSrcS8), the op (ProxOp) and the steps between the int32 flushes
-   int src8 = 0, op = 0, flush = 0;
-   // kModeInt: channels, the bytes from one channel's plane of the source and of the map to the
-   // next, and the 16-byte vectors from one channel's fragments to the next
-   int nch = 1;
-   size_t plane8 = 0, planef = 0, fragch = 0;
    // kF16x3: the peaks of source and template (split_range), the source's scale, the word that any
    // flagged tile sets, and the tile's flag (non-zero: prox_tile_f32_flagged computes it again)
    const unsigned *peaks = nullptr;
@@ -107,24 +98,7 @@ struct BatchDesc {
    int tw, th, tstep, KC, nub;
    u16x8 *frag0, *frag1;
    double *sums;
-   int src8 = 0;                 // template elements: F32 (0), U8 (kSrcU8), S8 (kSrcS8)
-   // interleaved channels (8-bit templates), the one described, and the vectors from one channel's
-   // fragments to the next
-   int nch = 1, ch = 0;
-   size_t fragch = 0;
 };
-
-// 8-bit integer element types of kModeInt (their values and products are exact in BF16 and
-// FP32)
-enum { kSrcU8 = 1, kSrcS8 = 2 };
-
-// Element u of a template row as float: F32, or an 8-bit integer (exact)
-__host__ __device__ inline float tmpl_elem(const char *row, int u, int src8)
-{
-   if (src8 == kSrcU8) return (float)reinterpret_cast<const unsigned char *>(row)[u];
-   if (src8 == kSrcS8) return (float)reinterpret_cast<const signed char *>(row)[u];
-   return reinterpret_cast<const float *>(row)[u];
-}
 
 __host__ __device__ constexpr int lcols_for(int KC, int NT) { return 16 * (2 * (NT - 1) + KC); }
 
@@ -231,7 +205,7 @@ __device__ __forceinline__ void template_sqsum(const BatchDesc &d, double *red)
          const int k = k0 + 256 * i;
          const int v = k / pitch, u = k - v * pitch;
          t[i] = (k < total && u < d.tw)
-                    ? tmpl_elem(d.tptr + (size_t)v * d.tstep, u * d.nch + d.ch, d.src8) : 0.f;
+                    ? reinterpret_cast<const float *>(d.tptr + (size_t)v * d.tstep)[u] : 0.f;
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) s2 += (double)t[i] * (double)t[i];
@@ -282,9 +256,6 @@ typedef float f32x4_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef __attribute__((address_space(1))) float gmem_f32;
 typedef __attribute__((address_space(1))) f32x4_t gmem_f32x4;
 typedef __attribute__((address_space(1))) char gmem_char;
-typedef __attribute__((address_space(1))) int gmem_i32;
-typedef int i32x4_t __attribute__((ext_vector_type(4), aligned(4)));
-typedef __attribute__((address_space(1))) i32x4_t gmem_i32x4;
 __device__ __forceinline__ gmem_f32 *out_row(const TileArgs &a, int y)
 {
    return reinterpret_cast<gmem_f32 *>((gmem_char *)a.dst + (size_t)y * a.dstep);
@@ -343,12 +314,10 @@ __device__ __forceinline__ void row_mfma(f32x16 (&acc)[NT], const unsigned short
 
 // Stage source rows [row0, row0 + nrows) x columns [col0, col0 + LCOLS) into LDS as 16-bit
 // values (zero outside the image), 8 columns per item, four items per thread in flight, each
-// item two 16-byte loads (one 8-byte load of 8-bit sources) whatever its alignment.  Against
-// eight loads of single elements wherever tw/2 or the row pitch left the columns unaligned:
-// CrossCorr_Norm BF16 4096^2/63x64 220 -> 187 us, 4095-wide 8-bit SqrDistance 32x32 167 -> 118 us,
+// item two 16-byte loads whatever its alignment.  Against eight loads of single elements wherever
+// tw/2 or the row pitch left the columns unaligned: CrossCorr_Norm BF16 4096^2/63x64 220 -> 187 us,
 // 48 BF16 templates of 8..96 px on 2048^2 2217 -> 1966 us; aligned calls unchanged.
-// SRC8: the source holds 8-bit integers (a.src8 gives the sign), exact in BF16.
-template <int P, int LCOLS, bool SRC8 = false>
+template <int P, int LCOLS>
 __device__ __forceinline__ void stage_rows(const TileArgs &a, unsigned short *lds, int ldsp,
                                            size_t plane, int row0, int col0, int nrows)
 {
@@ -356,55 +325,6 @@ __device__ __forceinline__ void stage_rows(const TileArgs &a, unsigned short *ld
    constexpr int groups = LCOLS / 8;
    const int W = a.W, H = a.H;
    const int total = nrows * groups;
-   if constexpr (SRC8) {
-      // 8-bit sources: eight items per thread in flight, each held as its raw bytes (two
-      // dwords) until every load of the batch is out
-      constexpr int K = 8;
-      for (int it0 = threadIdx.x; it0 < total; it0 += 256 * K) {
-         uint32_t lo[K], hi[K];
-#pragma unroll
-         for (int k = 0; k < K; ++k) {
-            const int it = it0 + 256 * k;
-            const int r = it / groups, g = it - r * groups;
-            const int sy = row0 + r, sx = col0 + 8 * g;
-            const bool rowin = it < total && sy >= 0 && sy < H;
-            const unsigned char *brow = reinterpret_cast<const unsigned char *>(a.src) +
-                                        (size_t)(rowin ? sy : 0) * a.sstep;
-            if (rowin && sx >= 0 && sx + 8 <= W) {
-               const u32x2_u q = *reinterpret_cast<const u32x2_u *>(brow + sx);
-               lo[k] = q.x;
-               hi[k] = q.y;
-            } else {
-               lo[k] = hi[k] = 0;
-#pragma unroll
-               for (int i = 0; i < 8; ++i) {
-                  const int x = sx + i;
-                  const uint32_t b = (rowin && x >= 0 && x < W) ? brow[x] : 0u;
-                  if (i < 4) lo[k] |= b << (8 * i); else hi[k] |= b << (8 * (i - 4));
-               }
-            }
-         }
-#pragma unroll
-         for (int k = 0; k < K; ++k) {
-            const int it = it0 + 256 * k;
-            if (it >= total) break;
-            const int r = it / groups, g = it - r * groups;
-            u16x8 h0, h1;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-               const unsigned b = ((i < 4 ? lo[k] : hi[k]) >> (8 * (i & 3))) & 0xffu;
-               const float f = a.src8 == kSrcS8 ? (float)(int)(signed char)b : (float)b;
-               unsigned short e0, e1;
-               encode<P>(f, e0, e1);
-               h0[i] = e0;
-               h1[i] = e1;
-            }
-            *reinterpret_cast<u16x8 *>(lds + (size_t)r * ldsp + 8 * g) = h0;
-            if (NPL == 2) *reinterpret_cast<u16x8 *>(lds + plane + (size_t)r * ldsp + 8 * g) = h1;
-         }
-      }
-      return;
-   }
    for (int it0 = threadIdx.x; it0 < total; it0 += 256 * 4) {
       float f[4][8];
 #pragma unroll
@@ -621,8 +541,7 @@ __host__ __device__ constexpr int pair_frag_steps(int th, int nub)
 template <int P>
 __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep, int tw, int th,
                                                     int KC, int nub, int f, int lane, u16x8 *frag,
-                                                    u16x8 *frag1, int src8, float scale = 1.f,
-                                                    int nch = 1, int ch = 0)
+                                                    u16x8 *frag1, float scale = 1.f)
 {
    const int S = pair_frag_steps(th, nub);
    const int kc = f % KC, s = (f / KC) % S, ub = f / (KC * S);
@@ -635,7 +554,7 @@ __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep,
 #pragma unroll
    for (int i = 0; i < 8; ++i) {
       const int u = 16 * kc + kb + i - dx;
-      const float t = (v < th && u >= 0 && u < wb) ? tmpl_elem(trow, (u0 + u) * nch + ch, src8) : 0.f;
+      const float t = (v < th && u >= 0 && u < wb) ? reinterpret_cast<const float *>(trow)[u0 + u] : 0.f;
       unsigned short h0, h1;
       encode<P>(P == kF16x3 ? t * scale : t, h0, h1);
       h[i] = h0;
@@ -646,14 +565,11 @@ __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep,
 }
 
 // Fragments of the row-pair kernel, one per wavefront, the FP64 sum of squares (same order
-// as single_prep) in the last block, alongside; blockIdx.y = channel (sums[0] per channel).
+// as single_prep) in the last block, alongside.
 template <int P>
 __global__ __launch_bounds__(256) void pair_prep(BatchDesc d)
 {
    __shared__ double red[4];
-   d.ch = blockIdx.y;
-   d.sums += d.ch;
-   d.frag0 += d.ch * d.fragch;
    if (blockIdx.x == gridDim.x - 1) {
       template_sqsum(d, red);
       return;
@@ -662,7 +578,7 @@ __global__ __launch_bounds__(256) void pair_prep(BatchDesc d)
    const int f = blockIdx.x * 4 + (threadIdx.x >> 6);
    if (f < nfrag)
       build_pair_fragment<P>(d.tptr, d.tstep, d.tw, d.th, d.KC, d.nub, f, threadIdx.x & 63,
-                             d.frag0, d.frag1, d.src8, 1.f, d.nch, d.ch);
+                             d.frag0, d.frag1);
 }
 
 // Batch: for template blockIdx.y, workgroups 0 .. gridDim.x - 2 build its fragments (in the
@@ -681,7 +597,7 @@ __global__ __launch_bounds__(256) void batch_prep(const BatchDesc *__restrict__ 
    for (int k = blockIdx.x * 256 + threadIdx.x; k < nfrag * 64; k += (gridDim.x - 1) * 256) {
       if constexpr (PAIR)
          build_pair_fragment<P>(d.tptr, d.tstep, d.tw, d.th, d.KC, d.nub, k >> 6, k & 63,
-                                d.frag0, d.frag1, d.src8);
+                                d.frag0, d.frag1);
       else
          build_fragment<P>(d.tptr, d.tstep, d.tw, d.th, d.KC, d.nub, k >> 6, k & 63, d.frag0,
                            d.frag1);
@@ -727,23 +643,10 @@ __device__ __forceinline__ void pair_mfma(f32x16 (&acc)[NT], const unsigned shor
 // CrossCorr map; kModeNCC / kModeSSDN store CrossCorr_Norm / SqrDistance_Norm with the window
 // sums of s^2 from the FP64 integral a.integ (the batch kernel's epilogue, the same
 // expressions as mfma_tile).
-//
-// kModeInt (8-bit integer images, BF16 operands): every value and product is an integer that
-// BF16 and FP32 hold exactly, and so is every partial sum below 2^24.  Each step adds one
-// template row to each accumulator, at most tw max|s t| in magnitude, so after a.flush steps
-// (a.flush tw max|s t| < 2^24, set by the host) the FP32 accumulators are converted to and
-// added into int32 accumulators and cleared: the sums are exact (below 2^31, also checked by
-// the host).  The epilogue pairs the int32 halves and forms the op from the exact cross term
-// (and the window sum of squares, exact in int32, which ss_box8 wrote into the map before)
-// with the same FP64 expressions as prox_tile_int, so the maps equal that kernel's bit for bit.
 template <int P, int KC, int NT, int MODE>
 __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, unsigned short *lds,
                                           int ldsp)
 {
-   static_assert(MODE == kModeCC || MODE == kModeNCC || MODE == kModeSSDN ||
-                     (MODE == kModeInt && P == kBF16 && NT == 4),
-                 "float maps, or exact integer sums (BF16, 4 n-tiles)");
-   constexpr bool INT = MODE == kModeInt;
    // operand planes: two for split BF16 (hi and lo), the lo plane of the staged rows at
    // `plane` 16-bit elements past the hi plane (the rows a band of a.vb steps stages)
    constexpr int NPL = planes_of(P);
@@ -761,39 +664,12 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[j][i] = 0.f;
-   // kModeInt: the int32 sums, and the steps since the last flush
-   int iacc[INT ? NT : 1][16];
-   int since = 0;
-   auto flush = [&]() {
-      if constexpr (INT) {
-#pragma unroll
-         for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-               iacc[j][i] += (int)acc[j][i];
-               acc[j][i] = 0.f;
-            }
-         since = 0;
-      }
-   };
-   auto stepped = [&]() {
-      if constexpr (INT) {
-         if (++since == a.flush) flush();
-      }
-   };
-   if constexpr (INT) {
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-         for (int i = 0; i < 16; ++i) iacc[j][i] = 0;
-   }
-
    for (int ub = 0; ub < a.nub; ++ub) {
       for (int s0 = 0; s0 < S; s0 += a.vb) {
          const int ns = min(a.vb, S - s0);
          __syncthreads();
          // LDS row r = source row Y0 - cy + 2 s0 + r; wave w reads rows 32 w + m + 2 (s - s0)
-         stage_rows<P, lcols, INT>(a, lds, ldsp, plane, Y0 - cy + 2 * s0, x0 - cx + ub * kBlockW,
+         stage_rows<P, lcols>(a, lds, ldsp, plane, Y0 - cy + 2 * s0, x0 - cx + ub * kBlockW,
                                    kTileRows - 2 + 2 * ns);
          __syncthreads();
 
@@ -810,20 +686,16 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
             load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)(q + 1) * KC * 64, pb, pb1);
             __builtin_amdgcn_sched_barrier(0);
             pair_mfma<P, KC, NT>(acc, arow + (size_t)(2 * q) * ldsp, plane, pa, pa1);
-            stepped();
             const int qn = q + 2 < ns ? q + 2 : q + 1;
             load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)qn * KC * 64, pa, pa1);
             __builtin_amdgcn_sched_barrier(0);
             pair_mfma<P, KC, NT>(acc, arow + (size_t)(2 * q + 2) * ldsp, plane, pb, pb1);
-            stepped();
          }
          if (q < ns) {
             pair_mfma<P, KC, NT>(acc, arow + (size_t)(2 * q) * ldsp, plane, pa, pa1);
-            stepped();
          }
       }
    }
-   flush();
 
    // Norm modes: groups of four consecutive outputs of one row per thread (kNormIters of them,
    // kEpiGroups per batch).  A group's window sums of s^2 are differences of the FP64
@@ -885,38 +757,10 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    };
    Corners qa, qb;
    if constexpr (NORM) load_corners(0, qa);
-   // kModeInt: the window sums of s^2 that ss_box8 left in the map (all ops but CrossCorr),
-   // the thread's groups of four outputs in the epilogue's order, loaded before the halves
-   // are paired so that their latency passes under it
-   constexpr int kIntIters = (kPairRows * (C / 4) + 255) / 256;
-   int4 ssq[INT ? kIntIters : 1];
-   if constexpr (INT) {
-#pragma unroll
-      for (int i = 0; i < kIntIters; ++i) {
-         const int k = threadIdx.x + 256 * i;
-         const int r = k / (C / 4), c = 4 * (k - r * (C / 4));
-         const int y = Y0 + r, x = x0 + c;
-         ssq[i] = make_int4(0, 0, 0, 0);
-         if (a.op == kCC || k >= kPairRows * (C / 4) || y >= a.H || x >= a.W) continue;
-         const gmem_i32 *oi = reinterpret_cast<const gmem_i32 *>(out_row(a, y) + x);
-         if (x + 4 <= a.W) {
-            const i32x4_t q = *reinterpret_cast<const gmem_i32x4 *>(oi);
-            ssq[i] = make_int4(q[0], q[1], q[2], q[3]);
-         } else {
-            int e4[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-               if (x + e < a.W) e4[e] = oi[e];
-            ssq[i] = make_int4(e4[0], e4[1], e4[2], e4[3]);
-         }
-      }
-   }
-
    // Pair the halves in LDS: tile row r = 32 w + m + dy holds output row Y0 - 1 + r.
    // C fragment: lane holds column n = lane % 32 of each n-tile, rows
-   // m = 8 * (i / 4) + 4 * (lane / 32) + i % 4.  (kModeInt: int32 halves, exact sums.)
+   // m = 8 * (i / 4) + 4 * (lane / 32) + i % 4.
    float *tile = reinterpret_cast<float *>(lds);
-   int *itile = reinterpret_cast<int *>(lds);
    const int n = lane & 31, dy = n >> 4, dx = n & 15;
    const int rb = 32 * wave + 4 * (lane >> 5) + dy;
    __syncthreads();
@@ -926,7 +770,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
 #pragma unroll
          for (int i = 0; i < 16; ++i) {
             const int at = (rb + 8 * (i / 4) + (i % 4)) * TP + 16 * j + dx;
-            if constexpr (INT) itile[at] = iacc[j][i]; else tile[at] = acc[j][i];
+            tile[at] = acc[j][i];
          }
    }
    __syncthreads();
@@ -936,47 +780,10 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
 #pragma unroll
          for (int i = 0; i < 16; ++i) {
             const int at = (rb + 8 * (i / 4) + (i % 4)) * TP + 16 * j + dx;
-            if constexpr (INT) itile[at] = iacc[j][i] + itile[at];
-            else tile[at] = acc[j][i] + tile[at];
+            tile[at] = acc[j][i] + tile[at];
          }
    }
    __syncthreads();
-   if constexpr (INT) {
-      // each output's op from its exact cross term CC (and for all but CrossCorr the window's
-      // sum of squares SS, an exact int32 that ss_box8 left in the map), as prox_tile_int forms
-      // it; four consecutive columns per thread, one 16-byte store where the row allows
-      const double tt = a.tsums[0];
-      const int itt = (int)tt;
-#pragma unroll
-      for (int i = 0; i < kIntIters; ++i) {
-         const int k = threadIdx.x + 256 * i;
-         const int r = k / (C / 4), c = 4 * (k - r * (C / 4));
-         const int y = Y0 + r, x = x0 + c;
-         if (k >= kPairRows * (C / 4) || y >= a.H || x >= a.W) continue;
-         const int4 cc = *reinterpret_cast<const int4 *>(&itile[(r + 1) * TP + c]);
-         const int ci[4] = {cc.x, cc.y, cc.z, cc.w};
-         gmem_f32 *o = out_row(a, y) + x;
-         const int si[4] = {ssq[i].x, ssq[i].y, ssq[i].z, ssq[i].w};
-         float v[4];
-#pragma unroll
-         for (int e = 0; e < 4; ++e) {
-            // (every sum is an exact integer below 2^31, so int32 arithmetic rounds to float as
-            // the FP64 expression does)
-            const int d = a.op == kSSD || a.op == kSSDNorm ? si[e] - 2 * ci[e] + itt : ci[e];
-            v[e] = a.op == kCC || a.op == kSSD
-                       ? (float)d
-                       : (float)((double)d * rsqrt64((double)si[e] * tt));
-         }
-         if (x + 4 <= a.W) {
-            *reinterpret_cast<gmem_f32x4 *>(o) = f32x4_t{v[0], v[1], v[2], v[3]};
-         } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-               if (x + e < a.W) o[e] = v[e];
-         }
-      }
-      return;
-   }
    // rows 1..127 are whole: four consecutive columns per thread (the tile pitch keeps them
    // 16-byte aligned in LDS), one at a time at the right edge
    static_assert(TP % 4 == 0 && C % 4 == 0, "16-byte groups of the LDS tile");
@@ -1077,15 +884,6 @@ void crosscorr_mfma_pair(TileArgs a, int ldsp, int tiles_x, int tiles, ZImages z
       a.src = z.src[zi];
       a.dst = z.dst[zi];
       a.sstep = z.sstep[zi];
-   }
-   if constexpr (MODE == kModeInt) {
-      // channel by channel
-      const int ch = blockIdx.x / tiles;
-      t = xcd_tile(blockIdx.x - ch * tiles, tiles);
-      a.src = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.src) + ch * a.plane8);
-      a.dst = reinterpret_cast<float *>(reinterpret_cast<char *>(a.dst) + ch * a.planef);
-      a.frag0 += ch * a.fragch;
-      a.tsums += ch;
    }
    if constexpr (P == kF16x3) {
       const SplitRange sr = split_range(a.peaks, a.tw * a.th);

@@ -250,13 +250,18 @@ bool sad8_ok(int op, const View &src, const View &T);
 size_t sad8_work_bytes(const View &src, const View &T);
 void launch_sad8(hipStream_t s, const View &src, const View &T, void *dst, int dst_step, void *work);
 
-// Exact integer sums of 8-bit images on BF16 MFMA (CrossCorr, CrossCorr_Norm, SqrDistance,
-// SqrDistance_Norm of U8/S8 images, every channel in one launch): int_mfma_ok tells whether the
-// path takes the call; tsums[ch] receives sum t^2.  The maps equal prox_tile_int's bit for bit.
+// Exact integer sums on int8 MFMA, bit for bit prox_tile_int's maps (OCIP_INT_MFMA=0 turns both
+// off); the _ok functions tell whether they take the call.  8-bit images, CrossCorr,
+// CrossCorr_Norm, SqrDistance and SqrDistance_Norm, every channel in one launch:
 bool int_mfma_ok(int op, const View &src, const View &T);
 size_t int_mfma_work_bytes(const View &src, const View &T);
-void launch_int_mfma(hipStream_t s, int op, const View &src, const View &T, double *tsums,
-                     float *dst, int dst_step, void *work);
+void launch_int_mfma(hipStream_t s, int op, const View &src, const View &T, float *dst, int dst_step,
+                     void *work);
+// 16-bit 1-channel images, CrossCorr and CrossCorr_Norm (`integ`: the integral of s^2):
+bool int16_mfma_ok(int op, const View &src, const View &T);
+size_t i8_work_bytes(const View &T);
+void launch_int16_mfma(hipStream_t s, int op, const View &src, const View &T, const double *integ,
+                       float *dst, int dst_step, void *work);
 
 // Batched MFMA CrossCorr_Norm (ssd = false) or SqrDistance_Norm (ssd = true) of F32 1-channel
 // templates against one F32 1-channel source, recorded into a HIP graph on first use and
