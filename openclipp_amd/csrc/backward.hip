@@ -20,7 +20,7 @@
 // templates up to 32 x 32, weight_corr in FP32 otherwise; partials reduced in FP64), the FP32
 // correlation of a map with the flipped template (the plain tiled kernel with anchor
 // (tw-1-cx, th-1-cy)), and window sums of maps in FP64 (box_f64; from an FP64 integral for
-// templates too large for its tile).
+// templates too large for it).
 #include <algorithm>
 
 #include "device_common.h"
@@ -94,19 +94,21 @@ __device__ __forceinline__ void grad_pixel(bool has1, bool has2, double c, doubl
 //              maps M and Eb of every pixel (grad_pixel) and the workgroup's partial sums;
 //   kBoxSource (the flipped window sums of Eb, anchor (tw-1-tw/2, th-1-th/2)): the source
 //              gradient dS = F + s * box, in FP64, rounded once (a null dS: nothing written).
-// One workgroup per 32 x 64 outputs of image blockIdx.y: the map region (31 + th rows by
-// 63 + tw columns) is staged in LDS as F32; a vertical pass (thread = column) keeps two FP64
-// running sums down the rows from the region's top, `lead` taking each row as it enters the
-// window and `lag` each row as it leaves, so the column sum V = lead - lag is a difference of
-// two prefixes of one sequence (exactly 0 for a column whose window rows are all zero); V goes
-// to LDS in FP64; a horizontal pass (thread = output row and 8 columns) does the same along
-// the row.  Every value of f is exact in FP64 (a float or the square of a float), and the
-// prefixes start at the tile, so the relative error stays near 2^-53 times (tile energy /
-// window energy).  Bound by instruction issue and LDS latency: staging without an index division
-// per element, 16-byte accesses to every map, and grad_pixel without square root and divisions
-// took kBoxMaps from 257 to 150 us and kBoxSource from 145 to 112 us for 16 x 1024^2 / 31x31 (400 and
-// 270 MB: 2.7 and 2.4 TB/s).
+// One workgroup per 32 x 64 outputs of image blockIdx.y.  A vertical pass straight from the map
+// (wavefront = 8 output rows, lane = column) keeps two FP64 running sums down the rows from its
+// first window's top, `lead` taking each row as it enters the window and `lag` each row as it
+// leaves, so the column sum V = lead - lag is a difference of two prefixes of one sequence
+// (exactly 0 for a column whose window rows are all zero); V goes to LDS in FP64; a horizontal pass
+// (thread = output row and 8 columns) does the same along the row.  Every value of f is exact in
+// FP64 (a float or the square of a float), and the prefixes start at most a window before, so
+// the relative error stays near 2^-53 times (tile energy / window energy).  Bound by latency (loads
+// eight rows at a time, then the serial sums), four workgroups per CU over one another.  With the
+// map region staged in LDS and one wavefront and a half on the columns: kBoxMaps 157 -> 128 us,
+// kBoxSource 119 -> 94 us for 16 x 1024^2 / 31x31 (400 and 270 MB: 3.1 and 2.9 TB/s); 16 rows per
+// thread 137 and 96, the epilogue's maps loaded ahead of the vertical pass 133 and 101, the next rows' loads
+// ahead of the sums 136 and 100.
 constexpr int kBxRows = 32, kBxCols = 64;
+constexpr int kBxRun = kBxRows / 4;   // output rows per wavefront of the vertical pass
 enum { kBoxMaps = 1, kBoxSource = 2 };
 
 // Epilogue arguments of box_f64: image z's maps C (= F), M, Eb at z * zstride elements from
@@ -122,14 +124,13 @@ struct BoxEpi {
    double *sncc, *sssd;
 };
 
-size_t box_f64_lds(int tw, int th)
+size_t box_f64_lds(int tw)
 {
-   const size_t ncols = kBxCols - 1 + tw, nrows = kBxRows - 1 + th;
-   return (size_t)kBxRows * (ncols | 1) * sizeof(double) + nrows * ncols * sizeof(float);
+   return (size_t)kBxRows * ((kBxCols - 1 + tw) | 1) * sizeof(double);
 }
 
 template <int EPI>
-__global__ __launch_bounds__(kThreads) void box_f64(ZPtrs maps, int W, int H, int tw, int th,
+__global__ __launch_bounds__(kThreads, 4) void box_f64(ZPtrs maps, int W, int H, int tw, int th,
                                                      int ax, int ay, int sqr, BoxEpi ep,
                                                      int tiles_x)
 {
@@ -138,50 +139,53 @@ __global__ __launch_bounds__(kThreads) void box_f64(ZPtrs maps, int W, int H, in
    const int z = blockIdx.y;
    const char *m = maps.p[z];
    const int mstep = maps.step[z];
-   const int ncols = kBxCols - 1 + tw, nrows = kBxRows - 1 + th;
+   const int ncols = kBxCols - 1 + tw;
    // column sums V at an odd pitch of doubles: the horizontal pass's lanes (eight rows by
    // eight 8-column groups per wavefront) then read 16 distinct pairs of LDS banks, not 8
    const int vp = ncols | 1;
-   double *vs = bx_lds;                                            // kBxRows x vp
-   float *ms = reinterpret_cast<float *>(vs + kBxRows * vp);      // nrows x ncols
+   double *vs = bx_lds;   // kBxRows x vp
    const int x0 = (blockIdx.x % tiles_x) * kBxCols, y0 = (blockIdx.x / tiles_x) * kBxRows;
-   const int c0 = x0 - ax, r0 = y0 - ay;
-   // staging: wavefront = rows w, w + 4, ..., lane = columns lane, lane + 64, ... (no index to
-   // divide out), 16 rows' loads of each lane in flight at a time
-   {
-      const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-      for (int cc = lane; cc < ncols; cc += 64) {
-         const int x = c0 + cc;
-         const bool colin = x >= 0 && x < W;
-         const float *col = reinterpret_cast<const float *>(m) + (colin ? x : 0);
-         for (int rb = wave; rb < nrows; rb += 64) {
-            float f[16];
+   // vertical pass: wavefront = kBxRun output rows, lane = columns lane, lane + 64, ...
+   const int wave = threadIdx.x >> 6, c0 = x0 - ax, r0 = y0 - ay + wave * kBxRun;
+   for (int c = threadIdx.x & 63; c < ncols; c += 64) {
+      const int x = c0 + c;
+      const bool colin = x >= 0 && x < W;
+      const char *col = m + sizeof(float) * (size_t)(colin ? x : 0);
+      auto load = [&](int i) {
+         return *reinterpret_cast<const float *>(col + (size_t)min(max(r0 + i, 0), H - 1) * mstep);
+      };
+      auto f = [&](float v, int i) {
+         const double d = colin && (unsigned)(r0 + i) < (unsigned)H ? (double)v : 0.0;
+         return sqr ? d * d : d;
+      };
+      // rows 0 .. kBxRun - 1 (the ones that leave the window), the rows between, in batches, and
+      // rows th - 1 .. th + kBxRun - 2 (the ones that enter it); `lead` in row order
+      float first[kBxRun], more[kBxRun];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-               const int y = r0 + rb + 4 * j;
-               const float *q = reinterpret_cast<const float *>(
-                   reinterpret_cast<const char *>(col) + (size_t)min(max(y, 0), H - 1) * mstep);
-               f[j] = *q;
-               if (!colin || y < 0 || y >= H) f[j] = 0.f;
-            }
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-               if (rb + 4 * j < nrows) ms[(rb + 4 * j) * ncols + cc] = f[j];
-         }
-      }
-   }
-   __syncthreads();
-   auto fv = [&](int r, int c) {
-      const double v = ms[r * ncols + c];
-      return sqr ? v * v : v;
-   };
-   for (int c = threadIdx.x; c < ncols; c += kThreads) {
+      for (int i = 0; i < kBxRun; ++i) first[i] = load(i);
       double lead = 0.0, lag = 0.0;
-      for (int i = 0; i < th - 1; ++i) lead += fv(i, c);
-      for (int r = 0; r < kBxRows; ++r) {
-         lead += fv(r + th - 1, c);
-         vs[r * vp + c] = lead - lag;
-         lag += fv(r, c);
+      for (int b = kBxRun; b < th - 1; b += kBxRun) {
+#pragma unroll
+         for (int i = 0; i < kBxRun; ++i) more[i] = load(b + i);
+         if (b == kBxRun) {
+#pragma unroll
+            for (int i = 0; i < kBxRun; ++i) lead += f(first[i], i);
+         }
+#pragma unroll
+         for (int i = 0; i < kBxRun; ++i) lead += b + i < th - 1 ? f(more[i], b + i) : 0.0;
+      }
+#pragma unroll
+      for (int i = 0; i < kBxRun; ++i) more[i] = load(th - 1 + i);
+      if (th - 1 <= kBxRun) {
+#pragma unroll
+         for (int i = 0; i < kBxRun; ++i) lead += i < th - 1 ? f(first[i], i) : 0.0;
+      }
+      double *v = vs + wave * kBxRun * vp + c;
+#pragma unroll
+      for (int i = 0; i < kBxRun; ++i) {
+         lead += f(more[i], th - 1 + i);
+         v[i * vp] = lead - lag;
+         lag += f(first[i], i);
       }
    }
    __syncthreads();
@@ -276,7 +280,7 @@ void launch_box_f64(hipStream_t s, const ZPtrs &maps, int n, int W, int H, int t
                     int ax, int ay, bool sqr, const BoxEpi &ep)
 {
    const int tiles_x = (W + kBxCols - 1) / kBxCols;
-   const size_t lds = box_f64_lds(tw, th);
+   const size_t lds = box_f64_lds(tw);
    if (lds > 64 * 1024)
       hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(box_f64<EPI>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
@@ -287,7 +291,7 @@ void launch_box_f64(hipStream_t s, const ZPtrs &maps, int n, int W, int H, int t
 }
 
 // The gradient maps (grad_pixel) of every pixel with SS from the exclusive FP64 integral
-// `integ` (templates whose box tile does not fit LDS), or without SS (has1 = 0), and
+// `integ` (templates too large for box_f64), or without SS (has1 = 0), and
 // per-block partial sums.  Image z = blockIdx.y: C, M and Eb at z * zstride elements from their
 // bases (W x H, rows W apart), G1 / G2 from the tables, partial sums at sncc / sssd +
 // z * gridDim.x.
@@ -723,7 +727,7 @@ BwLayout bw_layout(int n, int W, int H, int tw, int th)
    L.F = o;       o = align_up(o + maps);
    L.M = o;       o = align_up(o + maps);
    L.E = o;       o = align_up(o + maps);
-   L.I = o;       o = align_up(o + excl_bytes(W, H));   // templates too large for box_f64
+   L.I = o;       o = align_up(o + excl_bytes(W, H));   // templates too large for box_f64 (use_box)
    L.partial = o; o = align_up(o + (size_t)n * L.nb * tw * th * sizeof(float));
    L.red = o;     o = align_up(o + (size_t)((n * L.nb + kRedBlocks - 1) / kRedBlocks) * tw * th *
                                    sizeof(double));
@@ -770,8 +774,10 @@ void launch_backward_batch(hipStream_t s, int n, const View *S, const View *G1, 
    float *tflip = reinterpret_cast<float *>(w + L.tflip);
    double *sums = reinterpret_cast<double *>(w + L.sums);
    // window sums straight from the maps (box_f64, its epilogues forming the gradient maps
-   // and dS) when its LDS tile fits, else from integrals
-   const bool use_box = box_f64_lds(tw, th) <= (size_t)(160 * 1024 - 256);
+   // and dS) up to 256 rows (each wavefront reads th + 7 rows for 8; 4 images of 1000x700, with box_f64
+   // and with integrals: 128x128 3416 and 3482 us, 8x256 1017 and 1055, 8x400 1628 and 1562) and
+   // where its LDS row fits, else from integrals
+   const bool use_box = th <= 256 && box_f64_lds(tw) <= (size_t)(160 * 1024 - 256);
    // partial sums per image: one per tile of box_f64<kBoxMaps>, else per block of grad_maps
    const int nscal = use_box && G1 ? box_tiles(W, H) : grid_for((long long)px);
    const int taps = tw * th;
