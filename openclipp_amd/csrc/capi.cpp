@@ -177,9 +177,8 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
    }
    if (precision == ocipPrecisionF32 && int16_mfma_ok(op, view(S), view(T))) {
       c.stats.ensure(i8_work_bytes(view(T)));
-      const double *integ = norm ? sqr_integral_for(c, S, 0) : nullptr;
-      launch_int16_mfma(c.stream, op, view(S), view(T), integ, static_cast<float *>(D.dev),
-                        D.desc.Step, c.stats.ptr);
+      launch_int16_mfma(c.stream, op, view(S), view(T), static_cast<float *>(D.dev), D.desc.Step,
+                        c.stats.ptr);
       D.in_device = true;
       return;
    }

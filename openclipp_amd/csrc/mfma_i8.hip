@@ -1,4 +1,5 @@
-// mfma_i8.hip -- exact cross terms of 8- and 16-bit integer images on int8 matrix cores.
+// mfma_i8.hip -- CrossCorr, CrossCorr_Norm, SqrDistance and SqrDistance_Norm of 8- and 16-bit integer
+// images on int8 matrix cores, exact whole-number sums throughout.
 //
 // v_mfma_i32_32x32x32_i8 takes 32 source columns per instruction (a BF16 product takes 16) and adds
 // into int32, so sums are exact without flushes.  Source values become signed bytes,
@@ -44,8 +45,13 @@ __host__ __device__ constexpr int i8_steps(int th) { return (th + 1) / 2; }
 // n-tiles of 16 columns per wavefront.  8-bit: two, against four SqrDistance 4096^2/32x32 50 -> 47.6 us,
 // colour CrossCorr_Norm 1280x960/24x24 42 -> 33 (twice the wavefronts per SIMD), one 60 and 33.5.
 // 16-bit: one, against two CrossCorr_Norm 2048x1536/31x31 60 -> 51 us (48x48 of 4000x3000 233 -> 248).
+// (kernel times without the window sums)
 __host__ __device__ constexpr int i8_nt(int npa) { return npa == 1 ? 2 : 1; }
 __host__ __device__ constexpr int i8_lcols(int npa, int KC) { return 16 * (i8_nt(npa) - 1) + 32 * KC; }
+
+// pitch of the row sums of window_sums: 36 dwords, an odd multiple of 4 (16-byte stores of 8
+// consecutive rows on distinct banks)
+__host__ __device__ constexpr int hsum_pitch(int type) { return type == SImage::U16 || type == SImage::S16 ? 18 : 36; }
 
 // B fragments (NPB digits, lowest first) of channel blockIdx.y, one (row pair, chunk) per wavefront;
 // the last block the sums of the template: sums[2 ch] = sum t^2 (of t - 128 for U8 in one digit),
@@ -121,9 +127,6 @@ struct I8Args {
    int tw, th;
    const i32x4 *frag;
    const double *sums;          // i8_prep
-   // 8-bit ops but CrossCorr: the int32 window sums of s^2 (of (s - 128)^2 for U8 in one digit) lie
-   // in dst; 16-bit CrossCorr_Norm: the integral of s^2
-   const double *integ;
    float *dst;
    int dstep, op;
    size_t plane8, planef;       // bytes from one channel's source and map to the next
@@ -196,17 +199,102 @@ __device__ __forceinline__ void stage_i8(const I8Args &a, const unsigned char *s
    }
 }
 
+// Window sums of s^2 (of (s - 128)^2 for U8 in one digit) from the staged rows: SS of output column
+// `col` of C, rows row0 .. row0 + 128 C / 256 - 1, exact integers.  First the sums over tw columns
+// for every staged row and output column, thread = row, running along it; then over th rows,
+// thread = output column and a run of rows.  Differences of running sums that only ever grow (sums
+// that took squares off were compiled into byte dot products that added them).  It adds 12 us to
+// the 49 of SqrDistance U8 4096^2/32x32 and saves the 23 us of a kernel that wrote these sums to
+// memory; for 16-bit types 4 to 51 (2048x1536/31x31) and the integral's 25.
+template <int TYPE, int NPB, int C, class Sum>
+__device__ __forceinline__ void window_sums(const unsigned char *lds, int ldsp, int plane, int nrows,
+                                            Sum *hs, int tw, int th, int col, int row0,
+                                            Sum (&ss)[kTileRows * C / 256])
+{
+   constexpr bool B16 = is16(TYPE);
+   constexpr int HP = hsum_pitch(TYPE), kRun = kTileRows * C / 256;
+   // four elements: the staged bytes back to s
+   struct Px { uint32_t l, h; };
+   auto dword = [&](const unsigned char *row, int k) {
+      Px q;
+      q.l = reinterpret_cast<const uint32_t *>(row)[k];
+      q.h = B16 ? reinterpret_cast<const uint32_t *>(row + plane)[k] : 0u;
+      if (B16 || (TYPE == SImage::U8 && NPB == 2)) q.l ^= 0x80808080u;
+      if (TYPE == SImage::U16) q.h ^= 0x80808080u;
+      return q;
+   };
+   auto add = [&](Sum acc, const Px &q, int e) -> Sum {
+      if constexpr (B16) {
+         const uint32_t u = (q.h >> (8 * e) & 0xffu) << 8 | (q.l >> (8 * e) & 0xffu);
+         const uint32_t v = TYPE == SImage::S16 ? (uint32_t)abs((int)(int16_t)u) : u;
+         return acc + (uint64_t)v * v;
+      } else {
+         const int v = TYPE == SImage::U8 && NPB == 2 ? (int)(q.l >> (8 * e) & 0xffu)
+                                                      : (int)(q.l << (24 - 8 * e)) >> 24;
+         return acc + __mul24(v, v);
+      }
+   };
+   for (int r = threadIdx.x; r < nrows; r += 256) {
+      const unsigned char *row = lds + (size_t)r * ldsp;
+      Sum lead = 0, lag = 0;
+      int k = 0;
+      for (; 4 * k + 4 <= tw; ++k) {
+         const Px q = dword(row, k);
+#pragma unroll
+         for (int e = 0; e < 4; ++e) lead = add(lead, q, e);
+      }
+      Px q = dword(row, k);   // (the bytes past the row's last are never used)
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+         if (e < (tw & 3)) lead = add(lead, q, e);
+      Sum *out = hs + (size_t)r * HP;
+#pragma unroll
+      for (int j = 0; j < C / 4; ++j) {
+         // elements tw + 4 j .. of the row enter, elements 4 j .. leave
+         const Px n = dword(row, k + j + 1), o = dword(row, j);
+         const Px in = {__builtin_amdgcn_alignbyte(n.l, q.l, tw & 3), __builtin_amdgcn_alignbyte(n.h, q.h, tw & 3)};
+         q = n;
+         Sum w[4];
+#pragma unroll
+         for (int e = 0; e < 4; ++e) {
+            w[e] = lead - lag;
+            lead = add(lead, in, e);
+            lag = add(lag, o, e);
+         }
+         int4 *at = reinterpret_cast<int4 *>(out + 4 * j);
+         if constexpr (B16) {
+            at[0] = make_int4((int)w[0], (int)(w[0] >> 32), (int)w[1], (int)(w[1] >> 32));
+            at[1] = make_int4((int)w[2], (int)(w[2] >> 32), (int)w[3], (int)(w[3] >> 32));
+         } else {
+            at[0] = make_int4(w[0], w[1], w[2], w[3]);
+         }
+      }
+   }
+   __syncthreads();
+   const Sum *h = hs + (size_t)row0 * HP + col;
+   Sum lead = 0, lag = 0;
+   for (int i = 0; i < th - 1; ++i) lead += h[i * HP];
+#pragma unroll
+   for (int i = 0; i < kRun; ++i) {
+      lead += h[(th - 1 + i) * HP];
+      ss[i] = lead - lag;
+      lag += h[i * HP];
+   }
+}
+
 __device__ __forceinline__ i32x16 mma_i8(i32x4 a, i32x4 b, i32x16 c)
 {
    return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
 }
 
-// Bound by latency (staging, then the products, then the epilogue, two to six workgroups per CU over
-// one another) above the map's bytes (8-bit SqrDistance 4096^2/32x32: 49 us, 144 MB = 28 us at the copy rate) and
-// the MFMAs (U16 2048x1536/31x31: 51 us, of it 22 in the products, 17 us of MFMA issue).  Against
-// BF16 products flushed into int32 every few rows: SqrDistance 4096^2/32x32 82 -> 49 us, colour
-// CrossCorr_Norm 1280x960/24x24 37.5 -> 33 us; 16-bit images against the tile kernel's int64 sums:
-// 120 -> 51 us.  More wavefronts per SIMD by bounds on the registers (3, 4): no faster, spills at 4.
+// Bound by latency (staging, window sums, products and epilogue, three or four workgroups per CU over one
+// another) above the map's bytes (SqrDistance U8 4096^2/32x32: 61 us, 84 MB = 16 us at the copy rate,
+// 14 us of MFMA issue; CrossCorr_Norm U16 2048x1536/31x31: 55 us, of it 22 in the products, 17 us of
+// MFMA issue).  Whole calls, against BF16 products flushed into int32 every few rows and the window sums
+// from a kernel of their own: SqrDistance U8 4096^2/32x32 98 -> 56 us, colour CrossCorr_Norm
+// 1280x960/24x24 68 -> 50 us; against the tile kernel's int64 sums and the integral: CrossCorr_Norm U16
+// 2048x1536/31x31 154 -> 50 us.  More wavefronts per SIMD by bounds on the registers (3, 4): no
+// faster, spills at 4.
 template <int TYPE, int NPB, int KC>
 __global__ __launch_bounds__(256, is16(TYPE) && KC > 2 ? 1 : 2)
 void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
@@ -231,6 +319,16 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
    // LDS row r = source row Y0 - cy + r; wave w reads rows 32 w + m + 2 s
    stage_i8<TYPE, i8_lcols(NPA, KC) / 16>(a, src, lds, ldsp, plane, Y0 - a.th / 2, x0 - a.tw / 2, nrows);
    __syncthreads();
+   // the op's window sums, in registers until the epilogue: thread = output column `col`, kRun rows
+   // from `row0` on
+   constexpr int kRun = kTileRows * C / 256;
+   const int col = threadIdx.x % C, row0 = threadIdx.x / C * kRun;
+   typedef typename std::conditional<B16, uint64_t, int>::type Sum;
+   Sum ss[kRun];
+   if (a.op != kCC)
+      window_sums<TYPE, NPB, C>(lds, ldsp, plane, nrows, reinterpret_cast<Sum *>(lds + NPA * plane), a.tw,
+                                a.th, col, row0, ss);
+
    i32x16 acc[NL][NT];
 #pragma unroll
    for (int l = 0; l < NL; ++l)
@@ -309,73 +407,19 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
          for (int i = 0; i < 16; ++i) tile[(rb + 8 * (i / 4) + (i % 4)) * TP + 16 * j + dx] += half(j, i);
    }
    __syncthreads();
-   // four consecutive columns per thread
-   const int itt = (int)tt;
    constexpr int K = TYPE == SImage::U16 ? 32896 : TYPE == SImage::S16 || (TYPE == SImage::U8 && NPB == 2) ? 128 : 0;
-   const V kt = (V)K * (V)t1;
-   const int cx = a.tw / 2, cy = a.th / 2;
-   const size_t ip = excl_pitch(a.W);
-   for (int g = threadIdx.x; g < kPairRows * (C / 4); g += 256) {
-      const int r = g / (C / 4), c = 4 * (g - r * (C / 4));
-      const int y = Y0 + r, x = x0 + c;
-      if (y >= a.H || x >= a.W) continue;
-      const V *cc = &tile[(r + 1) * TP + c];
-      float *o = reinterpret_cast<float *>(dst + (size_t)y * a.dstep) + x;
-      const bool whole = x + 4 <= a.W;
-      float v[4];
-      if constexpr (B16) {
-         if (a.op == kCC) {
+   const V kt = (V)K * (V)t1, vtt = (V)tt;
+   const int x = x0 + col;
+   if (x >= a.W) return;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (float)(cc[e] + kt);
-         } else {
-            double ss[4];
-            if (x >= cx && x - cx + a.tw + 3 <= a.W && y >= cy && y - cy + a.th <= a.H) {
-               const double *p = a.integ + (size_t)(y - cy) * ip + (kExclOffset + x - cx);
-               const double *p1 = p + (size_t)a.th * ip;
-#pragma unroll
-               for (int e = 0; e < 4; e += 2) {
-                  const f64x2_u v0 = *reinterpret_cast<const f64x2_u *>(p + e);
-                  const f64x2_u v1 = *reinterpret_cast<const f64x2_u *>(p1 + e);
-                  const f64x2_u v2 = *reinterpret_cast<const f64x2_u *>(p + a.tw + e);
-                  const f64x2_u v3 = *reinterpret_cast<const f64x2_u *>(p1 + a.tw + e);
-#pragma unroll
-                  for (int h = 0; h < 2; ++h) ss[e + h] = (v3[h] - v2[h]) - (v1[h] - v0[h]);
-               }
-            } else {
-#pragma unroll
-               for (int e = 0; e < 4; ++e) ss[e] = window_sqsum(a.integ, a.W, a.H, x + e, y, a.tw, a.th);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (float)((cc[e] + kt) * rsqrt64(ss[e] * tt));
-         }
-      } else {
-         int ss[4] = {0, 0, 0, 0};
-         if (a.op != kCC) {
-            if (whole) {
-               const i32x4_u q = *reinterpret_cast<const i32x4_u *>(o);
-#pragma unroll
-               for (int e = 0; e < 4; ++e) ss[e] = q[e];
-            } else {
-#pragma unroll
-               for (int e = 0; e < 4; ++e)
-                  if (x + e < a.W) ss[e] = reinterpret_cast<const int *>(o)[e];
-            }
-         }
-#pragma unroll
-         for (int e = 0; e < 4; ++e) {
-            const int cross = cc[e] + kt;
-            const int d = a.op == kSSD || a.op == kSSDNorm ? ss[e] - 2 * cross + itt : cross;
-            v[e] = a.op == kCC || a.op == kSSD ? (float)d
-                                               : (float)((double)d * rsqrt64((double)ss[e] * tt));
-         }
-      }
-      if (whole) {
-         *reinterpret_cast<f32x4_u *>(o) = f32x4_u{v[0], v[1], v[2], v[3]};
-      } else {
-#pragma unroll
-         for (int e = 0; e < 4; ++e)
-            if (x + e < a.W) o[e] = v[e];
-      }
+   for (int i = 0; i < kRun; ++i) {
+      const int r = row0 + i, y = Y0 + r;
+      if (r >= kPairRows || y >= a.H) continue;
+      // (whole numbers, below 2^31 or 2^53)
+      const V cross = tile[(r + 1) * TP + col] + kt;
+      const V d = a.op == kSSD || a.op == kSSDNorm ? (V)ss[i] - 2 * cross + vtt : cross;
+      const float v = a.op == kCC || a.op == kSSD ? (float)d : (float)((double)d * rsqrt64((double)ss[i] * tt));
+      reinterpret_cast<float *>(dst + (size_t)y * a.dstep)[x] = v;
    }
 }
 
@@ -398,7 +442,9 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
    // an odd multiple of 16 bytes: the A reads of 8 consecutive rows on distinct banks
    int ldsp = i8_lcols(NPA, KC);
    if (ldsp % 32 == 0) ldsp += 16;
-   const size_t staging = (size_t)NPA * (kTileRows - 2 + 2 * steps) * ldsp;
+   const int nrows = kTileRows - 2 + 2 * steps;
+   const size_t sums = (size_t)(nrows + 1) * hsum_pitch(TYPE) * (B16 ? 8 : 4);
+   const size_t staging = (size_t)NPA * nrows * ldsp + (a.op == kCC ? 0 : sums);
    const size_t pairing = (size_t)(kTileRows + 1) * (16 * NT + (B16 ? 2 : 4)) * (B16 ? 8 : 4);
    const size_t lds = std::max(staging, pairing);
    const int tiles_x = (a.W + 16 * NT - 1) / (16 * NT), tiles_y = (a.H + kPairRows - 1) / kPairRows;
@@ -420,152 +466,7 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
    launch_check("crosscorr_i8");
 }
 
-// ------------------------------------------------------------------------- window sums, planes
-// Window sums of s^2 of an 8-bit image, exact in int32, into the map `dst` (as int32 bits):
-// SS(x, y) = sum over the template window of (x, y) (origin (-tw/2, -th/2), zero outside the
-// image).  One wavefront per band of box_band(th) output rows and 256 source columns, four adjacent
-// ones per lane, i.e. box_cols(tw) output columns:
-//  * each lane's four column sums of squares over the window's rows, running down the band: the
-//    squares of the rows entering the window (a dword each) less those of the rows leaving it;
-//  * per output row the inclusive prefix I of the column sums along the row: the lane's own four,
-//    a wavefront scan of the lanes' totals (DPP row shifts and broadcasts; U rows at once), then
-//    SS(i) = I[i + tw - 1] - I[i - 1]: the subtrahends are the lane's own, the minuends come through
-//    LDS; one 16-byte store per lane and row.
-// Integer arithmetic modulo 2^32 throughout and every result below 2^31 (checked by the host), so
-// the sums are exact in any order.  Bound by issue and the map's store: about 44 instructions per
-// row and 225 outputs (tw = 32) where a lane per output column with a ring of row sums in LDS
-// took 35 per 64 (4096^2/32x32: 38 -> 22 us).
-// Output rows per wavefront: 16, or 32 where the th - 1 rows before the first would outweigh them
-// (more wavefronts hide the chains' latency: colour 1280x960/24x24 15 us with 16, 18 with 32, 25 with 64)
-constexpr int box_band(int th) { return th <= 48 ? 16 : 32; }
-constexpr int kBoxOob = 0x40000000;   // a byte count past any image this kernel takes
-constexpr int box_cols(int tw) { return (256 - (tw - 1)) / 4 * 4; }
-
-// Inclusive scans across the 64 lanes of N values at once (the N scans interleaved, so that
-// each DPP step's wait on the previous one is filled by the others): within rows of 16 lanes
-// (lanes without a source add 0), then rows 1 and 3 take the last lane of rows 0 and 2, rows
-// 2 and 3 the last lane of row 1.
-template <int N>
-__device__ __forceinline__ void wave_incl_scan(int (&x)[N])
-{
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x111, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x112, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x114, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x118, 0xf, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x142, 0xa, 0xf, false);
-#pragma unroll
-   for (int k = 0; k < N; ++k) x[k] += __builtin_amdgcn_update_dpp(0, x[k], 0x143, 0xc, 0xf, false);
-}
-
-// FLIP: of s - 128 (U8).
-template <bool SIGNED, bool FLIP>
-__global__ __launch_bounds__(64) void ss_box8(const unsigned char *__restrict__ src, int W,
-                                              int H, int sstep, int tw, int th,
-                                              char *__restrict__ dst, int dstep, int bands,
-                                              size_t plane8, size_t planef)
-{
-   constexpr int U = 4;                          // rows at once (their loads one batch ahead)
-   __shared__ int pre[U][256 + 100];             // (lanes past the outputs read up to tw + 2 past 256)
-   typedef uint32_t u32_u __attribute__((aligned(1)));
-   typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
-   const int lane = threadIdx.x;
-   // consecutive blocks (one XCD's run) side by side along a band share halo columns in L2
-   const int b = xcd_tile(blockIdx.x, gridDim.x);
-   // blockIdx.y = channel
-   src += blockIdx.y * plane8;
-   dst += blockIdx.y * planef;
-   const int cblks = gridDim.x / bands, cols = box_cols(tw);
-   const int band = b / cblks, cblk = b % cblks;
-   const int x0 = cblk * cols, y0 = band * box_band(th);
-   const int cx = tw / 2, cy = th / 2;
-   const int n = min(box_band(th), H - y0);
-   // the lane's columns c .. c + 3 from the dword at column min(max(c, 0), W - 4), shifted into
-   // place, zero outside the image (mask 0: wholly outside)
-   const int c = x0 - cx + 4 * lane, cl = min(max(c, 0), W - 4);
-   const int lsh = min(max(-c, 0), 3) * 8, rsh = min(max(c - cl, 0), 3) * 8;
-   const uint32_t mask = c <= -4 || c >= W ? 0u : 0xffffffffu;
-   auto load = [&](int y) -> uint32_t {
-      return *reinterpret_cast<const u32_u *>(src + (size_t)min(max(y, 0), H - 1) * sstep + cl);
-   };
-   auto place = [&](uint32_t v, int y) -> uint32_t {
-      return ((unsigned)y < (unsigned)H ? (v << lsh) >> rsh & mask : 0u) ^ (FLIP ? 0x80808080u : 0u);
-   };
-   auto elem = [&](uint32_t v, int e) -> int {
-      return SIGNED ? (int)(v << (24 - 8 * e)) >> 24 : (int)(v >> (8 * e) & 0xffu);
-   };
-   // column sums lead - lag: squares are only ever added (sums that took squares off were compiled
-   // into byte dot products that added them)
-   int lead[4] = {0, 0, 0, 0}, lag[4] = {0, 0, 0, 0};
-   // the th - 1 rows before the first output row's last
-   for (int j0 = 0; j0 < th - 1; j0 += 8) {
-      uint32_t v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = load(y0 - cy + j0 + j);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-         const uint32_t q = j0 + j < th - 1 ? place(v[j], y0 - cy + j0 + j) : 0u;
-#pragma unroll
-         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(q, e), elem(q, e));
-      }
-   }
-   uint32_t in[U], out[U];
-   auto fetch = [&](int r) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         in[u] = load(y0 - cy + th - 1 + r + u);
-         out[u] = load(y0 - cy + r + u);
-      }
-   };
-   fetch(0);
-   const int x = x0 + 4 * lane;
-   const bool mine = 4 * lane < cols && x < W;
-   for (int r0 = 0; r0 < n; r0 += U) {
-      int q[U][4], inc[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         const uint32_t a = place(in[u], y0 - cy + th - 1 + r0 + u), o = place(out[u], y0 - cy + r0 + u);
-#pragma unroll
-         for (int e = 0; e < 4; ++e) lead[e] += __mul24(elem(a, e), elem(a, e));
-         q[u][0] = lead[0] - lag[0];
-#pragma unroll
-         for (int e = 1; e < 4; ++e) q[u][e] = q[u][e - 1] + (lead[e] - lag[e]);
-         inc[u] = q[u][3];
-#pragma unroll
-         for (int e = 0; e < 4; ++e) lag[e] += __mul24(elem(o, e), elem(o, e));
-      }
-      if (r0 + U < n) fetch(r0 + U);
-      wave_incl_scan<U>(inc);
-      __syncthreads();   // the reads of the batch before are done
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         inc[u] -= q[u][3];   // the sums of the lanes before
-         *reinterpret_cast<int4 *>(&pre[u][4 * lane]) =
-             make_int4(inc[u] + q[u][0], inc[u] + q[u][1], inc[u] + q[u][2], inc[u] + q[u][3]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-         const int *p = &pre[u][4 * lane + tw - 1];
-         const int s0 = p[0] - inc[u], s1 = p[1] - inc[u] - q[u][0], s2 = p[2] - inc[u] - q[u][1],
-                   s3 = p[3] - inc[u] - q[u][2];
-         if (!mine || r0 + u >= n) continue;
-         int *o = reinterpret_cast<int *>(dst + (size_t)(y0 + r0 + u) * dstep) + x;
-         if (x + 4 <= W) {
-            *reinterpret_cast<i32x4_u *>(o) = i32x4_u{s0, s1, s2, s3};
-         } else {
-            o[0] = s0;
-            if (x + 1 < W) o[1] = s1;
-            if (x + 2 < W) o[2] = s2;
-         }
-      }
-   }
-}
-
+// ------------------------------------------------------------------------- planes
 // Interleaved 8-bit channels into planes of their own (row pitch plane8_step, plane pitch H rows),
 // zeros between the width and the pitch, and the planes of the map back into interleaved
 // channels: the kernels between them take every channel of an image in one launch, as
@@ -668,10 +569,7 @@ bool int_mfma_ok(int op, const View &S, const View &T)
    if ((S.type != SImage::U8 && S.type != SImage::S8) || T.type != S.type) return false;
    if (S.channels != 1 && S.channels != 2 && S.channels != 4) return false;
    const int tw = T.width, th = T.height;
-   // (ss_box8: dwords of four columns)
-   if (tw <= 0 || th <= 0 || tw > 97 || th > 97 || (S.width < 4 && op != kCC)) return false;
-   if ((long long)S.height * std::max((long long)S.step, (long long)plane8_step(S.width)) >= kBoxOob)
-      return false;
+   if (tw <= 0 || th <= 0 || i8_chunks(tw) > 4 || th > 128) return false;
    // the whole sum in int32
    return (long long)tw * th * (S.type == SImage::U8 ? 255 * 255 : 128 * 128) < (1LL << 31);
 }
@@ -717,22 +615,6 @@ void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, fl
       a.dstep = 4 * S.step;
       a.planef = (size_t)S.height * a.dstep;
    }
-   if (op != kCC) {
-      // the window sums of s^2 go to the map first; the MFMA kernel's epilogue reads them
-      KernelTimer kt(s, "ss_box8");
-      const int bands = (S.height + box_band(T.height) - 1) / box_band(T.height);
-      const int cblks = (S.width + box_cols(T.width) - 1) / box_cols(T.width);
-      auto go = [&](auto kernel) {
-         kernel<<<dim3(bands * cblks, nch), 64, 0, s>>>(static_cast<const unsigned char *>(S.ptr),
-                                                       S.width, S.height, S.step, T.width, T.height,
-                                                       reinterpret_cast<char *>(a.dst), a.dstep, bands,
-                                                       a.plane8, a.planef);
-      };
-      if (T.type == SImage::S8) go(ss_box8<true, false>);
-      else if (op == kSSD) go(ss_box8<true, true>);
-      else go(ss_box8<false, false>);
-      launch_check("ss_box8");
-   }
    if (T.type == SImage::S8) launch_i8<SImage::S8, 1>(s, a, S, T);
    else if (op == kSSD) launch_i8<SImage::U8, 1>(s, a, S, T);
    else launch_i8<SImage::U8, 2>(s, a, S, T);
@@ -749,20 +631,19 @@ void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, fl
 
 // Every size up to the widest template of four chunks: against the tile kernel, CrossCorr 160x120/2x2
 // 9.2 -> 8.2 us, 640x480/3x3 11.1 -> 10.0, 1920x1080/11x11 27 -> 17, /49x49 232 -> 45, /113x128
-// 1355 -> 204.  (The height keeps the staged rows within the LDS and the sums within int32.)
+// 1355 -> 204; SqrDistance 640x480/5x5 12.6 -> 10.9, 2048x1536/31x31 192 -> 49.  (The height keeps the
+// staged rows and their sums within the LDS and the products within int32.)
 bool int16_mfma_ok(int op, const View &S, const View &T)
 {
    const char *e = getenv("OCIP_INT_MFMA");
-   if ((e && e[0] == '0') || (op != kCC && op != kCCNorm)) return false;
+   if ((e && e[0] == '0') || op == kSAD) return false;
    if (!is16(S.type) || T.type != S.type || S.channels != 1) return false;
    return T.width > 0 && T.height > 0 && i8_chunks(T.width) <= 4 && T.height <= 128;
 }
 
-void launch_int16_mfma(hipStream_t s, int op, const View &S, const View &T, const double *integ,
-                       float *dst, int dstep, void *work)
+void launch_int16_mfma(hipStream_t s, int op, const View &S, const View &T, float *dst, int dstep, void *work)
 {
    I8Args a = work_args(op, work);
-   a.integ = integ;
    a.dst = dst;
    a.dstep = dstep;
    if (S.type == SImage::U16) launch_i8<SImage::U16, 3>(s, a, S, T);

@@ -257,11 +257,11 @@ bool int_mfma_ok(int op, const View &src, const View &T);
 size_t int_mfma_work_bytes(const View &src, const View &T);
 void launch_int_mfma(hipStream_t s, int op, const View &src, const View &T, float *dst, int dst_step,
                      void *work);
-// 16-bit 1-channel images, CrossCorr and CrossCorr_Norm (`integ`: the integral of s^2):
+// the same of 16-bit 1-channel images:
 bool int16_mfma_ok(int op, const View &src, const View &T);
 size_t i8_work_bytes(const View &T);
-void launch_int16_mfma(hipStream_t s, int op, const View &src, const View &T, const double *integ,
-                       float *dst, int dst_step, void *work);
+void launch_int16_mfma(hipStream_t s, int op, const View &src, const View &T, float *dst, int dst_step,
+                       void *work);
 
 // Batched MFMA CrossCorr_Norm (ssd = false) or SqrDistance_Norm (ssd = true) of F32 1-channel
 // templates against one F32 1-channel source, recorded into a HIP graph on first use and
