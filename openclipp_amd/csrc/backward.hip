@@ -785,16 +785,13 @@ void launch_backward_batch(hipStream_t s, int n, const View *S, const View *G1, 
 
    bool any_ds = false;
    for (int i = 0; i < n; ++i) any_ds = any_ds || dS[i];
-   if (G1) {
-      const View tv{tstage, tw, th, tpitch * (int)sizeof(float), 1, SImage::F32};
-      prep_crosscorr_split(s, tv, w + L.fragT, sums);
-   }
+   SplitTemplate fwd{View{tstage, tw, th, tpitch * (int)sizeof(float), 1, SImage::F32}, w + L.fragT, sums};
+   SplitTemplate flip{View{tflip, L.twf, L.thf, L.twf * (int)sizeof(float), 1, SImage::F32}, w + L.fragF,
+                      sums + 4};
    if (any_ds) {
       flip_template<<<grid_for((long long)L.twf * L.thf), kThreads, 0, s>>>(tstage, tpitch, tw, th,
                                                                            L.twf, L.thf, tflip);
       launch_check("flip_template");
-      const View fv{tflip, L.twf, L.thf, L.twf * (int)sizeof(float), 1, SImage::F32};
-      prep_crosscorr_split(s, fv, w + L.fragF, sums + 4);
    }
    const float *src[kSplitImages];
    float *dst[kSplitImages];
@@ -829,7 +826,7 @@ void launch_backward_batch(hipStream_t s, int n, const View *S, const View *G1, 
             step[k] = S[c0 + k].step;
             dst[k] = F0 + (size_t)k * px;
          }
-         launch_crosscorr_split(s, m, src, step, dst, W * 4, W, H, tw, th, w + L.fragT, sums);
+         launch_crosscorr_split(s, m, src, step, dst, W * 4, W, H, fwd);
       }
       // the maps M and Eb (and partial sums): from the windows' sums of s^2 in the epilogue
       // of box_f64, or with those sums from integrals, or without them (no CrossCorr_Norm term)
@@ -906,7 +903,7 @@ void launch_backward_batch(hipStream_t s, int n, const View *S, const View *G1, 
          step[k] = W * 4;
          dst[k] = F0 + (size_t)k * px;
       }
-      launch_crosscorr_split(s, m, src, step, dst, W * 4, W, H, L.twf, L.thf, w + L.fragF, sums + 4);
+      launch_crosscorr_split(s, m, src, step, dst, W * 4, W, H, flip);
       // dS from F, s and the flipped window sums of Eb (window anchored at tw - 1 - cx,
       // th - 1 - cy)
       if (use_box) {

@@ -816,7 +816,7 @@ void launch_crosscorr_mfma(hipStream_t s, int precision, bool norm, const View &
 // Split-BF16 CrossCorr maps (anchor (tw/2, th/2), zero outside the image, no Norm) of several
 // sources of one size with one template: crosscorr_mfma (NT = 2 or 4) or the row-pair kernel
 // (NT = 4 or 6), the autotuner's choice, the images of up to kZImages sources in one launch.
-// The template's fragments, in both layouts, are prepared once by prep_crosscorr_split.
+// The template's fragments are prepared by the first launch that takes their layout.
 static_assert(kSplitImages == mfma::kZImages, "sources per launch");
 size_t crosscorr_split_frag_bytes(int tw, int th)
 {
@@ -831,33 +831,26 @@ static Geometry split_geometry(int tw, int th, int NT = 4)
    return g;
 }
 
-void prep_crosscorr_split(hipStream_t s, const View &T, void *frags, double *sums)
-{
-   const int tw = T.width, th = T.height, KC = kc_for(tw), KC2 = kc2_for(tw), nub = nub_for(tw);
-   (void)split_geometry(tw, th);
-   u16x8 *f0 = static_cast<u16x8 *>(frags);
-   const BatchDesc d{static_cast<const char *>(T.ptr), tw, th, T.step, KC, nub, f0,
-                     f0 + (size_t)nub * th * KC * 64, sums};
-   mfma::launch_single_prep<mfma::kBF16x3>(s, d);
-   // the row-pair layout after it (both preps write the same sum of squares)
-   u16x8 *g0 = reinterpret_cast<u16x8 *>(static_cast<char *>(frags) +
-                                         mfma_frag_bytes(mfma::kBF16x3, tw, th));
-   const BatchDesc e{static_cast<const char *>(T.ptr), tw, th, T.step, KC2, nub, g0,
-                     g0 + pair_frag_count(tw, th) * 64, sums};
-   mfma::launch_pair_prep<mfma::kBF16x3>(s, e);
-}
-
 void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const int *sstep,
-                            float *const *dst, int dstep, int W, int H, int tw, int th,
-                            const void *frags, const double *sums)
+                            float *const *dst, int dstep, int W, int H, SplitTemplate &t)
 {
+   const int tw = t.T.width, th = t.T.height;
    const int KC = kc_for(tw), KC2 = kc2_for(tw), nub = nub_for(tw);
    const int vb = split_geometry(tw, th).vb;
-   const u16x8 *f0 = static_cast<const u16x8 *>(frags);
-   const u16x8 *f1 = f0 + (size_t)nub * th * KC * 64;
-   const u16x8 *g0 = reinterpret_cast<const u16x8 *>(static_cast<const char *>(frags) +
-                                                     mfma_frag_bytes(mfma::kBF16x3, tw, th));
-   const u16x8 *g1 = g0 + pair_frag_count(tw, th) * 64;
+   u16x8 *f0 = static_cast<u16x8 *>(t.frags), *f1 = f0 + (size_t)nub * th * KC * 64;
+   // the row-pair layout after the other (both preps write the same sum of squares)
+   u16x8 *g0 = reinterpret_cast<u16x8 *>(static_cast<char *>(t.frags) +
+                                         mfma_frag_bytes(mfma::kBF16x3, tw, th));
+   u16x8 *g1 = g0 + pair_frag_count(tw, th) * 64;
+   auto prep = [&](bool pair) {
+      if (t.ready[pair]) return;
+      t.ready[pair] = true;
+      const char *tp = static_cast<const char *>(t.T.ptr);
+      if (pair)
+         mfma::launch_pair_prep<mfma::kBF16x3>(s, BatchDesc{tp, tw, th, t.T.step, KC2, nub, g0, g1, t.sums});
+      else
+         mfma::launch_single_prep<mfma::kBF16x3>(s, BatchDesc{tp, tw, th, t.T.step, KC, nub, f0, f1, t.sums});
+   };
    // one launch per kZImages sources: variant 2 or 4, crosscorr_mfma with NT = 2 or 4 column
    // tiles per workgroup; 14 or 16, the row-pair kernel with NT = 4 or 6
    auto run = [&](int variant) {
@@ -866,6 +859,7 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
       const Geometry g = pair ? pair_geometry(KC2, NT, th, mfma::kLdsMax, 2)
                               : split_geometry(tw, th, NT);
       if (g.vb < 1) fail(CL_INVALID_VALUE, "template too large for the MFMA tile");
+      prep(pair);
       for (int i0 = 0; i0 < n; i0 += mfma::kZImages) {
          SingleLaunch L;
          L.z.n = std::min(mfma::kZImages, n - i0);
@@ -879,13 +873,13 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
          L.ldsp = g.ldsp;
          L.lds = g.lds;
          if (pair) {
-            L.a = mfma::TileArgs{src[i0], W, H, sstep[i0], tw, th, nub, g0, g1, sums, nullptr,
+            L.a = mfma::TileArgs{src[i0], W, H, sstep[i0], tw, th, nub, g0, g1, t.sums, nullptr,
                                  dst[i0], dstep, g.vb, 0};
             L.KC = KC2;
             L.grid = dim3((W + 16 * NT - 1) / (16 * NT), (H + mfma::kPairRows - 1) / mfma::kPairRows);
             mfma::launch_pair<mfma::kBF16x3>(s, L);
          } else {
-            L.a = mfma::TileArgs{src[i0], W, H, sstep[i0], tw, th, nub, f0, f1, sums, nullptr,
+            L.a = mfma::TileArgs{src[i0], W, H, sstep[i0], tw, th, nub, f0, f1, t.sums, nullptr,
                                  dst[i0], dstep, vb, 0};
             L.KC = KC;
             L.grid = dim3((W + 32 * NT - 1) / (32 * NT), (H + mfma::kTileRows - 1) / mfma::kTileRows);

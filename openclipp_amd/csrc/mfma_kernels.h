@@ -178,7 +178,8 @@ __device__ __forceinline__ void build_fragment(const char *tptr, int tstep, int 
 #pragma unroll
    for (int i = 0; i < 8; ++i) {
       const int u = 16 * kc + kb + i - n;
-      const float t = (u >= 0 && u < wb) ? trow[u0 + u] : 0.f;
+      float t = trow[u0 + min(max(u, 0), wb - 1)];   // (in range: all 8 loads in flight)
+      if (u < 0 || u >= wb) t = 0.f;
       unsigned short h0, h1;
       encode<P>(t, h0, h1);
       a[i] = h0;
@@ -202,10 +203,10 @@ __device__ __forceinline__ void template_sqsum(const BatchDesc &d, double *red)
       float t[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-         const int k = k0 + 256 * i;
+         const int k = min(k0 + 256 * i, total - 1);
          const int v = k / pitch, u = k - v * pitch;
-         t[i] = (k < total && u < d.tw)
-                    ? reinterpret_cast<const float *>(d.tptr + (size_t)v * d.tstep)[u] : 0.f;
+         t[i] = reinterpret_cast<const float *>(d.tptr + (size_t)v * d.tstep)[min(u, d.tw - 1)];
+         if (k0 + 256 * i >= total || u >= d.tw) t[i] = 0.f;
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) s2 += (double)t[i] * (double)t[i];
@@ -554,7 +555,8 @@ __device__ __forceinline__ void build_pair_fragment(const char *tptr, int tstep,
 #pragma unroll
    for (int i = 0; i < 8; ++i) {
       const int u = 16 * kc + kb + i - dx;
-      const float t = (v < th && u >= 0 && u < wb) ? reinterpret_cast<const float *>(trow)[u0 + u] : 0.f;
+      float t = reinterpret_cast<const float *>(trow)[u0 + min(max(u, 0), wb - 1)];   // (as above)
+      if (v >= th || u < 0 || u >= wb) t = 0.f;
       unsigned short h0, h1;
       encode<P>(P == kF16x3 ? t * scale : t, h0, h1);
       h[i] = h0;

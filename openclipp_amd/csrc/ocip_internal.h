@@ -221,14 +221,19 @@ void launch_crosscorr_mfma(hipStream_t s, int precision, bool norm, const View &
 // The single-template MFMA Norm path forms its denominators from the source image; only
 // templates wider than 513 columns read the FP64 sum-of-squares integral instead.
 // Split-BF16 CrossCorr maps (no Norm) of n sources of one size (row pitches sstep[]) with one
-// template, whose fragments (crosscorr_split_frag_bytes) prep_crosscorr_split wrote to
-// `frags` (and sum t^2 to sums[0]); up to 16 sources per launch
+// template; up to 16 sources per launch.  The template, its fragments (crosscorr_split_frag_bytes;
+// the layout that the kernel variant reads is prepared by the first launch that takes it) and
+// sums (sum t^2 to sums[0]):
 constexpr int kSplitImages = 16;   // sources per launch of launch_crosscorr_split
 size_t crosscorr_split_frag_bytes(int tw, int th);
-void prep_crosscorr_split(hipStream_t s, const View &T, void *frags, double *sums);
+struct SplitTemplate {
+   View T;
+   void *frags;
+   double *sums;
+   bool ready[2] = {false, false};   // the layouts of crosscorr_mfma and crosscorr_mfma_pair
+};
 void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const int *sstep,
-                            float *const *dst, int dstep, int W, int H, int tw, int th,
-                            const void *frags, const double *sums);
+                            float *const *dst, int dstep, int W, int H, SplitTemplate &t);
 bool crosscorr_mfma_needs_integral(int tw);
 size_t crosscorr_mfma_work_bytes(int precision, int width, int height, int tw, int th);
 
