@@ -16,8 +16,10 @@
 //                  accumulates in the reference order (template row outer, column inner) with
 //                  one fused multiply-add per tap, which is the reference's order under
 //                  OpenCL's default FP contraction.
-//   prox_tile_int  8- and 16-bit integer sources: the same tiling with exact integer sums
-//                  (int32 where the bound allows, int64 otherwise), rounded once to float.
+//   prox_sad8      AbsDistance of 8-bit sources: the same tiling on dwords of four bytes.
+//   prox_tile_int  8- and 16-bit integer sources (what neither prox_sad8 nor the int8 matrix cores
+//                  of mfma_i8.hip take): the same tiling with exact integer sums (int32 where the
+//                  bound allows, int64 otherwise), rounded once to float.
 //   prox_direct    one output per thread, reference order, any type (F64 sources and
 //                  templates too wide for the LDS tile).
 // Norm denominators come from the FP64 sum-of-squares integral of the source (exclusive,
@@ -1004,7 +1006,7 @@ void launch_sad8(hipStream_t s, const View &image, const View &T, void *dst, int
              static_cast<const unsigned char *>(T.ptr), tw, th, T.step, nch, tq);
          launch_check("sad8_template");
       }
-      KernelTimer kt(s, "prox_tile_int");
+      KernelTimer kt(s, "prox_sad8");
       kernel<<<dim3(tiles, nch), 256, lds, s>>>(static_cast<const unsigned char *>(S.ptr), S.width,
                                                 S.height, S.step, plane8, tq, tw, th,
                                                 static_cast<char *>(dst), dstep, nch, vb, ldsw);
