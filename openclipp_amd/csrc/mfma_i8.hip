@@ -2,16 +2,18 @@
 // images on int8 matrix cores, exact whole-number sums throughout.
 //
 // v_mfma_i32_32x32x32_i8 takes 32 source columns per instruction (a BF16 product takes 16) and adds
-// into int32, so sums are exact without flushes.  Source values become signed bytes,
-//   S8   s                                                                         K = 0
-//   U8   s - 128                                                                   K = 128
-//   S16  s - 128   = 256 h + l, h the high byte, l the low byte - 128              K = 128
-//   U16  s - 32896 = 256 h + l, h the high byte - 128, l the low byte - 128        K = 32896
-// (pixels outside the image: 0 - K), template values t signed digits of base 256 (one for S8, two
-// for U8, three for 16-bit types, the top one 0 or 1), and
-//   sum s t = sum over the pairs of digits of 256^(place of both) sum s_i t_j + K sum t,
-// one int32 sum per place, put together in FP64 (16-bit: exact below 2^53) or int32.  SqrDistance
-// of U8 takes t - 128 in one digit instead: a difference keeps when both lose 128.
+// into int32, so sums are exact without flushes.  Values v of source and template become signed bytes
+// of v - K,
+//   S8   v                                                                         K = 0
+//   U8   v - 128                                                                   K = 128
+//   S16  v - 128   = 256 h + l, h the high byte, l the low byte - 128              K = 128
+//   U16  v - 32896 = 256 h + l, h the high byte - 128, l the low byte - 128        K = 32896
+// (pixels outside the image: 0 - K), products of 16-bit types one int32 sum per place, put together
+// in FP64 (exact below 2^53).  With s, t now the values less K, n taps, and window sums S1 of s, SS of
+// s^2 (window_sums), T1 and TT those of the template:
+//   SqrDistance = SS - 2 sum s t + TT   (a difference keeps when both lose K),
+//   CrossCorr = sum s t + K S1 + K T1 + K^2 n,
+//   and the true sums of squares SS + 2 K S1 + K^2 n, TT + 2 K T1 + K^2 n for the Norm ops.
 //
 // The contraction is the row-pair one of mfma_kernels.h (crosscorr_mfma_pair) with chunks of 32 source
 // columns: MFMA column n = 16 dy + dx, output row Y0 - 1 + 32 w + m + dy,
@@ -37,8 +39,13 @@ typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 typedef const i32x4 __attribute__((address_space(1))) *gfrag_i8;
 
 constexpr bool is16(int type) { return type == SImage::U16 || type == SImage::S16; }
-// digits of a source value, digits of a template value (U8: 1 = both less 128), places
+// digits of a value; its offset K
 __host__ __device__ constexpr int i8_npa(int type) { return type == SImage::U16 || type == SImage::S16 ? 2 : 1; }
+
+__host__ __device__ constexpr int i8_key(int type)
+{
+   return type == SImage::U16 ? 32896 : type == SImage::S8 ? 0 : 128;
+}
 
 __host__ __device__ constexpr int i8_chunks(int tw) { return (tw + 15 + 31) / 32; }
 __host__ __device__ constexpr int i8_steps(int th) { return (th + 1) / 2; }
@@ -49,18 +56,17 @@ __host__ __device__ constexpr int i8_steps(int th) { return (th + 1) / 2; }
 __host__ __device__ constexpr int i8_nt(int npa) { return npa == 1 ? 2 : 1; }
 __host__ __device__ constexpr int i8_lcols(int npa, int KC) { return 16 * (i8_nt(npa) - 1) + 32 * KC; }
 
-// pitch of the row sums of window_sums: 36 dwords, an odd multiple of 4 (16-byte stores of 8
-// consecutive rows on distinct banks)
-__host__ __device__ constexpr int hsum_pitch(int type) { return type == SImage::U16 || type == SImage::S16 ? 18 : 36; }
+// pitch of the row sums of window_sums over C columns: an odd multiple of 16 bytes (16-byte stores of
+// 8 consecutive rows on distinct banks)
+__host__ __device__ constexpr int hsum_pitch(int C, int bytes) { return C + 16 / bytes; }
 
-// B fragments (NPB digits, lowest first) of channel blockIdx.y, one (row pair, chunk) per wavefront;
-// the last block the sums of the template: sums[2 ch] = sum t^2 (of t - 128 for U8 in one digit),
-// sums[2 ch + 1] = sum t.
-template <int TYPE, int NPB>
+// B fragments (the digits, lowest first) of channel blockIdx.y, one (row pair, chunk) per wavefront;
+// the last block the sums of the template less K: sums[2 ch] = TT, sums[2 ch + 1] = T1.
+template <int TYPE>
 __global__ __launch_bounds__(256) void i8_prep(const char *tpl, int tw, int th, int tstep, int nch,
                                                i32x4 *frag, double *sums)
 {
-   constexpr bool kKey = TYPE == SImage::U8 && NPB == 1;
+   constexpr int K = i8_key(TYPE), NPB = i8_npa(TYPE);
    __shared__ double red[2][4];
    const int ch = blockIdx.y, KC = i8_chunks(tw), S = i8_steps(th);
    if (blockIdx.x == gridDim.x - 1) {
@@ -75,7 +81,7 @@ __global__ __launch_bounds__(256) void i8_prep(const char *tpl, int tw, int th, 
          }
 #pragma unroll
          for (int k = 0; k < 8; ++k) {
-            const double q = i0 + 256 * k < n ? (double)(kKey ? t[k] - 128 : t[k]) : 0.0;
+            const double q = i0 + 256 * k < n ? (double)(t[k] - K) : 0.0;
             s2 += q * q;
             s1 += q;
          }
@@ -107,7 +113,7 @@ __global__ __launch_bounds__(256) void i8_prep(const char *tpl, int tw, int th, 
    for (int i = 0; i < 16; ++i) {
       const int u = 32 * kc + kb + i - dx;
       int t = (int)ld<TYPE>(row, min(max(u, 0), tw - 1) * nch + ch);   // (in range: all 16 in flight)
-      t = v < th && u >= 0 && u < tw ? (kKey ? t - 128 : t) : 0;
+      t = v < th && u >= 0 && u < tw ? t - K : 0;
 #pragma unroll
       for (int p = 0; p < NPB; ++p) {
          const int digit = (int)(int8_t)t;
@@ -199,40 +205,34 @@ __device__ __forceinline__ void stage_i8(const I8Args &a, const unsigned char *s
    }
 }
 
-// Window sums of s^2 (of (s - 128)^2 for U8 in one digit) from the staged rows: SS of output column
-// `col` of C, rows row0 .. row0 + 128 C / 256 - 1, exact integers.  First the sums over tw columns
-// for every staged row and output column, thread = row, running along it; then over th rows,
-// thread = output column and a run of rows.  Differences of running sums that only ever grow (sums
-// that took squares off were compiled into byte dot products that added them).  It adds 12 us to
-// the 49 of SqrDistance U8 4096^2/32x32 and saves the 23 us of a kernel that wrote these sums to
-// memory; for 16-bit types 4 to 51 (2048x1536/31x31) and the integral's 25.
-template <int TYPE, int NPB, int C, class Sum>
+// Window sums of s^2 (SQ) or of s, s less K, from the staged rows: of output column `col` of C, rows
+// row0 .. row0 + 128 C / 256 - 1, exact integers.  First the sums over tw columns for every staged
+// row and output column (hs), thread = row, running along it; then over th rows, thread = output
+// column and a run of rows.  Differences of running sums (squares are only ever added: sums that
+// took some off were compiled into byte dot products that added them).  The sums of squares add 12 us
+// to the 49 of SqrDistance U8 4096^2/32x32 and save the 23 us of a kernel that wrote them to memory; for
+// 16-bit types 4 to 51 (2048x1536/31x31) and the integral's 25.
+template <int TYPE, int C, bool SQ, class Sum>
 __device__ __forceinline__ void window_sums(const unsigned char *lds, int ldsp, int plane, int nrows,
                                             Sum *hs, int tw, int th, int col, int row0,
                                             Sum (&ss)[kTileRows * C / 256])
 {
    constexpr bool B16 = is16(TYPE);
-   constexpr int HP = hsum_pitch(TYPE), kRun = kTileRows * C / 256;
-   // four elements: the staged bytes back to s
+   constexpr int HP = hsum_pitch(C, sizeof(Sum)), kRun = kTileRows * C / 256;
+   // four elements
    struct Px { uint32_t l, h; };
    auto dword = [&](const unsigned char *row, int k) {
       Px q;
       q.l = reinterpret_cast<const uint32_t *>(row)[k];
       q.h = B16 ? reinterpret_cast<const uint32_t *>(row + plane)[k] : 0u;
-      if (B16 || (TYPE == SImage::U8 && NPB == 2)) q.l ^= 0x80808080u;
-      if (TYPE == SImage::U16) q.h ^= 0x80808080u;
       return q;
    };
    auto add = [&](Sum acc, const Px &q, int e) -> Sum {
-      if constexpr (B16) {
-         const uint32_t u = (q.h >> (8 * e) & 0xffu) << 8 | (q.l >> (8 * e) & 0xffu);
-         const uint32_t v = TYPE == SImage::S16 ? (uint32_t)abs((int)(int16_t)u) : u;
-         return acc + (uint64_t)v * v;
-      } else {
-         const int v = TYPE == SImage::U8 && NPB == 2 ? (int)(q.l >> (8 * e) & 0xffu)
-                                                      : (int)(q.l << (24 - 8 * e)) >> 24;
-         return acc + __mul24(v, v);
-      }
+      int v = (int)(q.l << (24 - 8 * e)) >> 24;
+      if (B16) v += (int)(q.h << (24 - 8 * e)) >> 24 << 8;
+      if constexpr (!SQ) return acc + v;
+      else if constexpr (B16) return acc + (uint64_t)((uint32_t)abs(v) * (uint32_t)abs(v));
+      else return acc + __mul24(v, v);
    };
    for (int r = threadIdx.x; r < nrows; r += 256) {
       const unsigned char *row = lds + (size_t)r * ldsp;
@@ -262,7 +262,7 @@ __device__ __forceinline__ void window_sums(const unsigned char *lds, int ldsp, 
             lag = add(lag, o, e);
          }
          int4 *at = reinterpret_cast<int4 *>(out + 4 * j);
-         if constexpr (B16) {
+         if constexpr (sizeof(Sum) == 8) {
             at[0] = make_int4((int)w[0], (int)(w[0] >> 32), (int)w[1], (int)(w[1] >> 32));
             at[1] = make_int4((int)w[2], (int)(w[2] >> 32), (int)w[3], (int)(w[3] >> 32));
          } else {
@@ -289,18 +289,19 @@ __device__ __forceinline__ i32x16 mma_i8(i32x4 a, i32x4 b, i32x16 c)
 
 // Bound by latency (staging, window sums, products and epilogue, three or four workgroups per CU over one
 // another) above the map's bytes (SqrDistance U8 4096^2/32x32: 61 us, 84 MB = 16 us at the copy rate,
-// 14 us of MFMA issue; CrossCorr_Norm U16 2048x1536/31x31: 55 us, of it 22 in the products, 17 us of
-// MFMA issue).  Whole calls, against BF16 products flushed into int32 every few rows and the window sums
-// from a kernel of their own: SqrDistance U8 4096^2/32x32 98 -> 56 us, colour CrossCorr_Norm
-// 1280x960/24x24 68 -> 50 us; against the tile kernel's int64 sums and the integral: CrossCorr_Norm U16
-// 2048x1536/31x31 154 -> 50 us.  More wavefronts per SIMD by bounds on the registers (3, 4): no
-// faster, spills at 4.
-template <int TYPE, int NPB, int KC>
+// 14 us of MFMA issue) and, for large 16-bit templates, the MFMAs.  Whole calls, against BF16
+// products flushed into int32 every few rows and the window sums from a kernel of their own:
+// SqrDistance U8 4096^2/32x32 98 -> 55 us, CrossCorr 68 -> 53, /64x64 148 -> 108; against the tile
+// kernel's int64 sums and the integral: CrossCorr_Norm U16 2048x1536/31x31 154 -> 46 us.  With the
+// template's values whole (a digit more, 256 times 0 or 1) instead of less K and window sums of s:
+// CrossCorr U8 66 us (64x64 168), CrossCorr_Norm U16 51.  More wavefronts per SIMD by bounds on the
+// registers (3, 4): no faster, spills at 4.
+template <int TYPE, int KC>
 __global__ __launch_bounds__(256, is16(TYPE) && KC > 2 ? 1 : 2)
 void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
 {
    constexpr bool B16 = is16(TYPE);
-   constexpr int NPA = i8_npa(TYPE), NL = NPA + NPB - 1;
+   constexpr int NPA = i8_npa(TYPE), NPB = NPA, NL = NPA + NPB - 1, K = i8_key(TYPE);
    constexpr int NT = i8_nt(NPA), C = 16 * NT, NA = NT + 2 * KC - 2;
    typedef typename std::conditional<B16, double, int>::type V;   // a half row's cross term
    constexpr int TP = C + (B16 ? 2 : 4);                          // pitch of the paired tile
@@ -325,9 +326,14 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
    const int col = threadIdx.x % C, row0 = threadIdx.x / C * kRun;
    typedef typename std::conditional<B16, uint64_t, int>::type Sum;
    Sum ss[kRun];
+   int s1[kRun];
+   unsigned char *hs = lds + NPA * plane;
    if (a.op != kCC)
-      window_sums<TYPE, NPB, C>(lds, ldsp, plane, nrows, reinterpret_cast<Sum *>(lds + NPA * plane), a.tw,
-                                a.th, col, row0, ss);
+      window_sums<TYPE, C, true>(lds, ldsp, plane, nrows, reinterpret_cast<Sum *>(hs), a.tw, a.th, col, row0, ss);
+   if (K && a.op != kSSD) {
+      __syncthreads();
+      window_sums<TYPE, C, false>(lds, ldsp, plane, nrows, reinterpret_cast<int *>(hs), a.tw, a.th, col, row0, s1);
+   }
 
    i32x16 acc[NL][NT];
 #pragma unroll
@@ -356,15 +362,12 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
 #pragma unroll
          for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-            for (int k = 0; k < 6; ++k) {
-               // digit of s, digit of t: neighbours never add into the same place
-               constexpr int kA[6] = {0, 1, 0, 1, 1, 0}, kB[6] = {0, 1, 1, 2, 0, 2};
-               if (kA[k] >= NPA || kB[k] >= NPB) continue;
+            for (int k = 0; k < NPA * NPB; ++k) {
+               // digit of s, digit of t: (l, l), (h, l), (h, h), (l, h)
+               constexpr int kA[4] = {0, 1, 1, 0}, kB[4] = {0, 0, 1, 1};
 #pragma unroll
                for (int j = 0; j < NT; ++j)
-                  acc[kA[k] + kB[k]][j] =
-                      mma_i8(x[kA[k] < NPA ? kA[k] : 0][j + 2 * kc], q[kc][kB[k] < NPB ? kB[k] : 0],
-                             acc[kA[k] + kB[k] < NL ? kA[k] + kB[k] : 0][j]);
+                  acc[kA[k] + kB[k]][j] = mma_i8(x[kA[k]][j + 2 * kc], q[kc][kB[k]], acc[kA[k] + kB[k]][j]);
             }
       };
       fetch(0, b[0]);
@@ -407,23 +410,29 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
          for (int i = 0; i < 16; ++i) tile[(rb + 8 * (i / 4) + (i % 4)) * TP + 16 * j + dx] += half(j, i);
    }
    __syncthreads();
-   constexpr int K = TYPE == SImage::U16 ? 32896 : TYPE == SImage::S16 || (TYPE == SImage::U8 && NPB == 2) ? 128 : 0;
-   const V kt = (V)K * (V)t1, vtt = (V)tt;
+   // (whole numbers throughout, below 2^31 or 2^53)
+   const V n1 = (V)(a.tw * a.th), vtt = (V)tt, kt = K * (V)t1 + K * n1 * K;
+   const double ttrue = tt + 2.0 * K * t1 + (double)K * K * (double)(a.tw * a.th);
    const int x = x0 + col;
    if (x >= a.W) return;
 #pragma unroll
    for (int i = 0; i < kRun; ++i) {
       const int r = row0 + i, y = Y0 + r;
       if (r >= kPairRows || y >= a.H) continue;
-      // (whole numbers, below 2^31 or 2^53)
-      const V cross = tile[(r + 1) * TP + col] + kt;
-      const V d = a.op == kSSD || a.op == kSSDNorm ? (V)ss[i] - 2 * cross + vtt : cross;
-      const float v = a.op == kCC || a.op == kSSD ? (float)d : (float)((double)d * rsqrt64((double)ss[i] * tt));
+      const V cross = tile[(r + 1) * TP + col];
+      V d;
+      if (a.op == kSSD || a.op == kSSDNorm) d = (V)ss[i] - 2 * cross + vtt;
+      else d = cross + (K ? K * (V)s1[i] : (V)0) + kt;
+      float v = (float)d;
+      if (a.op == kSSDNorm || a.op == kCCNorm) {
+         const V sst = (V)ss[i] + (K ? 2 * K * (V)s1[i] + K * n1 * K : (V)0);
+         v = (float)((double)d * rsqrt64((double)sst * ttrue));
+      }
       reinterpret_cast<float *>(dst + (size_t)y * a.dstep)[x] = v;
    }
 }
 
-template <int TYPE, int NPB>
+template <int TYPE>
 void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
 {
    constexpr int NPA = i8_npa(TYPE), NT = i8_nt(NPA);
@@ -434,7 +443,7 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
    const int KC = i8_chunks(a.tw), steps = i8_steps(a.th), nch = T.channels;
    {
       KernelTimer kt(s, "template_prep");
-      i8_prep<TYPE, NPB><<<dim3((steps * KC + 3) / 4 + 1, nch), 256, 0, s>>>(
+      i8_prep<TYPE><<<dim3((steps * KC + 3) / 4 + 1, nch), 256, 0, s>>>(
           static_cast<const char *>(T.ptr), a.tw, a.th, T.step, nch, const_cast<i32x4 *>(a.frag),
           const_cast<double *>(a.sums));
       launch_check("i8_prep");
@@ -443,8 +452,9 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
    int ldsp = i8_lcols(NPA, KC);
    if (ldsp % 32 == 0) ldsp += 16;
    const int nrows = kTileRows - 2 + 2 * steps;
-   const size_t sums = (size_t)(nrows + 1) * hsum_pitch(TYPE) * (B16 ? 8 : 4);
-   const size_t staging = (size_t)NPA * nrows * ldsp + (a.op == kCC ? 0 : sums);
+   const int sum = B16 && a.op != kCC ? 8 : 4;
+   const size_t sums = (size_t)(nrows + 1) * hsum_pitch(16 * NT, sum) * sum;
+   const size_t staging = (size_t)NPA * nrows * ldsp + (a.op == kCC && i8_key(TYPE) == 0 ? 0 : sums);
    const size_t pairing = (size_t)(kTileRows + 1) * (16 * NT + (B16 ? 2 : 4)) * (B16 ? 8 : 4);
    const size_t lds = std::max(staging, pairing);
    const int tiles_x = (a.W + 16 * NT - 1) / (16 * NT), tiles_y = (a.H + kPairRows - 1) / kPairRows;
@@ -457,10 +467,10 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
       kernel<<<tiles_x * tiles_y * nch, 256, lds, s>>>(a, ldsp, tiles_x, tiles_x * tiles_y);
    };
    switch (KC) {
-   case 1: go(crosscorr_i8<TYPE, NPB, 1>); break;
-   case 2: go(crosscorr_i8<TYPE, NPB, 2>); break;
-   case 3: go(crosscorr_i8<TYPE, NPB, 3>); break;
-   case 4: go(crosscorr_i8<TYPE, NPB, 4>); break;
+   case 1: go(crosscorr_i8<TYPE, 1>); break;
+   case 2: go(crosscorr_i8<TYPE, 2>); break;
+   case 3: go(crosscorr_i8<TYPE, 3>); break;
+   case 4: go(crosscorr_i8<TYPE, 4>); break;
    default: fail(CL_INVALID_VALUE, "template width");
    }
    launch_check("crosscorr_i8");
@@ -574,12 +584,12 @@ bool int_mfma_ok(int op, const View &S, const View &T)
    return (long long)tw * th * (S.type == SImage::U8 ? 255 * 255 : 128 * 128) < (1LL << 31);
 }
 
-// Sums (two per channel), then the fragments of every channel (three digits at most).
+// Sums (two per channel), then the fragments of every channel (two digits at most).
 constexpr size_t kSumsBytes = 256;
 
 size_t i8_work_bytes(const View &T)
 {
-   const size_t n = 3 * (size_t)T.channels * i8_steps(T.height) * i8_chunks(T.width) * 64 * sizeof(i32x4);
+   const size_t n = 2 * (size_t)T.channels * i8_steps(T.height) * i8_chunks(T.width) * 64 * sizeof(i32x4);
    return kSumsBytes + (n + 255) / 256 * 256;
 }
 
@@ -615,9 +625,8 @@ void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, fl
       a.dstep = 4 * S.step;
       a.planef = (size_t)S.height * a.dstep;
    }
-   if (T.type == SImage::S8) launch_i8<SImage::S8, 1>(s, a, S, T);
-   else if (op == kSSD) launch_i8<SImage::U8, 1>(s, a, S, T);
-   else launch_i8<SImage::U8, 2>(s, a, S, T);
+   if (T.type == SImage::S8) launch_i8<SImage::S8>(s, a, S, T);
+   else launch_i8<SImage::U8>(s, a, S, T);
    if (nch > 1) {
       KernelTimer kt(s, "join_planes");
       auto go = [&](auto kernel) {
@@ -630,9 +639,9 @@ void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, fl
 }
 
 // Every size up to the widest template of four chunks: against the tile kernel, CrossCorr 160x120/2x2
-// 9.2 -> 8.2 us, 640x480/3x3 11.1 -> 10.0, 1920x1080/11x11 27 -> 17, /49x49 232 -> 45, /113x128
-// 1355 -> 204; SqrDistance 640x480/5x5 12.6 -> 10.9, 2048x1536/31x31 192 -> 49.  (The height keeps the
-// staged rows and their sums within the LDS and the products within int32.)
+// 9.9 -> 9.0 us, 640x480/3x3 11.2 -> 10.5, 4096^2/8x8 120 -> 75, /64x64 2428 -> 358; SqrDistance
+// 160x120/4x4 11.3 -> 9.4, 2048x1536/31x31 192 -> 49.  (The height keeps the staged rows and their
+// sums within the LDS and the products within int32.)
 bool int16_mfma_ok(int op, const View &S, const View &T)
 {
    const char *e = getenv("OCIP_INT_MFMA");
@@ -646,8 +655,8 @@ void launch_int16_mfma(hipStream_t s, int op, const View &S, const View &T, floa
    I8Args a = work_args(op, work);
    a.dst = dst;
    a.dstep = dstep;
-   if (S.type == SImage::U16) launch_i8<SImage::U16, 3>(s, a, S, T);
-   else launch_i8<SImage::S16, 3>(s, a, S, T);
+   if (S.type == SImage::U16) launch_i8<SImage::U16>(s, a, S, T);
+   else launch_i8<SImage::S16>(s, a, S, T);
 }
 
 }  // namespace ocip

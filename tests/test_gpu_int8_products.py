@@ -1,6 +1,6 @@
 """Cross terms of 8- and 16-bit integer images as products of signed bytes: against exact integer
 sums.  The largest and smallest values of each type are among the data (they reach every digit, the
-carry into the top one included)."""
+both halves of 16-bit values included)."""
 import numpy as np
 import pytest
 
