@@ -44,8 +44,8 @@ constexpr int kFftThreads = 1024;
 // Workgroups of the proximity passes for transforms of up to kFftSmallLen points: 8 wavefronts, two
 // on each SIMD, with 128 registers and half a CU's LDS (lengths up to about 4600 with their
 // twiddles), so that two workgroups share a CU and one computes while the other waits at a
-// barrier or for memory.  4320 points: 278 + 110 + 118 us for the three passes at 4096^2/256x256
-// against 350 + 131 + 162 us with 10 wavefronts (640 threads, one round for a radix-8 stage), whose
+// barrier or for memory.  4320 points: 278 + 110 + 118 us for the three passes at 4096^2/256x256 (before
+// map_at) against 350 + 131 + 162 us with 10 wavefronts (640 threads, one round for a radix-8 stage), whose
 // 3 + 3 + 2 + 2 on the SIMDs leaves no room for a second workgroup.  Longer transforms take
 // kFftThreads, one workgroup per CU.
 constexpr int kFftSmallThreads = 512, kFftSmallLen = kFftMaxLen / 2;
@@ -356,9 +356,20 @@ __global__ OCIP_FFT_BOUNDS(SMALL) void fft_rows_pair(const char *__restrict__ S,
    }
 }
 
+// Where the map's half spectra between passes 2 and 3 hold row y, column kx: blocks of kMapRows rows, a
+// column's values of a block side by side.  Pass 2 stores a column, so a row apart each would be 16 bytes of
+// a line, which left L2 before its neighbours' columns filled it (338 MB written for 142 at 4320 points);
+// pass 3 reads two rows at a time.  Passes 2 + 3 at 4096^2/256x256: 273 + 116 us with rows apart,
+// 265 + 120 with blocks of 2, 249 + 125 of 4, 251 + 152 of 8.
+constexpr int kMapRows = 4;
+__host__ __device__ constexpr size_t map_at(int y, int kx, int half)
+{
+   return ((size_t)(y / kMapRows) * half + kx) * kMapRows + y % kMapRows;
+}
+
 // Pass 2: spectrum column kx <= Wb / 2: FFT along y of the template's column (at y = 0) and of the
 // source's (at y = th/2), the conjugated product, FFT along y again; rows y < H stored
-// transposed: out[y * half + kx].  One column in LDS at a time, the template's spectrum in
+// transposed (map_at).  One column in LDS at a time, the template's spectrum in
 // registers meanwhile.
 template <bool SMALL>
 __global__ OCIP_FFT_BOUNDS(SMALL) void fft_cols(const double2 *__restrict__ ins,
@@ -397,7 +408,7 @@ __global__ OCIP_FFT_BOUNDS(SMALL) void fft_cols(const double2 *__restrict__ ins,
    }
    lds_barrier();
    lds_fft<true, THREADS, MAXN>(fbuf, 1, ph, ltw);
-   for (int y = threadIdx.x; y < H; y += THREADS) out[(size_t)y * half + kx] = fbuf[y];
+   for (int y = threadIdx.x; y < H; y += THREADS) out[map_at(y, kx, half)] = fbuf[y];
 }
 
 // Pass 3: output rows 2 j and 2 j + 1: FFT along x of Q_a + i Q_b = the two correlation rows, the
@@ -417,15 +428,15 @@ __global__ OCIP_FFT_BOUNDS(SMALL) void fft_rows_epi(const double2 *__restrict__ 
    const bool two = y + 1 < H;
    double2 *ltw = fbuf + Wb;
    for (int i = threadIdx.x; i < pw->twsize; i += THREADS) ltw[i] = tww[i];
-   const double2 *qa = in + (size_t)y * half, *qb = two ? qa + half : qa;
+   const double2 *qa = in + map_at(y, 0, half), *qb = two ? qa + 1 : qa;   // (y even: one block)
    {
       constexpr int PER = (FftShape<SMALL>::maxn / 2 + THREADS) / THREADS;
       double2 a[PER], b[PER];
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
          const int k = min((int)threadIdx.x + i * THREADS, half - 1);
-         a[i] = qa[k];
-         b[i] = qb[k];
+         a[i] = qa[(size_t)k * kMapRows];
+         b[i] = qb[(size_t)k * kMapRows];
       }
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
@@ -707,7 +718,7 @@ void fft_prepare(hipStream_t s, FftState *st, int W, int H, int tw, int th)
    // any image and template of this padded size
    const size_t half = Wb / 2 + 1;
    st->a.ensure(half * spectrum_pitch(Hb) * sizeof(double2));
-   st->b.ensure(half * Hb * sizeof(double2));
+   st->b.ensure(half * ((Hb + kMapRows - 1) / kMapRows * kMapRows) * sizeof(double2));
    st->t.ensure(half * spectrum_pitch(Hb) * sizeof(double2));
    st->tpart.ensure((size_t)((Hb + 1) / 2) * sizeof(double));
    st->Wb = Wb;
