@@ -135,7 +135,8 @@ struct I8Args {
    const double *sums;          // i8_prep
    float *dst;
    int dstep, op;
-   size_t plane8, planef;       // bytes from one channel's source and map to the next
+   size_t plane8;               // bytes from one channel's source to the next
+   int nch;                     // channels, interleaved in the map
 };
 
 // Source rows [row0, row0 + nrows) x columns [col0, col0 + 16 groups) as signed bytes, 16 columns
@@ -307,13 +308,15 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
    constexpr int TP = C + (B16 ? 2 : 4);                          // pitch of the paired tile
    extern __shared__ uint4 lds_v[];
    unsigned char *lds = reinterpret_cast<unsigned char *>(lds_v);
-   const int ch = blockIdx.x / tiles;
-   const int t = xcd_tile(blockIdx.x - ch * tiles, tiles);
+   // a tile's channels one after the other on one XCD, whose L2 puts their interleaved stores together
+   // (each channel's map in a plane of its own and a kernel to join them: colour CrossCorr_Norm
+   // 1280x960/24x24 50 us instead of 38.5, SqrDistance 4096^2/32x32 338 instead of 225)
+   const int tc = xcd_tile(blockIdx.x, tiles * a.nch), t = tc / a.nch, ch = tc - t * a.nch;
    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
    const int x0 = (t % tiles_x) * C, Y0 = (t / tiles_x) * kPairRows;
    const int S = i8_steps(a.th), nrows = kTileRows - 2 + 2 * S, plane = nrows * ldsp;
    const unsigned char *src = a.src + ch * a.plane8;
-   char *dst = reinterpret_cast<char *>(a.dst) + ch * a.planef;
+   char *dst = reinterpret_cast<char *>(a.dst + ch);
    const gfrag_i8 fr = (gfrag_i8)(a.frag + (size_t)ch * S * KC * NPB * 64 + lane);
    const double tt = a.sums[2 * ch], t1 = a.sums[2 * ch + 1];
 
@@ -428,7 +431,7 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
          const V sst = (V)ss[i] + (K ? 2 * K * (V)s1[i] + K * n1 * K : (V)0);
          v = (float)((double)d * rsqrt64((double)sst * ttrue));
       }
-      reinterpret_cast<float *>(dst + (size_t)y * a.dstep)[x] = v;
+      reinterpret_cast<float *>(dst + (size_t)y * a.dstep)[x * a.nch] = v;
    }
 }
 
@@ -440,6 +443,7 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
    a.src = static_cast<const unsigned char *>(S.ptr);
    a.W = S.width; a.H = S.height; a.sstep = S.step;
    a.tw = T.width; a.th = T.height;
+   a.nch = T.channels;
    const int KC = i8_chunks(a.tw), steps = i8_steps(a.th), nch = T.channels;
    {
       KernelTimer kt(s, "template_prep");
@@ -478,11 +482,9 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
 
 // ------------------------------------------------------------------------- planes
 // Interleaved 8-bit channels into planes of their own (row pitch plane8_step, plane pitch H rows),
-// zeros between the width and the pitch, and the planes of the map back into interleaved
-// channels: the kernels between them take every channel of an image in one launch, as
-// 1-channel images with wide loads and stores (with the channels' maps interleaved by those
-// kernels themselves, 4 bytes of every 16 a store, the row-pair kernel ran 60 instead of 40 us
-// at 1280x960/24x24).  Four pixels per thread.  Bound by HBM: 2 W H NCH and 8 W H NCH bytes.
+// zeros between the width and the pitch: the kernels after it take every channel of an image in one
+// launch, as 1-channel images with wide loads.  Four pixels per thread.  Bound by HBM: 2 W H NCH
+// bytes.
 int plane8_step(int W) { return (W + 15) / 16 * 16; }
 
 template <int NCH>
@@ -518,33 +520,6 @@ __global__ __launch_bounds__(256) void split_planes8(const unsigned char *__rest
    }
 }
 
-template <int NCH>
-__global__ __launch_bounds__(256) void join_planes(const float *__restrict__ src, int W, int H,
-                                                   int sstep, float *__restrict__ dst, int dstep)
-{
-   const int k = blockIdx.x * 256 + threadIdx.x, groups = sstep / 16;
-   const int y = k / groups, x = 4 * (k - y * groups);
-   if (y >= H) return;
-   float v[4 * NCH];
-#pragma unroll
-   for (int c = 0; c < NCH; ++c) {
-      const float4 q = *reinterpret_cast<const float4 *>(
-          reinterpret_cast<const char *>(src) + ((size_t)c * H + y) * sstep + 4 * x);
-      v[c] = q.x; v[NCH + c] = q.y; v[2 * NCH + c] = q.z; v[3 * NCH + c] = q.w;
-   }
-   float *d = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + (size_t)y * dstep) + x * NCH;
-   if (x + 4 <= W) {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i)
-         reinterpret_cast<f32x4_u *>(d)[i] = f32x4_u{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-   } else {
-#pragma unroll
-      for (int i = 0; i < 4 * NCH; ++i)
-         if (x + i / NCH < W) d[i] = v[i];
-   }
-}
-
-// one thread per 4 columns of a plane
 static unsigned plane_blocks(int H, int step) { return (unsigned)(((long long)H * (step / 4) + 255) / 256); }
 
 }  // namespace
@@ -595,8 +570,7 @@ size_t i8_work_bytes(const View &T)
 
 size_t int_mfma_work_bytes(const View &S, const View &T)
 {
-   // several channels: a plane of bytes and a plane of the map each
-   return i8_work_bytes(T) + 5 * planes8_bytes(S);
+   return i8_work_bytes(T) + planes8_bytes(S);
 }
 
 static I8Args work_args(int op, void *work)
@@ -612,30 +586,14 @@ void launch_int_mfma(hipStream_t s, int op, const View &image, const View &T, fl
                      void *work)
 {
    const int nch = image.channels;
-   // S, map: the image and its map, or (several channels) their first planes, the others plane8
-   // and planef bytes apart
+   // S: the image or (several channels) its first plane, the others plane8 bytes apart
    View S = image;
    I8Args a = work_args(op, work);
    a.dst = dst;
    a.dstep = dstep;
-   if (nch > 1) {
-      char *planes = static_cast<char *>(work) + i8_work_bytes(T);
-      S = launch_planes8(s, image, planes, &a.plane8);
-      a.dst = reinterpret_cast<float *>(planes + nch * a.plane8);
-      a.dstep = 4 * S.step;
-      a.planef = (size_t)S.height * a.dstep;
-   }
+   if (nch > 1) S = launch_planes8(s, image, static_cast<char *>(work) + i8_work_bytes(T), &a.plane8);
    if (T.type == SImage::S8) launch_i8<SImage::S8>(s, a, S, T);
    else launch_i8<SImage::U8>(s, a, S, T);
-   if (nch > 1) {
-      KernelTimer kt(s, "join_planes");
-      auto go = [&](auto kernel) {
-         kernel<<<plane_blocks(S.height, S.step), 256, 0, s>>>(a.dst, S.width, S.height, a.dstep, dst,
-                                                               dstep);
-      };
-      if (nch == 2) go(join_planes<2>); else go(join_planes<4>);
-      launch_check("join_planes");
-   }
 }
 
 // Every size up to the widest template of four chunks: against the tile kernel, CrossCorr 160x120/2x2
