@@ -640,6 +640,24 @@ __device__ __forceinline__ void pair_mfma(f32x16 (&acc)[NT], const unsigned shor
    }
 }
 
+// kF16x3: whether the source pixels under the windows of the C columns from x0 and kPairRows rows
+// from Y0 hold, among the calling thread's share, a non-zero value below 1 once scaled: lo is an
+// FP16 subnormal or 0 there, and the value held to fewer bits than one above.  Read again from
+// the source (by the few tiles with a dark window) rather than noted by every staging.
+__device__ __forceinline__ int split_loses(const TileArgs &a, int x0, int Y0, int C)
+{
+   const int r0 = max(Y0 - a.th / 2, 0), r1 = min(Y0 + kPairRows - 1 - a.th / 2 + a.th, a.H);
+   const int c0 = max(x0 - a.tw / 2, 0), c1 = min(x0 + C - 1 - a.tw / 2 + a.tw, a.W);
+   int loses = 0;
+   for (int r = r0 + (int)(threadIdx.x >> 6); r < r1; r += 4) {
+      const float *row = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.src) +
+                                                         (size_t)r * a.sstep);
+      for (int c = c0 + (int)(threadIdx.x & 63); c < c1; c += 64)
+         loses |= row[c] != 0.f && __builtin_fabsf(row[c]) * a.scale < 1.f;
+   }
+   return loses;
+}
+
 // Output tile (bx, by): 127 rows x 16 NT columns; a.vb = steps (template row pairs) per LDS
 // band.  Starts with a barrier, so consecutive calls may reuse the LDS.  kModeCC stores the
 // CrossCorr map; kModeNCC / kModeSSDN store CrossCorr_Norm / SqrDistance_Norm with the window
@@ -792,7 +810,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    if constexpr (NORM) {
       const double tt = tmpl_sqsum(a);
       // kF16x3: the sums' scale undone, the division in FP64 (as prox_tile_f32 has it), and
-      // outputs whose window is too dark for the split (split_range)
+      // outputs whose window may be too dark for the split (split_range)
       SplitRange sr;
       if constexpr (P == kF16x3) sr = split_range(a.peaks, a.tw * a.th);
       int dark = 0;
@@ -811,7 +829,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
                const double ss = (q[u][3][e] - q[u][2][e]) - (q[u][1][e] - q[u][0][e]);
                if constexpr (P == kF16x3) {
                   v[e] = (float)((double)cc[e] * sr.unscale * rsqrt64(ss * tt));
-                  dark |= cc[e] != 0.f && ss < sr.least_ss && x + e < a.W;
+                  dark |= !(ss >= sr.least_ss) && x + e < a.W;
                } else {
                   const double num = MODE == kModeNCC ? (double)cc[e] : ss - 2.0 * (double)cc[e] + tt;
                   v[e] = (float)num * inv_sqrt(ss * tt);
@@ -839,7 +857,9 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
          }
       }
       if constexpr (P == kF16x3) {
-         dark = __syncthreads_or(dark);
+         // dark windows: all zero, or data that the split does not hold (a sum of 0 says nothing:
+         // it may be values that both planes round to 0)
+         if (__syncthreads_or(dark)) dark = __syncthreads_or(split_loses(a, x0, Y0, C));
          if (threadIdx.x == 0) {
             *a.flags = (unsigned)dark;
             if (dark) *a.any = 1u;
