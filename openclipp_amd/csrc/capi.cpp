@@ -197,11 +197,12 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
       launch_template_prep(c.stream, view(T), 0, tpitch, 0, c.tmpl.data.ptr,
                            c.tmpl.sums.as<double>(), peaks + 1);
       const double *integ = sqr_integral_for(c, S, 0, peaks);
+      const bool tile_sums = prox_norm_from_tile(op, view(S), view(T));
       const SplitFlags f = launch_split_ncc(c.stream, view(S), view(T), c.tmpl.sums.as<double>(),
-                                            integ, peaks, static_cast<float *>(D.dev), D.desc.Step,
-                                            c.stats.as<char>() + head);
+                                            integ, tile_sums, peaks, static_cast<float *>(D.dev),
+                                            D.desc.Step, c.stats.as<char>() + head);
       launch_proximity_flagged(c.stream, view(S), view(T), D.dev, D.desc.Step, c.tmpl.data.ptr,
-                               tpitch, c.tmpl.sums.as<double>(), integ, f);
+                               tpitch, c.tmpl.sums.as<double>(), tile_sums ? nullptr : integ, f);
       D.in_device = true;
       return;
    }

@@ -900,6 +900,12 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
 
 // ======================================================================= split FP16
 constexpr int kSplitNT = 4;
+// Windows whose sum of squares is a smaller part of the integral's value than this are left to the
+// window sums of prox_tile_f32's tiles, where that kernel has them.  The four corners together are
+// off by up to 12 2^-53 of the last one (1.5 rms; 1920x1080 to 4096^2, with and without one large
+// pixel ahead of the others), so by up to 1.8e-7 (2e-8) of a window sum on the line, the map by half
+// of that.
+constexpr double kSplitIll = 0x1p-27;
 
 // Where the path is taken: prox_tile_f32 costs about 2 us + Mpx (11 us + 0.04 us taps) where it
 // forms the window sums in its tiles, and this path 46 us (seven launches, the integral's
@@ -932,8 +938,8 @@ size_t split_ncc_work_bytes(const View &S, const View &T)
 }
 
 SplitFlags launch_split_ncc(hipStream_t s, const View &S, const View &T, const double *tsums,
-                            const double *integ, const unsigned *peaks, float *dst, int dstep,
-                            void *work)
+                            const double *integ, bool tile_sums, const unsigned *peaks, float *dst,
+                            int dstep, void *work)
 {
    const int tw = T.width, th = T.height, KC2 = kc2_for(tw), NT = kSplitNT;
    u16x8 *g0 = static_cast<u16x8 *>(work);
@@ -952,6 +958,7 @@ SplitFlags launch_split_ncc(hipStream_t s, const View &S, const View &T, const d
    L.a.peaks = peaks;
    L.a.any = any;
    L.a.flags = any + 1;
+   if (tile_sums) L.a.ill = kSplitIll;
    L.KC = KC2;
    L.NT = NT;
    L.mode = mfma::kModeNCC;

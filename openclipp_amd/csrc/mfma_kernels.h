@@ -70,6 +70,9 @@ struct TileArgs {
    const unsigned *peaks = nullptr;
    unsigned *any = nullptr, *flags = nullptr;
    float scale = 1.f;
+   // kF16x3 where prox_tile_f32 forms the window sums in its tiles (-1 elsewhere): the least part
+   // of the integral up to a window's last corner that the window's own sum of squares may be
+   double ill = -1.0;
 };
 
 // Several sources of one size and template with crosscorr_mfma in one launch: the source, its
@@ -640,22 +643,42 @@ __device__ __forceinline__ void pair_mfma(f32x16 (&acc)[NT], const unsigned shor
    }
 }
 
-// kF16x3: whether the source pixels under the windows of the C columns from x0 and kPairRows rows
-// from Y0 hold, among the calling thread's share, a non-zero value below 1 once scaled: lo is an
-// FP16 subnormal or 0 there, and the value held to fewer bits than one above.  Read again from
-// the source (by the few tiles with a dark window) rather than noted by every staging.
-__device__ __forceinline__ int split_loses(const TileArgs &a, int x0, int Y0, int C)
+// kF16x3: what the source pixels under the windows of the outputs in `box` (first column and row, last
+// column and row) hold, the calling thread's share of them: data, a value other than 0; loses, a
+// non-zero value below 1 once scaled, where lo is an FP16 subnormal or 0 and the value held to
+// fewer bits than one above.  Read again from the source by the few tiles that ask.
+__device__ __forceinline__ void split_source(const TileArgs &a, int4 box, int &data, int &loses)
 {
-   const int r0 = max(Y0 - a.th / 2, 0), r1 = min(Y0 + kPairRows - 1 - a.th / 2 + a.th, a.H);
-   const int c0 = max(x0 - a.tw / 2, 0), c1 = min(x0 + C - 1 - a.tw / 2 + a.tw, a.W);
-   int loses = 0;
-   for (int r = r0 + (int)(threadIdx.x >> 6); r < r1; r += 4) {
-      const float *row = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.src) +
-                                                         (size_t)r * a.sstep);
-      for (int c = c0 + (int)(threadIdx.x & 63); c < c1; c += 64)
-         loses |= row[c] != 0.f && __builtin_fabsf(row[c]) * a.scale < 1.f;
+   const int r0 = max(box.y - a.th / 2, 0), r1 = min(box.w - a.th / 2 + a.th, a.H);
+   const int c0 = max(box.x - a.tw / 2, 0), c1 = min(box.z - a.tw / 2 + a.tw, a.W);
+   // four columns an item (the last ones of a row again where they do not fill it), eight items in
+   // flight
+   constexpr int K = 8;
+   const int groups = (c1 - c0 + 3) / 4, total = (r1 - r0) * groups;
+   for (int it0 = threadIdx.x; it0 < total; it0 += 256 * K) {
+      float f[K][4];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+         const int it = min(it0 + 256 * k, total - 1), r = it / groups, c = c0 + 4 * (it - r * groups);
+         const float *row = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.src) +
+                                                            (size_t)(r0 + r) * a.sstep);
+         if (c1 - c0 >= 4) {
+            const f32x4_u q = *reinterpret_cast<const f32x4_u *>(row + min(c, c1 - 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[k][e] = q[e];
+         } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[k][e] = row[min(c + e, c1 - 1)];
+         }
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+         for (int e = 0; e < 4; ++e) {
+            data |= f[k][e] != 0.f;
+            loses |= f[k][e] != 0.f && __builtin_fabsf(f[k][e]) * a.scale < 1.f;
+         }
    }
-   return loses;
 }
 
 // Output tile (bx, by): 127 rows x 16 NT columns; a.vb = steps (template row pairs) per LDS
@@ -813,7 +836,8 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
       // outputs whose window may be too dark for the split (split_range)
       SplitRange sr;
       if constexpr (P == kF16x3) sr = split_range(a.peaks, a.tw * a.th);
-      int dark = 0;
+      int dark = 0, ill = 0;
+      int4 box = make_int4(a.W, a.H, -1, -1);   // first and last columns and rows of such outputs
       auto finish = [&](int i0, const Corners &q) {
 #pragma unroll
          for (int u = 0; u < kEpiGroups; ++u) {
@@ -829,7 +853,15 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
                const double ss = (q[u][3][e] - q[u][2][e]) - (q[u][1][e] - q[u][0][e]);
                if constexpr (P == kF16x3) {
                   v[e] = (float)((double)cc[e] * sr.unscale * rsqrt64(ss * tt));
-                  dark |= !(ss >= sr.least_ss) && x + e < a.W;
+                  const bool d = !(ss >= sr.least_ss), b = !(ss >= a.ill * q[u][3][e]);
+                  if ((d || b) && x + e < a.W) {
+                     dark |= d;
+                     ill |= b;
+                     box.x = min(box.x, x + e);
+                     box.y = min(box.y, y);
+                     box.z = max(box.z, x + e);
+                     box.w = max(box.w, y);
+                  }
                } else {
                   const double num = MODE == kModeNCC ? (double)cc[e] : ss - 2.0 * (double)cc[e] + tt;
                   v[e] = (float)num * inv_sqrt(ss * tt);
@@ -858,11 +890,39 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
       }
       if constexpr (P == kF16x3) {
          // dark windows: all zero, or data that the split does not hold (a sum of 0 says nothing:
-         // it may be values that both planes round to 0)
-         if (__syncthreads_or(dark)) dark = __syncthreads_or(split_loses(a, x0, Y0, C));
+         // it may be values that both planes round to 0); windows that the integral does not hold
+         int flag = 0;
+         if (__syncthreads_or(dark | ill)) {
+            int *const b = reinterpret_cast<int *>(lds);   // the workgroup's box
+            if (threadIdx.x == 0) {
+               b[0] = a.W;
+               b[1] = a.H;
+               b[2] = b[3] = -1;
+            }
+            __syncthreads();
+            if (dark | ill) {
+               atomicMin(&b[0], box.x);
+               atomicMin(&b[1], box.y);
+               atomicMax(&b[2], box.z);
+               atomicMax(&b[3], box.w);
+            }
+            __syncthreads();
+            box = make_int4(b[0], b[1], b[2], b[3]);
+            int data = 0, loses = 0;
+            split_source(a, box, data, loses);
+            dark = __syncthreads_or(dark);
+            ill = __syncthreads_or(ill);
+            data = __syncthreads_or(data);
+            flag = __syncthreads_or(loses) && dark;
+            flag |= data && ill;
+            // no data: sums of squares of 0 where the integral leaves its rounding
+            if (ill && !data)
+               for (int y = box.y + wave; y <= box.w; y += 4)
+                  for (int x = box.x + lane; x <= box.z; x += 64) out_row(a, y)[x] = __builtin_nanf("");
+         }
          if (threadIdx.x == 0) {
-            *a.flags = (unsigned)dark;
-            if (dark) *a.any = 1u;
+            *a.flags = (unsigned)flag;
+            if (flag) *a.any = 1u;
          }
       }
       return;

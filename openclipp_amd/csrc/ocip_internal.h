@@ -195,9 +195,10 @@ bool prox_norm_from_tile(int op, const View &src, const View &tpl);
 // CrossCorr_Norm of F32 1-channel images on split-FP16 MFMA (as accurate as the FP32 sums of
 // launch_proximity, mfma_kernels.h): split_ncc_ok tells whether the path takes the call.  peaks
 // (launch_integral's of the source, launch_template_prep's of the template, in this order)
-// and integ come first; the tiles that the split cannot hold are then computed by
-// launch_proximity_flagged, from the flags (one per tile_w x tile_h outputs, tiles_x a row)
-// that launch_split_ncc left in `work`.
+// and integ come first; the tiles that the split cannot hold, or (tile_sums: prox_norm_from_tile
+// holds for the call) whose sums of squares the integral cannot, are then computed by
+// launch_proximity_flagged (tile_sums: integ null), from the flags (one per tile_w x tile_h
+// outputs, tiles_x a row) that launch_split_ncc left in `work`.
 struct SplitFlags {
    const unsigned *any, *flags;   // any: 0 where no tile is flagged
    int tiles_x, tile_w, tile_h;
@@ -205,8 +206,8 @@ struct SplitFlags {
 bool split_ncc_ok(int op, const View &src, const View &T);
 size_t split_ncc_work_bytes(const View &src, const View &T);
 SplitFlags launch_split_ncc(hipStream_t s, const View &src, const View &T, const double *tsums,
-                            const double *integ, const unsigned *peaks, float *dst, int dst_step,
-                            void *work);
+                            const double *integ, bool tile_sums, const unsigned *peaks, float *dst,
+                            int dst_step, void *work);
 void launch_proximity_flagged(hipStream_t s, const View &src, const View &T, void *dst,
                               int dst_step, const void *tstage, int tpitch, const double *tsums,
                               const double *integ, const SplitFlags &f);

@@ -1020,15 +1020,22 @@ void launch_proximity_flagged(hipStream_t s, const View &S, const View &T, void 
                               const void *tstage, int tpitch, const double *tsums,
                               const double *integ, const SplitFlags &f)
 {
-   constexpr int R = 16;
    const int W = S.width, H = S.height, tw = T.width, th = T.height;
+   // window sums in the tiles: 8 outputs per thread and one band, as launch_proximity has them
+   const int R = integ ? 16 : 8;
    const int ldsw = lds_pitch(kWaves * R + tw - 1);
    const int vb = min(th, kLdsBudget / (ldsw * 4) - (kTileRows - 1));   // >= 1: split_ncc_ok
+   const size_t lds = integ ? (size_t)(kTileRows + vb - 1) * ldsw * 4
+                            : tile_sqsum_offset(kTileRows + vb - 1, ldsw) + tile_sqsum_lds(R, th);
+   if (!integ && !prox_norm_from_tile(kCCNorm, S, T)) fail(CL_INVALID_VALUE, "integral required");
    const int tiles = ((W + kWaves * R - 1) / (kWaves * R)) * ((H + kTileRows - 1) / kTileRows);
    KernelTimer kt(s, "prox_flagged");
-   prox_tile_f32_flagged<R><<<min(tiles, 512), 256, (size_t)(kTileRows + vb - 1) * ldsw * 4, s>>>(
-       static_cast<const char *>(S.ptr), W, H, S.step, static_cast<const float *>(tstage), tpitch,
-       tw, th, tsums, integ, static_cast<char *>(dst), dstep, vb, ldsw, f);
+   auto go = [&](auto kernel) {
+      kernel<<<min(tiles, 512), 256, lds, s>>>(
+          static_cast<const char *>(S.ptr), W, H, S.step, static_cast<const float *>(tstage), tpitch,
+          tw, th, tsums, integ, static_cast<char *>(dst), dstep, vb, ldsw, f);
+   };
+   if (R == 16) go(prox_tile_f32_flagged<16>); else go(prox_tile_f32_flagged<8>);
    launch_check("prox_flagged");
 }
 
