@@ -907,13 +907,16 @@ constexpr int kSplitNT = 4;
 // of that.
 constexpr double kSplitIll = 0x1p-27;
 
-// Where the path is taken: prox_tile_f32 costs about 2 us + Mpx (11 us + 0.04 us taps) where it
-// forms the window sums in its tiles, and this path 46 us (seven launches, the integral's
-// three among them) + Mpx (5 us + 0.006 us taps), equal near Mpx (taps + 142) = 1420, where it is
-// taken from (1900^2/16x16 78 against 66 us, 1000x3000/24x24 96 against 79; 1400^2/24x24 66
-// against 73, 1000x3000/16x16 61 against 67).  Where prox_tile_f32 needs the integral too, it pays
-// its launches as well: taken from 200 taps or 2 Mpx on (160x120/31x31 78 against 57 us,
-// 2048x512/16x16 54 against 50, 2048x1024/5x5 56 against 55; 2048x512/5x5 40 against 47).
+// Where the path is taken.  For accuracy, templates of 64 taps and 8 columns on: below, prox_tile_f32's
+// few additions are the more exact ones (root mean square error against FP64, noise around 0.5: 3x3
+// 4.8e-8 against 4.5e-8 here, constant images up to 3e-9 against 2e-7; 8x8 1.0e-7 against 5.0e-8,
+// 64x64 7.4e-7 against 1.4e-7; 200 rows of 2, constant 0.1: 7e-7 against 1e-6).  For time, where
+// prox_tile_f32 forms the window sums in its tiles it costs about 2 us + Mpx (9 us + 0.04 us taps) and
+// this path 50 us (seven launches, the integral's three among them) + Mpx (5 us + 0.008 us taps):
+// taken from Mpx (taps + 100) = 1500 (1500^2/24x24 81 against 79 us, 2048^2/20x20 106 against 96,
+// 4000x2000/11x11 125 against 112; 1920x1080/24x24 63 against 74, 2048^2/16x16 81 against 86, 3000^2/8x8
+// 106 against 113).  Where prox_tile_f32 needs the integral too, it pays its launches as well: taken
+// from 200 taps or 2 Mpx on (160x120/31x31 78 against 61 us, 64 rows of 8 66 against 65).
 // OCIP_SPLIT_NCC=0 turns the path off (prox_tile_f32 then computes the maps), 1 has it take
 // every call that it can.
 bool split_ncc_ok(int op, const View &S, const View &T)
@@ -927,7 +930,8 @@ bool split_ncc_ok(int op, const View &S, const View &T)
    if (pair_geometry(kc2_for(tw), kSplitNT, th, mfma::kLdsMax, 2).vb < 1) return false;
    if (e && e[0] == '1') return true;
    const long long px = (long long)S.width * S.height, taps = (long long)tw * th;
-   return prox_norm_from_tile(op, S, T) ? px * (taps + 142) >= 1420000000LL
+   if (taps < 64 || tw < 8) return false;
+   return prox_norm_from_tile(op, S, T) ? px * (taps + 100) >= 1500000000LL
                                         : taps >= 200 || px >= 1 << 21;
 }
 

@@ -42,11 +42,12 @@ constexpr int kBlockW = 64;             // template column block for wide templa
 constexpr int kLdsMax = 160 * 1024 - 256;
 
 // kF16x3 (ocipCrossCorr_Norm of F32 images): split FP16, s = s_hi + s_lo of s scaled by a power of
-// two so that the image's largest magnitude lies in (2^14, 2^15], the template likewise.  hi
-// takes 11 significant bits and lo the next 11 to 13 (down to 2^-24, FP16 subnormals, which the
-// matrix cores keep), so a value within 2^15 of the largest is held to 2^-24 of itself, the rounding
-// unit of FP32, and every value to 2^-40 of the largest; the three products hi hi, hi lo, lo hi
-// leave out lo lo, at most 2^-24 of the product.
+// two so that the image's largest magnitude lies in (2^14, 2^15], the template likewise.  hi takes 11
+// significant bits and lo the next 11 and a sign (down to 2^-24, FP16 subnormals, which the matrix
+// cores keep): a value within 2^15 of the largest is held to 2^-23 of itself, three in four of them
+// exactly, and every value to 2^-40 of the largest.  All four products are taken, hi hi in one
+// accumulator and the others, 2^11 times smaller, in a second: added to the first they would lose
+// what lies below its grid (lo lo all of it).
 enum { kBF16 = 1, kF16 = 2, kBF16x3 = 3, kF16x3 = 4 };
 __host__ __device__ constexpr int planes_of(int P) { return P == kBF16x3 || P == kF16x3 ? 2 : 1; }
 // kModeCC: the CrossCorr map (the single-template call; CrossCorr_Norm scales it in place
@@ -643,6 +644,34 @@ __device__ __forceinline__ void pair_mfma(f32x16 (&acc)[NT], const unsigned shor
    }
 }
 
+// The same for split FP16: hi hi into acc, the products with a lo, lo lo among them, into low; chunk by
+// chunk of A, whose fragments then take 8 registers instead of 8 NA (two accumulators and the
+// prefetched B fragments fill the 256 of two waves per SIMD).  Without lo lo and in one accumulator
+// 4096^2/64x64 took 537 us instead of 649, at twice to three times the error on ordinary data and
+// 2^-22 on constant images of 1 + 2^-11, where the FP32 sums are off by 2^-23 to 2^-22.
+template <int KC, int NT>
+__device__ __forceinline__ void pair_mfma_f16x3(f32x16 (&acc)[NT], f32x16 (&low)[NT],
+                                                const unsigned short *ab, size_t plane,
+                                                const u16x8 (&b)[KC], const u16x8 (&b1)[KC])
+{
+#pragma unroll
+   for (int c = 0; c < NT + KC - 1; ++c) {
+      const u16x8 a0 = *reinterpret_cast<const u16x8 *>(ab + 16 * c);
+      const u16x8 a1 = *reinterpret_cast<const u16x8 *>(ab + plane + 16 * c);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+         for (int j = 0; j < NT; ++j) {
+            const int kc = c - j;
+            if (kc < 0 || kc >= KC) continue;
+            if (k == 0) acc[j] = mma<kF16x3>(a0, b[kc], acc[j]);
+            else if (k == 1) low[j] = mma<kF16x3>(a0, b1[kc], low[j]);
+            else if (k == 2) low[j] = mma<kF16x3>(a1, b[kc], low[j]);
+            else low[j] = mma<kF16x3>(a1, b1[kc], low[j]);
+         }
+   }
+}
+
 // kF16x3: what the source pixels under the windows of the outputs in `box` (first column and row, last
 // column and row) hold, the calling thread's share of them: data, a value other than 0; loses, a
 // non-zero value below 1 once scaled, where lo is an FP16 subnormal or 0 and the value held to
@@ -702,11 +731,18 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    const int cx = a.tw / 2, cy = a.th / 2;
    const int S = (a.th + 1) / 2;
 
-   f32x16 acc[NT];
+   f32x16 acc[NT], low[P == kF16x3 ? NT : 1];
 #pragma unroll
    for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[j][i] = 0.f;
+      for (int i = 0; i < 16; ++i) {
+         acc[j][i] = 0.f;
+         if constexpr (P == kF16x3) low[j][i] = 0.f;
+      }
+   auto step = [&](const unsigned short *ab, const u16x8 (&b)[KC], const u16x8 (&b1)[KC]) {
+      if constexpr (P == kF16x3) pair_mfma_f16x3<KC, NT>(acc, low, ab, plane, b, b1);
+      else pair_mfma<P, KC, NT>(acc, ab, plane, b, b1);
+   };
    for (int ub = 0; ub < a.nub; ++ub) {
       for (int s0 = 0; s0 < S; s0 += a.vb) {
          const int ns = min(a.vb, S - s0);
@@ -728,16 +764,23 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
          for (; q + 1 < ns; q += 2) {
             load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)(q + 1) * KC * 64, pb, pb1);
             __builtin_amdgcn_sched_barrier(0);
-            pair_mfma<P, KC, NT>(acc, arow + (size_t)(2 * q) * ldsp, plane, pa, pa1);
+            step(arow + (size_t)(2 * q) * ldsp, pa, pa1);
             const int qn = q + 2 < ns ? q + 2 : q + 1;
             load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)qn * KC * 64, pa, pa1);
             __builtin_amdgcn_sched_barrier(0);
-            pair_mfma<P, KC, NT>(acc, arow + (size_t)(2 * q + 2) * ldsp, plane, pb, pb1);
+            step(arow + (size_t)(2 * q + 2) * ldsp, pb, pb1);
          }
          if (q < ns) {
-            pair_mfma<P, KC, NT>(acc, arow + (size_t)(2 * q) * ldsp, plane, pa, pa1);
+            step(arow + (size_t)(2 * q) * ldsp, pa, pa1);
          }
       }
+   }
+
+   if constexpr (P == kF16x3) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int i = 0; i < 16; ++i) acc[j][i] += low[j][i];
    }
 
    // Norm modes: groups of four consecutive outputs of one row per thread (kNormIters of them,
