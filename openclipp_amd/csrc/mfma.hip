@@ -899,7 +899,7 @@ void launch_crosscorr_split(hipStream_t s, int n, const float *const *src, const
 }
 
 // ======================================================================= split FP16
-constexpr int kSplitNT = 4;
+using mfma::kSplitNT;
 // Windows whose sum of squares is a smaller part of the integral's value than this are left to the
 // window sums of prox_tile_f32's tiles, where that kernel has them.  The four corners together are
 // off by up to 12 2^-53 of the last one (1.5 rms; 1920x1080 to 4096^2, with and without one large
@@ -907,7 +907,7 @@ constexpr int kSplitNT = 4;
 // of that.
 constexpr double kSplitIll = 0x1p-27;
 
-// Where the path is taken.  For accuracy, templates of 64 taps and 8 columns on: below, prox_tile_f32's
+// Where the path is taken.  For accuracy, templates of 100 taps and 8 columns on: below, prox_tile_f32's
 // few additions are the more exact ones (root mean square error against FP64, noise around 0.5: 3x3
 // 4.8e-8 against 4.5e-8 here, constant images up to 3e-9 against 2e-7; 8x8 1.0e-7 against 5.0e-8,
 // 64x64 7.4e-7 against 1.4e-7; 200 rows of 2, constant 0.1: 7e-7 against 1e-6).  For time, where
@@ -915,7 +915,8 @@ constexpr double kSplitIll = 0x1p-27;
 // this path 50 us (seven launches, the integral's three among them) + Mpx (5 us + 0.008 us taps):
 // taken from Mpx (taps + 100) = 1500 (1500^2/24x24 81 against 79 us, 2048^2/20x20 106 against 96,
 // 4000x2000/11x11 125 against 112; 1920x1080/24x24 63 against 74, 2048^2/16x16 81 against 86, 3000^2/8x8
-// 106 against 113).  Where prox_tile_f32 needs the integral too, it pays its launches as well: taken
+// 106 against 113; 8x8 4096^2 180 against 174, not worth twice the time where a far brighter pixel
+// sends every tile back).  Where prox_tile_f32 needs the integral too, it pays its launches as well: taken
 // from 200 taps or 2 Mpx on (160x120/31x31 78 against 61 us, 64 rows of 8 66 against 65).
 // OCIP_SPLIT_NCC=0 turns the path off (prox_tile_f32 then computes the maps), 1 has it take
 // every call that it can.
@@ -930,7 +931,7 @@ bool split_ncc_ok(int op, const View &S, const View &T)
    if (pair_geometry(kc2_for(tw), kSplitNT, th, mfma::kLdsMax, 2).vb < 1) return false;
    if (e && e[0] == '1') return true;
    const long long px = (long long)S.width * S.height, taps = (long long)tw * th;
-   if (taps < 64 || tw < 8) return false;
+   if (taps < 100 || tw < 8) return false;
    return prox_norm_from_tile(op, S, T) ? px * (taps + 100) >= 1500000000LL
                                         : taps >= 200 || px >= 1 << 21;
 }
@@ -950,11 +951,6 @@ SplitFlags launch_split_ncc(hipStream_t s, const View &S, const View &T, const d
    u16x8 *g1 = g0 + pair_frag_count(tw, th) * 64;
    unsigned *any = reinterpret_cast<unsigned *>(static_cast<char *>(work) +
                                                 pair_frag_bytes(mfma::kF16x3, tw, th));
-   {
-      KernelTimer kt(s, "template_prep");
-      mfma::launch_split_prep(s, BatchDesc{static_cast<const char *>(T.ptr), tw, th, T.step, KC2,
-                                           1, g0, g1, nullptr}, peaks, any);
-   }
    const Geometry g = pair_geometry(KC2, NT, th, mfma::kLdsMax, 2);
    SingleLaunch L;
    L.a = mfma::TileArgs{static_cast<const float *>(S.ptr), S.width, S.height, S.step, tw, th, 1,
@@ -970,6 +966,11 @@ SplitFlags launch_split_ncc(hipStream_t s, const View &S, const View &T, const d
    L.lds = g.lds;
    L.grid = dim3((S.width + 16 * NT - 1) / (16 * NT),
                  (S.height + mfma::kPairRows - 1) / mfma::kPairRows);
+   {
+      KernelTimer kt(s, "template_prep");
+      mfma::launch_split_prep(s, BatchDesc{static_cast<const char *>(T.ptr), tw, th, T.step, KC2,
+                                           1, g0, g1, nullptr}, L.a, (int)L.grid.x, (int)(L.grid.x * L.grid.y));
+   }
    KernelTimer kt(s, "crosscorr_mfma_split");
    mfma::launch_split_pair(s, L);
    return SplitFlags{any, any + 1, (int)L.grid.x, 16 * NT, mfma::kPairRows};

@@ -6,23 +6,40 @@ namespace mfma {
 
 namespace {
 
-// Fragments of a split-FP16 template, one per wavefront (the sum of squares and the peaks come
-// from template_prep), and *any cleared.
-__global__ __launch_bounds__(256) void split_prep(BatchDesc d, const unsigned *__restrict__ peaks,
-                                                   unsigned *any)
+// Fragments of a split-FP16 template, one per wavefront of the first fblocks workgroups (the sum of
+// squares and the peaks come from template_prep), and *any cleared; then one wavefront per tile:
+// whether one of 64 outputs of it, 8 columns and 16 rows apart, has a window that the split or the
+// integral may not hold (the line of pair_tile's doubt).
+__global__ __launch_bounds__(256) void split_prep(BatchDesc d, TileArgs a, int fblocks, int tiles_x, int tiles)
 {
-   if (blockIdx.x == 0 && threadIdx.x == 0) *any = 0u;
-   const SplitRange sr = split_range(peaks, d.tw * d.th);
-   const int nfrag = pair_frag_steps(d.th, 1) * d.KC;
-   const int f = blockIdx.x * 4 + (threadIdx.x >> 6);
-   if (f < nfrag && sr.ok)
-      build_pair_fragment<kF16x3>(d.tptr, d.tstep, d.tw, d.th, d.KC, 1, f, threadIdx.x & 63,
-                                  d.frag0, d.frag1, pow2f(sr.kt));
+   if (blockIdx.x == 0 && threadIdx.x == 0) *a.any = 0u;
+   const SplitRange sr = split_range(a.peaks, d.tw * d.th);
+   if (!sr.ok) return;
+   const int lane = threadIdx.x & 63;
+   if ((int)blockIdx.x < fblocks) {
+      const int f = blockIdx.x * 4 + (threadIdx.x >> 6);
+      if (f < pair_frag_steps(d.th, 1) * d.KC)
+         build_pair_fragment<kF16x3>(d.tptr, d.tstep, d.tw, d.th, d.KC, 1, f, lane, d.frag0, d.frag1,
+                                     pow2f(sr.kt));
+      return;
+   }
+   const int t = (blockIdx.x - fblocks) * 4 + (threadIdx.x >> 6);
+   if (t >= tiles) return;
+   const int x = t % tiles_x * (16 * kSplitNT) + 8 * (lane & 7), y = t / tiles_x * kPairRows + 16 * (lane >> 3);
+   bool doubt = false;
+   if (x < a.W && y < a.H) {
+      const double last = a.integ[(size_t)min(y - a.th / 2 + a.th, a.H) * excl_pitch(a.W) + kExclOffset +
+                                  min(x - a.tw / 2 + a.tw, a.W)];
+      const double ss = window_sqsum(a.integ, a.W, a.H, x, y, a.tw, a.th);
+      doubt = !(ss >= sr.least_ss) || !(ss >= a.ill * last);
+   }
+   doubt = __any(doubt);
+   if (lane == 0) a.flags[t] = (unsigned)doubt;
 }
 
 template <int KC> void pair(hipStream_t s, const SingleLaunch &L)
 {
-   auto k = crosscorr_mfma_pair<kF16x3, KC, 4, kModeNCC>;
+   auto k = crosscorr_mfma_pair<kF16x3, KC, kSplitNT, kModeNCC>;
    // set for every call: the attribute belongs to the device that is current
    hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax),
@@ -48,10 +65,10 @@ void launch_split_pair(hipStream_t s, const SingleLaunch &L)
    launch_check("crosscorr_mfma_split");
 }
 
-void launch_split_prep(hipStream_t s, const BatchDesc &d, const unsigned *peaks, unsigned *any)
+void launch_split_prep(hipStream_t s, const BatchDesc &d, const TileArgs &a, int tiles_x, int tiles)
 {
-   const int nfrag = pair_frag_steps(d.th, 1) * d.KC;
-   split_prep<<<(nfrag + 3) / 4, 256, 0, s>>>(d, peaks, any);
+   const int nfrag = pair_frag_steps(d.th, 1) * d.KC, fblocks = (nfrag + 3) / 4;
+   split_prep<<<fblocks + (tiles + 3) / 4, 256, 0, s>>>(d, a, fblocks, tiles_x, tiles);
    launch_check("split_prep");
 }
 

@@ -67,7 +67,8 @@ struct TileArgs {
    int vb;                       // template rows per LDS band
    int vec;                      // 16-byte ring loads allowed (crosscorr_mfma_strip)
    // kF16x3: the peaks of source and template (split_range), the source's scale, the word that any
-   // flagged tile sets, and the tile's flag (non-zero: prox_tile_f32_flagged computes it again)
+   // flagged tile sets, and the tile's flag (non-zero: outputs in doubt as split_prep leaves it,
+   // prox_tile_f32_flagged computes the tile again as the kernel does)
    const unsigned *peaks = nullptr;
    unsigned *any = nullptr, *flags = nullptr;
    float scale = 1.f;
@@ -731,58 +732,6 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    const int cx = a.tw / 2, cy = a.th / 2;
    const int S = (a.th + 1) / 2;
 
-   f32x16 acc[NT], low[P == kF16x3 ? NT : 1];
-#pragma unroll
-   for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-         acc[j][i] = 0.f;
-         if constexpr (P == kF16x3) low[j][i] = 0.f;
-      }
-   auto step = [&](const unsigned short *ab, const u16x8 (&b)[KC], const u16x8 (&b1)[KC]) {
-      if constexpr (P == kF16x3) pair_mfma_f16x3<KC, NT>(acc, low, ab, plane, b, b1);
-      else pair_mfma<P, KC, NT>(acc, ab, plane, b, b1);
-   };
-   for (int ub = 0; ub < a.nub; ++ub) {
-      for (int s0 = 0; s0 < S; s0 += a.vb) {
-         const int ns = min(a.vb, S - s0);
-         __syncthreads();
-         // LDS row r = source row Y0 - cy + 2 s0 + r; wave w reads rows 32 w + m + 2 (s - s0)
-         stage_rows<P, lcols>(a, lds, ldsp, plane, Y0 - cy + 2 * s0, x0 - cx + ub * kBlockW,
-                                   kTileRows - 2 + 2 * ns);
-         __syncthreads();
-
-         // a wave whose output rows (from Y0 - 1 + 32 wave on) all lie below the image skips
-         // its products: its half rows are never stored
-         if (Y0 - 1 + 32 * wave >= a.H) continue;
-         // ping-pong: the B fragments of step s+1 load while step s multiplies
-         const size_t fb0 = ((size_t)(ub * pair_frag_steps(a.th, a.nub) + s0) * KC) * 64 + lane;
-         u16x8 pa[KC], pb[KC], pa1[KC], pb1[KC];   // (pa1, pb1: the lo planes, split BF16)
-         load_frags<NPL, KC>(a.frag0, a.frag1, fb0, pa, pa1);
-         const unsigned short *arow = lds + (size_t)(wave * 32 + (lane & 31)) * ldsp + 8 * (lane >> 5);
-         int q = 0;
-         for (; q + 1 < ns; q += 2) {
-            load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)(q + 1) * KC * 64, pb, pb1);
-            __builtin_amdgcn_sched_barrier(0);
-            step(arow + (size_t)(2 * q) * ldsp, pa, pa1);
-            const int qn = q + 2 < ns ? q + 2 : q + 1;
-            load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)qn * KC * 64, pa, pa1);
-            __builtin_amdgcn_sched_barrier(0);
-            step(arow + (size_t)(2 * q + 2) * ldsp, pb, pb1);
-         }
-         if (q < ns) {
-            step(arow + (size_t)(2 * q) * ldsp, pa, pa1);
-         }
-      }
-   }
-
-   if constexpr (P == kF16x3) {
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-         for (int i = 0; i < 16; ++i) acc[j][i] += low[j][i];
-   }
-
    // Norm modes: groups of four consecutive outputs of one row per thread (kNormIters of them,
    // kEpiGroups per batch).  A group's window sums of s^2 are differences of the FP64
    // integral at rows ya, yb (shared by the four) and columns xa + e, xb + e, all clamped to
@@ -842,6 +791,127 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
       }
    };
    Corners qa, qb;
+   // kF16x3: the outputs that the split or the integral may not hold (split_range, TileArgs::ill), by the
+   // whole workgroup: whether the tile is to be computed again (flag), and the outputs whose window has no
+   // data while the integral's rounding keeps their sums of squares from 0 (in `box`: first
+   // column and row, last column and row; none where blank is 0).
+   SplitRange sr;
+   int flag = 0, blank = 0, data = 1;
+   int4 box = make_int4(0, 0, -1, -1);
+   auto settle = [&]() {
+      int dark = 0, ill = 0, loses = 0;
+      int4 own = make_int4(a.W, a.H, -1, -1);
+#pragma unroll 1
+      for (int i0 = 0; i0 < kNormIters; i0 += kEpiGroups) {
+         load_corners(i0, qa);
+#pragma unroll
+         for (int u = 0; u < kEpiGroups; ++u) {
+            const int k = threadIdx.x + 256 * (i0 + u), r = k / (C / 4);
+            const int x = x0 + 4 * (k - r * (C / 4)), y = Y0 + r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+               const double ss = (qa[u][3][e] - qa[u][2][e]) - (qa[u][1][e] - qa[u][0][e]);
+               const bool in = k < kNormGroups && y < a.H && x + e < a.W;
+               const bool d = in && !(ss >= sr.least_ss), b = in && !(ss >= a.ill * qa[u][3][e]);
+               dark |= d;
+               ill |= b;
+               if (d || b) own = make_int4(min(own.x, x + e), min(own.y, y), max(own.z, x + e), max(own.w, y));
+            }
+         }
+      }
+      int *const b = reinterpret_cast<int *>(lds);
+      __syncthreads();
+      if (threadIdx.x < 4) b[threadIdx.x] = threadIdx.x < 2 ? 0x7fffffff : -1;
+      __syncthreads();
+      if (dark | ill) {
+         atomicMin(&b[0], own.x);
+         atomicMin(&b[1], own.y);
+         atomicMax(&b[2], own.z);
+         atomicMax(&b[3], own.w);
+      }
+      __syncthreads();
+      box = make_int4(b[0], b[1], b[2], b[3]);
+      // dark windows: all zero, or data that the split does not hold (a sum of 0 says nothing: it may
+      // be values that both planes round to 0); windows that the integral does not hold: data, or none
+      data = 0;
+      split_source(a, box, data, loses);
+      dark = __syncthreads_or(dark);
+      ill = __syncthreads_or(ill);
+      data = __syncthreads_or(data);
+      flag = (__syncthreads_or(loses) && dark) || (data && ill);
+      blank = ill && !data;
+   };
+   // Settled ahead of the products where split_prep found one output in 128 in doubt: a tile to be
+   // computed again then costs no products, nor does one without data.  4096^2/64x64 with one pixel
+   // 2^18 times the others 3020 -> 2313 us (2066 with FP32 sums alone), with 43 percent zeros in margins
+   // 715 -> 585; images without either 655 -> 663.
+   bool settled = false, empty = false;
+   if constexpr (P == kF16x3) {
+      sr = split_range(a.peaks, a.tw * a.th);
+      settled = *a.flags != 0u;
+      if (settled) {
+         settle();
+         if (flag) {
+            if (threadIdx.x == 0) *a.flags = *a.any = 1u;
+            return;
+         }
+         empty = !data && box.x <= x0 && box.y <= Y0 && box.z >= min(x0 + C, a.W) - 1 &&
+                 box.w >= min(Y0 + kPairRows, a.H) - 1;
+      }
+   }
+
+   f32x16 acc[NT], low[P == kF16x3 ? NT : 1];
+#pragma unroll
+   for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+         acc[j][i] = 0.f;
+         if constexpr (P == kF16x3) low[j][i] = 0.f;
+      }
+   auto step = [&](const unsigned short *ab, const u16x8 (&b)[KC], const u16x8 (&b1)[KC]) {
+      if constexpr (P == kF16x3) pair_mfma_f16x3<KC, NT>(acc, low, ab, plane, b, b1);
+      else pair_mfma<P, KC, NT>(acc, ab, plane, b, b1);
+   };
+   for (int ub = 0; ub < (empty ? 0 : a.nub); ++ub) {
+      for (int s0 = 0; s0 < S; s0 += a.vb) {
+         const int ns = min(a.vb, S - s0);
+         __syncthreads();
+         // LDS row r = source row Y0 - cy + 2 s0 + r; wave w reads rows 32 w + m + 2 (s - s0)
+         stage_rows<P, lcols>(a, lds, ldsp, plane, Y0 - cy + 2 * s0, x0 - cx + ub * kBlockW,
+                                   kTileRows - 2 + 2 * ns);
+         __syncthreads();
+
+         // a wave whose output rows (from Y0 - 1 + 32 wave on) all lie below the image skips
+         // its products: its half rows are never stored
+         if (Y0 - 1 + 32 * wave >= a.H) continue;
+         // ping-pong: the B fragments of step s+1 load while step s multiplies
+         const size_t fb0 = ((size_t)(ub * pair_frag_steps(a.th, a.nub) + s0) * KC) * 64 + lane;
+         u16x8 pa[KC], pb[KC], pa1[KC], pb1[KC];   // (pa1, pb1: the lo planes, split BF16)
+         load_frags<NPL, KC>(a.frag0, a.frag1, fb0, pa, pa1);
+         const unsigned short *arow = lds + (size_t)(wave * 32 + (lane & 31)) * ldsp + 8 * (lane >> 5);
+         int q = 0;
+         for (; q + 1 < ns; q += 2) {
+            load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)(q + 1) * KC * 64, pb, pb1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(arow + (size_t)(2 * q) * ldsp, pa, pa1);
+            const int qn = q + 2 < ns ? q + 2 : q + 1;
+            load_frags<NPL, KC>(a.frag0, a.frag1, fb0 + (size_t)qn * KC * 64, pa, pa1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(arow + (size_t)(2 * q + 2) * ldsp, pb, pb1);
+         }
+         if (q < ns) {
+            step(arow + (size_t)(2 * q) * ldsp, pa, pa1);
+         }
+      }
+   }
+
+   if constexpr (P == kF16x3) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int i = 0; i < 16; ++i) acc[j][i] += low[j][i];
+   }
+
    if constexpr (NORM) load_corners(0, qa);
    // Pair the halves in LDS: tile row r = 32 w + m + dy holds output row Y0 - 1 + r.
    // C fragment: lane holds column n = lane % 32 of each n-tile, rows
@@ -875,12 +945,8 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    static_assert(TP % 4 == 0 && C % 4 == 0, "16-byte groups of the LDS tile");
    if constexpr (NORM) {
       const double tt = tmpl_sqsum(a);
-      // kF16x3: the sums' scale undone, the division in FP64 (as prox_tile_f32 has it), and
-      // outputs whose window may be too dark for the split (split_range)
-      SplitRange sr;
-      if constexpr (P == kF16x3) sr = split_range(a.peaks, a.tw * a.th);
-      int dark = 0, ill = 0;
-      int4 box = make_int4(a.W, a.H, -1, -1);   // first and last columns and rows of such outputs
+      // kF16x3: the sums' scale undone, the division in FP64 (as prox_tile_f32 has it)
+      int doubt = 0;
       auto finish = [&](int i0, const Corners &q) {
 #pragma unroll
          for (int u = 0; u < kEpiGroups; ++u) {
@@ -896,15 +962,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
                const double ss = (q[u][3][e] - q[u][2][e]) - (q[u][1][e] - q[u][0][e]);
                if constexpr (P == kF16x3) {
                   v[e] = (float)((double)cc[e] * sr.unscale * rsqrt64(ss * tt));
-                  const bool d = !(ss >= sr.least_ss), b = !(ss >= a.ill * q[u][3][e]);
-                  if ((d || b) && x + e < a.W) {
-                     dark |= d;
-                     ill |= b;
-                     box.x = min(box.x, x + e);
-                     box.y = min(box.y, y);
-                     box.z = max(box.z, x + e);
-                     box.w = max(box.w, y);
-                  }
+                  doubt |= (!(ss >= sr.least_ss) | !(ss >= a.ill * q[u][3][e])) & (x + e < a.W);
                } else {
                   const double num = MODE == kModeNCC ? (double)cc[e] : ss - 2.0 * (double)cc[e] + tt;
                   v[e] = (float)num * inv_sqrt(ss * tt);
@@ -932,41 +990,15 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
          }
       }
       if constexpr (P == kF16x3) {
-         // dark windows: all zero, or data that the split does not hold (a sum of 0 says nothing:
-         // it may be values that both planes round to 0); windows that the integral does not hold
-         int flag = 0;
-         if (__syncthreads_or(dark | ill)) {
-            int *const b = reinterpret_cast<int *>(lds);   // the workgroup's box
-            if (threadIdx.x == 0) {
-               b[0] = a.W;
-               b[1] = a.H;
-               b[2] = b[3] = -1;
-            }
-            __syncthreads();
-            if (dark | ill) {
-               atomicMin(&b[0], box.x);
-               atomicMin(&b[1], box.y);
-               atomicMax(&b[2], box.z);
-               atomicMax(&b[3], box.w);
-            }
-            __syncthreads();
-            box = make_int4(b[0], b[1], b[2], b[3]);
-            int data = 0, loses = 0;
-            split_source(a, box, data, loses);
-            dark = __syncthreads_or(dark);
-            ill = __syncthreads_or(ill);
-            data = __syncthreads_or(data);
-            flag = __syncthreads_or(loses) && dark;
-            flag |= data && ill;
-            // no data: sums of squares of 0 where the integral leaves its rounding
-            if (ill && !data)
-               for (int y = box.y + wave; y <= box.w; y += 4)
-                  for (int x = box.x + lane; x <= box.z; x += 64) out_row(a, y)[x] = __builtin_nanf("");
-         }
+         // (the barrier: every thread's part of the map is stored)
+         if (__syncthreads_or(doubt) && !settled) settle();
          if (threadIdx.x == 0) {
             *a.flags = (unsigned)flag;
             if (flag) *a.any = 1u;
          }
+         if (blank)
+            for (int y = box.y + wave; y <= box.w; y += 4)
+               for (int x = box.x + lane; x <= box.z; x += 64) out_row(a, y)[x] = __builtin_nanf("");
       }
       return;
    }
@@ -1403,8 +1435,10 @@ template <int P> void launch_single_prep(hipStream_t s, const BatchDesc &d);
 template <int P> void launch_pair(hipStream_t s, const SingleLaunch &L);
 template <int P> void launch_pair_prep(hipStream_t s, const BatchDesc &d);
 template <int P> void launch_strip(hipStream_t s, const SingleLaunch &L, int tiles_y, int q_rows);
-// CrossCorr_Norm on split FP16 (mfma_f16x3.hip): the fragments, and the row-pair kernel
-void launch_split_prep(hipStream_t s, const BatchDesc &d, const unsigned *peaks, unsigned *any);
+constexpr int kSplitNT = 4;   // n-tiles of 16 columns per tile
+// CrossCorr_Norm on split FP16 (mfma_f16x3.hip): fragments and the tiles' first flags, and the row-pair
+// kernel (NT = kSplitNT)
+void launch_split_prep(hipStream_t s, const BatchDesc &d, const TileArgs &a, int tiles_x, int tiles);
 void launch_split_pair(hipStream_t s, const SingleLaunch &L);
 template <int P> void launch_batch_prep(hipStream_t s, const BatchDesc *descs, int n);
 // the batch on the row-pair tile (BF16, FP16): its kernel and its fragments

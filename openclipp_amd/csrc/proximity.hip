@@ -399,7 +399,8 @@ __global__ __launch_bounds__(256) void prox_tile_f32(const char *src, int W, int
 
 // CrossCorr_Norm of the tiles that the split-FP16 kernel flagged (SplitFlags): a workgroup walks
 // every gridDim.x-th tile and computes those that a flagged tile of that kernel overlaps.  With
-// no tile flagged it ends at once (4 us at 4096^2).
+// no tile flagged it ends at once (4.6 us at 4096^2).  All flagged, 4096^2/64x64 (a NaN in the source) takes
+// 2140 us in all, 2285 with 768 workgroups instead of up to 2048, 2066 by prox_tile_f32.
 template <int R>
 __global__ __launch_bounds__(256) void prox_tile_f32_flagged(const char *src, int W, int H,
                                                               int sstep,
@@ -1021,8 +1022,7 @@ void launch_proximity_flagged(hipStream_t s, const View &S, const View &T, void 
                               const double *integ, const SplitFlags &f)
 {
    const int W = S.width, H = S.height, tw = T.width, th = T.height;
-   // window sums in the tiles: 8 outputs per thread and one band, as launch_proximity has them
-   const int R = integ ? 16 : 8;
+   const int R = tile_r(kCCNorm, S, T);   // (8 where the tiles have the window sums)
    const int ldsw = lds_pitch(kWaves * R + tw - 1);
    const int vb = min(th, kLdsBudget / (ldsw * 4) - (kTileRows - 1));   // >= 1: split_ncc_ok
    const size_t lds = integ ? (size_t)(kTileRows + vb - 1) * ldsw * 4
@@ -1031,7 +1031,7 @@ void launch_proximity_flagged(hipStream_t s, const View &S, const View &T, void 
    const int tiles = ((W + kWaves * R - 1) / (kWaves * R)) * ((H + kTileRows - 1) / kTileRows);
    KernelTimer kt(s, "prox_flagged");
    auto go = [&](auto kernel) {
-      kernel<<<min(tiles, 512), 256, lds, s>>>(
+      kernel<<<min(tiles, 2048), 256, lds, s>>>(
           static_cast<const char *>(S.ptr), W, H, S.step, static_cast<const float *>(tstage), tpitch,
           tw, th, tsums, integ, static_cast<char *>(dst), dstep, vb, ldsw, f);
    };

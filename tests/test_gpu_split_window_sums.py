@@ -39,6 +39,23 @@ def test_bright_pixel(ocip, monkeypatch, tshape, bright):
     assert np.all(e <= 1), float(np.max(e))
 
 
+# zero windows (7 x 7 outputs) between the samples of split_prep, and the whole of one 127 x 64 tile
+@pytest.mark.parametrize("rows,cols", [((117, 147), (101, 131)), ((100, 300), (40, 160))])
+def test_hole(ocip, monkeypatch, rows, cols):
+    rng = np.random.default_rng(9)
+    src = rng.random((330, 260), dtype=np.float32)
+    src[slice(*rows), slice(*cols)] = 0
+    tpl = rng.random((24, 24), dtype=np.float32)
+    say("split hole", rows, cols)
+    maps = []
+    for on in ("0", "1"):
+        monkeypatch.setenv("OCIP_SPLIT_NCC", on)
+        maps.append(run_op(ocip, "CrossCorr_Norm", src, tpl))
+    assert np.isnan(maps[0]).sum() == (rows[1] - rows[0] - 23) * (cols[1] - cols[0] - 23)
+    np.testing.assert_array_equal(np.isnan(maps[1]), np.isnan(maps[0]))
+    np.testing.assert_allclose(maps[1], maps[0], rtol=0, atol=2 * (20 + tpl.size) * 2.0 ** -23)
+
+
 # the default rule takes the split at 1920x1080 / 24x24
 @pytest.mark.parametrize("what", [np.nan, np.inf, -np.inf, "margins"])
 @pytest.mark.parametrize("shape,forced", [((200, 190), True), ((1080, 1920), False)])
