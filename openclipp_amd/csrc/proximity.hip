@@ -938,12 +938,16 @@ void launch_template_prep(hipStream_t s, const View &t, int channel, int pitch, 
 // up to 1024 taps (F32 CrossCorr 4096^2: 8x8 57 us with 16, 64 with 8; 64x64 1994, 1951; 640x480/48x48
 // SqrDistance 172, 104; 2500x2001/61x64 AbsDistance 856, 695).  The F32 Norm ops, whose window sums
 // come from tiles of 8 but from an integral with 16, take 16 only where the integral is the
-// smaller part (SqrDistance_Norm 4096^2: 8x8 282, 189; 16x16 297, 323; 2048^2/16x16 103, 81).
+// smaller part (SqrDistance_Norm 4096^2: 8x8 282, 189; 16x16 297, 323; 2048^2/16x16 103, 81), and not
+// in images of less than 2048 columns: the tiles' sums round relative to the tile's energy, the
+// integral's to all of the image above and left, and one NaN there reaches the rest of the image
+// (SqrDistance_Norm 2000x4200/16x16 217 us with 16, 192 with 8; 2000x4400/24x24 322 and 323).
 static int tile_r(int op, const View &S, const View &T)
 {
    const long long px = (long long)S.width * S.height, taps = (long long)T.width * T.height;
    const bool norm = S.type == SImage::F32 && (op == kSSDNorm || op == kCCNorm);
-   if (taps >= 1024 || px < (norm ? 8 : 4) * (1 << 20) || (norm && taps < 200)) return 8;
+   if (taps >= 1024 || px < (norm ? 8 : 4) * (1 << 20)) return 8;
+   if (norm && (taps < 200 || S.width < 2048)) return 8;
    return 16;
 }
 
