@@ -811,9 +811,12 @@ void launch_backward_batch(hipStream_t s, int n, const View *S, const View *G1, 
    double *sums = reinterpret_cast<double *>(w + L.sums);
    // window sums straight from the maps (box_f64, its epilogues forming the gradient maps
    // and dS) up to 256 rows (each wavefront reads th + 7 rows for 8; 4 images of 1000x700, with box_f64
-   // and with integrals: 128x128 3416 and 3482 us, 8x256 1017 and 1055, 8x400 1628 and 1562) and
-   // where its LDS row fits, else from integrals
-   const bool use_box = th <= 256 && box_f64_lds(tw) <= (size_t)(160 * 1024 - 256);
+   // and with integrals: 128x128 3416 and 3482 us, 8x256 1017 and 1055) and where its LDS row fits, else
+   // from integrals.  Narrow templates keep them to 543 rows (one column) for their accuracy, which
+   // is relative to the sums' surroundings and not to all of the image above and left: one NaN or far
+   // larger value there spoils no other window (8x400 1611 and 1544 us, 1x543 1205 and 1240).
+   const bool use_box = (th <= 256 || (long long)(th + 31) * (tw + 63) <= 36 * 1024) &&
+                        box_f64_lds(tw) <= (size_t)(160 * 1024 - 256);
    // partial sums per image: one per tile of box_f64<kBoxMaps>, else per block of grad_maps
    const int nscal = use_box && G1 ? box_tiles(W, H) : grid_for((long long)px);
    const int taps = tw * th;
