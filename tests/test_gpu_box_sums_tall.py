@@ -56,4 +56,4 @@ def test_one_bright_weight(ocip, tshape, bright):
 def test_integral_sums_are_exact(ocip):
     s, g = whole_numbers(np.random.default_rng(270), (300, 130))
     say("integral sums")
-    np.testing.assert_array_equal(gradient(ocip, s, g, (270, 100)), exact(s, g, (270, 100)))
+    np.testing.assert_array_equal(gradient(ocip, s, g, (270, 62)), exact(s, g, (270, 62)))
