@@ -55,40 +55,43 @@ IntegralAux aux_layout(void *base, int W, int H)
    return a;
 }
 
-// Four elements read or written at once, at the element's own alignment (see f32x4_u)
-template <class T> struct __attribute__((packed, aligned(alignof(T)))) Vec4 {
-   T v[4];
+// Four elements read or written at once, at the element's own alignment (see f32x4_u).  (A vector
+// type: from a struct's array the selection of `values` was compiled into an indexed copy in scratch
+// memory; SqrIntegral of F64 3001x2003 into F32 49.6 -> 32.5 us.)
+template <class T> struct Vec4 {
+   typedef T type __attribute__((ext_vector_type(4), aligned(alignof(T))));
 };
 
 // The lane's 4 elements of a row as loaded, unconditionally, so that many rows can be in flight in
 // ragged tiles too: rows from y1 on read the row before, columns from W on the last ones inside
 // (VEC: 1-channel rows of at least 4 elements, one vector load at column min(x0, W - 4)).
 template <int TYPE, bool VEC>
-__device__ __forceinline__ Vec4<typename ElemT<TYPE>::type>
+__device__ __forceinline__ typename Vec4<typename ElemT<TYPE>::type>::type
 load_raw(const char *src, int step, int y, int y1, int x0, int W, int nch, int ch)
 {
    typedef typename ElemT<TYPE>::type T;
+   typedef typename Vec4<T>::type V;
    const char *row = src + (size_t)min(y, y1 - 1) * step;
-   if (VEC) return *reinterpret_cast<const Vec4<T> *>(row + (size_t)min(x0, W - 4) * sizeof(T));
-   Vec4<T> q;
+   if (VEC) return *reinterpret_cast<const V *>(row + (size_t)min(x0, W - 4) * sizeof(T));
+   V q;
 #pragma unroll
-   for (int j = 0; j < kVec; ++j) q.v[j] = ld<TYPE>(row, min(x0 + j, W - 1) * nch + ch);
+   for (int j = 0; j < kVec; ++j) q[j] = ld<TYPE>(row, min(x0 + j, W - 1) * nch + ch);
    return q;
 }
 
 // f(s) for the lane's 4 columns of row y from load_raw's elements, 0 outside [0, y1) x [0, W).
 // WHOLE: the tile lies inside the image.
-template <bool WHOLE, bool SQR, bool VEC, class A, class T>
-__device__ __forceinline__ void values(const Vec4<T> &q, int y, int y1, int x0, int W, A (&v)[kVec])
+template <class T, bool WHOLE, bool SQR, bool VEC, class A>
+__device__ __forceinline__ void values(typename Vec4<T>::type q, int y, int y1, int x0, int W, A (&v)[kVec])
 {
    const int d = VEC && !WHOLE ? x0 - min(x0, W - 4) : 0;   // the vector starts d columns early
 #pragma unroll
    for (int j = 0; j < kVec; ++j) {
-      T e = q.v[j];
+      T e = q[j];
       if (!WHOLE) {
 #pragma unroll
          for (int k = j + 1; k < kVec; ++k)
-            if (d == k - j) e = q.v[k];
+            if (d == k - j) e = q[k];
          if (y >= y1 || x0 + j >= W) e = (T)0;
       }
       const A f = (A)e;
@@ -129,14 +132,14 @@ __global__ __launch_bounds__(kThreads) void integral_aggregate(const char *src, 
    unsigned peak = 0;
    by_tile(cb, rb, W, H, [&](auto whole) {
       for (int y = y0; y < y1; y += kAggRows) {
-         Vec4<typename ElemT<TYPE>::type> q[kAggRows];
+         typename Vec4<typename ElemT<TYPE>::type>::type q[kAggRows];
 #pragma unroll
          for (int r = 0; r < kAggRows; ++r)
             q[r] = load_raw<TYPE, VEC>(src, step, y + r, y1, x0, W, nch, ch);
 #pragma unroll
          for (int r = 0; r < kAggRows; ++r) {
             A v[kVec], rs = 0;
-            values<decltype(whole)::value, SQR, VEC>(q[r], y + r, y1, x0, W, v);
+            values<typename ElemT<TYPE>::type, decltype(whole)::value, SQR, VEC>(q[r], y + r, y1, x0, W, v);
 #pragma unroll
             for (int j = 0; j < kVec; ++j) {
                col[j] += v[j];
@@ -263,10 +266,10 @@ template <class T>
 __device__ __forceinline__ void store4(T *o, int x0, int W, const double (&val)[kVec])
 {
    if (x0 + kVec <= W) {
-      Vec4<T> q;
+      typename Vec4<T>::type q;
 #pragma unroll
-      for (int j = 0; j < kVec; ++j) q.v[j] = (T)val[j];
-      *reinterpret_cast<Vec4<T> *>(o + x0) = q;
+      for (int j = 0; j < kVec; ++j) q[j] = (T)val[j];
+      *reinterpret_cast<typename Vec4<T>::type *>(o + x0) = q;
       return;
    }
 #pragma unroll
@@ -320,7 +323,7 @@ __global__ __launch_bounds__(kThreads) void integral_final(const char *src, int 
    double py = 0;
    by_tile(cb, rb, W, H, [&](auto whole) {
       for (int y = y0; y < y1; y += kRowUnroll) {
-         Vec4<typename ElemT<TYPE>::type> q[kRowUnroll];
+         typename Vec4<typename ElemT<TYPE>::type>::type q[kRowUnroll];
          double v[kRowUnroll][kVec];
          double rc[kRowUnroll];
 #pragma unroll
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(kThreads) void integral_final(const char *src, int 
          }
 #pragma unroll
          for (int r = 0; r < kRowUnroll; ++r)
-            values<decltype(whole)::value, SQR, VEC>(q[r], y + r, y1, x0, W, v[r]);
+            values<typename ElemT<TYPE>::type, decltype(whole)::value, SQR, VEC>(q[r], y + r, y1, x0, W, v[r]);
          // the lane's prefixes of the batch's rows, then their wavefront scans together
          double p[kRowUnroll][kVec], inc[kRowUnroll];
 #pragma unroll
