@@ -283,8 +283,11 @@ __device__ __forceinline__ void tile_sqsums(float *lds, int ldsw, int tw, int th
    for (int r = 0; r < R; ++r) ss[r] = sb[(size_t)lane * C4 + colbase + r];
 }
 
-// One output tile (x0, y0).  Starts with a barrier, so consecutive calls may reuse the LDS.
-template <int OP, int TYPE, int R>
+// One output tile (x0, y0).  Starts with a barrier, so consecutive calls may reuse the LDS.  1-channel F32
+// images are staged by stage_tile_f32_v4; with 8 outputs per thread (V4) in an instance of their own,
+// since its loads in flight take twice the registers of the other staging (several channels ran 6 to 20
+// percent slower with both: 34 -> 74 registers).
+template <int OP, int TYPE, int R, bool V4>
 __device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int H, int sstep,
                                          int nch, int ch, const float *__restrict__ tp, int tpitch,
                                          int tw, int th, const double *__restrict__ tsums,
@@ -300,7 +303,7 @@ __device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int
    float acc[R];
 #pragma unroll
    for (int r = 0; r < R; ++r) acc[r] = 0.f;
-   const bool v4 = TYPE == SImage::F32 && nch == 1;
+   const bool v4 = V4 || (TYPE == SImage::F32 && R == 16 && nch == 1);
    // sum t^2 where the host passes none: each workgroup its own from the template (in place), the
    // loads under the staging's
    __shared__ double red[4];
@@ -378,7 +381,7 @@ __device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int
    }
 }
 
-template <int OP, int TYPE, int R>
+template <int OP, int TYPE, int R, bool V4>
 __global__ __launch_bounds__(256) void prox_tile_f32(const char *src, int W, int H, int sstep,
                                                       int nch, int ch,
                                                       const float *__restrict__ tp, int tpitch,
@@ -392,7 +395,7 @@ __global__ __launch_bounds__(256) void prox_tile_f32(const char *src, int W, int
    // one-dimensional grid in XCD-aware tile order
    const int tiles_x = (W + kWaves * R - 1) / (kWaves * R);
    const int tile = xcd_tile(blockIdx.x, gridDim.x);
-   tile_f32<OP, TYPE, R>(lds, src, W, H, sstep, nch, ch, tp, tpitch, tw, th, tsums, integ, dst,
+   tile_f32<OP, TYPE, R, V4>(lds, src, W, H, sstep, nch, ch, tp, tpitch, tw, th, tsums, integ, dst,
                          dstep, vb, ldsw, cx, cy, (tile % tiles_x) * (kWaves * R),
                          (tile / tiles_x) * kTileRows);
 }
@@ -423,7 +426,7 @@ __global__ __launch_bounds__(256) void prox_tile_f32_flagged(const char *src, in
          for (int bx = x0 / f.tile_w; bx <= bx1 / f.tile_w; ++bx)
             any |= f.flags[by * f.tiles_x + bx] != 0u;
       if (any)
-         tile_f32<kCCNorm, SImage::F32, R>(lds, src, W, H, sstep, 1, 0, tp, tpitch, tw, th, tsums,
+         tile_f32<kCCNorm, SImage::F32, R, R == 8>(lds, src, W, H, sstep, 1, 0, tp, tpitch, tw, th, tsums,
                                            integ, dst, dstep, vb, ldsw, tw / 2, th / 2, x0, y0);
    }
 }
@@ -1112,8 +1115,8 @@ static void launch_op(hipStream_t s, const View &S, const View &T, void *dst, in
       lds = tile_sqsum_offset(kTileRows + vb - 1, ldsw) + tile_sqsum_lds(R, th);
    }
 
-#define OCIP_TILE_F32(TT_, R_)                                                                 \
-   prox_tile_f32<OP, TT_, R_><<<grid.x * grid.y, 256, lds, s>>>(                                         \
+#define OCIP_TILE_F32(TT_, R_, V4_)                                                            \
+   prox_tile_f32<OP, TT_, R_, V4_><<<grid.x * grid.y, 256, lds, s>>>(                          \
        src, W, H, S.step, S.channels, ch, static_cast<const float *>(tstage), tpitch, tw, th, \
        tsums, integ, static_cast<char *>(dst), dstep, vb, ldsw, tw / 2, th / 2)
 #define OCIP_TILE_INT(TT_, R_, ACC_)                                                             \
@@ -1134,9 +1137,17 @@ static void launch_op(hipStream_t s, const View &S, const View &T, void *dst, in
    } else {
       KernelTimer kt(s, "prox_tile_f32");
       switch (S.type) {
-      case SImage::F32: if (R == 16) OCIP_TILE_F32(SImage::F32, 16); else OCIP_TILE_F32(SImage::F32, 8); break;
-      case SImage::U32: if (R == 16) OCIP_TILE_F32(SImage::U32, 16); else OCIP_TILE_F32(SImage::U32, 8); break;
-      case SImage::S32: if (R == 16) OCIP_TILE_F32(SImage::S32, 16); else OCIP_TILE_F32(SImage::S32, 8); break;
+      case SImage::F32:
+         if (R == 16) OCIP_TILE_F32(SImage::F32, 16, false);
+         else if (S.channels == 1) OCIP_TILE_F32(SImage::F32, 8, true);
+         else OCIP_TILE_F32(SImage::F32, 8, false);
+         break;
+      case SImage::U32:
+         if (R == 16) OCIP_TILE_F32(SImage::U32, 16, false); else OCIP_TILE_F32(SImage::U32, 8, false);
+         break;
+      case SImage::S32:
+         if (R == 16) OCIP_TILE_F32(SImage::S32, 16, false); else OCIP_TILE_F32(SImage::S32, 8, false);
+         break;
       default: fail(CL_IMAGE_FORMAT_NOT_SUPPORTED, "type");
       }
       launch_check("prox_tile_f32");
