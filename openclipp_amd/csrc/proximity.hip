@@ -937,19 +937,33 @@ void launch_template_prep(hipStream_t s, const View &t, int channel, int pitch, 
 }
 
 // Output columns per lane of the tiled kernels: 8, twice the workgroups and less staged at once, or
-// 16, fewer LDS reads per tap, for images that fill the GPU with such tiles and templates of
-// up to 1024 taps (F32 CrossCorr 4096^2: 8x8 57 us with 16, 64 with 8; 64x64 1994, 1951; 640x480/48x48
-// SqrDistance 172, 104; 2500x2001/61x64 AbsDistance 856, 695).  The F32 Norm ops, whose window sums
-// come from tiles of 8 but from an integral with 16, take 16 only where the integral is the
-// smaller part (SqrDistance_Norm 4096^2: 8x8 282, 189; 16x16 297, 323; 2048^2/16x16 103, 81), and not
-// in images of less than 2048 columns: the tiles' sums round relative to the tile's energy, the
-// integral's to all of the image above and left, and one NaN there reaches the rest of the image
-// (SqrDistance_Norm 2000x4200/16x16 217 us with 16, 192 with 8; 2000x4400/24x24 322 and 323).
+// 16, fewer LDS reads per tap.  8 below 2 Mpx, whose workgroups of 16 do not fill the GPU (640x480/48x48
+// SqrDistance 172 us with 16, 104 with 8), 16 above where it is the faster one (us with 16, with 8):
+//   templates 96 columns wide, whose halo is a third of a tile of 16 and half of one of 8 (CrossCorr F32
+//   x 4 1920x1080/20x100 600, 668), or tall and a few columns wide (CrossCorr 2048x1024/150x4 U8 168, 235,
+//   U16 140, 193, F32 x 4 433, 534);
+//   AbsDistance of 16-bit unsigned images from 200 taps on (1920x1080/64x64 300, 419; 16x16 36, 40);
+//   SqrDistance(_Norm) and AbsDistance with 1024 taps where the tiles of 16 are about two workgroups
+//   per CU, all resident, and those of 8 a third and a fourth (1920x1080/64x64 F32 348, 375; 4000x2000
+//   the other way round: 1180, 1120);
+//   up to 1024 taps from 4 Mpx on (F32 CrossCorr 4096^2: 8x8 57, 64; 64x64 1994, 1951).
+// The F32 Norm ops, whose window sums come from tiles of 8 but from an integral with 16, take 16 up to
+// 1024 taps only where the integral is the smaller part (SqrDistance_Norm 4096^2: 8x8 282, 189; 16x16
+// 297, 323; 2048^2/16x16 103, 81), and not in images of less than 2048 columns: the tiles' sums round
+// relative to the tile's energy, the integral's to all of the image above and left, and one NaN there
+// reaches the rest of the image (SqrDistance_Norm 2000x4200/16x16 217, 192; 2000x4400/24x24 322, 323).
 static int tile_r(int op, const View &S, const View &T)
 {
    const long long px = (long long)S.width * S.height, taps = (long long)T.width * T.height;
    const bool norm = S.type == SImage::F32 && (op == kSSDNorm || op == kCCNorm);
-   if (taps >= 1024 || px < (norm ? 8 : 4) * (1 << 20)) return 8;
+   if (px < 2000000) return 8;
+   if (T.width >= 96 || (T.height >= 100 && T.width < 8)) return 16;   // (no tile holds their window sums)
+   if (op == kSAD && S.type == SImage::U16 && taps >= 200 && T.width >= 8) return 16;
+   if (taps >= 1024) {
+      const long long tiles = (long long)((S.width + 63) / 64) * ((S.height + kTileRows - 1) / kTileRows);
+      return (op == kSSD || op == kSSDNorm || op == kSAD) && tiles > 384 && tiles <= 512 ? 16 : 8;
+   }
+   if (px < (norm ? 8 : 4) * (1 << 20)) return 8;
    if (norm && (taps < 200 || S.width < 2048)) return 8;
    return 16;
 }
