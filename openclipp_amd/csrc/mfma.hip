@@ -907,10 +907,11 @@ using mfma::kSplitNT;
 // of that.
 constexpr double kSplitIll = 0x1p-27;
 
-// Where the path is taken.  For accuracy, templates of 100 taps and 8 columns on: below, prox_tile_f32's
-// few additions are the more exact ones (root mean square error against FP64, noise around 0.5: 3x3
-// 4.8e-8 against 4.5e-8 here, constant images up to 3e-9 against 2e-7; 8x8 1.0e-7 against 5.0e-8,
-// 64x64 7.4e-7 against 1.4e-7; 200 rows of 2, constant 0.1: 7e-7 against 1e-6).  For time, where
+// Where the path is taken.  For accuracy, templates of 100 taps and 5 columns on: below, prox_tile_f32's
+// few additions are the more exact ones on some images (root mean square error against FP64, FP32 sums
+// and split: 3x3 noise around 0.5 4.8e-8, 4.5e-8, but constant images 4e-8, 6e-8; 10x10 noise 1.2e-7,
+// 4.2e-8, constant 4.6e-7, 7.4e-8; 64x64 7.4e-7, 1.4e-7; 40 rows of 5 1.7e-7, 5.7e-8; 200 rows of 2,
+// constant 0.1 7e-7, 1e-6, at the most 8.9e-7, 1.4e-6).  For time, where
 // prox_tile_f32 forms the window sums in its tiles it costs about 2 us + Mpx (9 us + 0.04 us taps) and
 // this path 50 us (seven launches, the integral's three among them) + Mpx (5 us + 0.008 us taps):
 // taken from Mpx (taps + 100) = 1500 (1500^2/24x24 81 against 79 us, 2048^2/20x20 106 against 96,
@@ -931,7 +932,7 @@ bool split_ncc_ok(int op, const View &S, const View &T)
    if (pair_geometry(kc2_for(tw), kSplitNT, th, mfma::kLdsMax, 2).vb < 1) return false;
    if (e && e[0] == '1') return true;
    const long long px = (long long)S.width * S.height, taps = (long long)tw * th;
-   if (taps < 100 || tw < 8) return false;
+   if (taps < 100 || tw < 5) return false;
    return prox_norm_from_tile(op, S, T) ? px * (taps + 100) >= 1500000000LL
                                         : taps >= 200 || px >= 1 << 21;
 }

@@ -30,7 +30,7 @@ def test_products_of_the_low_parts(ocip, monkeypatch, tshape):
     assert worst[1] <= worst[0], worst
 
 
-@pytest.mark.parametrize("tshape", [(8, 8), (25, 8), (16, 16), (33, 64)])
+@pytest.mark.parametrize("tshape", [(8, 8), (25, 8), (20, 5), (2, 50), (16, 16), (33, 64)])
 @pytest.mark.parametrize("kind", ["noise", "signed", "levels"])
 def test_no_further_from_fp64_than_fp32_sums(ocip, monkeypatch, kind, tshape):
     rng = np.random.default_rng(tshape[1])
