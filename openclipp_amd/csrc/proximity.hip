@@ -34,7 +34,8 @@ namespace {
 
 constexpr int kTileRows = 64;      // output rows per workgroup (one per lane)
 constexpr int kWaves = 4;          // waves per workgroup, side by side in x
-constexpr int kLdsBudget = 64 * 1024;
+constexpr int kTileStatic = 32;    // the float tile kernels' static LDS (tile_f32's sums of t^2)
+constexpr int kLdsBudget = 64 * 1024 - kTileStatic;   // dynamic LDS that needs no attribute
 
 // ------------------------------------------------------------------------- template staging
 // The staged template and its sums, by one workgroup (the sums have one fixed order and no
@@ -307,6 +308,7 @@ __device__ __forceinline__ void tile_f32(float *lds, const char *src, int W, int
    // sum t^2 where the host passes none: each workgroup its own from the template (in place), the
    // loads under the staging's
    __shared__ double red[4];
+   static_assert(sizeof red == kTileStatic, "static LDS");
    if ((OP == kSSDNorm || OP == kCCNorm) && !tsums) {
       double t2 = 0.0;
       const int n = tw * th;
