@@ -7,9 +7,10 @@ includes everything the call does: template staging, the FP64 sum-of-squares int
 feeds the denominators, and the correlation itself.
 
 Metric: Gpix*tpix/s = W*H*tw*th / seconds / 1e9.  The headline uses BF16 MFMA products with
-FP32 accumulation; the plain FP32 VALU path is measured beside it on the same inputs, and the
-maximum / mean absolute NCC error of both against an FP64 evaluation at sampled pixels is
-reported.
+FP32 accumulation; the plain FP32 VALU kernel (plain_f32, OCIP_SPLIT_NCC=0) and what F32 precision runs
+by default (default_f32, split-FP16 MFMA products of FP32's accuracy) are measured beside it on the
+same inputs, and the maximum / mean absolute NCC error of each against an FP64 evaluation at sampled
+pixels is reported.
 
 Roofline: the dominant kernel's algorithmic FLOPs (2 per template pixel per output pixel)
 divided by its average duration, timed with HIP events on the library's own stream
@@ -79,8 +80,8 @@ def time_steps(ocip, fn, steps, warmup, kernel):
 
 def batch_bench(ocip, steps):
     """256 templates with sides 8..96 against one 2048x2048 F32 image, CrossCorr_Norm, one
-    ocipCrossCorr_NormBatch call per step (BF16 MFMA, one recorded graph), next to the plain
-    FP32 path on the same batch."""
+    ocipCrossCorr_NormBatch call per step (BF16 MFMA, one recorded graph), next to F32
+    precision on the same batch (split-FP16 MFMA, the FP32 kernel for the smallest templates)."""
     from openclipp_amd import workloads
     src, tpls, _ = workloads.batch_2048()
     H, W = src.shape
@@ -340,9 +341,15 @@ def main():
     ms_cc, kms_cc = time_steps(ocip, lambda: ocip.lib.ocipCrossCorrEx(S.handle, T.handle, D32.handle,
                                                                       PREC_CODE[prec]),
                                max(3, args.steps // 2), 1, DOMINANT[prec])
-    # plain FP32 VALU path on the same inputs
-    ms32, kms32 = time_steps(ocip, step(0), max(3, args.steps // 2), 1, DOMINANT["f32"])
-    value32 = tpix / (ms32 * 1e-3) / 1e9
+    # FP32 on the same inputs: the plain VALU kernel, and the default
+    def f32_figures(kernel):
+        ms32, kms32 = time_steps(ocip, step(0), max(3, args.steps // 2), 1, kernel)
+        return ms32, kms32, D32.read().copy()
+
+    os.environ["OCIP_SPLIT_NCC"] = "0"
+    plain32 = f32_figures("prox_tile_f32")
+    del os.environ["OCIP_SPLIT_NCC"]
+    default32 = f32_figures(DOMINANT["f32"])
 
     # accuracy against FP64 at sampled pixels (and the match location)
     rng = np.random.default_rng(123)
@@ -350,9 +357,16 @@ def main():
     ys = np.concatenate([rng.integers(0, H, 4095), [oy + th // 2]])
     want = ncc_f64_at(src, tpl, xs, ys)
     got = D.read()[ys, xs].astype(np.float64) if prec != "f32" else None
-    got32 = D32.read()[ys, xs].astype(np.float64)
-    err = np.abs(got - want) if got is not None else np.abs(got32 - want)
-    err32 = np.abs(got32 - want)
+    if got is None:
+        got = default32[2][ys, xs].astype(np.float64)
+    err = np.abs(got - want)
+
+    def f32_line(ms32, kms32, m):
+        e = np.abs(m[ys, xs].astype(np.float64) - want)
+        return {"value": round(tpix / (ms32 * 1e-3) / 1e9, 3), "ms_per_step": round(ms32, 4),
+                "kernel_ms": round(kms32, 4) if kms32 else None,
+                "achieved_tflops": round(2.0 * tpix / (kms32 * 1e-3) / 1e12, 2) if kms32 else None,
+                "max_abs_err": float(e.max()), "mean_abs_err": float(e.mean())}
 
     # the other MFMA precisions on the same workload: FP16 and split BF16 (hi + lo, three
     # products: the F32-accuracy figure)
@@ -371,7 +385,7 @@ def main():
 
     flops = 2.0 * tpix
     achieved = flops / (kms * 1e-3) / 1e12 if kms else None
-    peak = PEAK_TFLOPS[prec]
+    peak = PEAK_TFLOPS[prec if prec != "f32" else "f16"]   # (F32 by default: split FP16)
     line = {
         "metric": "NCC/SSD Gpix·tpix/s, 4096² F32, BF16-MFMA vs FP32 HIP, err≤1e-3",
         "value": round(value, 3), "unit": "Gpix·tpix/s", "n_gpus": 1,
@@ -381,7 +395,7 @@ def main():
         "config": {"workload": f"CrossCorr_Norm, {W}x{H} F32 N(0.5,0.2) clamped, {tw}x{th} "
                                f"crop x1.1, precision {prec}",
                    "image": [W, H], "template": [tw, th], "precision": prec},
-        "roofline": {"bound": "mfma" if prec != "f32" else "valu",
+        "roofline": {"bound": "mfma",
                      "kernel": DOMINANT[prec],
                      "achieved": round(achieved, 2) if achieved else None, "peak": peak,
                      "unit": "TFLOP/s",
@@ -389,11 +403,9 @@ def main():
                      "kernel_ms": round(kms, 4) if kms else None,
                      "traffic": measured_traffic() if prec == "bf16" else None},
         "max_abs_err": float(err.max()), "mean_abs_err": float(err.mean()),
-        "plain_f32": {"value": round(value32, 3), "ms_per_step": round(ms32, 4),
-                      "kernel_ms": round(kms32, 4) if kms32 else None,
-                      "achieved_tflops": round(flops / (kms32 * 1e-3) / 1e12, 2) if kms32 else None,
-                      "max_abs_err": float(err32.max()), "mean_abs_err": float(err32.mean())},
-        "speedup_vs_plain_f32": round(value / value32, 3),
+        "plain_f32": f32_line(*plain32),
+        "default_f32": f32_line(*default32),
+        "speedup_vs_plain_f32": round(plain32[0] / ms, 3),
         "other_precisions": others,
         "crosscorr_same_precision": {"value": round(tpix / (ms_cc * 1e-3) / 1e9, 3),
                                      "ms_per_step": round(ms_cc, 4),
