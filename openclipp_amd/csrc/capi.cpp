@@ -162,7 +162,7 @@ void run_proximity(int op, ocipImage hs, ocipImage ht, ocipImage hd, int precisi
    const int esz = kind == 1 ? 8 : 4;
    const int tpitch = tpitch_for(tw);
    c.tmpl.data.ensure((size_t)tpitch * (th > 0 ? th : 1) * esz);
-   c.tmpl.sums.ensure(4 * sizeof(double));
+   c.tmpl.sums.ensure(2 * sizeof(double));
 
    // SqrDistance on 8-bit sources is formed from the cross term and the window sums of
    // squares, which come from the integral as for the Norm ops
@@ -292,7 +292,7 @@ void run_backward_batch(uint n, const ocipImage *hs, ocipImage ht, const ocipIma
    const int W = S[0]->desc.Width, H = S[0]->desc.Height;
    const int tpitch = tpitch_for(tw);
    c.tmpl.data.ensure((size_t)tpitch * th * sizeof(float));
-   c.tmpl.sums.ensure(4 * sizeof(double));
+   c.tmpl.sums.ensure(2 * sizeof(double));
    c.integ_aux.ensure(integral_aux_bytes(W, H));
    launch_template_prep(c.stream, view(T), 0, tpitch, 0, c.tmpl.data.ptr, c.tmpl.sums.as<double>());
    c.work.ensure(backward_work_bytes((int)n, W, H, tw, th, tpitch));

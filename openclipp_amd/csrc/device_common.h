@@ -25,12 +25,14 @@ __device__ __forceinline__ typename ElemT<TYPE>::type ld(const char *row, int i)
    return reinterpret_cast<const typename ElemT<TYPE>::type *>(row)[i];
 }
 
-// Vectors read and written at their elements' alignment: on gfx950 a 16-byte global access needs
-// only 4-byte aligned addresses and a 4- or 8-byte one none, at one more cache line for the
-// wavefront, so image rows need no particular pitch, width or template offset for them.
+// Vectors read and written at their elements' alignment, bytes included: a global access of 4, 8 or
+// 16 bytes takes any address on gfx950 (the compiler makes one instruction of each, as the target's
+// unaligned access mode has it), at one more cache line for the wavefront, so image rows need no
+// particular pitch, width or template offset for them.  LDS accesses are aligned.
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 typedef double f64x2_u __attribute__((ext_vector_type(2), aligned(8)));
-typedef uint32_t u32x2_u __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32_b __attribute__((aligned(1)));
+typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
 
 // Dispatch a runtime SImage type to a template parameter.
 #define OCIP_TYPE_SWITCH(t, TT, ...)                                     \

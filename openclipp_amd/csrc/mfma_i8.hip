@@ -34,13 +34,12 @@ using mfma::kTileRows;
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
 typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 typedef const i32x4 __attribute__((address_space(1))) *gfrag_i8;
 
 constexpr bool is16(int type) { return type == SImage::U16 || type == SImage::S16; }
 // digits of a value; its offset K
-__host__ __device__ constexpr int i8_npa(int type) { return type == SImage::U16 || type == SImage::S16 ? 2 : 1; }
+__host__ __device__ constexpr int i8_digits(int type) { return type == SImage::U16 || type == SImage::S16 ? 2 : 1; }
 
 __host__ __device__ constexpr int i8_key(int type)
 {
@@ -53,8 +52,8 @@ __host__ __device__ constexpr int i8_steps(int th) { return (th + 1) / 2; }
 // colour CrossCorr_Norm 1280x960/24x24 42 -> 33 (twice the wavefronts per SIMD), one 60 and 33.5.
 // 16-bit: one, against two CrossCorr_Norm 2048x1536/31x31 60 -> 51 us (48x48 of 4000x3000 233 -> 248).
 // (kernel times without the window sums)
-__host__ __device__ constexpr int i8_nt(int npa) { return npa == 1 ? 2 : 1; }
-__host__ __device__ constexpr int i8_lcols(int npa, int KC) { return 16 * (i8_nt(npa) - 1) + 32 * KC; }
+__host__ __device__ constexpr int i8_nt(int digits) { return digits == 1 ? 2 : 1; }
+__host__ __device__ constexpr int i8_lcols(int digits, int KC) { return 16 * (i8_nt(digits) - 1) + 32 * KC; }
 
 // pitch of the row sums of window_sums over C columns: an odd multiple of 16 bytes (16-byte stores of
 // 8 consecutive rows on distinct banks)
@@ -66,7 +65,7 @@ template <int TYPE>
 __global__ __launch_bounds__(256) void i8_prep(const char *tpl, int tw, int th, int tstep, int nch,
                                                i32x4 *frag, double *sums)
 {
-   constexpr int K = i8_key(TYPE), NPB = i8_npa(TYPE);
+   constexpr int K = i8_key(TYPE), ND = i8_digits(TYPE);
    __shared__ double red[2][4];
    const int ch = blockIdx.y, KC = i8_chunks(tw), S = i8_steps(th);
    if (blockIdx.x == gridDim.x - 1) {
@@ -104,9 +103,9 @@ __global__ __launch_bounds__(256) void i8_prep(const char *tpl, int tw, int th, 
    const int n = lane & 31, dy = n >> 4, dx = n & 15, kb = 16 * (lane >> 5);
    const int v = 2 * s + 1 - dy;
    const char *row = tpl + (size_t)(v < th ? v : 0) * tstep;
-   uint32_t q[NPB][4];
+   uint32_t q[ND][4];
 #pragma unroll
-   for (int p = 0; p < NPB; ++p)
+   for (int p = 0; p < ND; ++p)
 #pragma unroll
       for (int i = 0; i < 4; ++i) q[p][i] = 0;
 #pragma unroll
@@ -115,15 +114,15 @@ __global__ __launch_bounds__(256) void i8_prep(const char *tpl, int tw, int th, 
       int t = (int)ld<TYPE>(row, min(max(u, 0), tw - 1) * nch + ch);   // (in range: all 16 in flight)
       t = v < th && u >= 0 && u < tw ? t - K : 0;
 #pragma unroll
-      for (int p = 0; p < NPB; ++p) {
+      for (int p = 0; p < ND; ++p) {
          const int digit = (int)(int8_t)t;
          q[p][i / 4] |= ((uint32_t)digit & 0xffu) << (8 * (i % 4));
          t = (t - digit) >> 8;
       }
    }
-   i32x4 *out = frag + ((size_t)(ch * S * KC + f) * NPB) * 64 + lane;
+   i32x4 *out = frag + ((size_t)(ch * S * KC + f) * ND) * 64 + lane;
 #pragma unroll
-   for (int p = 0; p < NPB; ++p)
+   for (int p = 0; p < ND; ++p)
       out[64 * p] = i32x4{(int)q[p][0], (int)q[p][1], (int)q[p][2], (int)q[p][3]};
 }
 
@@ -146,12 +145,12 @@ __device__ __forceinline__ void stage_i8(const I8Args &a, const unsigned char *s
                                          int ldsp, int plane, int row0, int col0, int nrows)
 {
    constexpr bool B16 = is16(TYPE);
-   constexpr int ND = B16 ? 8 : 4;   // dwords of 16 elements
+   constexpr int DW = B16 ? 8 : 4;   // dwords of 16 elements
    constexpr int K = 4;              // items in flight
    constexpr uint32_t kFlip = 0x80808080u;
    const int total = nrows * GROUPS;
    for (int it0 = threadIdx.x; it0 < total; it0 += 256 * K) {
-      uint32_t q[K][ND];
+      uint32_t q[K][DW];
 #pragma unroll
       for (int k = 0; k < K; ++k) {
          const int it = it0 + 256 * k, r = it / GROUPS, g = it - r * GROUPS;
@@ -160,14 +159,14 @@ __device__ __forceinline__ void stage_i8(const I8Args &a, const unsigned char *s
          const unsigned char *row = src + (size_t)(rowin ? sy : 0) * a.sstep;
          if (rowin && sx >= 0 && sx + 16 <= a.W) {
 #pragma unroll
-            for (int j = 0; j < ND / 4; ++j) {
+            for (int j = 0; j < DW / 4; ++j) {
                const u32x4_b b = *reinterpret_cast<const u32x4_b *>(row + sx * (B16 ? 2 : 1) + 16 * j);
 #pragma unroll
                for (int e = 0; e < 4; ++e) q[k][4 * j + e] = b[e];
             }
          } else {
 #pragma unroll
-            for (int j = 0; j < ND; ++j) q[k][j] = 0;
+            for (int j = 0; j < DW; ++j) q[k][j] = 0;
             if (rowin && sx + 16 > 0 && sx < a.W) {
 #pragma unroll
                for (int j = 0; j < 16; ++j) {
@@ -289,8 +288,8 @@ __device__ __forceinline__ i32x16 mma_i8(i32x4 a, i32x4 b, i32x16 c)
 }
 
 // Bound by latency (staging, window sums, products and epilogue, three or four workgroups per CU over one
-// another) above the map's bytes (SqrDistance U8 4096^2/32x32: 61 us, 84 MB = 16 us at the copy rate,
-// 14 us of MFMA issue) and, for large 16-bit templates, the MFMAs.  Whole calls, against BF16
+// another) above the map's bytes (SqrDistance U8 4096^2/32x32: 55 us in all, 84 MB = 16 us at the copy
+// rate, 14 us of MFMA issue) and, for large 16-bit templates, the MFMAs.  Whole calls, against BF16
 // products flushed into int32 every few rows and the window sums from a kernel of their own:
 // SqrDistance U8 4096^2/32x32 98 -> 55 us, CrossCorr 68 -> 53, /64x64 148 -> 108; against the tile
 // kernel's int64 sums and the integral: CrossCorr_Norm U16 2048x1536/31x31 154 -> 46 us.  With the
@@ -302,8 +301,8 @@ __global__ __launch_bounds__(256, is16(TYPE) && KC > 2 ? 1 : 2)
 void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
 {
    constexpr bool B16 = is16(TYPE);
-   constexpr int NPA = i8_npa(TYPE), NPB = NPA, NL = NPA + NPB - 1, K = i8_key(TYPE);
-   constexpr int NT = i8_nt(NPA), C = 16 * NT, NA = NT + 2 * KC - 2;
+   constexpr int ND = i8_digits(TYPE), NL = 2 * ND - 1, K = i8_key(TYPE);   // digits, int32 sums
+   constexpr int NT = i8_nt(ND), C = 16 * NT, NA = NT + 2 * KC - 2;
    typedef typename std::conditional<B16, double, int>::type V;   // a half row's cross term
    constexpr int TP = C + (B16 ? 2 : 4);                          // pitch of the paired tile
    extern __shared__ uint4 lds_v[];
@@ -317,11 +316,11 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
    const int S = i8_steps(a.th), nrows = kTileRows - 2 + 2 * S, plane = nrows * ldsp;
    const unsigned char *src = a.src + ch * a.plane8;
    char *dst = reinterpret_cast<char *>(a.dst + ch);
-   const gfrag_i8 fr = (gfrag_i8)(a.frag + (size_t)ch * S * KC * NPB * 64 + lane);
+   const gfrag_i8 fr = (gfrag_i8)(a.frag + (size_t)ch * S * KC * ND * 64 + lane);
    const double tt = a.sums[2 * ch], t1 = a.sums[2 * ch + 1];
 
    // LDS row r = source row Y0 - cy + r; wave w reads rows 32 w + m + 2 s
-   stage_i8<TYPE, i8_lcols(NPA, KC) / 16>(a, src, lds, ldsp, plane, Y0 - a.th / 2, x0 - a.tw / 2, nrows);
+   stage_i8<TYPE, i8_lcols(ND, KC) / 16>(a, src, lds, ldsp, plane, Y0 - a.th / 2, x0 - a.tw / 2, nrows);
    __syncthreads();
    // the op's window sums, in registers until the epilogue: thread = output column `col`, kRun rows
    // from `row0` on
@@ -330,7 +329,7 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
    typedef typename std::conditional<B16, uint64_t, int>::type Sum;
    Sum ss[kRun];
    int s1[kRun];
-   unsigned char *hs = lds + NPA * plane;
+   unsigned char *hs = lds + ND * plane;
    if (a.op != kCC)
       window_sums<TYPE, C, true>(lds, ldsp, plane, nrows, reinterpret_cast<Sum *>(hs), a.tw, a.th, col, row0, ss);
    if (K && a.op != kSSD) {
@@ -347,25 +346,25 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
          for (int i = 0; i < 16; ++i) acc[l][j][i] = 0;
    // (a wave whose output rows all lie below the image has nothing to multiply)
    if (Y0 - 1 + 32 * wave < a.H) {
-      i32x4 b[2][KC][NPB];
-      auto fetch = [&](int s, i32x4 (&q)[KC][NPB]) {
+      i32x4 b[2][KC][ND];
+      auto fetch = [&](int s, i32x4 (&q)[KC][ND]) {
 #pragma unroll
          for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-            for (int p = 0; p < NPB; ++p) q[kc][p] = fr[(size_t)((s * KC + kc) * NPB + p) * 64];
+            for (int p = 0; p < ND; ++p) q[kc][p] = fr[(size_t)((s * KC + kc) * ND + p) * 64];
       };
       const unsigned char *arow = lds + (size_t)(wave * 32 + (lane & 31)) * ldsp + 16 * (lane >> 5);
-      auto step = [&](int s, const i32x4 (&q)[KC][NPB]) {
-         i32x4 x[NPA][NA];
+      auto step = [&](int s, const i32x4 (&q)[KC][ND]) {
+         i32x4 x[ND][NA];
 #pragma unroll
          for (int c = 0; c < NA; ++c)
 #pragma unroll
-            for (int p = 0; p < NPA; ++p)
+            for (int p = 0; p < ND; ++p)
                x[p][c] = *reinterpret_cast<const i32x4 *>(arow + p * plane + (size_t)(2 * s) * ldsp + 16 * c);
 #pragma unroll
          for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-            for (int k = 0; k < NPA * NPB; ++k) {
+            for (int k = 0; k < ND * ND; ++k) {
                // digit of s, digit of t: (l, l), (h, l), (h, h), (l, h)
                constexpr int kA[4] = {0, 1, 1, 0}, kB[4] = {0, 0, 1, 1};
 #pragma unroll
@@ -438,7 +437,7 @@ void crosscorr_i8(I8Args a, int ldsp, int tiles_x, int tiles)
 template <int TYPE>
 void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
 {
-   constexpr int NPA = i8_npa(TYPE), NT = i8_nt(NPA);
+   constexpr int ND = i8_digits(TYPE), NT = i8_nt(ND);
    constexpr bool B16 = is16(TYPE);
    a.src = static_cast<const unsigned char *>(S.ptr);
    a.W = S.width; a.H = S.height; a.sstep = S.step;
@@ -453,12 +452,12 @@ void launch_i8(hipStream_t s, I8Args a, const View &S, const View &T)
       launch_check("i8_prep");
    }
    // an odd multiple of 16 bytes: the A reads of 8 consecutive rows on distinct banks
-   int ldsp = i8_lcols(NPA, KC);
+   int ldsp = i8_lcols(ND, KC);
    if (ldsp % 32 == 0) ldsp += 16;
    const int nrows = kTileRows - 2 + 2 * steps;
    const int sum = B16 && a.op != kCC ? 8 : 4;
    const size_t sums = (size_t)(nrows + 1) * hsum_pitch(16 * NT, sum) * sum;
-   const size_t staging = (size_t)NPA * nrows * ldsp + (a.op == kCC && i8_key(TYPE) == 0 ? 0 : sums);
+   const size_t staging = (size_t)ND * nrows * ldsp + (a.op == kCC && i8_key(TYPE) == 0 ? 0 : sums);
    const size_t pairing = (size_t)(kTileRows + 1) * (16 * NT + (B16 ? 2 : 4)) * (B16 ? 8 : 4);
    const size_t lds = std::max(staging, pairing);
    const int tiles_x = (a.W + 16 * NT - 1) / (16 * NT), tiles_y = (a.H + kPairRows - 1) / kPairRows;
@@ -498,9 +497,8 @@ __global__ __launch_bounds__(256) void split_planes8(const unsigned char *__rest
    const unsigned char *row = src + (size_t)y * sstep;
    uint32_t q[NCH];   // the 4 NCH bytes of the thread's pixels
    if (x + 4 <= W) {
-      typedef uint32_t u32_u __attribute__((aligned(1)));
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) q[i] = reinterpret_cast<const u32_u *>(row + x * NCH)[i];
+      for (int i = 0; i < NCH; ++i) q[i] = reinterpret_cast<const u32_b *>(row + x * NCH)[i];
    } else {
 #pragma unroll
       for (int i = 0; i < NCH; ++i) q[i] = 0;

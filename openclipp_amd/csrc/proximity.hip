@@ -737,7 +737,6 @@ __global__ __launch_bounds__(256) void prox_sad8(const unsigned char *src, int W
    extern __shared__ uint32_t ldsp[];
    constexpr int R = kSad8R;
    constexpr uint32_t kKey = TYPE == SImage::S8 ? 0x80808080u : 0u;
-   typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ch = blockIdx.y;
    const int tiles_x = (W + kWaves * R - 1) / (kWaves * R);
    const int tile = xcd_tile(blockIdx.x, gridDim.x);
