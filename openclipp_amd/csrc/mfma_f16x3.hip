@@ -37,9 +37,9 @@ __global__ __launch_bounds__(256) void split_prep(BatchDesc d, TileArgs a, int f
    if (lane == 0) a.flags[t] = (unsigned)doubt;
 }
 
-template <int KC> void pair(hipStream_t s, const SingleLaunch &L)
+template <int KC, bool LOLO> void pair(hipStream_t s, const SingleLaunch &L)
 {
-   auto k = crosscorr_mfma_pair<kF16x3, KC, kSplitNT, kModeNCC>;
+   auto k = crosscorr_mfma_pair<kF16x3, KC, kSplitNT, kModeNCC, LOLO>;
    // set for every call: the attribute belongs to the device that is current
    hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax),
@@ -50,18 +50,30 @@ template <int KC> void pair(hipStream_t s, const SingleLaunch &L)
 
 }  // namespace
 
-void launch_split_pair(hipStream_t s, const SingleLaunch &L)
+template <bool LOLO> static void pairs(hipStream_t s, const SingleLaunch &L)
 {
    switch (L.KC) {
-   case 1: pair<1>(s, L); break;
-   case 2: pair<2>(s, L); break;
-   case 3: pair<3>(s, L); break;
-   case 4: pair<4>(s, L); break;
-   case 5: pair<5>(s, L); break;
-   case 6: pair<6>(s, L); break;
-   case 7: pair<7>(s, L); break;
+   case 1: pair<1, LOLO>(s, L); break;
+   case 2: pair<2, LOLO>(s, L); break;
+   case 3: pair<3, LOLO>(s, L); break;
+   case 4: pair<4, LOLO>(s, L); break;
+   case 5: pair<5, LOLO>(s, L); break;
+   case 6: pair<6, LOLO>(s, L); break;
+   case 7: pair<7, LOLO>(s, L); break;
    default: fail(CL_INVALID_VALUE, "template width");
    }
+}
+
+// lo lo (pair_mfma_f16x3) is taken below kLoLoTaps taps.  It matters where all of a window's lo are alike:
+// constant images of 1 + 2^-11 are off by 7e-8 with it (8x8 to 24x24) and 2.4e-7 without, FP32 sums by
+// 1.2e-7 to 2e-7.  With more taps the roundings of FP32 sums have long outgrown its 2^-22 (constant images
+// at 32x32, root mean square 5.4e-6 against 3.2e-7; noise 3.7e-7 against 8.4e-8), and a fourth product
+// costs 19 percent of 4096^2/64x64 (556 -> 663 us) against 4 of 4000x2000/31x31 (157 -> 164).
+constexpr int kLoLoTaps = 1024;
+
+void launch_split_pair(hipStream_t s, const SingleLaunch &L)
+{
+   if (L.a.tw * L.a.th < kLoLoTaps) pairs<true>(s, L); else pairs<false>(s, L);
    launch_check("crosscorr_mfma_split");
 }
 

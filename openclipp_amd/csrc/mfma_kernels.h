@@ -45,9 +45,9 @@ constexpr int kLdsMax = 160 * 1024 - 256;
 // two so that the image's largest magnitude lies in (2^14, 2^15], the template likewise.  hi takes 11
 // significant bits and lo the next 11 and a sign (down to 2^-24, FP16 subnormals, which the matrix
 // cores keep): a value within 2^15 of the largest is held to 2^-23 of itself, three in four of them
-// exactly, and every value to 2^-40 of the largest.  All four products are taken, hi hi in one
-// accumulator and the others, 2^11 times smaller, in a second: added to the first they would lose
-// what lies below its grid (lo lo all of it).
+// exactly, and every value to 2^-40 of the largest.  hi hi goes into one accumulator, hi lo, lo hi and
+// (templates of few taps: kLoLoTaps) lo lo, 2^11 and 2^22 times smaller, into a second: added to the
+// first they would lose what lies below its grid (lo lo all of it).
 enum { kBF16 = 1, kF16 = 2, kBF16x3 = 3, kF16x3 = 4 };
 __host__ __device__ constexpr int planes_of(int P) { return P == kBF16x3 || P == kF16x3 ? 2 : 1; }
 // kModeCC: the CrossCorr map (the single-template call; CrossCorr_Norm scales it in place
@@ -645,12 +645,11 @@ __device__ __forceinline__ void pair_mfma(f32x16 (&acc)[NT], const unsigned shor
    }
 }
 
-// The same for split FP16: hi hi into acc, the products with a lo, lo lo among them, into low; chunk by
-// chunk of A, whose fragments then take 8 registers instead of 8 NA (two accumulators and the
-// prefetched B fragments fill the 256 of two waves per SIMD).  Without lo lo and in one accumulator
-// 4096^2/64x64 took 537 us instead of 649, at twice to three times the error on ordinary data and
-// 2^-22 on constant images of 1 + 2^-11, where the FP32 sums are off by 2^-23 to 2^-22.
-template <int KC, int NT>
+// The same for split FP16: hi hi into acc, the products with a lo into low; chunk by chunk of A, whose
+// fragments then take 8 registers instead of 8 NA (two accumulators and the prefetched B fragments fill
+// the 256 of two waves per SIMD).  4096^2/64x64, us and error against FP64: one accumulator 537, 3.1e-7;
+// two 556, 1.8e-7; with lo lo 663, 1.8e-7 (FP32 sums 2070, 9.4e-7).
+template <int KC, int NT, bool LOLO>
 __device__ __forceinline__ void pair_mfma_f16x3(f32x16 (&acc)[NT], f32x16 (&low)[NT],
                                                 const unsigned short *ab, size_t plane,
                                                 const u16x8 (&b)[KC], const u16x8 (&b1)[KC])
@@ -660,7 +659,7 @@ __device__ __forceinline__ void pair_mfma_f16x3(f32x16 (&acc)[NT], f32x16 (&low)
       const u16x8 a0 = *reinterpret_cast<const u16x8 *>(ab + 16 * c);
       const u16x8 a1 = *reinterpret_cast<const u16x8 *>(ab + plane + 16 * c);
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < (LOLO ? 4 : 3); ++k)
 #pragma unroll
          for (int j = 0; j < NT; ++j) {
             const int kc = c - j;
@@ -716,7 +715,7 @@ __device__ __forceinline__ void split_source(const TileArgs &a, int4 box, int &d
 // CrossCorr map; kModeNCC / kModeSSDN store CrossCorr_Norm / SqrDistance_Norm with the window
 // sums of s^2 from the FP64 integral a.integ (the batch kernel's epilogue, the same
 // expressions as mfma_tile).
-template <int P, int KC, int NT, int MODE>
+template <int P, int KC, int NT, int MODE, bool LOLO = false>
 __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, unsigned short *lds,
                                           int ldsp)
 {
@@ -844,7 +843,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
    // Settled ahead of the products where split_prep found one output in 128 in doubt: a tile to be
    // computed again then costs no products, nor does one without data.  4096^2/64x64 with one pixel
    // 2^18 times the others 3020 -> 2313 us (2066 with FP32 sums alone), with 43 percent zeros in margins
-   // 715 -> 585; images without either 655 -> 663.
+   // 715 -> 585; images without either 655 -> 663 (all three with lo lo; 2310, 498 and 556 without).
    bool settled = false, empty = false;
    if constexpr (P == kF16x3) {
       sr = split_range(a.peaks, a.tw * a.th);
@@ -869,7 +868,7 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
          if constexpr (P == kF16x3) low[j][i] = 0.f;
       }
    auto step = [&](const unsigned short *ab, const u16x8 (&b)[KC], const u16x8 (&b1)[KC]) {
-      if constexpr (P == kF16x3) pair_mfma_f16x3<KC, NT>(acc, low, ab, plane, b, b1);
+      if constexpr (P == kF16x3) pair_mfma_f16x3<KC, NT, LOLO>(acc, low, ab, plane, b, b1);
       else pair_mfma<P, KC, NT>(acc, ab, plane, b, b1);
    };
    for (int ub = 0; ub < (empty ? 0 : a.nub); ++ub) {
@@ -1029,7 +1028,7 @@ __host__ __device__ constexpr int pair_waves(int P, int KC, int NT, int MODE)
 // One 127 x 16 NT tile per workgroup, XCD-aware order (the single-template call): tiles_x *
 // tiles_y workgroups per image, images z.n of them one after the other (or the one image of
 // `a`).
-template <int P, int KC, int NT, int MODE>
+template <int P, int KC, int NT, int MODE, bool LOLO = false>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(pair_waves(P, KC, NT, MODE), pair_waves(P, KC, NT, MODE))))
 void crosscorr_mfma_pair(TileArgs a, int ldsp, int tiles_x, int tiles, ZImages z)
@@ -1051,8 +1050,8 @@ void crosscorr_mfma_pair(TileArgs a, int ldsp, int tiles_x, int tiles, ZImages z
       }
       a.scale = pow2f(sr.ks);
    }
-   pair_tile<P, KC, NT, MODE>(a, t % tiles_x, t / tiles_x, reinterpret_cast<unsigned short *>(lds_v),
-                              ldsp);
+   pair_tile<P, KC, NT, MODE, LOLO>(a, t % tiles_x, t / tiles_x, reinterpret_cast<unsigned short *>(lds_v),
+                                    ldsp);
 }
 
 // Persistent batch kernel on the row-pair tile (the batch of BF16 / FP16 templates).  The
