@@ -1018,11 +1018,14 @@ __device__ __forceinline__ void pair_tile(const TileArgs &a, int bx, int by, uns
 }
 
 // Waves per SIMD the row-pair kernel's registers are sized for: 3 for the narrow one-plane
-// CrossCorr tile, 1 for the widest split-BF16 tiles (whose two staged planes leave LDS for one
-// workgroup per CU at these template widths, and whose three fragment sets would spill at 2).
+// CrossCorr tile, 1 for the widest split tiles (whose two staged planes leave LDS for one
+// workgroup per CU at these template widths, and whose fragments would spill at 2: split FP16
+// 2048^2/96x96 378 -> 337 us; with 6 chunks, 36 bytes spilled at 2, 256 -> 263).
 __host__ __device__ constexpr int pair_waves(int P, int KC, int NT, int MODE)
 {
-   return NT <= 4 && MODE == kModeCC && planes_of(P) == 1 ? 3 : P == kBF16x3 && NT == 6 && KC >= 7 ? 1 : 2;
+   return NT <= 4 && MODE == kModeCC && planes_of(P) == 1        ? 3
+          : KC >= 7 && (P == kF16x3 || (P == kBF16x3 && NT == 6)) ? 1
+                                                                  : 2;
 }
 
 // One 127 x 16 NT tile per workgroup, XCD-aware order (the single-template call): tiles_x *
