@@ -172,15 +172,21 @@ ocipError ocip_API ocipCrossCorrFFT_Norm(ocipProgram Program, ocipImage Source,
 /* Arithmetic used by the cross-correlation sums. */
 enum ocipPrecision
 {
-   ocipPrecisionF32    = 0,  /* FP32 VALU, same as ocipCrossCorr / ocipCrossCorr_Norm        */
+   ocipPrecisionF32    = 0,  /* same as ocipCrossCorr / ocipCrossCorr_Norm: FP32 FMAs, and for
+                              * CrossCorr_Norm of larger F32 images split hi+lo FP16 MFMA
+                              * products, FP32 accumulation (operands held to 2^-23; the maps'
+                              * error is below that of FP32 sums, but for constant images of a
+                              * few values; what the split cannot hold is computed in FP32;
+                              * OCIP_SPLIT_NCC=0: always FP32)                                */
    ocipPrecisionBF16   = 1,  /* BF16 MFMA products, FP32 accumulation                         */
    ocipPrecisionF16    = 2,  /* FP16 MFMA products, FP32 accumulation                         */
    ocipPrecisionBF16x3 = 3   /* split hi+lo BF16, three MFMA products, FP32 accumulation      */
 };
 
 /* ocipCrossCorr / ocipCrossCorr_Norm with an explicit arithmetic (F32 1-channel sources for
- * the MFMA precisions).  Norm denominators always come from the FP64 sum-of-squares
- * integral of Source and the FP64 sum of squares of Template. */
+ * the MFMA precisions).  Norm denominators are FP64 sums of squares of Source's windows (formed
+ * from its tiles or from its integral; the MFMA precisions round a window's column sums to FP32)
+ * and the FP64 sum of squares of Template. */
 ocipError ocip_API ocipCrossCorrEx(ocipImage Source, ocipImage Template, ocipImage Dest,
                                    int Precision);
 ocipError ocip_API ocipCrossCorr_NormEx(ocipImage Source, ocipImage Template, ocipImage Dest,
@@ -208,8 +214,8 @@ ocipError ocip_API ocipSqrDistance_NormBatch(ocipImage Source, const ocipImage *
 
 /* Gradients of L = sum(GradDest * op(Source, Template)) for F32 1-channel images.
  * GradSource is Source-sized, GradTemplate is Template-sized (both F32, overwritten).
- * Either gradient output may be NULL to skip it.  The Norm statistics are recomputed from
- * the FP64 integral of squares, not stored by the forward call. */
+ * Either gradient output may be NULL to skip it.  The Norm statistics are recomputed as FP64
+ * sums of squares, not stored by the forward call. */
 ocipError ocip_API ocipCrossCorr_NormBackward(ocipImage Source, ocipImage Template,
                                               ocipImage GradDest, ocipImage GradSource,
                                               ocipImage GradTemplate);

@@ -22,8 +22,9 @@
 //                  bound allows, int64 otherwise), rounded once to float.
 //   prox_direct    one output per thread, reference order, any type (F64 sources and
 //                  templates too wide for the LDS tile).
-// Norm denominators come from the FP64 sum-of-squares integral of the source (exclusive,
-// (W+1) x (H+1) layout) by four corners and the FP64 sum of squares of the template.
+// Norm denominators: FP64 window sums of squares, of F32 sources from the staged tile where it holds them
+// (prox_norm_from_tile), else from the sum-of-squares integral of the source (exclusive, (W+1) x (H+1)
+// layout) by four corners; and the FP64 sum of squares of the template.
 #include <algorithm>
 
 #include "device_common.h"
